@@ -458,7 +458,7 @@ void launch_adj_stage(int stage, const AdjArgs<R>& a, hipStream_t s) {
 
 template <typename R>
 void launch_adj_combine(const AdjCombineArgs<R>& a, hipStream_t s) {
-    hipLaunchKernelGGL((k_adj_combine<R>), dim3(2048), dim3(256), 0, s, a);
+    hipLaunchKernelGGL((k_adj_combine<R>), dim3(mesh_grid((int64_t)a.nx * a.ny * a.nzp)), dim3(256), 0, s, a);
 }
 
 template <typename R>

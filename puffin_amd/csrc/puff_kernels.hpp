@@ -105,6 +105,13 @@ struct CombineArgs {
     int clear_from;        // d[k] with k >= clear_from are cleared after the update
 };
 
+// Workgroups of 256 threads of a grid-stride kernel over (a part of) a mesh
+// of nmesh nodes: no more than the mesh fills, at most eight per CU.
+inline unsigned mesh_grid(int64_t nmesh) {
+    const int64_t b = (nmesh + 255) / 256;
+    return (unsigned)(b < 1 ? 1 : (b > 2048 ? 2048 : b));
+}
+
 template <typename R>
 void launch_stage(int stage, const StageArgs<R>& a, hipStream_t s);
 void launch_step_begin(int* flags, Box* box, hipStream_t s);

@@ -435,7 +435,8 @@ void launch_det_scale(const PartPtrs<double>& y, const double* chi, int64_t n, c
 
 void launch_det_convert(const DetState& d, cplx<double>* dA, const Box* box, int nx, int ny, int nzp,
                         int periodic, int one_d, hipStream_t s) {
-    hipLaunchKernelGGL(k_det_convert, dim3(2048), dim3(256), 0, s, d, dA, box, nx, ny, nzp, periodic, one_d);
+    hipLaunchKernelGGL(k_det_convert, dim3(mesh_grid((int64_t)nx * ny * nzp)), dim3(256), 0, s, d, dA, box, nx, ny,
+                       nzp, periodic, one_d);
 }
 
 void launch_step_begin(int* flags, Box* box, hipStream_t s) {
@@ -444,7 +445,7 @@ void launch_step_begin(int* flags, Box* box, hipStream_t s) {
 
 template <typename R>
 void launch_combine(const CombineArgs<R>& a, hipStream_t s) {
-    hipLaunchKernelGGL((k_field_combine<R>), dim3(2048), dim3(256), 0, s, a);
+    hipLaunchKernelGGL((k_field_combine<R>), dim3(mesh_grid((int64_t)a.nx * a.ny * a.nzp)), dim3(256), 0, s, a);
 }
 
 void launch_wrap(double* z2, int64_t n, double lenz2, hipStream_t s) {

@@ -204,18 +204,19 @@ __device__ __forceinline__ void box_coords(const BoxDiv& d, int q, int& lx, int&
     ly = r - lz * d.ty;
 }
 
-// Union of the spread box copies.
+// Union of the spread box copies, one copy per lane and six wavefront
+// reductions.  Every lane of the wavefront must be active.  (Each thread
+// reading all 64 copies in turn is a chain of 384 loads: it held the field
+// combination at 24 us on any mesh, however small.)
 __device__ __forceinline__ Box merged_box(const Box* box) {
+    static_assert(BOX_COPIES == 64, "one copy per lane");
+    const Box mine = box[threadIdx.x & 63];
     Box b;
+#pragma unroll
     for (int d = 0; d < 3; ++d) {
-        b.lo[d] = 0x7fffffff;
-        b.hi[d] = -1;
+        b.lo[d] = wave_min(mine.lo[d]);
+        b.hi[d] = wave_max(mine.hi[d]);
     }
-    for (int k = 0; k < BOX_COPIES; ++k)
-        for (int d = 0; d < 3; ++d) {
-            b.lo[d] = min(b.lo[d], box[k].lo[d]);
-            b.hi[d] = max(b.hi[d], box[k].hi[d]);
-        }
     return b;
 }
 
