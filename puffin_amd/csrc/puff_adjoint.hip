@@ -75,15 +75,16 @@ __global__ __launch_bounds__(ADJ_THREADS) void k_adj_stage(AdjArgs<R> a) {
     if (in) {
         const R x0 = a.y0.x[i], y0 = a.y0.y[i], pr0 = a.y0.pr[i], pi0 = a.y0.pi[i];
         const double z20 = a.y0.z2[i], g0 = a.y0.g[i];
-        R kx = 0, ky = 0, kpr = 0, kpi = 0;
-        double kz2 = 0.0, kg = 0.0;
+        R kr = 0, ki = 0, kg = 0, qr = 0, qi = 0, qg = 0;
         if (STAGE > 1) {
-            kx = a.kin.x[i];
-            ky = a.kin.y[i];
-            kz2 = a.kin.z2[i];
-            kpr = a.kin.pr[i];
-            kpi = a.kin.pi[i];
+            kr = a.kin.pr[i];
+            ki = a.kin.pi[i];
             kg = a.kin.g[i];
+        }
+        if (STAGE > 2) {
+            qr = a.kprev.pr[i];
+            qi = a.kprev.pi[i];
+            qg = a.kprev.g[i];
         }
         chi = a.chi[i];
         const bool ev = ph.electrons_evolve;
@@ -108,13 +109,9 @@ __global__ __launch_bounds__(ADJ_THREADS) void k_adj_stage(AdjArgs<R> a) {
         if (STAGE == 1) {
             x = x0; y = y0; z2 = z20; pr = pr0; pi = pi0; g = g0;
         } else {
-            const R c = (R)a.cin;
-            x = fma(c, kx, x0);
-            y = fma(c, ky, y0);
-            z2 = fma(a.cin, kz2, z20);
-            pr = fma(c, kpr, pr0);
-            pi = fma(c, kpi, pi0);
-            g = fma(a.cin, kg, g0);
+            const Trial<R> t = trial_state<R, STAGE>(ph, x0, y0, z20, pr0, pi0, g0, kr, ki, kg, qr, qi, qg, a.cin,
+                                                     a.cprev);
+            x = t.x; y = t.y; z2 = t.z2; pr = t.pr; pi = t.pi; g = t.g;
         }
         if (ev) {
             ax = a.ws * Lx;

@@ -34,7 +34,7 @@ struct Particles {
     KPtrs<R> k[3];
     R* chi = nullptr;
     // the sort's spare z2 and Gamma arrays in the mixed form (its spare x, y,
-    // p_r, p_i are k[0]'s; the FP64 form's k[0] serves whole)
+    // p_r, p_i are k[0]'s and k[1]'s, as are the FP64 form's z2 and Gamma)
     double* z2_spare = nullptr;
     double* g_spare = nullptr;
 };
@@ -514,9 +514,6 @@ static int alloc_particles(Ctx* c) {
         return PUFF_OK;
     };
     auto setk = [&](KPtrs<R>& q) -> int {
-        PUFF_TRY(dalloc(c, (void**)&q.x, sizeof(R) * c->n));
-        PUFF_TRY(dalloc(c, (void**)&q.y, sizeof(R) * c->n));
-        PUFF_TRY(dalloc(c, (void**)&q.z2, sizeof(R) * c->n));
         PUFF_TRY(dalloc(c, (void**)&q.pr, sizeof(R) * c->n));
         PUFF_TRY(dalloc(c, (void**)&q.pi, sizeof(R) * c->n));
         PUFF_TRY(dalloc(c, (void**)&q.g, sizeof(R) * c->n));
@@ -705,7 +702,7 @@ static void release(Ctx* c) {
 // ---- step capture ---------------------------------------------------------------
 // A step's start state and stage data kept in caller-owned device memory for
 // the adjoint: 256-byte header, x y z2 pr pi Gamma, chi, orig, A, then k1, k2,
-// k3 (six arrays each) and dA1, dA2, dA3, each section 256-byte aligned.
+// k3 (p_r, p_i, Gamma) and dA1, dA2, dA3, each section 256-byte aligned.
 
 template <typename R>
 struct CaptureView {
@@ -738,9 +735,6 @@ static size_t capture_view(const Ctx* c, char* base, CaptureView<R>* v) {
         q.g = reinterpret_cast<double*>(take(sizeof(double) * n));
     };
     auto take_k = [&](KPtrs<R>& q) {
-        q.x = reinterpret_cast<R*>(take(sizeof(R) * n));
-        q.y = reinterpret_cast<R*>(take(sizeof(R) * n));
-        q.z2 = reinterpret_cast<R*>(take(sizeof(R) * n));
         q.pr = reinterpret_cast<R*>(take(sizeof(R) * n));
         q.pi = reinterpret_cast<R*>(take(sizeof(R) * n));
         q.g = reinterpret_cast<R*>(take(sizeof(R) * n));
@@ -765,12 +759,14 @@ static void sort_particles(Ctx* c) {
     a.ncell = c->ncell;
     a.mesh = c->mesh;
     a.y = &P.y;
-    // spare state arrays: k[0]'s, with z2 and Gamma of the state's type
+    // spare state arrays: those of k[0] and k[1], with z2 and Gamma of the
+    // state's type
     KPtrs<R>& k0 = P.k[0];
-    PartPtrs<R> spare{k0.x, k0.y, nullptr, k0.pr, k0.pi, nullptr};
+    KPtrs<R>& k1 = P.k[1];
+    PartPtrs<R> spare{k0.pr, k0.pi, nullptr, k1.pr, k1.pi, nullptr};
     if constexpr (sizeof(R) == sizeof(double)) {
-        spare.z2 = reinterpret_cast<double*>(k0.z2);
-        spare.g = reinterpret_cast<double*>(k0.g);
+        spare.z2 = reinterpret_cast<double*>(k0.g);
+        spare.g = reinterpret_cast<double*>(k1.g);
     } else {
         spare.z2 = P.z2_spare;
         spare.g = P.g_spare;
@@ -788,13 +784,13 @@ static void sort_particles(Ctx* c) {
     a.tile_sums = c->sort_tiles;
     launch_sort<R>(a, c->stream);
     // the sort swapped the state and spare pointers: the spares go back
-    k0.x = spare.x;
-    k0.y = spare.y;
-    k0.pr = spare.pr;
-    k0.pi = spare.pi;
+    k0.pr = spare.x;
+    k0.pi = spare.y;
+    k1.pr = spare.pr;
+    k1.pi = spare.pi;
     if constexpr (sizeof(R) == sizeof(double)) {
-        k0.z2 = reinterpret_cast<R*>(spare.z2);
-        k0.g = reinterpret_cast<R*>(spare.g);
+        k0.g = reinterpret_cast<R*>(spare.z2);
+        k1.g = reinterpret_cast<R*>(spare.g);
     } else {
         P.z2_spare = spare.z2;
         P.g_spare = spare.g;
@@ -871,12 +867,11 @@ static int rk4par(Ctx* c, double sz, double h, char* cap = nullptr, void* cap_hd
         a.s = sc[st - 1];
         a.cin = cin[st - 1];
         a.cnext = cnext[st - 1];
+        a.cprev = (st > 2) ? cin[st - 2] : 0.0;
         a.kin = (st > 1) ? K[st - 2] : KPtrs<R>{};
+        a.kprev = (st > 2) ? K[st - 3] : KPtrs<R>{};
+        a.k1 = K[0];
         a.kout = (st < 4) ? K[st - 1] : KPtrs<R>{};
-        if (st == 4) {
-            a.k1 = K[0];
-            a.k2 = K[1];
-        }
         a.dAin = (st > 1) ? D[st - 2] : nullptr;
         a.dAout = D[st - 1];
         if (cap && st == 1) {
@@ -1338,7 +1333,9 @@ static int replay_stages(Ctx* c, const StageScalars* sc, const double* cin, cons
         a.s = sc[st - 1];
         a.cin = cin[st - 1];
         a.cnext = cnext[st - 1];
+        a.cprev = (st > 2) ? cin[st - 2] : 0.0;
         a.kin = (st > 1) ? P.k[st - 2] : KPtrs<R>{};
+        a.kprev = (st > 2) ? P.k[st - 3] : KPtrs<R>{};
         a.kout = P.k[st - 1];
         a.dAin = (st > 1) ? reinterpret_cast<const cplx<R>*>(c->dA[st - 2]) : nullptr;
         a.dAout = reinterpret_cast<cplx<R>*>(c->dA[st - 1]);
@@ -1441,7 +1438,9 @@ static int rk4par_adjoint(Ctx* c, double sz, double h, double* dn2col, int32_t* 
     for (int st = 4; st >= 1; --st) {
         b.s = sc[st - 1];
         b.cin = cin[st - 1];
+        b.cprev = (st > 2) ? cin[st - 2] : 0.0;
         b.kin = (st > 1) ? K[st - 2] : KPtrs<R>{};
+        b.kprev = (st > 2) ? K[st - 3] : KPtrs<R>{};
         b.dAin = (st > 1) ? D[st - 2] : nullptr;
         b.ws = wts[st - 1] * h6;
         b.cnext = (st < 4) ? cin[st] : 0.0;

@@ -26,24 +26,31 @@ struct Physics {
     int coupling, electrons_evolve, field_evolve;
 };
 
-// Six particle coordinates: x, y, p_r, p_i in R; z2 and Gamma in Z (FP64
-// for the state).
-template <typename R, typename Z = double>
+// Six particle coordinates: x, y, p_r, p_i in R; z2 and Gamma in FP64.
+template <typename R>
 struct PartPtrs {
     R* x;
     R* y;
-    Z* z2;
+    double* z2;
     R* pr;
     R* pi;
-    Z* g;
+    double* g;
 };
 
-// RK4 stage derivatives k_s: all six components in R.  In the mixed form the
-// derivatives of z2 and Gamma are stored in FP32, while the trial states
-// y0 + c k and the step's accumulation y0 + h/6 (k1 + 2 k2 + 2 k3 + k4) of z2
-// and Gamma are formed in FP64 (24 instead of 32 bytes per derivative).
+// RK4 stage derivatives k_s of the momenta p_r, p_i and Gamma, in R.  The
+// derivatives of x, y and z2 are functions of the stage's trial momenta alone
+// (rates(), puff_stage.hpp), so a later stage forms them again from y0 and
+// k_{s-2} instead of reading them: of the 656 bytes per macroparticle and
+// step that storing all six moved in the FP64 form (368 in the mixed form),
+// 488 (284) are left.  In the mixed form the derivative of Gamma is stored in
+// FP32, while the trial states y0 + c k and the step's accumulation
+// y0 + h/6 (k1 + 2 k2 + 2 k3 + k4) of z2 and Gamma are formed in FP64.
 template <typename R>
-using KPtrs = PartPtrs<R, R>;
+struct KPtrs {
+    R* pr;
+    R* pi;
+    R* g;
+};
 
 // Deterministic deposit of the FP64 form.  Every contribution v = w_k s of a
 // macroparticle to a node is split into two fixed-point integers,
@@ -71,11 +78,13 @@ template <typename R>
 struct StageArgs {
     int64_t n;
     PartPtrs<R> y0;     // state at the start of the step (written by stage 4)
-    KPtrs<R> kin;       // derivative of the previous stage
-    KPtrs<R> kout;      // derivative of this stage (stages 1-3)
-    KPtrs<R> k1, k2;    // stage 4: first two derivatives (k3 = kin)
+    KPtrs<R> kin;       // k_{s-1} (stages 2-4)
+    KPtrs<R> kprev;     // k_{s-2} (stages 3, 4)
+    KPtrs<R> k1;        // stage 4
+    KPtrs<R> kout;      // k_s (stages 1-3)
     const R* chi;
     double cin;         // trial coefficient of this stage (0, h/2, h/2, h)
+    double cprev;       // of the stage before (stages 3, 4: h/2)
     double cnext;       // trial coefficient of the next stage
     double h6;
     const cplx<R>* A0;
@@ -139,8 +148,9 @@ struct AdjArgs {
     int64_t n;
     PartPtrs<R> y0;
     KPtrs<R> kin;          // k_{s-1} (stages 2-4)
+    KPtrs<R> kprev;        // k_{s-2} (stages 3, 4)
     const R* chi;
-    double cin;
+    double cin, cprev;     // trial coefficients of this stage and the one before
     const cplx<R>* A0;
     const cplx<R>* dAin;   // dA_{s-1} (stages 2-4)
     PartPtrs<R> L;         // cotangent of the step's end state

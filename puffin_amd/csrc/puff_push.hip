@@ -59,39 +59,42 @@ __global__ __launch_bounds__(STAGE_THREADS) void k_stage(StageArgs<R> a) {
                 a.chicap[i] = chi;
             }
         } else {
-            const R c = (R)a.cin;
-            const R k3x = a.kin.x[i], k3y = a.kin.y[i], k3pr = a.kin.pr[i], k3pi = a.kin.pi[i];
-            const double k3z2 = a.kin.z2[i], k3g = a.kin.g[i];
-            x = fma(c, k3x, x0);
-            y = fma(c, k3y, y0);
-            z2 = fma(a.cin, k3z2, z20);
-            pr = fma(c, k3pr, pr0);
-            pi = fma(c, k3pi, pi0);
-            g = fma(a.cin, k3g, g0);
+            const R kr = a.kin.pr[i], ki = a.kin.pi[i], kg = a.kin.g[i];
+            R qr = 0, qi = 0, qg = 0;
+            if (STAGE > 2) {
+                qr = a.kprev.pr[i];
+                qi = a.kprev.pi[i];
+                qg = a.kprev.g[i];
+            }
+            const Trial<R> t = trial_state<R, STAGE>(ph, x0, y0, z20, pr0, pi0, g0, kr, ki, kg, qr, qi, qg, a.cin,
+                                                     a.cprev);
+            x = t.x; y = t.y; z2 = t.z2; pr = t.pr; pi = t.pi; g = t.g;
             if (STAGE == 4) {
                 // y0 + h/6 (k1 + 2 (k2 + k3)) formed now, with k1 and k2 loaded
                 // beside y0 and k3: the end of the kernel adds h/6 k4 only, and
-                // no k array is read after the deposit (puffin_mpi_RK4.f90:274-279)
-                const R h6 = (R)a.h6;
-                x0 = fma(h6, a.k1.x[i] + (R)2 * (a.k2.x[i] + k3x), x0);
-                y0 = fma(h6, a.k1.y[i] + (R)2 * (a.k2.y[i] + k3y), y0);
-                z20 = fma(a.h6, a.k1.z2[i] + 2.0 * (a.k2.z2[i] + k3z2), z20);
-                pr0 = fma(h6, a.k1.pr[i] + (R)2 * (a.k2.pr[i] + k3pr), pr0);
-                pi0 = fma(h6, a.k1.pi[i] + (R)2 * (a.k2.pi[i] + k3pi), pi0);
-                g0 = fma(a.h6, a.k1.g[i] + 2.0 * (a.k2.g[i] + k3g), g0);
+                // no k array is read after the deposit (puffin_mpi_RK4.f90:274-279).
+                // The rates of y0, y0 + h/2 k1 and y0 + h/2 k2 are k1 to k3 of
+                // x, y and z2.
+                const R h6 = (R)a.h6, hh = (R)a.cprev;
+                const R k1r = a.k1.pr[i], k1i = a.k1.pi[i], k1g = a.k1.g[i];
+                const Rates<R> v1 = rates<R>(ph, drift_of(ph, (double)pr0, (double)pi0, g0), pr0, pi0);
+                const R p2r = fma(hh, k1r, pr0), p2i = fma(hh, k1i, pi0);
+                const Rates<R> v2 =
+                    rates<R>(ph, drift_of(ph, (double)p2r, (double)p2i, fma(a.cprev, (double)k1g, g0)), p2r, p2i);
+                x0 = fma(h6, v1.x + (R)2 * (v2.x + t.v.x), x0);
+                y0 = fma(h6, v1.y + (R)2 * (v2.y + t.v.y), y0);
+                z20 = fma(a.h6, v1.z2 + 2.0 * (v2.z2 + t.v.z2), z20);
+                pr0 = fma(h6, k1r + (R)2 * (qr + kr), pr0);
+                pi0 = fma(h6, k1i + (R)2 * (qi + ki), pi0);
+                g0 = fma(a.h6, (double)k1g + 2.0 * ((double)qg + (double)kg), g0);
             }
         }
     }
 
-    // ---- p2 in FP64 (gamma_to_p2.f90:84-85), with 1/eta and 1/gamma_r^2
-    // from the host and 1/Gamma formed once
+    // ---- p2 in FP64 and (1 + eta p2) / Gamma
     const double prd = (double)pr, pid = (double)pi;
-    const double invg = 1.0 / g;
-    const double p2 = in ? ((1.0 / sqrt(1.0 - ph.inv_gr2 * invg * invg *
-                                               (1.0 + ph.aw * ph.aw * (prd * prd + pid * pid)))) -
-                            1.0) * ph.inv_eta
-                         : 0.0;
-    const double fac = (1.0 + ph.eta * p2) * invg;   // (1 + eta p2) / Gamma
+    const Drift dr = drift_of(ph, prd, pid, g);
+    const double p2 = dr.p2, fac = dr.fac;
 
     // ---- node and weights
     Cell<R> c{};
@@ -220,45 +223,39 @@ __global__ __launch_bounds__(STAGE_THREADS) void k_stage(StageArgs<R> a) {
     if (!ph.coupling) { fr = 0; fi = 0; }   // rhs.f90:221-224
 
     // ---- equations (puffin_equations.f90:17-176)
-    R kx_ = 0, ky_ = 0, kpr = 0, kpi = 0;
-    double kz2 = 0.0, kg = 0.0;
+    const Rates<R> v = rates<R>(ph, dr, pr, pi);
+    R kpr = 0, kpi = 0;
+    double kg = 0.0;
     if (ph.electrons_evolve) {
         R bx, by, bz;
         bfield<R>(a.s, x, y, bx, by, bz);
         const R facr = (R)fac;
         const R n2col = (R)a.s.n2col;
         const R ep2k = (R)(ph.eta * p2 / (ph.kappa * ph.kappa));
-        kz2 = p2;
-        kx_ = (R)ph.c_dx * facr * pr;
-        ky_ = -(R)ph.c_dx * facr * pi;
         kpr = (R)ph.inv2rho * (n2col * by - ep2k * fr) + (R)ph.kappa * pi * facr * n2col * bz;
         kpi = (R)ph.inv2rho * (n2col * bx - ep2k * fi) - (R)ph.kappa * pr * facr * n2col * bz;
         kg = -ph.rho * fac * 2.0 * ((double)pr * (double)fr + (double)pi * (double)fi);
     }
 
     if (STAGE < 4) {
-        // stored in R (FP32 in the mixed form: see KPtrs)
-        const R kz2s = (R)kz2;
-        a.kout.x[i] = kx_;
-        a.kout.y[i] = ky_;
-        a.kout.z2[i] = kz2s;
         a.kout.pr[i] = kpr;
         a.kout.pi[i] = kpi;
-        a.kout.g[i] = (R)kg;
+        a.kout.g[i] = (R)kg;   // FP32 in the mixed form (see KPtrs)
         // next stage's trial state must lie inside the mesh, else the next
-        // derivs call would raise the flag (checked here, on the stored
-        // derivative, so that no later kernel writes state when it does)
+        // derivs call would raise the flag (checked here, on the rates the
+        // next stage forms again, so that no later kernel writes state when
+        // it does)
         const R cn = (R)a.cnext;
         Cell<R> cc;
-        const int nf = locate<R>(m, fma(cn, kx_, x0), fma(cn, ky_, y0), fma(a.cnext, (double)kz2s, z20), cc);
+        const int nf = locate<R>(m, fma(cn, v.x, x0), fma(cn, v.y, y0), fma(a.cnext, v.z2, z20), cc);
         if (nf) atomicOr(a.flags, nf);
     } else {
         // y = (y0 + h/6 (k1 + 2 (k2 + k3))) + h/6 k4  (puffin_mpi_RK4.f90:274-279, 307-312)
         if (rejected) return;   // the step is rejected
         const R h6 = (R)a.h6;
-        a.y0.x[i] = fma(h6, kx_, x0);
-        a.y0.y[i] = fma(h6, ky_, y0);
-        a.y0.z2[i] = fma(a.h6, kz2, z20);
+        a.y0.x[i] = fma(h6, v.x, x0);
+        a.y0.y[i] = fma(h6, v.y, y0);
+        a.y0.z2[i] = fma(a.h6, v.z2, z20);
         a.y0.pr[i] = fma(h6, kpr, pr0);
         a.y0.pi[i] = fma(h6, kpi, pi0);
         a.y0.g[i] = fma(a.h6, kg, g0);

@@ -66,6 +66,73 @@ __device__ __forceinline__ int locate(const MeshGeom& m, R x, R y, double z2,
     return 0;
 }
 
+// p2 (gamma_to_p2.f90:84-85) and (1 + eta p2) / Gamma of one macroparticle,
+// in FP64, with 1/eta and 1/gamma_r^2 from the host and 1/Gamma formed once.
+// Without contraction and with its FMAs written out, as in rates(): a stage
+// forms the previous trial state's derivatives of x, y and z2 again, and they
+// are the bits that the previous stage checked its successor's trial position
+// with.
+struct Drift {
+    double p2, fac;
+};
+
+__device__ __forceinline__ Drift drift_of(const Physics& ph, double pr, double pi, double g) {
+#pragma clang fp contract(off)
+    const double invg = 1.0 / g;
+    const double s = fma(ph.aw * ph.aw, fma(pr, pr, pi * pi), 1.0);
+    const double p2 = ((1.0 / sqrt(fma(-(ph.inv_gr2 * invg * invg), s, 1.0))) - 1.0) * ph.inv_eta;
+    return {p2, fma(ph.eta, p2, 1.0) * invg};
+}
+
+// Derivatives of x, y and z2 (puffin_equations.f90:115-117, 144-146, 172):
+// zero when the electrons do not evolve (rhs.f90:301-308).
+template <typename R>
+struct Rates {
+    R x, y;
+    double z2;
+};
+
+template <typename R>
+__device__ __forceinline__ Rates<R> rates(const Physics& ph, const Drift& d, R pr, R pi) {
+#pragma clang fp contract(off)
+    if (!ph.electrons_evolve) return {(R)0, (R)0, 0.0};
+    const R v = (R)ph.c_dx * (R)d.fac;
+    return {v * pr, -v * pi, d.p2};
+}
+
+// Trial state y0 + c k_{s-1} of one macroparticle (puffin_mpi_RK4.f90:190-195
+// etc.): p_r, p_i and Gamma from the stored derivative, x, y and z2 from the
+// rates of the previous trial state's momenta, y0 + cprev k_{s-2} (those of
+// y0 itself in stage 2).
+template <typename R>
+struct Trial {
+    R x, y, pr, pi;
+    double z2, g;
+    Rates<R> v;     // rates of the previous trial state
+};
+
+template <typename R, int STAGE>
+__device__ __forceinline__ Trial<R> trial_state(const Physics& ph, R x0, R y0, double z20, R pr0, R pi0, double g0,
+                                                R kr, R ki, R kg, R qr, R qi, R qg, double cin, double cprev) {
+    Trial<R> t;
+    R ppr = pr0, ppi = pi0;
+    double pg = g0;
+    if (STAGE > 2) {
+        ppr = fma((R)cprev, qr, pr0);
+        ppi = fma((R)cprev, qi, pi0);
+        pg = fma(cprev, (double)qg, g0);
+    }
+    const R c = (R)cin;
+    t.v = rates<R>(ph, drift_of(ph, (double)ppr, (double)ppi, pg), ppr, ppi);
+    t.x = fma(c, t.v.x, x0);
+    t.y = fma(c, t.v.y, y0);
+    t.z2 = fma(cin, t.v.z2, z20);
+    t.pr = fma(c, kr, pr0);
+    t.pi = fma(c, ki, pi0);
+    t.g = fma(cin, (double)kg, g0);
+    return t;
+}
+
 // Scaled undulator field at one particle from the stage coefficients
 // (bfields.f90): see stage_scalars() on the host for the coefficient map.
 template <typename R>
