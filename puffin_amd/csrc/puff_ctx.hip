@@ -33,10 +33,14 @@ struct Particles {
     PartPtrs<R> y;
     KPtrs<R> k[3];
     R* chi = nullptr;
-    // the sort's spare z2 and Gamma arrays in the mixed form (its spare x, y,
-    // p_r, p_i are k[0]'s and k[1]'s, as are the FP64 form's z2 and Gamma)
-    double* z2_spare = nullptr;
-    double* g_spare = nullptr;
+};
+
+// The eight arrays of a set of slots: state, chi, reference index.
+template <typename R>
+struct Slots {
+    PartPtrs<R> y;
+    R* chi;
+    int* orig;
 };
 
 constexpr int DN2_TABLE_CAP = 4096;   // taper-table slots of the deferred adjoint
@@ -84,8 +88,15 @@ struct Ctx {
     Physics phys{};
     // particle order: orig[j] = reference index of slot j
     int* orig = nullptr;
-    int* orig_spare = nullptr;
-    void* chi_spare = nullptr;
+    // One allocation holds two sets of slots with the stage derivatives
+    // between them: slots 0 | k | slots 1.  The macroparticles are in set
+    // slot_set; a re-sort moves them to the other.  Outside a step the other
+    // set and k are free, and are one contiguous stretch of at least 64 bytes
+    // per macroparticle in either form (132 and 76): the records of a sort or
+    // of a move between slot and reference order (records_region).
+    char* slots_base = nullptr;
+    size_t slots_bytes = 0, k_bytes = 0;   // of one set, of k
+    int slot_set = 0;
     int* sort_key = nullptr;
     int* sort_counts = nullptr;
     int* sort_perm = nullptr;
@@ -501,34 +512,56 @@ static double advance_taper(Ctx* c, double z) {
 
 // ---- context creation -------------------------------------------------------
 
+static size_t align256c(size_t v) { return (v + 255) & ~(size_t)255; }
+
+// Arrays of the set of slots at base, each 256-byte aligned; returns its bytes.
+template <typename R>
+static size_t slots_view(size_t n, char* base, Slots<R>* v) {
+    size_t o = 0;
+    auto take = [&](size_t bytes) -> char* {
+        char* p = base ? base + o : nullptr;
+        o = align256c(o + bytes);
+        return p;
+    };
+    v->y.x = reinterpret_cast<R*>(take(sizeof(R) * n));
+    v->y.y = reinterpret_cast<R*>(take(sizeof(R) * n));
+    v->y.z2 = reinterpret_cast<double*>(take(sizeof(double) * n));
+    v->y.pr = reinterpret_cast<R*>(take(sizeof(R) * n));
+    v->y.pi = reinterpret_cast<R*>(take(sizeof(R) * n));
+    v->y.g = reinterpret_cast<double*>(take(sizeof(double) * n));
+    v->chi = reinterpret_cast<R*>(take(sizeof(R) * n));
+    v->orig = reinterpret_cast<int*>(take(sizeof(int) * n));
+    return o;
+}
+
+template <typename R>
+static Slots<R> slot_arrays(const Ctx* c, int set) {
+    Slots<R> v;
+    slots_view<R>((size_t)c->n, c->slots_base + (set ? c->slots_bytes + c->k_bytes : 0), &v);
+    return v;
+}
+
+static uint4* records_region(const Ctx* c) {
+    return reinterpret_cast<uint4*>(c->slots_base + (c->slot_set ? 0 : c->slots_bytes));
+}
+
 template <typename R>
 static int alloc_particles(Ctx* c) {
     Particles<R>& P = parts<R>(c);
-    auto setp = [&](PartPtrs<R>& q) -> int {
-        PUFF_TRY(dalloc(c, (void**)&q.x, sizeof(R) * c->n));
-        PUFF_TRY(dalloc(c, (void**)&q.y, sizeof(R) * c->n));
-        PUFF_TRY(dalloc(c, (void**)&q.z2, sizeof(double) * c->n));
-        PUFF_TRY(dalloc(c, (void**)&q.pr, sizeof(R) * c->n));
-        PUFF_TRY(dalloc(c, (void**)&q.pi, sizeof(R) * c->n));
-        PUFF_TRY(dalloc(c, (void**)&q.g, sizeof(double) * c->n));
-        return PUFF_OK;
-    };
-    auto setk = [&](KPtrs<R>& q) -> int {
-        PUFF_TRY(dalloc(c, (void**)&q.pr, sizeof(R) * c->n));
-        PUFF_TRY(dalloc(c, (void**)&q.pi, sizeof(R) * c->n));
-        PUFF_TRY(dalloc(c, (void**)&q.g, sizeof(R) * c->n));
-        return PUFF_OK;
-    };
-    PUFF_TRY(setp(P.y));
-    for (int k = 0; k < 3; ++k) PUFF_TRY(setk(P.k[k]));
-    if constexpr (sizeof(R) != sizeof(double)) {
-        PUFF_TRY(dalloc(c, (void**)&P.z2_spare, sizeof(double) * c->n));
-        PUFF_TRY(dalloc(c, (void**)&P.g_spare, sizeof(double) * c->n));
+    const size_t n = (size_t)c->n;
+    Slots<R> v;
+    c->slots_bytes = slots_view<R>(n, nullptr, &v);
+    const size_t kb = align256c(sizeof(R) * n);
+    c->k_bytes = 9 * kb;
+    PUFF_TRY(dalloc(c, (void**)&c->slots_base, 2 * c->slots_bytes + c->k_bytes));
+    v = slot_arrays<R>(c, 0);
+    P.y = v.y;
+    P.chi = v.chi;
+    c->orig = v.orig;
+    for (int k = 0; k < 3; ++k) {
+        char* q = c->slots_base + c->slots_bytes + 3 * k * kb;
+        P.k[k] = {reinterpret_cast<R*>(q), reinterpret_cast<R*>(q + kb), reinterpret_cast<R*>(q + 2 * kb)};
     }
-    PUFF_TRY(dalloc(c, (void**)&P.chi, sizeof(R) * c->n));
-    PUFF_TRY(dalloc(c, &c->chi_spare, sizeof(R) * c->n));
-    PUFF_TRY(dalloc(c, (void**)&c->orig, sizeof(int) * c->n));
-    PUFF_TRY(dalloc(c, (void**)&c->orig_spare, sizeof(int) * c->n));
     PUFF_TRY(dalloc(c, (void**)&c->sort_key, sizeof(int) * c->n));
     PUFF_TRY(dalloc(c, (void**)&c->sort_perm, sizeof(int) * c->n));
     const int64_t bins = sort_bins(c->p.nx, c->p.ny, c->nzp(), c->p.one_d != 0);
@@ -714,8 +747,6 @@ struct CaptureView {
     cplx<R>* dA[3];
 };
 
-static size_t align256c(size_t v) { return (v + 255) & ~(size_t)255; }
-
 // Pointers into the capture at base (null base: sizes only); returns its bytes.
 template <typename R>
 static size_t capture_view(const Ctx* c, char* base, CaptureView<R>* v) {
@@ -754,49 +785,31 @@ template <typename R>
 static void sort_particles(Ctx* c) {
     const int slot = prof_start(c, 11);
     Particles<R>& P = parts<R>(c);
+    const Slots<R> spare = slot_arrays<R>(c, 1 - c->slot_set);
     SortArgs<R> a{};
     a.n = c->n;
     a.ncell = c->ncell;
     a.mesh = c->mesh;
-    a.y = &P.y;
-    // spare state arrays: those of k[0] and k[1], with z2 and Gamma of the
-    // state's type
-    KPtrs<R>& k0 = P.k[0];
-    KPtrs<R>& k1 = P.k[1];
-    PartPtrs<R> spare{k0.pr, k0.pi, nullptr, k1.pr, k1.pi, nullptr};
-    if constexpr (sizeof(R) == sizeof(double)) {
-        spare.z2 = reinterpret_cast<double*>(k0.g);
-        spare.g = reinterpret_cast<double*>(k1.g);
-    } else {
-        spare.z2 = P.z2_spare;
-        spare.g = P.g_spare;
-    }
-    a.spare = &spare;
-    a.chi = &P.chi;
-    R* spare_chi = reinterpret_cast<R*>(c->chi_spare);
-    a.chi_spare = &spare_chi;
-    a.orig = &c->orig;
-    a.orig_spare = &c->orig_spare;
+    a.y = P.y;
+    a.spare = spare.y;
+    a.chi = P.chi;
+    a.chi_spare = spare.chi;
+    a.orig = c->orig;
+    a.orig_spare = spare.orig;
     a.key = c->sort_key;
     a.counts = c->sort_counts;
     a.cursor = c->sort_counts;
     a.perm = c->sort_perm;
     a.tile_sums = c->sort_tiles;
+    a.rec = c->identity_order ? records_region(c) : nullptr;
     launch_sort<R>(a, c->stream);
-    // the sort swapped the state and spare pointers: the spares go back
-    k0.pr = spare.x;
-    k0.pi = spare.y;
-    k1.pr = spare.pr;
-    k1.pi = spare.pi;
-    if constexpr (sizeof(R) == sizeof(double)) {
-        k0.g = reinterpret_cast<R*>(spare.z2);
-        k1.g = reinterpret_cast<R*>(spare.g);
-    } else {
-        P.z2_spare = spare.z2;
-        P.g_spare = spare.g;
+    if (!a.rec) {
+        c->slot_set = 1 - c->slot_set;
+        P.y = spare.y;
+        P.chi = spare.chi;
+        c->orig = spare.orig;
     }
     prof_stop(c, slot);
-    c->chi_spare = spare_chi;
     c->sorted = true;
     c->identity_order = false;
     c->steps_since_sort = 0;
@@ -977,6 +990,29 @@ static int diffraction(Ctx* c, double h) {
 
 // ---- data exchange ------------------------------------------------------------
 
+// Whether the kernels may read or write the caller's n doubles at p: memory
+// of this context's device, the whole range inside one allocation.  Anything
+// else that was passed as device memory (a peer's, pinned or managed memory)
+// goes through the copy engine, which checks it.
+static bool on_device(const Ctx* c, const void* p, int64_t n) {
+    hipPointerAttribute_t at{};
+    hipDeviceptr_t base = nullptr;
+    size_t bytes = 0;
+    const bool ok = p && hipPointerGetAttributes(&at, p) == hipSuccess && at.type == hipMemoryTypeDevice &&
+                    at.device == c->device && ((uintptr_t)p & 7) == 0 &&
+                    hipMemGetAddressRange(&base, &bytes, const_cast<void*>(p)) == hipSuccess &&
+                    (const char*)p + sizeof(double) * (size_t)n <= (const char*)base + bytes;
+    if (!ok) (void)hipGetLastError();
+    return ok;
+}
+
+template <size_t K, typename T>
+static bool all_on_device(const Ctx* c, T* const (&p)[K], int64_t n) {
+    for (T* q : p)
+        if (!on_device(c, q, n)) return false;
+    return true;
+}
+
 // One coordinate array from the reference order (FP64) into the slot order
 // and storage type T of the device.
 template <typename T>
@@ -1023,6 +1059,13 @@ static int upload_particles(Ctx* c, int kind, const double* x, const double* y, 
         c->identity_order = true;
         c->sorted = false;
         c->order_id = ++c->order_counter;
+        const double* const in[7] = {x, y, z2, px, py, g, chi};
+        if (kind == PUFF_MEM_DEVICE && all_on_device(c, in, c->n)) {
+            launch_load_state<R>(in, c->n, P.y, P.chi, c->stream);
+            PUFF_HIP(hipGetLastError());
+            PUFF_HIP(hipStreamSynchronize(c->stream));
+            return PUFF_OK;
+        }
     }
     PUFF_TRY(upload_array<R>(c, kind, x, P.y.x));
     PUFF_TRY(upload_array<R>(c, kind, y, P.y.y));
@@ -1038,6 +1081,14 @@ template <typename R>
 static int download_particles(Ctx* c, int kind, double* x, double* y, double* z2, double* px,
                               double* py, double* g) {
     Particles<R>& P = parts<R>(c);
+    double* const out[6] = {x, y, z2, px, py, g};
+    if (kind == PUFF_MEM_DEVICE && !c->identity_order && all_on_device(c, out, c->n)) {
+        launch_records_scatter<R>(P.y, c->orig, c->n, records_region(c), c->stream);
+        launch_records_unpack<R>(records_region(c), c->n, out, c->stream);
+        PUFF_HIP(hipGetLastError());
+        PUFF_HIP(hipStreamSynchronize(c->stream));
+        return PUFF_OK;
+    }
     PUFF_TRY(download_array<R>(c, kind, P.y.x, x));
     PUFF_TRY(download_array<R>(c, kind, P.y.y, y));
     PUFF_TRY(download_array<double>(c, kind, P.y.z2, z2));
@@ -1047,35 +1098,50 @@ static int download_particles(Ctx* c, int kind, double* x, double* y, double* z2
     return PUFF_OK;
 }
 
+// Split FP64 arrays into an interleaved field buffer: from device arrays in
+// one pass, others through the staging buffer.  alias: fill the last plane of
+// a periodic mesh with plane 1, which it copies (para_field.f90:1075-1138).
 template <typename R>
-static int upload_field(Ctx* c, int kind, const double* ar, const double* ai) {
+static int field_in(Ctx* c, int kind, const double* ar, const double* ai, cplx<R>* A, bool alias) {
     const int64_t nm = c->nmesh();
-    const hipMemcpyKind k = kind == PUFF_MEM_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
-    PUFF_HIP(hipMemcpyAsync(c->stage_buf, ar, sizeof(double) * nm, k, c->stream));
-    PUFF_HIP(hipMemcpyAsync(c->stage_buf + nm, ai, sizeof(double) * nm, k, c->stream));
-    launch_pack_field<R>(c->stage_buf, c->stage_buf + nm, reinterpret_cast<cplx<R>*>(c->A), nm, c->stream);
+    const double* const in[2] = {ar, ai};
+    if (kind != PUFF_MEM_DEVICE || !all_on_device(c, in, nm)) {
+        const hipMemcpyKind k = kind == PUFF_MEM_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
+        PUFF_HIP(hipMemcpyAsync(c->stage_buf, ar, sizeof(double) * nm, k, c->stream));
+        PUFF_HIP(hipMemcpyAsync(c->stage_buf + nm, ai, sizeof(double) * nm, k, c->stream));
+        ar = c->stage_buf;
+        ai = c->stage_buf + nm;
+    }
+    const int64_t from = (alias && c->p.periodic) ? (int64_t)c->p.nx * c->p.ny * (c->p.nz2 - 1) : nm;
+    launch_pack_field<R>(ar, ai, A, nm, from, c->stream);
     PUFF_HIP(hipGetLastError());
-    if (c->p.periodic) {
-        // the last plane of a periodic mesh aliases plane 1 (para_field.f90:1075-1138)
-        const int64_t ntr = (int64_t)c->p.nx * c->p.ny;
-        cplx<R>* A = reinterpret_cast<cplx<R>*>(c->A);
-        PUFF_HIP(hipMemcpyAsync(A + (int64_t)(c->p.nz2 - 1) * ntr, A, sizeof(cplx<R>) * ntr,
-                                hipMemcpyDeviceToDevice, c->stream));
+    PUFF_HIP(hipStreamSynchronize(c->stream));
+    return PUFF_OK;
+}
+
+template <typename R>
+static int field_out(Ctx* c, int kind, const cplx<R>* A, double* ar, double* ai) {
+    const int64_t nm = c->nmesh();
+    const bool direct = kind == PUFF_MEM_DEVICE && (!ar || on_device(c, ar, nm)) && (!ai || on_device(c, ai, nm));
+    launch_unpack_field<R>(A, direct ? ar : c->stage_buf, direct ? ai : c->stage_buf + nm, nm, c->stream);
+    PUFF_HIP(hipGetLastError());
+    if (!direct) {
+        const hipMemcpyKind k = kind == PUFF_MEM_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost;
+        if (ar) PUFF_HIP(hipMemcpyAsync(ar, c->stage_buf, sizeof(double) * nm, k, c->stream));
+        if (ai) PUFF_HIP(hipMemcpyAsync(ai, c->stage_buf + nm, sizeof(double) * nm, k, c->stream));
     }
     PUFF_HIP(hipStreamSynchronize(c->stream));
     return PUFF_OK;
 }
 
 template <typename R>
+static int upload_field(Ctx* c, int kind, const double* ar, const double* ai) {
+    return field_in<R>(c, kind, ar, ai, reinterpret_cast<cplx<R>*>(c->A), true);
+}
+
+template <typename R>
 static int download_field(Ctx* c, int kind, double* ar, double* ai) {
-    const int64_t nm = c->nmesh();
-    const hipMemcpyKind k = kind == PUFF_MEM_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost;
-    launch_unpack_field<R>(reinterpret_cast<const cplx<R>*>(c->A), c->stage_buf, c->stage_buf + nm, nm, c->stream);
-    PUFF_HIP(hipGetLastError());
-    if (ar) PUFF_HIP(hipMemcpyAsync(ar, c->stage_buf, sizeof(double) * nm, k, c->stream));
-    if (ai) PUFF_HIP(hipMemcpyAsync(ai, c->stage_buf + nm, sizeof(double) * nm, k, c->stream));
-    PUFF_HIP(hipStreamSynchronize(c->stream));
-    return PUFF_OK;
+    return field_out<R>(c, kind, reinterpret_cast<const cplx<R>*>(c->A), ar, ai);
 }
 
 template <typename R>
@@ -1240,17 +1306,8 @@ static void fill_zero_typed(T* p, int64_t n, hipStream_t s) {
 template <typename R>
 static int repermute_cotangent(Ctx* c, const int* orig_from, const int* orig_to) {
     AdjBufs<R>& B = adjb<R>(c);
-    hipStream_t s = c->stream;
-    R* rr[4] = {B.L.x, B.L.y, B.L.pr, B.L.pi};
-    double* dd[2] = {B.L.z2, B.L.g};
-    for (R* a : rr) {
-        launch_unpermute<R>(a, orig_from, c->n, c->stage_buf, s);
-        launch_permute_in<R>(c->stage_buf, orig_to, c->n, a, s);
-    }
-    for (double* a : dd) {
-        launch_unpermute<double>(a, orig_from, c->n, c->stage_buf, s);
-        launch_permute_in<double>(c->stage_buf, orig_to, c->n, a, s);
-    }
+    launch_records_scatter<R>(B.L, orig_from, c->n, records_region(c), c->stream);
+    launch_records_gather<R>(records_region(c), orig_to, c->n, B.L, c->stream);
     PUFF_HIP(hipGetLastError());
     return PUFF_OK;
 }
@@ -1551,15 +1608,7 @@ static int adjoint_upload(Ctx* c, int kind, const double* x, const double* y, co
     PUFF_TRY(upload_array<R>(c, kind, px, B.L.pr));
     PUFF_TRY(upload_array<R>(c, kind, py, B.L.pi));
     PUFF_TRY(upload_array<double>(c, kind, g, B.L.g));
-    if (ar && ai) {
-        const int64_t nm = c->nmesh();
-        const hipMemcpyKind k = kind == PUFF_MEM_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
-        PUFF_HIP(hipMemcpyAsync(c->stage_buf, ar, sizeof(double) * nm, k, c->stream));
-        PUFF_HIP(hipMemcpyAsync(c->stage_buf + nm, ai, sizeof(double) * nm, k, c->stream));
-        launch_pack_field<R>(c->stage_buf, c->stage_buf + nm, reinterpret_cast<cplx<R>*>(c->LA), nm, c->stream);
-        PUFF_HIP(hipGetLastError());
-        PUFF_HIP(hipStreamSynchronize(c->stream));
-    }
+    if (ar && ai) PUFF_TRY(field_in<R>(c, kind, ar, ai, reinterpret_cast<cplx<R>*>(c->LA), false));
     return PUFF_OK;
 }
 
@@ -1575,16 +1624,7 @@ static int adjoint_download(Ctx* c, int kind, double* x, double* y, double* z2, 
     PUFF_TRY(download_array<R>(c, kind, B.L.pr, px));
     PUFF_TRY(download_array<R>(c, kind, B.L.pi, py));
     PUFF_TRY(download_array<double>(c, kind, B.L.g, g));
-    if (ar || ai) {
-        const int64_t nm = c->nmesh();
-        const hipMemcpyKind k = kind == PUFF_MEM_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost;
-        launch_unpack_field<R>(reinterpret_cast<const cplx<R>*>(c->LA), c->stage_buf, c->stage_buf + nm, nm,
-                               c->stream);
-        PUFF_HIP(hipGetLastError());
-        if (ar) PUFF_HIP(hipMemcpyAsync(ar, c->stage_buf, sizeof(double) * nm, k, c->stream));
-        if (ai) PUFF_HIP(hipMemcpyAsync(ai, c->stage_buf + nm, sizeof(double) * nm, k, c->stream));
-        PUFF_HIP(hipStreamSynchronize(c->stream));
-    }
+    if (ar || ai) PUFF_TRY(field_out<R>(c, kind, reinterpret_cast<const cplx<R>*>(c->LA), ar, ai));
     return PUFF_OK;
 }
 

@@ -154,18 +154,25 @@ __global__ __launch_bounds__(256) void k_current(const double* z2, const R* chi,
     if (p0 == 0 && (threadIdx.x & 63) == 0 && bad > 0.0) atomicAdd(&acc[npts], bad);
 }
 
+// Split FP64 arrays of the caller to the mesh's interleaved field and back:
+// both ways bound by their own bytes (32 per node in the FP64 form).
 template <typename R>
-__global__ void k_pack(const double* ar, const double* ai, cplx<R>* a, int64_t n) {
+__global__ __launch_bounds__(256) void k_pack(const double* ar, const double* ai, cplx<R>* a, int64_t n,
+                                              int64_t alias_from) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) a[i] = {(R)ar[i], (R)ai[i]};
+    if (i < n) {
+        const int64_t j = i < alias_from ? i : i - alias_from;
+        a[i] = {(R)ar[j], (R)ai[j]};
+    }
 }
 
 template <typename R>
-__global__ void k_unpack(const cplx<R>* a, double* ar, double* ai, int64_t n) {
+__global__ __launch_bounds__(256) void k_unpack(const cplx<R>* a, double* ar, double* ai, int64_t n) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) {
-        ar[i] = (double)a[i].x;
-        ai[i] = (double)a[i].y;
+        const cplx<R> v = a[i];
+        if (ar) ar[i] = (double)v.x;
+        if (ai) ai[i] = (double)v.y;
     }
 }
 
@@ -270,8 +277,8 @@ void launch_current(const double* z2, const R* chi, int64_t n, int npts, double 
 }
 
 template <typename R>
-void launch_pack_field(const double* ar, const double* ai, cplx<R>* a, int64_t n, hipStream_t s) {
-    hipLaunchKernelGGL((k_pack<R>), grid_for(n), dim3(256), 0, s, ar, ai, a, n);
+void launch_pack_field(const double* ar, const double* ai, cplx<R>* a, int64_t n, int64_t alias_from, hipStream_t s) {
+    hipLaunchKernelGGL((k_pack<R>), grid_for(n), dim3(256), 0, s, ar, ai, a, n, alias_from);
 }
 template <typename R>
 void launch_unpack_field(const cplx<R>* a, double* ar, double* ai, int64_t n, hipStream_t s) {
@@ -295,7 +302,7 @@ void launch_convert_back(const R* src, double* dst, int64_t n, hipStream_t s) {
                                           double*, hipStream_t);                                  \
     template void launch_current<R>(const double*, const R*, int64_t, int, double, int, double*,  \
                                     hipStream_t);                                                 \
-    template void launch_pack_field<R>(const double*, const double*, cplx<R>*, int64_t,           \
+    template void launch_pack_field<R>(const double*, const double*, cplx<R>*, int64_t, int64_t,  \
                                        hipStream_t);                                              \
     template void launch_unpack_field<R>(const cplx<R>*, double*, double*, int64_t, hipStream_t); \
     template void launch_convert<R>(const double*, R*, int64_t, hipStream_t);                     \

@@ -254,21 +254,48 @@ struct SortArgs {
     int64_t n;
     int ncell;             // bins on the mesh (sort_bins); bin ncell collects particles off it
     MeshGeom mesh;
-    PartPtrs<R>* y;        // sorted in place (pointers swapped with spare)
-    PartPtrs<R>* spare;
-    R** chi;
-    R** chi_spare;
-    int** orig;            // reference index of each slot
-    int** orig_spare;
+    PartPtrs<R> y;
+    PartPtrs<R> spare;
+    R* chi;
+    R* chi_spare;
+    int* orig;             // reference index of each slot
+    int* orig_spare;
     int* key;
     int* counts;           // ncell + 1 bins, scanned in place
     int* cursor;
     int* perm;
     int* tile_sums;
+    uint4* rec;            // n records (RecordQuads) for a sort out of the reference order, else null
 };
 
+// Sorts the macroparticles by cell.  With a.rec (a.orig is the identity: the
+// macroparticles come in any order) the result is in a.y, a.chi and a.orig;
+// without it (a re-sort, nearly in order) in the spare arrays.
 template <typename R>
-void launch_sort(SortArgs<R>& a, hipStream_t s);
+void launch_sort(const SortArgs<R>& a, hipStream_t s);
+
+// One macroparticle's values together, in 16-byte quads: x, y, z2, pr, pi,
+// Gamma, chi and the reference index (the sort), or the first six (the moves
+// between slot and reference order).  An array moved to or from scattered
+// places one 8-byte value at a time costs a memory transaction per value;
+// the record is one 64-byte (32-byte) transaction for all of them, and the
+// pass between records and arrays is contiguous on both sides.
+template <typename R>
+constexpr int RecordQuads = 4;          // with chi and the reference index
+template <typename R>
+constexpr int StateQuads = sizeof(R) == 8 ? 4 : 2;
+// rec[to[j]] = state of slot j
+template <typename R>
+void launch_records_scatter(const PartPtrs<R>& y, const int* to, int64_t n, uint4* rec, hipStream_t s);
+// slot j of y = rec[from[j]]
+template <typename R>
+void launch_records_gather(const uint4* rec, const int* from, int64_t n, const PartPtrs<R>& y, hipStream_t s);
+// x, y, z2, pr, pi, gam[i] = rec[i] as FP64
+template <typename R>
+void launch_records_unpack(const uint4* rec, int64_t n, double* const out[6], hipStream_t s);
+// y, chi = x, y, z2, px, py, gam, chi (FP64, the same order)
+template <typename R>
+void launch_load_state(const double* const in[7], int64_t n, const PartPtrs<R>& y, R* chi, hipStream_t s);
 
 // Lattice elements between undulator modules (puff_lattice.hip).
 enum LatticeKind { LAT_DRIFT, LAT_CHICANE, LAT_QUAD, LAT_MODULATION, LAT_CORRECT_TRANS, LAT_MATCH };
@@ -381,8 +408,10 @@ struct CopySections {
 };
 void launch_copy_sections(const CopySections& c, hipStream_t s);
 void launch_fill_zero(double* p, int64_t n, hipStream_t s);
+// a[i] = (ar, ai)[i] for i < n; from alias_from on, the values of i - alias_from
+// (the last plane of a periodic mesh; n: none).
 template <typename R>
-void launch_pack_field(const double* ar, const double* ai, cplx<R>* a, int64_t n, hipStream_t s);
+void launch_pack_field(const double* ar, const double* ai, cplx<R>* a, int64_t n, int64_t alias_from, hipStream_t s);
 template <typename R>
 void launch_unpack_field(const cplx<R>* a, double* ar, double* ai, int64_t n, hipStream_t s);
 template <typename R>
