@@ -10,7 +10,8 @@
 // Radices 2, 3, 4 and 16 have explicit butterflies (16 as 4 x 4 in
 // registers, halving the passes and barriers of power-of-two lines); any
 // other factor (11, 43, 127, ...) is a direct DFT pass; a prime line length
-// with a power-of-two n - 1 (17, 257) uses Rader's algorithm.
+// with a power-of-two n - 1 (17, 257) uses Rader's algorithm (transverse lines
+// of 257 points with their own kernels, k_rader_x and k_rader_y).
 //
 // DiffractionStep (diffraction.f90:209-348) becomes nine line passes:
 //   x fwd | y fwd | z fwd . multiplyexp . z inv | y inv |
@@ -28,14 +29,6 @@ namespace puff {
 #ifndef PUFF_Z_THREADS
 #define PUFF_Z_THREADS 256
 #endif
-// Threads per x/y workgroup on a Rader axis.  Its radix-16 sub-passes keep
-// B x 16 of them busy; with the ping-pong transform (7 lines of C4's 257
-// points, 112 busy) 128 and 192 threads measured 15 % and 7 % slower C4
-// events than 256.
-#ifndef PUFF_RADER_THREADS
-#define PUFF_RADER_THREADS 256
-#endif
-
 // LDS word of flat element e of a line-major buffer (IL false): one spare
 // slot after every 16 elements.  A radix-16 pass with p = 1 has each lane
 // write 16 consecutive outputs, so lanes write 16 elements apart, all on the
@@ -182,24 +175,21 @@ __device__ __forceinline__ void dft16(cplx<R>* v, int sign) {
 template <int N>
 struct CtPlan {
     static constexpr int np = 0;
-    static constexpr int rader = 0;
     static constexpr int r[1] = {0};
 };
-#define PUFF_CT_PLAN(N_, RADER_, ...)                         \
+#define PUFF_CT_PLAN(N_, ...)                                 \
     template <>                                               \
     struct CtPlan<N_> {                                       \
         static constexpr int r[] = {__VA_ARGS__};             \
         static constexpr int np = sizeof(r) / sizeof(int);    \
-        static constexpr int rader = RADER_;                  \
     };
-PUFF_CT_PLAN(33, 0, 11, 3)
-PUFF_CT_PLAN(129, 0, 43, 3)
-PUFF_CT_PLAN(257, 1, 16, 16)   // Rader: transforms of M = 256
-PUFF_CT_PLAN(128, 0, 16, 4, 2)
-PUFF_CT_PLAN(256, 0, 16, 16)
-PUFF_CT_PLAN(1024, 0, 16, 16, 4)
-PUFF_CT_PLAN(4096, 0, 16, 16, 16)
-PUFF_CT_PLAN(64, 0, 16, 4)   // the four-step sub-lines of 4096-point z2 lines
+PUFF_CT_PLAN(33, 11, 3)
+PUFF_CT_PLAN(129, 43, 3)
+PUFF_CT_PLAN(128, 16, 4, 2)
+PUFF_CT_PLAN(256, 16, 16)
+PUFF_CT_PLAN(1024, 16, 16, 4)
+PUFF_CT_PLAN(4096, 16, 16, 16)
+PUFF_CT_PLAN(64, 16, 4)   // the four-step sub-lines of 4096-point z2 lines
 #undef PUFF_CT_PLAN
 
 // Direct DFT pass for an odd prime r (a radix pass of lds_pass), folded:
@@ -492,10 +482,9 @@ __device__ __forceinline__ cplx<R>* ct_passes(cplx<R>* src, cplx<R>* dst, int B,
         return src;
     } else {
         constexpr int r = CtPlan<NC>::r[K];
-        constexpr int NN = CtPlan<NC>::rader ? NC - 1 : NC;   // the transform's length
-        if constexpr (r != 2 && r != 3 && r != 4 && r != 16 && !CtPlan<NC>::rader) {
+        if constexpr (r != 2 && r != 3 && r != 4 && r != 16) {
             constexpr int nq = r >= PUFF_DFT_WIDE_MIN ? PUFF_DFT_WIDE : 2;
-            direct_pass_ct<R, IL, nq, NN, r, P>(src, dst, B, tw, sign);
+            direct_pass_ct<R, IL, nq, NC, r, P>(src, dst, B, tw, sign);
         } else {
             lds_pass<R, IL>(src, dst, B, LD, N, r, P, tw, sign);
         }
@@ -504,23 +493,15 @@ __device__ __forceinline__ cplx<R>* ct_passes(cplx<R>* src, cplx<R>* dst, int B,
     }
 }
 
-// Plan NC's passes when NC > 0, else the runtime plan of ax.
-template <typename R, bool IL, int NC>
-__device__ __forceinline__ cplx<R>* plan_passes(cplx<R>* src, cplx<R>* dst, int B, int LD, int N,
-                                                const FftAxis& ax, const cplx<R>* tw, int sign) {
-    if constexpr (NC > 0) return ct_passes<R, IL, NC>(src, dst, B, LD, N, tw, sign);
-    else return lds_passes<R, IL>(src, dst, B, LD, N, ax.npass, ax.radix, tw, sign);
-}
-
 // Rader's algorithm for a prime N with N - 1 = M a power of two (FftAxis):
 // a_j = x[g^j], A = DFT_M(a), C = A . rb_s, c = IDFT_M(C) (unnormalised; rb
 // carries the 1/M), X[g^-q] = x_0 + c_q, X_0 = x_0 + A_0.  Element M of each
 // line buffer is outside the M-point transforms: it keeps x_0 in dst and
 // X_0 in src until the final permutation.
-template <typename R, bool IL, int NC>
+template <typename R, bool IL>
 __device__ __forceinline__ cplx<R>* lds_rader(cplx<R>* src, cplx<R>* dst, int B, const FftAxis& ax,
                                               const cplx<R>* tw, int sign) {
-    const int N = NC ? NC : ax.n, M = N - 1;
+    const int N = ax.n, M = N - 1;
     const cplx<R>* rb = reinterpret_cast<const cplx<R>*>(ax.rb) + (sign > 0 ? M : 0);
     cplx<R>* P = dst;   // element M: x_0
     cplx<R>* Q = src;   // element M: X_0
@@ -530,7 +511,7 @@ __device__ __forceinline__ cplx<R>* lds_rader(cplx<R>* src, cplx<R>* dst, int B,
         P[lidx<IL>(b, j, B, N)] = src[lidx<IL>(b, j < M ? ax.rperm[j] : 0, B, N)];
     }
     __syncthreads();
-    cplx<R>* res = plan_passes<R, IL, NC>(P, Q, B, N, M, ax, tw, -1);
+    cplx<R>* res = lds_passes<R, IL>(P, Q, B, N, M, ax.npass, ax.radix, tw, -1);
     for (int w = threadIdx.x; w < B * M; w += blockDim.x) {
         int b, k;
         if (IL) { b = w % B; k = w / B; } else { k = w % M; b = w / M; }
@@ -543,7 +524,7 @@ __device__ __forceinline__ cplx<R>* lds_rader(cplx<R>* src, cplx<R>* dst, int B,
     }
     __syncthreads();
     cplx<R>* other = (res == P) ? Q : P;
-    res = plan_passes<R, IL, NC>(res, other, B, N, M, ax, tw, +1);
+    res = lds_passes<R, IL>(res, other, B, N, M, ax.npass, ax.radix, tw, +1);
     cplx<R>* out = (res == P) ? Q : P;
     // every output element except element M (which holds x_0 or X_0 in out)
     const int qm = M / 2;   // g^-(M/2) = -1 = M (mod N)
@@ -708,126 +689,10 @@ template <typename R, bool IL, int NC>
 __device__ __forceinline__ cplx<R>* lds_fft(cplx<R>* src, cplx<R>* dst, int B, const FftAxis& ax,
                                             const cplx<R>* tw, int sign) {
     if constexpr (NC > 0) {
-        if constexpr (CtPlan<NC>::rader) return lds_rader<R, IL, NC>(src, dst, B, ax, tw, sign);
-        else return ct_passes<R, IL, NC>(src, dst, B, NC, NC, tw, sign);
+        return ct_passes<R, IL, NC>(src, dst, B, NC, NC, tw, sign);
     } else {
-        if (ax.rader) return lds_rader<R, IL, 0>(src, dst, B, ax, tw, sign);
+        if (ax.rader) return lds_rader<R, IL>(src, dst, B, ax, tw, sign);
         return lds_passes<R, IL>(src, dst, B, ax.n, ax.n, ax.npass, ax.radix, tw, sign);
-    }
-}
-
-// Rader's algorithm in place, for the compile-time prime lengths (257): one
-// LDS buffer of BC lines instead of two, so twice the lines per workgroup at
-// the same LDS, and the radix-16 passes of the (N - 1)-point transforms
-// keep BC x 16 threads busy.  The two permutations go through registers
-// (each thread reads its elements, the workgroup passes a barrier, the
-// elements go to their new places); X_0 = x_0 + A_0 waits in x0s[b].  The
-// permutation tables are read from LDS (rps: g^j at j < N - 1, then g^-q at
-// N + q), staged by the kernel: read from global memory, the compiler kept
-// both tables' entries in registers across the kernel (191 VGPRs).
-template <typename R, int NC>
-constexpr bool rader_ip() { return sizeof(R) == 4 && NC > 0 && CtPlan<NC>::rader; }
-
-// rps[j] = g^j (j < n - 1), rps[n + q] = g^-q (q < n - 1).
-__device__ __forceinline__ void stage_rader_perm(int* rps, const FftAxis& ax) {
-    for (int w = threadIdx.x; w < ax.n - 1; w += blockDim.x) {
-        rps[w] = ax.rperm[w];
-        rps[ax.n + w] = ax.riperm[w];
-    }
-}
-
-// The middle of the in-place Rader transform, between the permutations:
-// buf holds a_j = x[g^j] at element j < M and x_0 at element M; on return
-// element q < M holds c_q (X[g^-q] = x_0 + c_q, x_0 still at element M) and
-// x0s[b] holds X_0.
-template <typename R, bool IL, int NC, int BC>
-__device__ __forceinline__ void rader_ip_core(cplx<R>* buf, cplx<R>* x0s, const FftAxis& ax, const cplx<R>* tw,
-                                              int sign) {
-    constexpr int N = NC, M = N - 1;
-    constexpr int THR = PUFF_RADER_THREADS;
-    const cplx<R>* rb = reinterpret_cast<const cplx<R>*>(ax.rb) + (sign > 0 ? M : 0);
-    ct_passes_inplace<R, IL, M, BC, N, THR>(buf, tw, -1);
-    // C = A . rb_s (rb carries 1/M); X_0 = x_0 + A_0
-    for (int w = threadIdx.x; w < BC * M; w += THR) {
-        int b, k;
-        if (IL) { b = w % BC; k = w / BC; } else { k = w % M; b = w / M; }
-        const cplx<R> v = buf[lidx<IL>(b, k, BC, N)];
-        if (k == 0) x0s[b] = cadd(buf[lidx<IL>(b, M, BC, N)], v);
-        buf[lidx<IL>(b, k, BC, N)] = cmul(v, rb[k]);
-    }
-    __syncthreads();
-    ct_passes_inplace<R, IL, M, BC, N, THR>(buf, tw, +1);
-}
-
-template <typename R, bool IL, int NC, int BC>
-__device__ __forceinline__ void lds_rader_ip(cplx<R>* buf, cplx<R>* x0s, const int* rps, const FftAxis& ax,
-                                             const cplx<R>* tw, int sign) {
-    constexpr int N = NC, M = N - 1;
-    constexpr int THR = PUFF_RADER_THREADS;
-    constexpr int KP = (BC * N + THR - 1) / THR;   // elements per thread in a permutation
-    // a_j = x[g^j] at element j < M; x_0 to element M
-    {
-        cplx<R> v[KP];
-        const int tid = opaque_tid();
-#pragma unroll
-        for (int u = 0; u < KP; ++u) {
-            const int w = tid + u * THR;
-            int b, j;
-            if (IL) { b = w % BC; j = w / BC; } else { j = w % N; b = w / N; }
-            const bool in = w < BC * N;
-            v[u] = buf[in ? lidx<IL>(b, j < M ? rps[j] : 0, BC, N) : 0];
-        }
-        __syncthreads();
-        const int tid2 = opaque_tid();
-#pragma unroll
-        for (int u = 0; u < KP; ++u) {
-            const int w = tid2 + u * THR;
-            int b, j;
-            if (IL) { b = w % BC; j = w / BC; } else { j = w % N; b = w / N; }
-            if (w < BC * N) buf[lidx<IL>(b, j < M ? j : M, BC, N)] = v[u];
-        }
-        __syncthreads();
-    }
-    rader_ip_core<R, IL, NC, BC>(buf, x0s, ax, tw, sign);
-    // X[g^-q] = x_0 + c_q; X_0 to element 0
-    {
-        cplx<R> v[KP];
-        const int tid = opaque_tid();
-#pragma unroll
-        for (int u = 0; u < KP; ++u) {
-            const int w = tid + u * THR;
-            int b, q;
-            if (IL) { b = w % BC; q = w / BC; } else { q = w % N; b = w / N; }
-            const bool in = w < BC * N;
-            const int bb = in ? b : 0;
-            const cplx<R> c = buf[lidx<IL>(bb, q < M ? q : 0, BC, N)];
-            const cplx<R> x0 = buf[lidx<IL>(bb, M, BC, N)];
-            v[u] = q < M ? cadd(x0, c) : x0s[bb];
-        }
-        __syncthreads();
-        const int tid2 = opaque_tid();
-#pragma unroll
-        for (int u = 0; u < KP; ++u) {
-            const int w = tid2 + u * THR;
-            int b, q;
-            if (IL) { b = w % BC; q = w / BC; } else { q = w % N; b = w / N; }
-            if (w < BC * N) buf[lidx<IL>(b, q < M ? rps[N + q] : 0, BC, N)] = v[u];
-        }
-        __syncthreads();
-    }
-}
-
-// Line transform of the x / y passes: in place for rader_ip lengths (dst
-// unused; x0s holds BC values and then the permutation tables), else
-// lds_fft.  Returns the buffer holding the result.
-template <typename R, bool IL, int NC, int BC>
-__device__ __forceinline__ cplx<R>* line_fft(cplx<R>* src, cplx<R>* dst, cplx<R>* x0s, int B, const FftAxis& ax,
-                                             const cplx<R>* tw, int sign) {
-    if constexpr (rader_ip<R, NC>()) {
-        lds_rader_ip<R, IL, NC, BC>(src, x0s, reinterpret_cast<const int*>(x0s + BC), ax, tw, sign);
-        return src;
-    } else {
-        return lds_fft<R, IL, NC>(src, dst, B, ax, tw, sign);
     }
 }
 
@@ -844,6 +709,276 @@ __device__ __forceinline__ cplx<R>* z_fft(cplx<R>* src, cplx<R>* dst, int B, con
     }
 }
 
+// ---- Rader passes of 257-point transverse lines ------------------------------
+// The n-point DFT of a prime n as a cyclic convolution of M = n - 1 = 256
+// points: a_k = x[g^k], A = DFT_M(a), C = A . rb_s, c = IDFT_M(C) (rb carries
+// the 1/M), X[g^-k] = x_0 + c_k, X_0 = x_0 + A_0.
+//
+// Sixteen threads hold a line, thread u its elements u + 16 j (j = 0 .. 15) in
+// registers, and a workgroup holds BL lines.  With M = 16 x 16,
+//   A[q + 16 p] = sum_u W256^(u q) W16^(u p) sum_j a[u + 16 j] W16^(j q),
+// the transform is a 16-point DFT per thread, one exchange through LDS, and a
+// second one that leaves thread q with A[q + 16 p]; the product with rb and
+// the inverse's first 16-point DFT stay in the thread, and a second exchange
+// brings c[u + 16 j] back to thread u.  Two LDS round trips and three barriers
+// per transform, every thread busy, and the y pass moves its rows between
+// memory and registers directly (the permutation moves whole rows of BL
+// x-columns).  The x passes turn their lines through LDS in natural order, so
+// that memory sees contiguous lines, and apply masks, scalings and the kept
+// copies there.
+//
+// On 257 x 257 x 4096 (FP32) the y pass takes 0.99 ms and the x passes (forward,
+// split, recombination) 0.80, 2.25 and 1.33 ms; moving the field once takes
+// 0.89 ms at the rate of a large copy.  With the lines in LDS throughout (eight
+// per workgroup, half the threads idle in the 16-point passes, seven LDS round
+// trips per transform) they took 1.55 and 1.54, 3.31 and 1.80 ms.
+constexpr int RAD_N = 257, RAD_M = 256;
+constexpr int RAD_LD = 272;   // LDS elements of a line: 256 + 256 / 16, see rad_at
+
+// Lines per workgroup: 35 KiB of LDS in either form, four workgroups per CU.
+template <typename R>
+constexpr int rad_lines() { return sizeof(R) == 8 ? 8 : 16; }
+
+constexpr int rad_pow(int b, int e) {
+    int r = 1;
+    for (; e > 0; --e) r = r * b % RAD_N;
+    return r;
+}
+// g^(16 j) for j < 16; inverse powers with b = g^-1
+template <int B>
+struct RadPowers {
+    int v[16];
+    constexpr RadPowers() : v() {
+        for (int j = 0; j < 16; ++j) v[j] = rad_pow(B, 16 * j);
+    }
+};
+constexpr int RAD_G = 3;                                 // the host's generator of 257 (make_axis)
+constexpr int RAD_GI = rad_pow(RAD_G, RAD_M - 1);        // its inverse
+static_assert(rad_pow(RAD_G, RAD_M / 2) == RAD_N - 1 && RAD_G * RAD_GI % RAD_N == 1, "primitive root of 257");
+
+// x mod 257 for 0 <= x <= 65536: 256 = -1, so the low byte less the rest, and
+// the wrapped one of r and r + 257 is the larger as unsigned.
+__device__ __forceinline__ int rad_mod(int x) {
+    const unsigned r = (unsigned)(x & 255) - (unsigned)(x >> 8);
+    return (int)min(r, r + 257u);
+}
+
+// b^u mod 257 for u < 16.
+template <int B>
+__device__ __forceinline__ int rad_pow16(int u) {
+    constexpr int b2 = rad_pow(B, 2), b4 = rad_pow(B, 4), b8 = rad_pow(B, 8);
+    int r = (u & 1) ? B : 1;
+    r = rad_mod(r * ((u & 2) ? b2 : 1));
+    r = rad_mod(r * ((u & 4) ? b4 : 1));
+    return rad_mod(r * ((u & 8) ? b8 : 1));
+}
+
+// LDS element e of line b.  XL (x lines: the 16 threads of a line
+// consecutive): line-major, a spare element after every 16, so that a wave's
+// writes (16 consecutive elements of four lines) and reads (elements 16
+// apart) each touch every bank once.  Otherwise (y: the BL columns of an
+// element consecutive) rows of BL with a spare row after every 16.
+template <int BL, bool XL>
+__device__ __forceinline__ int rad_at(int b, int e) {
+    return XL ? b * RAD_LD + e + (e >> 4) : (e + (e >> 4)) * BL + b;
+}
+
+// Index of X_k in dft16's output.
+__host__ __device__ constexpr int dft16_at(int k) { return 4 * (k & 3) + (k >> 2); }
+
+// v[j] = a[u + 16 j] -> v[j] = c[u + 16 j]; returns A_0 (in thread u = 0).
+// rb: the table of the transform's sign (global memory, L2).  The buffer may
+// be in use when called; every thread has passed a barrier after its last
+// read of it, except of its own elements u + 16 j, on return.
+template <typename R, int BL, bool XL>
+__device__ __forceinline__ cplx<R> rader_core(cplx<R> (&v)[16], int b, int u, cplx<R>* buf, const cplx<R>* tw,
+                                              const cplx<R>* rb) {
+    dft16(v, -1);
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+        const cplx<R> y = q ? cmul(v[dft16_at(q)], tw[u * q]) : v[0];
+        buf[rad_at<BL, XL>(b, q * 16 + u)] = y;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < 16; ++t) v[t] = buf[rad_at<BL, XL>(b, u * 16 + t)];
+    dft16(v, -1);
+    const cplx<R> a0 = v[0];
+    cplx<R> c[16];
+#pragma unroll
+    for (int p = 0; p < 16; ++p) c[p] = cmul(v[dft16_at(p)], rb[u + 16 * p]);
+    dft16(c, +1);
+    // back to the elements this thread read: no barrier before the writes
+#pragma unroll
+    for (int t = 0; t < 16; ++t) {
+        const cplx<R> y = t ? cmul(c[dft16_at(t)], tw_get(tw, u * t, +1)) : c[0];
+        buf[rad_at<BL, XL>(b, u * 16 + t)] = y;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 16; ++q) c[q] = buf[rad_at<BL, XL>(b, q * 16 + u)];
+    dft16(c, +1);
+#pragma unroll
+    for (int j = 0; j < 16; ++j) v[j] = c[dft16_at(j)];
+    return a0;
+}
+
+template <typename R>
+__global__ __launch_bounds__(16 * rad_lines<R>()) void k_rader_y(DiffArgs<R> a, int sign) {
+    constexpr int BL = rad_lines<R>();
+    __shared__ cplx<R> buf[RAD_LD * BL];
+    __shared__ cplx<R> tw[RAD_M];
+    const int b = (int)threadIdx.x % BL, u = (int)threadIdx.x / BL;
+    // blocks of BL x-columns, x fastest; neighbouring blocks share the cache
+    // lines at their edges, so they go to one XCD
+    const int nxb = (a.nx + BL - 1) / BL;
+    const int64_t blk = xcd_block((int64_t)nxb * a.nzp);
+    if (blk >= (int64_t)nxb * a.nzp) return;
+    const int x = (int)(blk % nxb) * BL + b;
+    const bool in = x < a.nx;
+    cplx<R>* col = a.a + (blk / nxb) * (int64_t)a.nx * RAD_N + x;
+    const cplx<R>* twg = reinterpret_cast<const cplx<R>*>(a.ay.tw);
+    const cplx<R>* rb = reinterpret_cast<const cplx<R>*>(a.ay.rb) + (sign > 0 ? RAD_M : 0);
+    constexpr RadPowers<RAD_G> GP;
+    constexpr RadPowers<RAD_GI> GI;
+    cplx<R> v[16];
+    const int gu = rad_pow16<RAD_G>(u);
+#pragma unroll
+    for (int j = 0; j < 16; ++j)
+        v[j] = in ? col[rad_mod(gu * GP.v[j]) * a.nx] : cplx<R>{0, 0};
+    const cplx<R> x0 = in ? col[0] : cplx<R>{0, 0};
+    for (int w = threadIdx.x; w < RAD_M; w += 16 * BL) tw[w] = twg[w];
+    const cplx<R> a0 = rader_core<R, BL, false>(v, b, u, buf, tw, rb);
+    if (!in) return;
+    const int hu = rad_pow16<RAD_GI>(u);
+#pragma unroll
+    for (int j = 0; j < 16; ++j) col[rad_mod(hu * GI.v[j]) * a.nx] = cadd(x0, v[j]);
+    if (u == 0) col[0] = cadd(x0, a0);
+}
+
+// The DFT of the BL lines held in natural order in buf (element x of line b at
+// b * RAD_LD + x), back in natural order.  Starts and ends with a barrier.
+template <typename R, int BL>
+__device__ __forceinline__ void rader_natural(int b, int u, cplx<R>* buf, const cplx<R>* tw, const cplx<R>* rb) {
+    constexpr RadPowers<RAD_G> GP;
+    constexpr RadPowers<RAD_GI> GI;
+    cplx<R>* line = buf + b * RAD_LD;
+    __syncthreads();
+    cplx<R> v[16];
+    const int gu = rad_pow16<RAD_G>(u);
+#pragma unroll
+    for (int j = 0; j < 16; ++j) v[j] = line[rad_mod(gu * GP.v[j])];
+    const cplx<R> x0 = line[0];
+    const cplx<R> a0 = rader_core<R, BL, true>(v, b, u, buf, tw, rb);
+    __syncthreads();
+    const int hu = rad_pow16<RAD_GI>(u);
+#pragma unroll
+    for (int j = 0; j < 16; ++j) line[rad_mod(hu * GI.v[j])] = cadd(x0, v[j]);
+    if (u == 0) line[0] = cadd(x0, a0);
+    __syncthreads();
+}
+
+// x lines of 257 points, OP an XOP_ value as in k_fft_x.
+template <typename R, int OP>
+__global__ __launch_bounds__(16 * rad_lines<R>()) void k_rader_x(DiffArgs<R> a, int sign) {
+    constexpr int BL = rad_lines<R>();
+    constexpr int T = 16 * BL;
+    constexpr int KE = 17;   // elements per thread: 16, and one more for the first BL threads
+    __shared__ cplx<R> buf[RAD_LD * BL];
+    __shared__ cplx<R> tw[RAD_M];
+    const int b = (int)threadIdx.x / 16, u = (int)threadIdx.x % 16;
+    const int64_t L0 = (int64_t)blockIdx.x * BL;
+    const int nb = (int)min<int64_t>(BL, (int64_t)a.ny * a.nzp - L0);
+    cplx<R>* base = a.a + L0 * RAD_N;
+    cplx<R>* keep = a.anb + L0 * RAD_N;
+    const cplx<R>* twg = reinterpret_cast<const cplx<R>*>(a.ax.tw);
+    const cplx<R>* rbg = reinterpret_cast<const cplx<R>*>(a.ax.rb);
+    const int64_t alias = (int64_t)(a.nz2 - 1) * a.nx * a.ny;   // the last plane of a periodic mesh
+    const double rff = 1.0 / a.ffact;
+    // the backward transform's 1/ffact: a divide in FP64 (the reference's
+    // arithmetic), a reciprocal multiply in the mixed form
+    auto unscale = [&](R s) -> double {
+        if constexpr (sizeof(R) == 8) return (double)s / a.ffact;
+        else return (double)s * rff;
+    };
+    // f(k, w, lb, x) for the thread's elements w = x + 257 lb of the block's lines
+    auto each = [&](auto f) {
+#pragma unroll
+        for (int k = 0; k < KE; ++k) {
+            const int w = (int)threadIdx.x + k * T;
+            const int lb = w / RAD_N;
+            if (w < nb * RAD_N) f(k, w, lb, w - lb * RAD_N);
+        }
+    };
+    // mask of element x of line lb
+    const int iy0 = (int)(L0 % a.ny), iz0 = (int)(L0 / a.ny);
+    auto mask = [&](int lb, int x) {
+        const int l = iy0 + lb;
+        const double mxy = a.mxy[(int64_t)(l % a.ny) * a.nx + x];
+        return mxy + (a.mz[iz0 + l / a.ny] * (1.0 - mxy));
+    };
+    cplx<R> in[KE];
+#pragma unroll
+    for (int k = 0; k < KE; ++k) in[k] = cplx<R>{0, 0};
+    each([&](int k, int w, int, int) { in[k] = base[w]; });
+    for (int w = threadIdx.x; w < RAD_M; w += T) tw[w] = twg[w];
+    if constexpr (OP == XOP_ADJ_FOLD_SAVE_FWD) {
+        each([&](int k, int w, int lb, int x) {
+            const int64_t L = L0 + lb;
+            if (a.periodic && L < a.ny) {
+                // the output's aliased plane copies plane 1: fold its cotangent
+                cplx<R>* al = a.a + alias + L * RAD_N + x;
+                in[k] = cadd(in[k], *al);
+                *al = cplx<R>{0, 0};
+            }
+            keep[w] = in[k];
+        });
+    }
+#pragma unroll
+    for (int k = 0; k < KE; ++k) {   // zeros on lines past the end
+        const int w = (int)threadIdx.x + k * T;
+        if (w < BL * RAD_N) buf[(w / RAD_N) * RAD_LD + w % RAD_N] = in[k];
+    }
+    const int s1 = OP == XOP_FORWARD ? sign : (OP == XOP_ADJ_FOLD_SAVE_FWD ? -1 : +1);
+    rader_natural<R, BL>(b, u, buf, tw, rbg + (s1 > 0 ? RAD_M : 0));
+    // the kept copy, all loads before the first use (held across the
+    // transform it cost 40 to 90 registers, one to two waves per SIMD)
+    cplx<R> kept[OP == XOP_INV_RECOMBINE || OP == XOP_ADJ_INV_MIX_FWD ? KE : 1];
+    if constexpr (OP == XOP_INV_RECOMBINE || OP == XOP_ADJ_INV_MIX_FWD)
+        each([&](int k, int w, int, int) { kept[k] = keep[w]; });
+    if constexpr (OP == XOP_INV_SPLIT_FWD || OP == XOP_ADJ_INV_MIX_FWD) {
+        each([&](int k, int w, int lb, int x) {
+            cplx<R>* e = buf + lb * RAD_LD + x;
+            const double m = mask(lb, x);
+            const double vr = unscale(e->x), vi = unscale(e->y);
+            if constexpr (OP == XOP_INV_SPLIT_FWD) {
+                // /ffact then AbsorptionStep's split (diffraction.f90:310, 454-470)
+                keep[w] = {(R)((1.0 - m) * vr), (R)((1.0 - m) * vi)};
+                *e = {(R)(m * vr), (R)(m * vi)};
+            } else {
+                // adjoint of the split: (1 - m) cotangent + m W^H G W cotangent / ffact
+                *e = {(R)((1.0 - m) * (double)kept[k].x + m * vr), (R)((1.0 - m) * (double)kept[k].y + m * vi)};
+            }
+        });
+        rader_natural<R, BL>(b, u, buf, tw, rbg);
+    }
+    each([&](int k, int w, int lb, int x) {
+        cplx<R> v = buf[lb * RAD_LD + x];
+        if constexpr (OP == XOP_INV_RECOMBINE) {
+            // /ffact + interior (diffraction.f90:513-517)
+            if constexpr (sizeof(R) == 8) v = {unscale(v.x) + kept[k].x, unscale(v.y) + kept[k].y};
+            else v = {(R)unscale(v.x) + kept[k].x, (R)unscale(v.y) + kept[k].y};
+            // keep the aliased plane NZ2 equal to plane 1 (para_field.f90:3197-3244)
+            const int64_t L = L0 + lb;
+            if (a.periodic && L < a.ny) a.a[alias + L * RAD_N + x] = v;
+        } else if constexpr (OP == XOP_ADJ_INV_SCALE) {
+            v = {(R)unscale(v.x), (R)unscale(v.y)};
+        }
+        base[w] = v;
+    });
+}
+
 // ---- x lines (contiguous) --------------------------------------------------
 // OP (an XOP_ value) is a template parameter: each fused operation gets its
 // own register allocation.
@@ -855,120 +990,19 @@ __global__ __launch_bounds__(256) void k_fft_x(DiffArgs<R> a, int Bp, int sign) 
     const int B = BC ? BC : Bp;
     const FftAxis& ax = a.ax;
     cplx<R>* s0 = reinterpret_cast<cplx<R>*>(smem_raw);
-    cplx<R>* s1 = rader_ip<R, NC>() ? s0 : s0 + lpad<false>(B * N);
+    cplx<R>* s1 = s0 + lpad<false>(B * N);
     const int64_t nlines = (int64_t)a.ny * a.nzp;
     const int64_t L0 = (int64_t)blockIdx.x * B;
     const int nb = (int)min<int64_t>(B, nlines - L0);
     const cplx<R>* twg = reinterpret_cast<const cplx<R>*>(ax.tw);
     cplx<R>* tw = s1 + lpad<false>(B * N);   // twiddle table staged in LDS
-    cplx<R>* x0s = tw + N;            // in-place Rader's X_0 per line and permutations
     for (int w = threadIdx.x; w < N; w += blockDim.x) tw[w] = twg[w];
-    if constexpr (rader_ip<R, NC>()) stage_rader_perm(reinterpret_cast<int*>(x0s + B), ax);
     cplx<R>* base = a.a + L0 * N;
     const int64_t ntr = (int64_t)a.nx * a.ny;
     // plane and row of the block's first line; line L0 + b is row iy0 + b
     // counted on from there (b < B)
     const int iy0 = (int)(L0 % a.ny), iz0 = (int)(L0 / a.ny);
     const double rff = 1.0 / a.ffact;
-    if constexpr (rader_ip<R, NC>() && (OP == XOP_FORWARD || OP == XOP_INV_SPLIT_FWD || OP == XOP_INV_RECOMBINE)) {
-        // Rader's permutations folded into the global reads and writes (as
-        // in the y pass; here they scatter within each line's 2 KB): the
-        // input permutation into the loads, the output permutation into the
-        // stores, and for the split, the inverse transform's output
-        // permutation and the forward transform's input permutation into
-        // one move within LDS (natural index g^-q = g^(M - q): element q
-        // goes to element (M - q) mod M, X_0 to element M)
-        constexpr int M = NC - 1;
-        constexpr int THR = PUFF_RADER_THREADS;
-        constexpr int KP = (BC * NC + THR - 1) / THR;
-        const int* rps = reinterpret_cast<const int*>(x0s + BC);
-        __syncthreads();   // rps staged
-        // the recombination's interior part, read with the lines (read in
-        // the final loop, each load waits on the memory latency there)
-        cplx<R> anbp[OP == XOP_INV_RECOMBINE ? KP : 1];
-        if constexpr (OP == XOP_INV_RECOMBINE) {
-            const int tid = opaque_tid();
-#pragma unroll
-            for (int u = 0; u < KP; ++u) {
-                const int w = tid + u * THR;
-                const int ww = w < BC * NC ? w : 0;
-                const int b = ww / NC, q = ww % NC;
-                const int n = q < M ? rps[NC + q] : 0;
-                anbp[u] = (w < BC * NC && b < nb) ? a.anb[(L0 + b) * N + n] : cplx<R>{0, 0};
-            }
-        }
-        lds_fill<false, STAGE_UNROLL>(s0, BC * NC, [&](int w) {
-            const int b = w / NC, k = w % NC;
-            const int j = k < M ? rps[k] : 0;   // element k < M: x[g^k]; element M: x_0
-            return b < nb ? base[b * NC + j] : cplx<R>{0, 0};
-        });
-        __syncthreads();
-        rader_ip_core<R, false, NC, BC>(s0, x0s, ax, tw, OP == XOP_FORWARD ? sign : +1);
-        if constexpr (OP == XOP_INV_SPLIT_FWD) {
-            // /ffact then AbsorptionStep's split (diffraction.f90:310, 454-470)
-            cplx<R>* anb = a.anb + L0 * N;
-            cplx<R> v[KP];
-            int e[KP];
-            const int tid = opaque_tid();
-#pragma unroll
-            for (int u = 0; u < KP; ++u) {
-                const int w = tid + u * THR;
-                const int ww = w < BC * NC ? w : 0;
-                const int b = ww / NC, q = ww % NC;
-                const cplx<R> c = s0[lidx<false>(b, q < M ? q : 0, BC, NC)];
-                const cplx<R> xz = s0[lidx<false>(b, M, BC, NC)];
-                const cplx<R> x = q < M ? cadd(xz, c) : x0s[b];   // X[g^-q] = x_0 + c_q; X_0
-                const int n = q < M ? rps[NC + q] : 0;
-                e[u] = lidx<false>(b, q < M ? (q ? M - q : 0) : M, BC, NC);
-                const int lb = iy0 + b;   // (iy, iz) of line L0 + b
-                const int iy = lb % a.ny, iz = iz0 + lb / a.ny;
-                const bool st = w < BC * NC && b < nb;
-                const double mxy = st ? a.mxy[(int64_t)iy * a.nx + n] : 0.0;
-                const double m = mxy + ((st ? a.mz[iz] : 0.0) * (1.0 - mxy));
-                const double vr = (double)x.x * rff, vi = (double)x.y * rff;
-                if (st) anb[b * NC + n] = {(R)((1.0 - m) * vr), (R)((1.0 - m) * vi)};
-                v[u] = {(R)(m * vr), (R)(m * vi)};
-            }
-            __syncthreads();
-#pragma unroll
-            for (int u = 0; u < KP; ++u)
-                if (tid + u * THR < BC * NC) s0[e[u]] = v[u];
-            __syncthreads();
-            rader_ip_core<R, false, NC, BC>(s0, x0s, ax, tw, -1);
-        }
-        {
-            cplx<R> v[KP];
-            int n[KP];
-            const int tid = opaque_tid();
-#pragma unroll
-            for (int u = 0; u < KP; ++u) {
-                const int w = tid + u * THR;
-                const int ww = w < BC * NC ? w : 0;
-                const int b = ww / NC, q = ww % NC;
-                const cplx<R> c = s0[lidx<false>(b, q < M ? q : 0, BC, NC)];
-                const cplx<R> xz = s0[lidx<false>(b, M, BC, NC)];
-                v[u] = q < M ? cadd(xz, c) : x0s[b];   // X[g^-q] = x_0 + c_q; X_0
-                n[u] = q < M ? rps[NC + q] : 0;
-            }
-#pragma unroll
-            for (int u = 0; u < KP; ++u) {
-                const int w = tid + u * THR;
-                const int b = w / NC;
-                if (w >= BC * NC || b >= nb) continue;
-                cplx<R> x = v[u];
-                if constexpr (OP == XOP_INV_RECOMBINE) {
-                    // /ffact + interior (diffraction.f90:513-517)
-                    const cplx<R> qn = anbp[u];
-                    x = {(R)((double)x.x * rff) + qn.x, (R)((double)x.y * rff) + qn.y};
-                    // keep the aliased plane NZ2 equal to plane 1 (para_field.f90:3197-3244)
-                    const int64_t L = L0 + b;
-                    if (a.periodic && L < a.ny) a.a[(int64_t)(a.nz2 - 1) * ntr + L * N + n[u]] = x;
-                }
-                base[b * NC + n[u]] = x;
-            }
-        }
-        return;
-    }
     if (op == XOP_ADJ_FOLD_SAVE_FWD) {
         for (int w = threadIdx.x; w < B * N; w += blockDim.x) {
             const int b = w / N;
@@ -999,7 +1033,7 @@ __global__ __launch_bounds__(256) void k_fft_x(DiffArgs<R> a, int Bp, int sign) 
         if constexpr (sizeof(R) == 8) return (double)v / a.ffact;
         else return (double)v * rff;
     };
-    cplx<R>* res = line_fft<R, false, NC, BC>(s0, s1, x0s, B, ax, tw, first_sign);
+    cplx<R>* res = lds_fft<R, false, NC>(s0, s1, B, ax, tw, first_sign);
     if (op == XOP_ADJ_INV_MIX_FWD) {
         // adjoint of the absorption split: (1 - m) cotangent + m W^H G W cotangent / ffact
         const cplx<R>* lam = a.anb + L0 * N;
@@ -1016,7 +1050,7 @@ __global__ __launch_bounds__(256) void k_fft_x(DiffArgs<R> a, int Bp, int sign) 
         }
         __syncthreads();
         cplx<R>* other = (res == s0) ? s1 : s0;
-        res = line_fft<R, false, NC, BC>(res, other, x0s, B, ax, tw, -1);
+        res = lds_fft<R, false, NC>(res, other, B, ax, tw, -1);
     } else if (op == XOP_ADJ_INV_SCALE) {
         for (int w = threadIdx.x; w < nb * N; w += blockDim.x) {
             const cplx<R> v = res[lpad<false>(w)];
@@ -1039,7 +1073,7 @@ __global__ __launch_bounds__(256) void k_fft_x(DiffArgs<R> a, int Bp, int sign) 
         }
         __syncthreads();
         cplx<R>* other = (res == s0) ? s1 : s0;
-        res = line_fft<R, false, NC, BC>(res, other, x0s, B, ax, tw, -1);
+        res = lds_fft<R, false, NC>(res, other, B, ax, tw, -1);
     } else if (op == XOP_INV_RECOMBINE) {
         // /ffact + interior (diffraction.f90:513-517)
         const cplx<R>* anb = a.anb + L0 * N;
@@ -1064,34 +1098,6 @@ __global__ __launch_bounds__(256) void k_fft_x(DiffArgs<R> a, int Bp, int sign) 
     }
 }
 
-// ---- persistent tile loops -----------------------------------------------------
-// With compile-time plans the x and y passes run persistent workgroups (as
-// many as fit the device at once): each loops over its tiles of B lines,
-// loading tile t + stride into registers while tile t is transformed in LDS
-// and stored.  A one-tile workgroup has its loads in flight only between
-// its start and its first barrier; here they overlap the transform and the
-// stores of the previous tile.  The tiles are dealt to the XCDs in
-// contiguous ranges (workgroup g runs on XCD g mod 8, the grid being a
-// multiple of 8), so that neighbouring tiles, which share cache lines at
-// their edges, meet in one L2.
-// Off by default: on the C1 and C4 meshes the persistent y pass measured
-// 1-2 % slower events than one tile per workgroup (its prefetch registers
-// cost a wave per SIMD of occupancy).
-#ifndef PUFF_PERSIST_Y
-#define PUFF_PERSIST_Y 0
-#endif
-struct TileRange {
-    int64_t t, end;
-    int stride;
-};
-__device__ __forceinline__ TileRange tile_range(int64_t ntile) {
-    const int per_xcd = (int)gridDim.x / NXCD;
-    const int xcd = (int)blockIdx.x % NXCD, l = (int)blockIdx.x / NXCD;
-    const int64_t per = (ntile + NXCD - 1) / NXCD;
-    const int64_t lo = xcd * per;
-    return {lo + l, min(lo + per, ntile), per_xcd};
-}
-
 // ---- y lines (stride nx), B consecutive x per block -------------------------
 template <typename R, int NC, int BC>
 __global__ __launch_bounds__(256) void k_fft_y(DiffArgs<R> a, int Bp, int sign) {
@@ -1100,104 +1106,25 @@ __global__ __launch_bounds__(256) void k_fft_y(DiffArgs<R> a, int Bp, int sign) 
     const int B = BC ? BC : Bp;
     const FftAxis& ay = a.ay;
     cplx<R>* s0 = reinterpret_cast<cplx<R>*>(smem_raw);
-    cplx<R>* s1 = rader_ip<R, NC>() ? s0 : s0 + lpad<true>(B * N);
+    cplx<R>* s1 = s0 + lpad<true>(B * N);
     // blocks of B x-columns, x fastest; neighbouring blocks share the cache
     // lines at their edges, so they go to one XCD
     const int nxb = (a.nx + B - 1) / B;
-    constexpr bool persist = NC > 0 && PUFF_PERSIST_Y;
-    const int64_t blk = persist ? 0 : xcd_block((int64_t)nxb * a.nzp);
+    const int64_t blk = xcd_block((int64_t)nxb * a.nzp);
     if (blk >= (int64_t)nxb * a.nzp) return;
     const int x0 = (int)(blk % nxb) * B;
     const int iz = (int)(blk / nxb);
     const int nb = min(B, a.nx - x0);
     const cplx<R>* twg = reinterpret_cast<const cplx<R>*>(ay.tw);
     cplx<R>* tw = s1 + lpad<true>(B * N);   // twiddle table staged in LDS
-    cplx<R>* x0s = tw + N;            // in-place Rader's X_0 per line and permutations
     for (int w = threadIdx.x; w < N; w += blockDim.x) tw[w] = twg[w];
-    if constexpr (rader_ip<R, NC>()) stage_rader_perm(reinterpret_cast<int*>(x0s + B), ay);
-    if constexpr (persist) {
-        // persistent: tiles of B x-columns of one plane, x fastest
-        static_assert(PUFF_RADER_THREADS == 256, "the tile loop assumes 256 threads");
-        constexpr int U = (BC * NC + 255) / 256;   // elements per thread (256 threads)
-        const int64_t ntile = (int64_t)nxb * a.nzp;
-        const TileRange tr = tile_range(ntile);
-        cplx<R> v[U];
-        auto load = [&](int64_t t) {
-            const int tx0 = (int)(t % nxb) * BC, tz = (int)(t / nxb);
-            const int tnb = min(BC, a.nx - tx0);
-            const cplx<R>* tb = a.a + (int64_t)tz * a.nx * a.ny + tx0;
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int w = (int)threadIdx.x + u * 256;
-                const int b = w % BC, j = w / BC;
-                v[u] = (w < BC * NC && b < tnb) ? tb[(int64_t)j * a.nx + b] : cplx<R>{0, 0};
-            }
-        };
-        if (tr.t < tr.end) load(tr.t);
-        for (int64_t t = tr.t; t < tr.end; t += tr.stride) {
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int w = (int)threadIdx.x + u * 256;
-                if (w < BC * NC) s0[lpad<true>(w)] = v[u];
-            }
-            __syncthreads();
-            if (t + tr.stride < tr.end) load(t + tr.stride);
-            cplx<R>* res = line_fft<R, true, NC, BC>(s0, s1, x0s, BC, ay, tw, sign);
-            const int tx0 = (int)(t % nxb) * BC, tz = (int)(t / nxb);
-            const int tnb = min(BC, a.nx - tx0);
-            cplx<R>* tb = a.a + (int64_t)tz * a.nx * a.ny + tx0;
-            lds_drain<true, STAGE_UNROLL>(res, BC * NC, [&](int w, const cplx<R>& vv) {
-                const int b = w % BC, j = w / BC;
-                if (b < tnb) tb[(int64_t)j * a.nx + b] = vv;
-            });
-            __syncthreads();
-        }
-        return;
-    }
     cplx<R>* base = a.a + (int64_t)iz * a.nx * a.ny + x0;
-    if constexpr (rader_ip<R, NC>()) {
-        // Rader's permutations folded into the global reads and writes: the
-        // permutation moves whole rows of B x-columns, so the accesses stay
-        // as contiguous as the plain ones, and the transform saves two LDS
-        // round trips and their barriers
-        constexpr int M = NC - 1;
-        const int* rps = reinterpret_cast<const int*>(x0s + BC);
-        __syncthreads();   // rps staged
-        lds_fill<true, STAGE_UNROLL>(s0, BC * NC, [&](int w) {
-            const int b = w % BC, k = w / BC;
-            const int j = k < M ? rps[k] : 0;   // element k < M: x[g^k]; element M: x_0
-            return (b < nb) ? base[(int64_t)j * a.nx + b] : cplx<R>{0, 0};
-        });
-        __syncthreads();
-        rader_ip_core<R, true, NC, BC>(s0, x0s, ay, tw, sign);
-        for (int w0 = threadIdx.x; w0 < BC * NC; w0 += STAGE_UNROLL * (int)blockDim.x) {
-            cplx<R> v[STAGE_UNROLL];
-            int j[STAGE_UNROLL];
-#pragma unroll
-            for (int u = 0; u < STAGE_UNROLL; ++u) {
-                const int w = w0 + u * (int)blockDim.x;
-                const int ww = w < BC * NC ? w : 0;
-                const int b = ww % BC, q = ww / BC;
-                const cplx<R> c = s0[lidx<true>(b, q < M ? q : 0, BC, NC)];
-                const cplx<R> xz = s0[lidx<true>(b, M, BC, NC)];
-                v[u] = q < M ? cadd(xz, c) : x0s[b];   // X[g^-q] = x_0 + c_q; X_0
-                j[u] = q < M ? rps[NC + q] : 0;
-            }
-#pragma unroll
-            for (int u = 0; u < STAGE_UNROLL; ++u) {
-                const int w = w0 + u * (int)blockDim.x;
-                const int b = w % BC;
-                if (w < BC * NC && b < nb) base[(int64_t)j[u] * a.nx + b] = v[u];
-            }
-        }
-        return;
-    }
     lds_fill<true, STAGE_UNROLL>(s0, B * N, [&](int w) {
         const int b = w % B, j = w / B;
         return (b < nb) ? base[(int64_t)j * a.nx + b] : cplx<R>{0, 0};
     });
     __syncthreads();
-    cplx<R>* res = line_fft<R, true, NC, BC>(s0, s1, x0s, B, ay, tw, sign);
+    cplx<R>* res = lds_fft<R, true, NC>(s0, s1, B, ay, tw, sign);
     lds_drain<true, STAGE_UNROLL>(res, B * N, [&](int w, const cplx<R>& v) {
         const int b = w % B, j = w / B;
         if (b < nb) base[(int64_t)j * a.nx + b] = v;
@@ -1499,41 +1426,16 @@ static constexpr ZPlan z_plan(int n, size_t elem, bool rader, int npass, const i
     return ZPlan{B, inplace};
 }
 
-// Lines per workgroup of the in-place Rader passes: one line buffer, the
-// twiddle table, X_0 and the permutation tables within `budget`; at most 16
-// lines (one butterfly per thread in the radix-16 passes).  22 KiB (8 of
-// C4's 257-point FP32 lines, 7 workgroups per CU) measured 20.7 ms per C4
-// event against 21.7 (18 KiB, 6 lines), 21.6 (26 KiB, 10 lines) and 22.1
-// (40 KiB, 16 lines).
-#ifndef PUFF_RADER_LDS_BUDGET
-#define PUFF_RADER_LDS_BUDGET (22 * 1024)
-#endif
-static constexpr int lines_per_block_ip(int n, size_t elem, bool il, size_t budget = PUFF_RADER_LDS_BUDGET) {
-    int b = 16;
-    while (b > 1 && ((size_t)(il ? lpad<true>(b * n) : lpad<false>(b * n)) + n + b) * elem +
-                            2 * n * sizeof(int) > budget)
-        --b;
-    return b;
-}
-template <typename R, int NC, bool IL>
-static constexpr size_t xy_lds_elems(int B) {
-    // in-place Rader: line buffer, twiddles, X_0 per line, two int tables of NC
-    return rader_ip<R, NC>() ? (size_t)lpad<IL>(B * NC) + NC + B +
-                                   (2 * NC * sizeof(int) + sizeof(cplx<R>) - 1) / sizeof(cplx<R>)
-                             : 2 * (size_t)lpad<IL>(B * NC) + NC;
-}
-template <typename R, int NC>
-static constexpr int ct_lines_x() {
-    return rader_ip<R, NC>() ? lines_per_block_ip(NC, sizeof(cplx<R>), false)
-                             : lines_per_block(NC, sizeof(cplx<R>), 64, PUFF_XY_LDS_BUDGET, false);
-}
 #ifndef PUFF_Y_LDS_BUDGET
 #define PUFF_Y_LDS_BUDGET PUFF_XY_LDS_BUDGET
 #endif
 template <typename R, int NC>
+static constexpr int ct_lines_x() {
+    return lines_per_block(NC, sizeof(cplx<R>), 64, PUFF_XY_LDS_BUDGET, false);
+}
+template <typename R, int NC>
 static constexpr int ct_lines_y() {
-    return rader_ip<R, NC>() ? lines_per_block_ip(NC, sizeof(cplx<R>), true)
-                             : lines_per_block(NC, sizeof(cplx<R>), 16, PUFF_Y_LDS_BUDGET, true);
+    return lines_per_block(NC, sizeof(cplx<R>), 16, PUFF_Y_LDS_BUDGET, true);
 }
 // Compile-time plans may give a thread several butterflies of an in-place
 // pass (inplace_pass<KB>), up to Z_MAX_HELD complex values per thread
@@ -1542,7 +1444,7 @@ template <typename R>
 constexpr int z_max_held() { return sizeof(R) == 8 ? 16 : 32; }
 template <typename R, int NC>
 static constexpr ZPlan ct_zplan() {
-    bool inplace = !CtPlan<NC>::rader;
+    bool inplace = true;
     for (int k = 0; k < CtPlan<NC>::np; ++k) {
         const int r = CtPlan<NC>::r[k];
         if (r != 2 && r != 3 && r != 4 && r != 16) inplace = false;
@@ -1568,12 +1470,29 @@ static constexpr ZPlan ct_zplan() {
 template <typename R, int NC, int BC, int OP>
 static void launch_x_op(const DiffArgs<R>& a, int B, int sign, hipStream_t s) {
     const int64_t nlines = (int64_t)a.ny * a.nzp;
-    const size_t sh = (NC ? xy_lds_elems<R, NC, false>(B) : 2 * (size_t)lpad<false>(B * a.nx) + a.nx) *
-                      sizeof(cplx<R>);
+    const size_t sh = (2 * (size_t)lpad<false>(B * a.nx) + a.nx) * sizeof(cplx<R>);
     lds_opt_in(reinterpret_cast<const void*>(&k_fft_x<R, NC, BC, OP>), sh);
-    const int thr = a.ax.rader ? PUFF_RADER_THREADS : 256;
-    hipLaunchKernelGGL((k_fft_x<R, NC, BC, OP>), dim3((unsigned)((nlines + B - 1) / B)), dim3(thr), sh, s, a, B,
+    hipLaunchKernelGGL((k_fft_x<R, NC, BC, OP>), dim3((unsigned)((nlines + B - 1) / B)), dim3(256), sh, s, a, B,
                        sign);
+}
+
+template <typename R, int OP>
+static void launch_rader_x(const DiffArgs<R>& a, int sign, hipStream_t s) {
+    constexpr int BL = rad_lines<R>();
+    const int64_t nlines = (int64_t)a.ny * a.nzp;
+    hipLaunchKernelGGL((k_rader_x<R, OP>), dim3((unsigned)((nlines + BL - 1) / BL)), dim3(16 * BL), 0, s, a, sign);
+}
+
+template <typename R>
+static void run_rader_x(const DiffArgs<R>& a, int op, int sign, hipStream_t s) {
+    switch (op) {
+        case XOP_FORWARD: return launch_rader_x<R, XOP_FORWARD>(a, sign, s);
+        case XOP_INV_SPLIT_FWD: return launch_rader_x<R, XOP_INV_SPLIT_FWD>(a, sign, s);
+        case XOP_INV_RECOMBINE: return launch_rader_x<R, XOP_INV_RECOMBINE>(a, sign, s);
+        case XOP_ADJ_FOLD_SAVE_FWD: return launch_rader_x<R, XOP_ADJ_FOLD_SAVE_FWD>(a, sign, s);
+        case XOP_ADJ_INV_MIX_FWD: return launch_rader_x<R, XOP_ADJ_INV_MIX_FWD>(a, sign, s);
+        default: return launch_rader_x<R, XOP_ADJ_INV_SCALE>(a, sign, s);
+    }
 }
 
 template <typename R, int NC, int BC>
@@ -1591,51 +1510,32 @@ static void launch_x(const DiffArgs<R>& a, int B, int op, int sign, hipStream_t 
 
 template <typename R>
 static void run_x(const DiffArgs<R>& a, int op, int sign, hipStream_t s) {
+    if (a.nx == RAD_N) return run_rader_x(a, op, sign, s);
     const int B = lines_per_block(a.nx, sizeof(cplx<R>), 64, PUFF_XY_LDS_BUDGET, false);
     if (a.nx == 129) return launch_x<R, 129, ct_lines_x<R, 129>()>(a, B, op, sign, s);
-    if (a.nx == 257) return launch_x<R, 257, ct_lines_x<R, 257>()>(a, B, op, sign, s);
     if (a.nx == 33) return launch_x<R, 33, ct_lines_x<R, 33>()>(a, B, op, sign, s);
     launch_x<R, 0, 0>(a, B, op, sign, s);
-}
-
-// Workgroups of a persistent pass: as many as the device holds at once (the
-// kernel's occupancy at `sh` bytes of LDS times the CUs), a multiple of the
-// XCD count, and no more than the tiles.
-static int64_t persistent_grid(const void* kernel, int threads, size_t sh, int64_t ntile, int* cache) {
-    if (*cache <= 0) {
-        int dev = 0, cus = 0, per = 0;
-        (void)hipGetDevice(&dev);
-        (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-        (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, threads, sh);
-        *cache = (per < 1 ? 1 : per) * (cus < 1 ? 1 : cus);
-    }
-    int64_t g = *cache;
-    const int64_t cap = (ntile + NXCD - 1) / NXCD * NXCD;
-    if (g > cap) g = cap;
-    g = g / NXCD * NXCD;
-    return g < NXCD ? NXCD : g;
 }
 
 template <typename R, int NC, int BC>
 static void launch_y(const DiffArgs<R>& a, int B, int sign, hipStream_t s) {
     if (BC) B = BC;   // compile-time plans fix their lines per workgroup
-    const size_t sh = (NC ? xy_lds_elems<R, NC, true>(B) : 2 * (size_t)lpad<true>(B * a.ny) + a.ny) *
-                      sizeof(cplx<R>);
+    const size_t sh = (2 * (size_t)lpad<true>(B * a.ny) + a.ny) * sizeof(cplx<R>);
     lds_opt_in(reinterpret_cast<const void*>(&k_fft_y<R, NC, BC>), sh);
-    const int thr = a.ay.rader ? PUFF_RADER_THREADS : 256;
-    const int64_t ntile = (int64_t)((a.nx + B - 1) / B) * a.nzp;
-    static int cache = 0;   // resident workgroups (one device)
-    const int64_t blocks = (NC > 0 && PUFF_PERSIST_Y) ? persistent_grid(reinterpret_cast<const void*>(&k_fft_y<R, NC, BC>), thr, sh,
-                                                    ntile, &cache)
-                                  : xcd_grid(ntile);
-    hipLaunchKernelGGL((k_fft_y<R, NC, BC>), dim3((unsigned)blocks), dim3(thr), sh, s, a, B, sign);
+    hipLaunchKernelGGL((k_fft_y<R, NC, BC>), dim3((unsigned)xcd_grid((int64_t)((a.nx + B - 1) / B) * a.nzp)),
+                       dim3(256), sh, s, a, B, sign);
 }
 
 template <typename R>
 static void run_y(const DiffArgs<R>& a, int sign, hipStream_t s) {
+    if (a.ny == RAD_N) {
+        constexpr int BL = rad_lines<R>();
+        const int64_t blocks = xcd_grid((int64_t)((a.nx + BL - 1) / BL) * a.nzp);
+        hipLaunchKernelGGL((k_rader_y<R>), dim3((unsigned)blocks), dim3(16 * BL), 0, s, a, sign);
+        return;
+    }
     const int B = lines_per_block(a.ny, sizeof(cplx<R>), 16, PUFF_Y_LDS_BUDGET, true);
     if (a.ny == 129) return launch_y<R, 129, ct_lines_y<R, 129>()>(a, B, sign, s);
-    if (a.ny == 257) return launch_y<R, 257, ct_lines_y<R, 257>()>(a, B, sign, s);
     if (a.ny == 33) return launch_y<R, 33, ct_lines_y<R, 33>()>(a, B, sign, s);
     launch_y<R, 0, 0>(a, B, sign, s);
 }
