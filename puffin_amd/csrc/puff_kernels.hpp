@@ -278,12 +278,10 @@ void launch_sort(const SortArgs<R>& a, hipStream_t s);
 // Gamma, chi and the reference index (the sort), or the first six (the moves
 // between slot and reference order).  An array moved to or from scattered
 // places one 8-byte value at a time costs a memory transaction per value;
-// the record is one 64-byte (32-byte) transaction for all of them, and the
-// pass between records and arrays is contiguous on both sides.
-template <typename R>
-constexpr int RecordQuads = 4;          // with chi and the reference index
-template <typename R>
-constexpr int StateQuads = sizeof(R) == 8 ? 4 : 2;
+// the record is one 64-byte transaction for all of them, and the pass between
+// records and arrays is contiguous on both sides.  Always whole 64 bytes: of
+// 2^24 scattered writes, 32-byte ones took 696 us and 64-byte ones 502 us.
+constexpr int RECORD_QUADS = 4;
 // rec[to[j]] = state of slot j
 template <typename R>
 void launch_records_scatter(const PartPtrs<R>& y, const int* to, int64_t n, uint4* rec, hipStream_t s);
@@ -318,6 +316,8 @@ struct LatticeOp {
     MatchArgs match;
 };
 
+// sums: scratch of the transverse corrector, LATTICE_SUMS doubles.
+constexpr int LATTICE_SUMS = 8 + 5 * 512;
 template <typename R>
 void launch_lattice(const LatticeOp& op, PartPtrs<R> y, const R* chi, int64_t n, const Physics& ph,
                     const MeshGeom& m, double* sums, hipStream_t s);

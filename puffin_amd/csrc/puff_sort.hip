@@ -338,7 +338,7 @@ __device__ __forceinline__ OneState<R> unpack_state(const uint4 (&q)[Q]) {
 template <typename R>
 __global__ __launch_bounds__(256) void k_scatter_records(PartPtrs<R> y, const R* chi, const int* key, int64_t n,
                                                          int* cursor, uint4* rec) {
-    constexpr int Q = RecordQuads<R>;
+    constexpr int Q = RECORD_QUADS;
     __shared__ uint4 sh[4 * 64 * (Q + 1)];
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const bool valid = i < n;
@@ -360,7 +360,7 @@ __global__ __launch_bounds__(256) void k_scatter_records(PartPtrs<R> y, const R*
 template <typename R>
 __global__ __launch_bounds__(256) void k_slots_from_records(const uint4* rec, int64_t n, PartPtrs<R> y, R* chi,
                                                             int* orig) {
-    constexpr int Q = RecordQuads<R>;
+    constexpr int Q = RECORD_QUADS;
     __shared__ uint4 sh[4 * 64 * (Q + 1)];
     const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     uint4 q[Q];
@@ -378,7 +378,7 @@ __global__ __launch_bounds__(256) void k_slots_from_records(const uint4* rec, in
 
 template <typename R>
 __global__ __launch_bounds__(256) void k_records_scatter(PartPtrs<R> y, const int* to, int64_t n, uint4* rec) {
-    constexpr int Q = StateQuads<R>;
+    constexpr int Q = RECORD_QUADS;
     __shared__ uint4 sh[4 * 64 * (Q + 1)];
     const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     uint4 q[Q] = {};
@@ -388,7 +388,7 @@ __global__ __launch_bounds__(256) void k_records_scatter(PartPtrs<R> y, const in
 
 template <typename R>
 __global__ __launch_bounds__(256) void k_records_gather(const uint4* rec, const int* from, int64_t n, PartPtrs<R> y) {
-    constexpr int Q = StateQuads<R>;
+    constexpr int Q = RECORD_QUADS;
     __shared__ uint4 sh[4 * 64 * (Q + 1)];
     const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     uint4 q[Q];
@@ -401,7 +401,7 @@ struct StateOut {
 };
 template <typename R>
 __global__ __launch_bounds__(256) void k_records_unpack(const uint4* rec, int64_t n, StateOut out) {
-    constexpr int Q = StateQuads<R>;
+    constexpr int Q = RECORD_QUADS;
     __shared__ uint4 sh[4 * 64 * (Q + 1)];
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     uint4 q[Q];
