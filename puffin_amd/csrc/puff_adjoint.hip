@@ -110,7 +110,7 @@ __global__ __launch_bounds__(ADJ_THREADS) void k_adj_stage(AdjArgs<R> a) {
             x = x0; y = y0; z2 = z20; pr = pr0; pi = pi0; g = g0;
         } else {
             const Trial<R> t = trial_state<R, STAGE>(ph, x0, y0, z20, pr0, pi0, g0, kr, ki, kg, qr, qi, qg, a.cin,
-                                                     a.cprev);
+                                                     a.cprev, a.cin_r, a.cprev_r);
             x = t.x; y = t.y; z2 = t.z2; pr = t.pr; pi = t.pi; g = t.g;
         }
         if (ev) {
@@ -152,7 +152,9 @@ __global__ __launch_bounds__(ADJ_THREADS) void k_adj_stage(AdjArgs<R> a) {
     if (flag) atomicOr(a.flags, flag);
     const int lane = threadIdx.x & 63;
     const int wv = threadIdx.x >> 6;
-    const TileBox tb = workgroup_box<R>(m, ok, c, a.box);
+    LaneBox lb = lane_box();
+    lane_box_add<R>(lb, ok, c);
+    const TileBox tb = workgroup_box<6>(m, lb, a.box);
     const bool scat = ph.coupling && ph.electrons_evolve;
     const bool use_tile = scat && tile_fits<ADJ_TILE_NODES>(m, tb);
     const int nnb = m.one_d ? 2 : 8;
@@ -180,7 +182,7 @@ __global__ __launch_bounds__(ADJ_THREADS) void k_adj_stage(AdjArgs<R> a) {
     // workgroup's node box is small (the dense part of the beam), both are
     // formed once per node of the box in LDS and the corners read from there
     // (same arithmetic as the global reads).
-    const R cA = (R)a.cin;
+    const R cA = a.cin_r;
     const bool lds_field = tile_fits<ADJ_TILE_NODES>(m, tb) && tb.tx * tb.ty * tb.tz <= ADJ_FIELD_TILE_NODES;
     __shared__ cplx<R> s_v[ADJ_FIELD_TILE_NODES];
     __shared__ double2 s_g[ADJ_FIELD_TILE_NODES];
@@ -240,9 +242,17 @@ __global__ __launch_bounds__(ADJ_THREADS) void k_adj_stage(AdjArgs<R> a) {
 
     // ---- field cotangent of this stage: w_k (dL/dFr, dL/dFi) at the nodes
     if (scat) {
-        __shared__ double s_tile[2 * ADJ_TILE_NODES];
-        scatter_cells<R>(m, tb, use_tile, ok, c, cr, ok ? (R)Lfr : (R)0,
-                         ok ? (R)Lfi : (R)0, a.mAout, s_tile);
+        const R sr = ok ? (R)Lfr : (R)0, si = ok ? (R)Lfi : (R)0;
+        if (use_tile) {
+            __shared__ double s_tile[2 * ADJ_TILE_NODES];
+            for (int t = threadIdx.x; t < 2 * tb.tx * tb.ty * tb.tz; t += blockDim.x) s_tile[t] = 0.0;
+            __syncthreads();
+            if (ok) tile_add<R, double>(m, tb, c, cr, sr, si, s_tile);
+            __syncthreads();
+            tile_flush<R, double>(m, tb, a.mAout, s_tile);
+        } else {
+            global_add<R>(m, ok, c, cr, sr, si, a.mAout);
+        }
     }
 
     // ---- dJ/dn2col of this stage: workgroup sum into a spread accumulator

@@ -71,9 +71,20 @@ constexpr int BOX_COPIES = 64;
 #define PUFF_STAGE_THREADS 256
 #endif
 constexpr int STAGE_THREADS = PUFF_STAGE_THREADS;
-// (256 or 512: the packed tile's rounding needs STAGE_THREADS >= 256)
-constexpr int STAGE_THREADS_LOG2 = STAGE_THREADS == 512 ? 9 : STAGE_THREADS == 256 ? 8 : -1;
-static_assert(STAGE_THREADS_LOG2 > 0, "stage workgroups of 256 or 512 threads");
+// Macroparticles per thread of a stage workgroup, and its workgroups.
+#ifndef PUFF_STAGE_WIDE
+#define PUFF_STAGE_WIDE 1
+#endif
+constexpr int STAGE_WIDE = PUFF_STAGE_WIDE;
+constexpr int64_t STAGE_WIDE_MIN = (int64_t)4 * 256 * STAGE_THREADS * STAGE_WIDE;
+inline int stage_per_thread(int stage, int64_t n, int precision, bool general) {
+    return (precision == PUFF_MIXED && stage < 4 && n >= STAGE_WIDE_MIN && !general) ? STAGE_WIDE : 1;
+}
+inline bool stage_pole(int und_type) { return und_type == PUFF_UND_PLANEPOLE || und_type == PUFF_UND_CURVED; }
+inline int64_t stage_workgroups(int64_t n, int per_thread) {
+    const int64_t w = (int64_t)STAGE_THREADS * per_thread;
+    return (n + w - 1) / w;
+}
 #ifndef PUFF_TILE_NODES_FP64
 #define PUFF_TILE_NODES_FP64 1280
 #endif
@@ -93,9 +104,10 @@ constexpr int stage_tile_nodes() {
 }
 // Node capacity of the stage kernels' LDS copy of the field over the
 // workgroup's node box (one complex per node; larger boxes gather from
-// global memory).
+// global memory); the box of two macroparticles per thread fits 512 nodes as
+// often as that of one fits 256.
 #ifndef PUFF_FIELD_TILE_NODES
-#define PUFF_FIELD_TILE_NODES 256
+#define PUFF_FIELD_TILE_NODES 512
 #endif
 constexpr int FIELD_TILE_NODES = PUFF_FIELD_TILE_NODES;
 
@@ -109,7 +121,8 @@ constexpr int ADJ_THREADS = 256;
 // against 888 ms.
 constexpr int ADJ_TILE_NODES = 2000;
 constexpr int ADJ_FIELD_TILE_NODES = 256;   // LDS copy of the trial field and source cotangent
-constexpr int MAX_BOX_WAVES = (STAGE_THREADS > ADJ_THREADS ? STAGE_THREADS : ADJ_THREADS) / 64;
+constexpr int MAX_BOX_WAVES = STAGE_THREADS / 64;
+static_assert(STAGE_THREADS == ADJ_THREADS, "one count of wavefronts per workgroup");
 
 // Flag words of the step kernels: [0] flag bits of the current step;
 // [FLAG_WORD_FALLBACK] the stage workgroups of the step whose node box did not
@@ -157,6 +170,18 @@ struct StageScalars {
     double n2col;
     double c[8];
     int und_type;
+    float n2col_f;   // the same in FP32
+    float c_f[8];
+    template <typename R>
+    __device__ __forceinline__ R coef(int k) const {
+        if constexpr (sizeof(R) == 8) return c[k];
+        else return c_f[k];
+    }
+    template <typename R>
+    __device__ __forceinline__ R strength() const {
+        if constexpr (sizeof(R) == 8) return n2col;
+        else return n2col_f;
+    }
 };
 
 // 1-D FFT plan of one axis.  Mixed radix: radices (product n) and the

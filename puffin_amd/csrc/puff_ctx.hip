@@ -483,6 +483,8 @@ static int stage_scalars(const puff_params& p, double z, double n2col, StageScal
             s.c[2] = 0.0;
         }
     }
+    s.n2col_f = (float)s.n2col;
+    for (int k = 0; k < 8; ++k) s.c_f[k] = (float)s.c[k];
     return PUFF_OK;
 }
 
@@ -629,6 +631,8 @@ static int create(Ctx* c) {
     m.inv_dz2 = 1.0 / p.dz2;
     m.halfx = ((p.nx - 1) / 2.0) * p.dx;   // rhs.f90:395-396
     m.halfy = ((p.ny - 1) / 2.0) * p.dy;
+    m.sd = {m.dx, m.dy, m.inv_dx, m.inv_dy, m.halfx, m.halfy};
+    m.sf = {(float)m.dx, (float)m.dy, (float)m.inv_dx, (float)m.inv_dy, (float)m.halfx, (float)m.halfy};
     Physics& ph = c->phys;
     ph.eta = p.eta;
     ph.rho = p.rho;
@@ -640,6 +644,10 @@ static int create(Ctx* c) {
     ph.c_dx = 2 * p.rho * p.kappa / std::sqrt(p.eta);
     ph.inv_eta = 1.0 / p.eta;
     ph.inv_gr2 = 1.0 / (p.gamma_r * p.gamma_r);
+    ph.aw2 = p.aw * p.aw;
+    ph.eta_k2 = p.eta / (p.kappa * p.kappa);
+    ph.sd = {ph.c_dx, ph.inv2rho, ph.kappa};
+    ph.sf = {(float)ph.c_dx, (float)ph.inv2rho, (float)ph.kappa};
     ph.coupling = p.coupling;
     ph.electrons_evolve = p.electrons_evolve;
     ph.field_evolve = p.field_evolve;
@@ -881,6 +889,10 @@ static int rk4par(Ctx* c, double sz, double h, char* cap = nullptr, void* cap_hd
         a.cin = cin[st - 1];
         a.cnext = cnext[st - 1];
         a.cprev = (st > 2) ? cin[st - 2] : 0.0;
+        a.cin_r = (R)a.cin;
+        a.cprev_r = (R)a.cprev;
+        a.cnext_r = (R)a.cnext;
+        a.h6_r = (R)a.h6;
         a.kin = (st > 1) ? K[st - 2] : KPtrs<R>{};
         a.kprev = (st > 2) ? K[st - 3] : KPtrs<R>{};
         a.k1 = K[0];
@@ -931,7 +943,10 @@ static int rk4par(Ctx* c, double sz, double h, char* cap = nullptr, void* cap_hd
         // could not use the LDS tile exceeds twice its value after the sort
         // (measured on the bunched C1 beam: sorting at that point beats
         // letting the share grow until the fallback has cost one sort)
-        const double groups = 4.0 * (double)((c->n + STAGE_THREADS - 1) / STAGE_THREADS);
+        const bool general = c->det || stage_pole(c->p.und_type);
+        double groups = 0.0;
+        for (int st = 1; st <= 4; ++st)
+            groups += (double)stage_workgroups(c->n, stage_per_thread(st, c->n, c->precision, general));
         const double share = groups > 0 ? (double)c->h_flags[FLAG_WORD_FALLBACK] / groups : 0.0;
         c->fallback_last = share;
         if (c->steps_since_sort == 1) c->fallback_base = share;
@@ -1391,6 +1406,10 @@ static int replay_stages(Ctx* c, const StageScalars* sc, const double* cin, cons
         a.cin = cin[st - 1];
         a.cnext = cnext[st - 1];
         a.cprev = (st > 2) ? cin[st - 2] : 0.0;
+        a.cin_r = (R)a.cin;
+        a.cprev_r = (R)a.cprev;
+        a.cnext_r = (R)a.cnext;
+        a.h6_r = (R)a.h6;
         a.kin = (st > 1) ? P.k[st - 2] : KPtrs<R>{};
         a.kprev = (st > 2) ? P.k[st - 3] : KPtrs<R>{};
         a.kout = P.k[st - 1];
@@ -1496,6 +1515,8 @@ static int rk4par_adjoint(Ctx* c, double sz, double h, double* dn2col, int32_t* 
         b.s = sc[st - 1];
         b.cin = cin[st - 1];
         b.cprev = (st > 2) ? cin[st - 2] : 0.0;
+        b.cin_r = (R)b.cin;
+        b.cprev_r = (R)b.cprev;
         b.kin = (st > 1) ? K[st - 2] : KPtrs<R>{};
         b.kprev = (st > 2) ? K[st - 3] : KPtrs<R>{};
         b.dAin = (st > 1) ? D[st - 2] : nullptr;

@@ -8,22 +8,51 @@ namespace puff {
 // Mesh geometry as seen by the push kernels.  The whole mesh is the
 // interpolation window: halfx = ((NX-1)/2) dx (rhs.f90:395-396 with
 // nspinDX = NX).  nzp is the z2 period (NZ2-1) on a periodic mesh, else NZ2.
+// Constants that the kernels use in the form's own type are held in both: a
+// conversion of a scalar argument is a vector instruction per lane (some 25 of
+// a mixed stage kernel's 600).
+template <typename R>
+struct MeshScale {
+    R dx, dy, inv_dx, inv_dy, halfx, halfy;
+};
+
 struct MeshGeom {
     int nx, ny, nz2, nzp;
     int periodic, one_d;
     double dx, dy, dz2;
     double inv_dx, inv_dy, inv_dz2;
     double halfx, halfy;
+    MeshScale<double> sd;
+    MeshScale<float> sf;
+    template <typename R>
+    __device__ __forceinline__ const MeshScale<R>& scale() const {
+        if constexpr (sizeof(R) == 8) return sd;
+        else return sf;
+    }
+};
+
+template <typename R>
+struct PhysScale {
+    R c_dx, inv2rho, kappa;
 };
 
 struct Physics {
     double eta, rho, kappa, gamma_r, aw;
+    double aw2;         // aw^2
+    double eta_k2;      // eta / kappa^2
     double inv2rho;     // 1 / (2 rho)                    (rhs.f90:366)
     double inv_dV3;     // 1 / (dx dy dz2)                (rhs.f90:361)
     double c_dx;        // 2 rho kappa / sqrt(eta)        (puffin_equations.f90:115)
     double inv_eta;     // 1 / eta
     double inv_gr2;     // 1 / gamma_r^2
     int coupling, electrons_evolve, field_evolve;
+    PhysScale<double> sd;
+    PhysScale<float> sf;
+    template <typename R>
+    __device__ __forceinline__ const PhysScale<R>& scale() const {
+        if constexpr (sizeof(R) == 8) return sd;
+        else return sf;
+    }
 };
 
 // Six particle coordinates: x, y, p_r, p_i in R; z2 and Gamma in FP64.
@@ -87,6 +116,7 @@ struct StageArgs {
     double cprev;       // of the stage before (stages 3, 4: h/2)
     double cnext;       // trial coefficient of the next stage
     double h6;
+    R cin_r, cprev_r, cnext_r, h6_r;   // the same in R
     const cplx<R>* A0;
     const cplx<R>* dAin;
     cplx<R>* dAout;
@@ -151,6 +181,7 @@ struct AdjArgs {
     KPtrs<R> kprev;        // k_{s-2} (stages 3, 4)
     const R* chi;
     double cin, cprev;     // trial coefficients of this stage and the one before
+    R cin_r, cprev_r;      // the same in R
     const cplx<R>* A0;
     const cplx<R>* dAin;   // dA_{s-1} (stages 2-4)
     PartPtrs<R> L;         // cotangent of the step's end state

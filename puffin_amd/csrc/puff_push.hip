@@ -18,124 +18,34 @@
 
 namespace puff {
 
-// One RK4 stage.  STAGE = 1..4 (rk4par's four derivs calls).  DET: the
-// deterministic fixed-point deposit (FP64 form only; see DetState).
-template <typename R, int STAGE, bool DET>
+// A value through an empty asm statement: computed here, not later.
+template <typename T>
+__device__ __forceinline__ void hold(T& v) {
+    asm volatile("" : "+v"(v));
+}
+
+// One RK4 stage.  STAGE = 1..4 (rk4par's four derivs calls), P macroparticles
+// per thread (STAGE_THREADS apart).  DET: the deterministic fixed-point
+// deposit (FP64 form only; see DetState).
+//
+// Two macroparticles per thread halve what a workgroup pays per macroparticle
+// for its node box, field tile, flush and barriers, and give the memory twice
+// the loads per wavefront.
+template <typename R, int STAGE, bool DET, int P, bool POLE>
 __global__ __launch_bounds__(STAGE_THREADS) void k_stage(StageArgs<R> a) {
-    // Flags raised by an earlier kernel of this step do not stop stages 1-3:
-    // they write only the step's scratch (k_s, dA_s), and a particle whose
-    // trial position is off the mesh takes no part in the gather and deposit
-    // (locate raises the flag again).  Stage 4 writes the state, and only
-    // when no flag is set: read here, with the particle loads (no kernel of
-    // stage 4 raises a flag: stage 3 checked its trial positions).
-    const int rejected = (STAGE == 4) ? *a.flags : 0;
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const bool in = i < a.n;
-    const MeshGeom& m = a.mesh;
-    const Physics& ph = a.phys;
-
-    // ---- trial state y_s = y0 + c k_{s-1} (puffin_mpi_RK4.f90:190-195 etc.)
-    R x = 0, y = 0, pr = 0, pi = 0, chi = 0;
-    double z2 = 0.0, g = 1.0;
-    R x0 = 0, y0 = 0, pr0 = 0, pi0 = 0;
-    double z20 = 0.0, g0 = 1.0;
-    if (in) {
-        x0 = a.y0.x[i];
-        y0 = a.y0.y[i];
-        z20 = a.y0.z2[i];
-        pr0 = a.y0.pr[i];
-        pi0 = a.y0.pi[i];
-        g0 = a.y0.g[i];
-        chi = a.chi[i];
-        if (STAGE == 1) {
-            x = x0; y = y0; z2 = z20; pr = pr0; pi = pi0; g = g0;
-            if (a.ycap.x) {
-                a.ycap.x[i] = x0;
-                a.ycap.y[i] = y0;
-                a.ycap.z2[i] = z20;
-                a.ycap.pr[i] = pr0;
-                a.ycap.pi[i] = pi0;
-                a.ycap.g[i] = g0;
-                a.chicap[i] = chi;
-            }
-        } else {
-            const R kr = a.kin.pr[i], ki = a.kin.pi[i], kg = a.kin.g[i];
-            R qr = 0, qi = 0, qg = 0;
-            if (STAGE > 2) {
-                qr = a.kprev.pr[i];
-                qi = a.kprev.pi[i];
-                qg = a.kprev.g[i];
-            }
-            const Trial<R> t = trial_state<R, STAGE>(ph, x0, y0, z20, pr0, pi0, g0, kr, ki, kg, qr, qi, qg, a.cin,
-                                                     a.cprev);
-            x = t.x; y = t.y; z2 = t.z2; pr = t.pr; pi = t.pi; g = t.g;
-            if (STAGE == 4) {
-                // y0 + h/6 (k1 + 2 (k2 + k3)) formed now, with k1 and k2 loaded
-                // beside y0 and k3: the end of the kernel adds h/6 k4 only, and
-                // no k array is read after the deposit (puffin_mpi_RK4.f90:274-279).
-                // The rates of y0, y0 + h/2 k1 and y0 + h/2 k2 are k1 to k3 of
-                // x, y and z2.
-                const R h6 = (R)a.h6, hh = (R)a.cprev;
-                const R k1r = a.k1.pr[i], k1i = a.k1.pi[i], k1g = a.k1.g[i];
-                const Rates<R> v1 = rates<R>(ph, drift_of(ph, (double)pr0, (double)pi0, g0), pr0, pi0);
-                const R p2r = fma(hh, k1r, pr0), p2i = fma(hh, k1i, pi0);
-                const Rates<R> v2 =
-                    rates<R>(ph, drift_of(ph, (double)p2r, (double)p2i, fma(a.cprev, (double)k1g, g0)), p2r, p2i);
-                x0 = fma(h6, v1.x + (R)2 * (v2.x + t.v.x), x0);
-                y0 = fma(h6, v1.y + (R)2 * (v2.y + t.v.y), y0);
-                z20 = fma(a.h6, v1.z2 + 2.0 * (v2.z2 + t.v.z2), z20);
-                pr0 = fma(h6, k1r + (R)2 * (qr + kr), pr0);
-                pi0 = fma(h6, k1i + (R)2 * (qi + ki), pi0);
-                g0 = fma(a.h6, (double)k1g + 2.0 * ((double)qg + (double)kg), g0);
-            }
-        }
-    }
-
-    // ---- p2 in FP64 and (1 + eta p2) / Gamma
-    const double prd = (double)pr, pid = (double)pi;
-    const Drift dr = drift_of(ph, prd, pid, g);
-    const double p2 = dr.p2, fac = dr.fac;
-
-    // ---- node and weights
-    Cell<R> c{};
-    int flag = in ? locate<R>(m, x, y, z2, c) : 0;
-    const bool ok = in && flag == 0;
-    if (flag) atomicOr(a.flags, flag);
-
-    // ---- sources (getSource): s = chi / dV3 (1 + eta p2) p / Gamma
-    const R sr = ok ? (R)((double)chi * ph.inv_dV3 * fac * prd) : (R)0;
-    const R si = ok ? (R)((double)chi * ph.inv_dV3 * fac * pid) : (R)0;
-
-    // ---- node box of this workgroup's cells and the step's active box (and,
-    // for the packed fixed-point tile, the workgroup's largest |s|)
-    const int lane = threadIdx.x & 63;
-    constexpr bool PACKED = sizeof(R) == 4 && PUFF_MIXED_TILE == 0 && !DET;
-    const TileBox tb = workgroup_box<R, PACKED ? 7 : 6>(
-        m, ok, c, a.box, PACKED ? __float_as_int(fmaxf(fabsf((float)sr), fabsf((float)si))) : 0);
-    const bool use_tile = ph.field_evolve && tile_fits<stage_tile_nodes<R>()>(m, tb);
-    if (threadIdx.x == 0 && ph.field_evolve && tb.any && !use_tile) atomicAdd(a.flags + FLAG_WORD_FALLBACK, 1);
-
-    // ---- nodes of the cell (weights are formed per corner where used)
-    const int nnb = m.one_d ? 2 : 8;
-    const CellRef cr = cell_ref<R>(m, ok, c, tb, lane);
-
-    // ---- gather F = sum_k w_k (A0 + c dA_{s-1})[node_k]  (getFFelecs).
-    // When the workgroup's node box is small (the dense part of the beam),
-    // A0 + c dA_{s-1} is formed once per node of the box in LDS and the
-    // corners are read from there; else from global memory.  Same arithmetic
-    // either way.
-    // The field tile shares the deposit tile's LDS: it is used only for boxes
-    // of at most FIELD_TILE_NODES nodes, whose deposit needs the first
-    // WORDS x FIELD_TILE_NODES words, so it sits right after them.
     // Deposit tiles: two doubles per node in the FP64 form; DET_WORDS 8-byte
     // integers in its deterministic mode; one 8-byte packed fixed-point word
-    // in the mixed form (scatter_cells_packed: one ds_add_u64 per corner for
+    // in the mixed form (packed_add: one ds_add_u64 per corner for
     // both components).  Measured on the C1 beam, mixed form: an FP32 tile
     // (ds_add_f32) ran each stage 3.1x slower than the FP64 tile, and a
     // compensated FP32 tile (ds_add_rtn_f32 + TwoSum) 5.7x slower, with the
     // same count of LDS instructions per wave but 6x the LDS-active and 24x
     // the LDS-wait cycles of ds_add_f64; the packed tile cut the LDS-wait
     // cycles per wave from 398 to 6 and the step by 3-4 %.
+    // The field tile shares the deposit tile's LDS: it is used only for boxes
+    // of at most FIELD_TILE_NODES nodes, whose deposit needs the first
+    // WORDS x FIELD_TILE_NODES words, so it sits right after them.
+    constexpr bool PACKED = sizeof(R) == 4 && PUFF_MIXED_TILE == 0 && !DET;
     constexpr int TILE = stage_tile_nodes<R>();
     using D = typename std::conditional<
         PACKED, unsigned long long,
@@ -145,10 +55,183 @@ __global__ __launch_bounds__(STAGE_THREADS) void k_stage(StageArgs<R> a) {
                       WORDS * TILE * sizeof(D), "field tile inside the deposit tile");
     __shared__ D s_dep[WORDS * TILE];
     cplx<R>* s_fld = reinterpret_cast<cplx<R>*>(s_dep + WORDS * FIELD_TILE_NODES);
-    const R cA = (R)a.cin;
-    const bool lds_field = use_tile && tb.tx * tb.ty * tb.tz <= FIELD_TILE_NODES;
+
+    // Flags raised by an earlier kernel of this step do not stop stages 1-3:
+    // they write only the step's scratch (k_s, dA_s), and a particle whose
+    // trial position is off the mesh takes no part in the gather and deposit
+    // (locate raises the flag again).  Stage 4 writes the state, and only
+    // when no flag is set: read here, with the particle loads (no kernel of
+    // stage 4 raises a flag: stage 3 checked its trial positions).
+    const int rejected = (STAGE == 4) ? *a.flags : 0;
+    // Slots of the workgroup: s0 + t, with s0 scalar and t 32 bits, so that an
+    // access is a scalar base and one register of offset (64-bit lane addresses
+    // took two registers and three instructions per array).
+    const int64_t s0 = (int64_t)blockIdx.x * (STAGE_THREADS * P);
+    const unsigned left = (unsigned)min<int64_t>(a.n - s0, STAGE_THREADS * P);
+    auto at = [s0](auto* q, unsigned t) -> auto& { return (q + s0)[t]; };
+    const MeshGeom& m = a.mesh;
+    const Physics& ph = a.phys;
+
+    // ---- trial state y_s = y0 + c k_{s-1} (puffin_mpi_RK4.f90:190-195 etc.)
+    bool in[P];
+    R x[P], y[P], pr[P], pi[P], chi[P];
+    double z2[P], g[P];
+    R x0[P], y0[P], pr0[P], pi0[P];
+    double z20[P], g0[P];
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        const unsigned i = threadIdx.x + p * STAGE_THREADS;
+        in[p] = i < left;
+        x0[p] = y0[p] = pr0[p] = pi0[p] = chi[p] = 0;
+        z20[p] = 0.0;
+        g0[p] = 1.0;
+        if (in[p]) {
+            x0[p] = at(a.y0.x, i);
+            y0[p] = at(a.y0.y, i);
+            z20[p] = at(a.y0.z2, i);
+            pr0[p] = at(a.y0.pr, i);
+            pi0[p] = at(a.y0.pi, i);
+            g0[p] = at(a.y0.g, i);
+            chi[p] = at(a.chi, i);
+        }
+    }
+    if constexpr (STAGE == 1) {
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+            x[p] = x0[p]; y[p] = y0[p]; z2[p] = z20[p]; pr[p] = pr0[p]; pi[p] = pi0[p]; g[p] = g0[p];
+            const unsigned i = threadIdx.x + p * STAGE_THREADS;
+            if (in[p] && a.ycap.x) {
+                at(a.ycap.x, i) = x0[p];
+                at(a.ycap.y, i) = y0[p];
+                at(a.ycap.z2, i) = z20[p];
+                at(a.ycap.pr, i) = pr0[p];
+                at(a.ycap.pi, i) = pi0[p];
+                at(a.ycap.g, i) = g0[p];
+                at(a.chicap, i) = chi[p];
+            }
+        }
+    } else {
+        R kr[P], ki[P], kg[P], qr[P], qi[P], qg[P];
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+            const unsigned i = threadIdx.x + p * STAGE_THREADS;
+            kr[p] = ki[p] = kg[p] = qr[p] = qi[p] = qg[p] = 0;
+            if (in[p]) {
+                kr[p] = at(a.kin.pr, i);
+                ki[p] = at(a.kin.pi, i);
+                kg[p] = at(a.kin.g, i);
+                if (STAGE > 2) {
+                    qr[p] = at(a.kprev.pr, i);
+                    qi[p] = at(a.kprev.pi, i);
+                    qg[p] = at(a.kprev.g, i);
+                }
+            }
+        }
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+            const Trial<R> t = trial_state<R, STAGE>(ph, x0[p], y0[p], z20[p], pr0[p], pi0[p], g0[p], kr[p], ki[p],
+                                                     kg[p], qr[p], qi[p], qg[p], a.cin, a.cprev, a.cin_r, a.cprev_r);
+            x[p] = t.x; y[p] = t.y; z2[p] = t.z2; pr[p] = t.pr; pi[p] = t.pi; g[p] = t.g;
+            if (STAGE == 4) {
+                // y0 + h/6 (k1 + 2 (k2 + k3)) formed now: the end of the kernel
+                // adds h/6 k4 only, and no k array is read after the deposit
+                // (puffin_mpi_RK4.f90:274-279).  The rates of y0, y0 + h/2 k1
+                // and y0 + h/2 k2 are k1 to k3 of x, y and z2.
+                const unsigned i = threadIdx.x + p * STAGE_THREADS;
+                const R h6 = a.h6_r, hh = a.cprev_r;
+                R k1r = 0, k1i = 0, k1g = 0;
+                if (in[p]) {
+                    k1r = at(a.k1.pr, i);
+                    k1i = at(a.k1.pi, i);
+                    k1g = at(a.k1.g, i);
+                }
+                Rates<R> v1 = rates<R>(ph, drift_of(ph, (double)pr0[p], (double)pi0[p], g0[p]), pr0[p], pi0[p]);
+                // one rate after the other: side by side they take 20 registers more
+                hold(v1.x);
+                hold(v1.y);
+                hold(v1.z2);
+                hold(k1r);
+                const R p2r = fma(hh, k1r, pr0[p]), p2i = fma(hh, k1i, pi0[p]);
+                const Rates<R> v2 =
+                    rates<R>(ph, drift_of(ph, (double)p2r, (double)p2i, fma(a.cprev, (double)k1g, g0[p])), p2r, p2i);
+                x0[p] = fma(h6, v1.x + (R)2 * (v2.x + t.v.x), x0[p]);
+                y0[p] = fma(h6, v1.y + (R)2 * (v2.y + t.v.y), y0[p]);
+                z20[p] = fma(a.h6, v1.z2 + 2.0 * (v2.z2 + t.v.z2), z20[p]);
+                pr0[p] = fma(h6, k1r + (R)2 * (qr[p] + kr[p]), pr0[p]);
+                pi0[p] = fma(h6, k1i + (R)2 * (qi[p] + ki[p]), pi0[p]);
+                g0[p] = fma(a.h6, (double)k1g + 2.0 * ((double)qg[p] + (double)kg[p]), g0[p]);
+                // formed here: left alone, the compiler moves them behind the
+                // deposit, with their inputs live across it
+                hold(x0[p]);
+                hold(y0[p]);
+                hold(z20[p]);
+                hold(pr0[p]);
+                hold(pi0[p]);
+                hold(g0[p]);
+            }
+        }
+    }
+
+    // ---- p2 in FP64 and (1 + eta p2) / Gamma; node and weights; sources
+    // (getSource): s = chi / dV3 (1 + eta p2) p / Gamma
+    double fac[P];
+    R ep2k[P], sr[P], si[P];
+    Cell<R> c[P];
+    bool ok[P];
+    LaneBox lb = lane_box();
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        hold(g[p]);
+        const double prd = (double)pr[p], pid = (double)pi[p];
+        const Drift dr = drift_of(ph, prd, pid, g[p]);
+        fac[p] = dr.fac;
+        ep2k[p] = (R)(ph.eta_k2 * dr.p2);
+        c[p] = Cell<R>{};
+        int flag = in[p] ? locate<R>(m, x[p], y[p], z2[p], c[p]) : 0;
+        ok[p] = in[p] && flag == 0;
+        sr[p] = ok[p] ? (R)((double)chi[p] * ph.inv_dV3 * fac[p] * prd) : (R)0;
+        si[p] = ok[p] ? (R)((double)chi[p] * ph.inv_dV3 * fac[p] * pid) : (R)0;
+        lane_box_add<R>(lb, ok[p], c[p], PACKED ? __float_as_int(fmaxf(fabsf((float)sr[p]), fabsf((float)si[p]))) : 0);
+        const Rates<R> v = rates<R>(ph, dr, pr[p], pi[p]);
+        if (STAGE < 4) {
+            // next stage's trial state must lie inside the mesh, else the next
+            // derivs call would raise the flag (checked here, on the rates the
+            // next stage forms again, so that no later kernel writes state when
+            // it does)
+            const R cn = a.cnext_r;
+            Cell<R> cc;
+            if (in[p]) flag |= locate<R>(m, fma(cn, v.x, x0[p]), fma(cn, v.y, y0[p]), fma(a.cnext, v.z2, z20[p]), cc);
+        } else {
+            // x, y and z2 of the step's end do not wait for the field
+            const unsigned i = threadIdx.x + p * STAGE_THREADS;
+            if (in[p] && !rejected) {
+                at(a.y0.x, i) = fma(a.h6_r, v.x, x0[p]);
+                at(a.y0.y, i) = fma(a.h6_r, v.y, y0[p]);
+                at(a.y0.z2, i) = fma(a.h6, v.z2, z20[p]);
+            }
+        }
+        if (flag) atomicOr(a.flags, flag);
+        // kept as they stand across the barriers (see the sums above)
+        hold(fac[p]);
+        hold(ep2k[p]);
+    }
+
+    // ---- node box of this workgroup's cells and the step's active box (and,
+    // for the packed fixed-point tile, the workgroup's largest |s|)
+    const int lane = threadIdx.x & 63;
+    const TileBox tb = workgroup_box<PACKED ? 7 : 6>(m, lb, a.box);
+    const bool use_tile = ph.field_evolve && tile_fits<TILE>(m, tb);
+    if (threadIdx.x == 0 && ph.field_evolve && tb.any && !use_tile) atomicAdd(a.flags + FLAG_WORD_FALLBACK, 1);
+
+    // ---- gather F = sum_k w_k (A0 + c dA_{s-1})[node_k]  (getFFelecs).
+    // When the workgroup's node box is small (the dense part of the beam),
+    // A0 + c dA_{s-1} is formed once per node of the box in LDS and the
+    // corners are read from there; else from global memory.  Same arithmetic
+    // either way.
+    const R cA = a.cin_r;
+    const int nt = tb.tx * tb.ty * tb.tz;
+    const bool lds_field = use_tile && nt <= FIELD_TILE_NODES;
     if (lds_field) {
-        const int nt = tb.tx * tb.ty * tb.tz;
         const int ntr = m.nx * m.ny;
         const BoxDiv bd = box_div(tb);
         for (int q = threadIdx.x; q < nt; q += blockDim.x) {
@@ -163,102 +246,121 @@ __global__ __launch_bounds__(STAGE_THREADS) void k_stage(StageArgs<R> a) {
             }
             s_fld[q] = v;
         }
+    }
+    if (use_tile) {
+        tile_clear(s_dep, WORDS * nt);
         __syncthreads();
     }
-    R fr = 0, fi = 0;
-    if (ok && lds_field && !m.one_d) {
-        // getFFelecs' corner order, the weights formed once per lane
-        const CornerSet<R> cs = corner_set<R>(c, tb, 0);
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const cplx<R> v = s_fld[cr.t0 + cs.oxy[k & 3] + cs.oz[k >> 2]];
-            const R wk = cs.xy[k & 3] * cs.z[k >> 2];
-            fr = fma(wk, v.x, fr);
-            fi = fma(wk, v.y, fi);
+    const int nnb = m.one_d ? 2 : 8;
+    const int log2S = PACKED ? packed_scale_log2(tb.extra) : 0;
+    R fr[P], fi[P];
+    // ---- momentum equations (puffin_equations.f90:17-104)
+    auto equations = [&](int p) {
+        const unsigned i = threadIdx.x + p * STAGE_THREADS;
+        R kpr = 0, kpi = 0;
+        double kg = 0.0;
+        if (ph.electrons_evolve) {
+            R bx, by, bz;
+            bfield<R, POLE>(a.s, x[p], y[p], bx, by, bz);
+            const R facr = (R)fac[p];
+            const R n2col = a.s.template strength<R>(), kappa = ph.template scale<R>().kappa, inv2rho = ph.template scale<R>().inv2rho;
+            kpr = inv2rho * (n2col * by - ep2k[p] * fr[p]) + kappa * pi[p] * facr * n2col * bz;
+            kpi = inv2rho * (n2col * bx - ep2k[p] * fi[p]) - kappa * pr[p] * facr * n2col * bz;
+            kg = -ph.rho * fac[p] * 2.0 * ((double)pr[p] * (double)fr[p] + (double)pi[p] * (double)fi[p]);
         }
-    } else if (ok) {
+        if (STAGE < 4) {
+            if (in[p]) {
+                at(a.kout.pr, i) = kpr;
+                at(a.kout.pi, i) = kpi;
+                at(a.kout.g, i) = (R)kg;   // FP32 in the mixed form (see KPtrs)
+            }
+        } else if (in[p] && !rejected) {
+            // y = (y0 + h/6 (k1 + 2 (k2 + k3))) + h/6 k4 (puffin_mpi_RK4.f90:274-279, 307-312)
+            at(a.y0.pr, i) = fma(a.h6_r, kpr, pr0[p]);
+            at(a.y0.pi, i) = fma(a.h6_r, kpi, pi0[p]);
+            at(a.y0.g, i) = fma(a.h6, kg, g0[p]);
+        }
+    };
+    double det_scale = 0.0;
+    if constexpr (DET) det_scale = ldexp(1.0, *a.det.shift);
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            if (k < nnb) {
-                cplx<R> v;
-                if (lds_field) {
-                    v = s_fld[corner_tile(m, tb, cr, k)];
-                } else {
-                    const int node = corner_node(m, cr, k);
-                    v = a.A0[node];
-                    if (STAGE > 1) {
-                        const cplx<R> d = a.dAin[node];
-                        v.x = fma(cA, d.x, v.x);
-                        v.y = fma(cA, d.y, v.y);
+    for (int p = 0; p < P; ++p) {
+        const CellRef cr = cell_ref<R>(m, ok[p], c[p], tb, lane);
+        fr[p] = fi[p] = 0;
+        if (ok[p] && lds_field && !m.one_d) {
+            // getFFelecs' corner order, the weights formed once per lane
+            const CornerSet<R> cs = corner_set<R>(c[p], tb, 0);
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                const cplx<R> v = s_fld[cr.t0 + cs.oxy[q & 3] + cs.oz[q >> 2]];
+                const R wk = cs.xy[q & 3] * cs.z[q >> 2];
+                fr[p] = fma(wk, v.x, fr[p]);
+                fi[p] = fma(wk, v.y, fi[p]);
+            }
+        } else if (ok[p]) {
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                if (q < nnb) {
+                    cplx<R> v;
+                    if (lds_field) {
+                        v = s_fld[corner_tile(m, tb, cr, q)];
+                    } else {
+                        const int node = corner_node(m, cr, q);
+                        v = a.A0[node];
+                        if (STAGE > 1) {
+                            const cplx<R> d = a.dAin[node];
+                            v.x = fma(cA, d.x, v.x);
+                            v.y = fma(cA, d.y, v.y);
+                        }
                     }
+                    const R wk = corner_weight<R>(m, c[p], q);
+                    fr[p] = fma(wk, v.x, fr[p]);
+                    fi[p] = fma(wk, v.y, fi[p]);
                 }
-                const R wk = corner_weight<R>(m, c, k);
-                fr = fma(wk, v.x, fr);
-                fi = fma(wk, v.y, fi);
             }
         }
+        if (!ph.coupling) { fr[p] = 0; fi[p] = 0; }   // rhs.f90:221-224
+
+        if (!POLE) equations(p);
     }
 
     // ---- deposit w_k s into dA_s (getSource)
     if (ph.field_evolve) {
-        if constexpr (DET) {
-            // n |s| 2^F <= 2^62 keeps every node's integer sums in range
-            const int F = *a.det.shift;
-            const double lim = ldexp(1.0, 62 - F) / (double)a.n;
-            if (ok && (fabs((double)sr) > lim || fabs((double)si) > lim)) atomicOr(a.flags, FLAG_DET_RANGE);
-            scatter_cells_det(m, tb, use_tile, ok, c, cr, (double)sr, (double)si, ldexp(1.0, F), a.det.acc,
-                              reinterpret_cast<unsigned long long*>(s_dep));
-        } else if constexpr (PACKED) {
-            if (use_tile) {
-                scatter_cells_packed(m, tb, ok, c, cr, (float)sr, (float)si, packed_scale_log2(tb.extra),
-                                     reinterpret_cast<cplx<float>*>(a.dAout), s_dep);
-            } else {
-                scatter_cells<R, float>(m, tb, false, ok, c, cr, sr, si, a.dAout, (float*)nullptr);
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+            // the deposit's weights are formed here, not beside the gather's
+            hold(c[p].fx);
+            hold(c[p].fy);
+            hold(c[p].fz);
+            const CellRef cr = cell_ref<R>(m, ok[p], c[p], tb, lane);
+            if constexpr (DET) {
+                // n |s| 2^F <= 2^62 keeps every node's integer sums in range
+                const double lim = ldexp(1.0, 62) / det_scale / (double)a.n;
+                if (ok[p] && (fabs((double)sr[p]) > lim || fabs((double)si[p]) > lim))
+                    atomicOr(a.flags, FLAG_DET_RANGE);
+                if (!use_tile)
+                    det_global_add(m, ok[p], c[p], cr, (double)sr[p], (double)si[p], det_scale, a.det.acc);
+                else if (ok[p])
+                    det_add(m, tb, c[p], cr, (double)sr[p], (double)si[p], det_scale,
+                            reinterpret_cast<unsigned long long*>(s_dep));
+            } else if (!use_tile) {
+                global_add<R>(m, ok[p], c[p], cr, sr[p], si[p], a.dAout);
+            } else if (ok[p]) {
+                if constexpr (PACKED) packed_add(m, tb, c[p], cr, (float)sr[p], (float)si[p], log2S, s_dep);
+                else tile_add<R, D>(m, tb, c[p], cr, sr[p], si[p], s_dep);
             }
-        } else {
-            scatter_cells<R, D>(m, tb, use_tile, ok, c, cr, sr, si, a.dAout, s_dep);
         }
     }
-    if (!in) return;
-    if (!ph.coupling) { fr = 0; fi = 0; }   // rhs.f90:221-224
 
-    // ---- equations (puffin_equations.f90:17-176)
-    const Rates<R> v = rates<R>(ph, dr, pr, pi);
-    R kpr = 0, kpi = 0;
-    double kg = 0.0;
-    if (ph.electrons_evolve) {
-        R bx, by, bz;
-        bfield<R>(a.s, x, y, bx, by, bz);
-        const R facr = (R)fac;
-        const R n2col = (R)a.s.n2col;
-        const R ep2k = (R)(ph.eta * p2 / (ph.kappa * ph.kappa));
-        kpr = (R)ph.inv2rho * (n2col * by - ep2k * fr) + (R)ph.kappa * pi * facr * n2col * bz;
-        kpi = (R)ph.inv2rho * (n2col * bx - ep2k * fi) - (R)ph.kappa * pr * facr * n2col * bz;
-        kg = -ph.rho * fac * 2.0 * ((double)pr * (double)fr + (double)pi * (double)fi);
+    if constexpr (POLE) {   // the hyperbolic functions' registers after the deposit's
+#pragma unroll
+        for (int p = 0; p < P; ++p) equations(p);
     }
-
-    if (STAGE < 4) {
-        a.kout.pr[i] = kpr;
-        a.kout.pi[i] = kpi;
-        a.kout.g[i] = (R)kg;   // FP32 in the mixed form (see KPtrs)
-        // next stage's trial state must lie inside the mesh, else the next
-        // derivs call would raise the flag (checked here, on the rates the
-        // next stage forms again, so that no later kernel writes state when
-        // it does)
-        const R cn = (R)a.cnext;
-        Cell<R> cc;
-        const int nf = locate<R>(m, fma(cn, v.x, x0), fma(cn, v.y, y0), fma(a.cnext, v.z2, z20), cc);
-        if (nf) atomicOr(a.flags, nf);
-    } else {
-        // y = (y0 + h/6 (k1 + 2 (k2 + k3))) + h/6 k4  (puffin_mpi_RK4.f90:274-279, 307-312)
-        if (rejected) return;   // the step is rejected
-        const R h6 = (R)a.h6;
-        a.y0.x[i] = fma(h6, v.x, x0);
-        a.y0.y[i] = fma(h6, v.y, y0);
-        a.y0.z2[i] = fma(a.h6, v.z2, z20);
-        a.y0.pr[i] = fma(h6, kpr, pr0);
-        a.y0.pi[i] = fma(h6, kpi, pi0);
-        a.y0.g[i] = fma(a.h6, kg, g0);
+    if (use_tile) {
+        __syncthreads();
+        if constexpr (DET) det_flush(m, tb, a.det.acc, reinterpret_cast<const unsigned long long*>(s_dep));
+        else if constexpr (PACKED) packed_flush(m, tb, log2S, reinterpret_cast<cplx<float>*>(a.dAout), s_dep);
+        else tile_flush<R, D>(m, tb, a.dAout, s_dep);
     }
 }
 
@@ -397,27 +499,35 @@ __global__ void k_wrap_z2(double* z2, int64_t n, double lenz2) {
 
 // ---- host launchers --------------------------------------------------------
 
-template <typename R>
-void launch_stage(int stage, const StageArgs<R>& a, hipStream_t s) {
-    const int threads = STAGE_THREADS;
-    const int64_t blocks = (a.n + threads - 1) / threads;
-    dim3 grid((unsigned)(blocks > 0 ? blocks : 1));
+template <typename R, int STAGE>
+static void launch_stage_n(const StageArgs<R>& a, hipStream_t s) {
+    const bool pole = stage_pole(a.s.und_type);
+    const int per = stage_per_thread(STAGE, a.n, sizeof(R) == 8 ? PUFF_FP64 : PUFF_MIXED, pole || a.det.acc);
+    const int64_t blocks = stage_workgroups(a.n, per);
+    const dim3 grid((unsigned)(blocks > 0 ? blocks : 1)), thr(STAGE_THREADS);
     if constexpr (sizeof(R) == 8) {
         if (a.det.acc) {
-            switch (stage) {
-                case 1: hipLaunchKernelGGL((k_stage<R, 1, true>), grid, dim3(threads), 0, s, a); break;
-                case 2: hipLaunchKernelGGL((k_stage<R, 2, true>), grid, dim3(threads), 0, s, a); break;
-                case 3: hipLaunchKernelGGL((k_stage<R, 3, true>), grid, dim3(threads), 0, s, a); break;
-                default: hipLaunchKernelGGL((k_stage<R, 4, true>), grid, dim3(threads), 0, s, a); break;
-            }
+            hipLaunchKernelGGL((k_stage<R, STAGE, true, 1, true>), grid, thr, 0, s, a);
             return;
         }
     }
+    if constexpr (sizeof(R) == 4 && STAGE < 4) {
+        if (per > 1) {
+            hipLaunchKernelGGL((k_stage<R, STAGE, false, STAGE_WIDE, false>), grid, thr, 0, s, a);
+            return;
+        }
+    }
+    if (pole) hipLaunchKernelGGL((k_stage<R, STAGE, false, 1, true>), grid, thr, 0, s, a);
+    else hipLaunchKernelGGL((k_stage<R, STAGE, false, 1, false>), grid, thr, 0, s, a);
+}
+
+template <typename R>
+void launch_stage(int stage, const StageArgs<R>& a, hipStream_t s) {
     switch (stage) {
-        case 1: hipLaunchKernelGGL((k_stage<R, 1, false>), grid, dim3(threads), 0, s, a); break;
-        case 2: hipLaunchKernelGGL((k_stage<R, 2, false>), grid, dim3(threads), 0, s, a); break;
-        case 3: hipLaunchKernelGGL((k_stage<R, 3, false>), grid, dim3(threads), 0, s, a); break;
-        default: hipLaunchKernelGGL((k_stage<R, 4, false>), grid, dim3(threads), 0, s, a); break;
+        case 1: return launch_stage_n<R, 1>(a, s);
+        case 2: return launch_stage_n<R, 2>(a, s);
+        case 3: return launch_stage_n<R, 3>(a, s);
+        default: return launch_stage_n<R, 4>(a, s);
     }
 }
 

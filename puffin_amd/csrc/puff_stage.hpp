@@ -15,11 +15,14 @@
 
 namespace puff {
 
-// Cell of one particle and its interpolation fractions.
+// Cell of one particle and its interpolation fractions.  ix and iy share a
+// register (an FFT line fits a workgroup's LDS, so both are below 2^13).
 template <typename R>
 struct Cell {
-    int ix, iy, iz0, iz1;
+    int ixy, iz0;
     R fx, fy, fz;   // x_in2, y_in2, z2_in2
+    __device__ __forceinline__ int ix() const { return ixy & 0xffff; }
+    __device__ __forceinline__ int iy() const { return ixy >> 16; }
 };
 
 // Node and fractions of a particle (getInterps_3D / _1D).  Returns flag bits;
@@ -35,39 +38,50 @@ __device__ __forceinline__ int locate(const MeshGeom& m, R x, R y, double z2,
         long long r = q % m.nzp;
         if (r < 0) r += m.nzp;
         c.iz0 = (int)r;
-        c.iz1 = (c.iz0 + 1 == m.nzp) ? 0 : c.iz0 + 1;
     } else {
         // temporal mesh: z2node >= NZ2 stops the reference
         // (system_interpolation.f90:70-75); z2 < 0 is refused too.
         if (!(zq >= 0.0 && zq <= (double)(m.nzp - 2))) return FLAG_Z2MESH;
         c.iz0 = (int)zq;
-        c.iz1 = c.iz0 + 1;
     }
     const double locz2 = z2 - zq * m.dz2;
     c.fz = (R)(locz2 * m.inv_dz2);
     if (m.one_d) {
-        c.ix = 0;
-        c.iy = 0;
+        c.ixy = 0;
         c.fx = 0;
         c.fy = 0;
         return 0;
     }
-    const R tx = (x + (R)m.halfx) * (R)m.inv_dx;
-    const R ty = (y + (R)m.halfy) * (R)m.inv_dy;
+    const MeshScale<R>& q = m.template scale<R>();
+    const R tx = (x + q.halfx) * q.inv_dx;
+    const R ty = (y + q.halfy) * q.inv_dy;
     const R xq = floor(tx), yq = floor(ty);
     // xnode >= nspinDX .or. xnode < 1 (system_interpolation.f90:60-68)
     if (!(xq >= (R)0 && xq <= (R)(m.nx - 2))) flag |= FLAG_TRANSVERSE;
     if (!(yq >= (R)0 && yq <= (R)(m.ny - 2))) flag |= FLAG_TRANSVERSE;
     if (flag) return flag;
-    c.ix = (int)xq;
-    c.iy = (int)yq;
-    c.fx = (x + (R)m.halfx - xq * (R)m.dx) * (R)m.inv_dx;
-    c.fy = (y + (R)m.halfy - yq * (R)m.dy) * (R)m.inv_dy;
+    c.ixy = (int)xq | ((int)yq << 16);
+    c.fx = (x + q.halfx - xq * q.dx) * q.inv_dx;
+    c.fy = (y + q.halfy - yq * q.dy) * q.inv_dy;
     return 0;
 }
 
+// 1 / a by the hardware's estimate and two Newton steps: within an ulp of the
+// correctly rounded divide, in half its instructions.
+__device__ __forceinline__ double reciprocal(double a) {
+    double r = __builtin_amdgcn_rcp(a);
+    r = fma(r, fma(-a, r, 1.0), r);
+    return fma(r, fma(-a, r, 1.0), r);
+}
+
 // p2 (gamma_to_p2.f90:84-85) and (1 + eta p2) / Gamma of one macroparticle,
-// in FP64, with 1/eta and 1/gamma_r^2 from the host and 1/Gamma formed once.
+// in FP64.  The difference 1/sqrt(D) - 1 loses a factor 1/eta of its digits,
+// so the root and its reciprocal are formed with the bits of the correctly
+// rounded sqrt and divide (no difference in 1.2e7 draws over gamma_r 10 to
+// 1e4 and estimates off by 2^-23): the estimate of 1/sqrt(D), one coupled
+// Newton step for the root r and h = 1/(2 r), one for the residue of r, one
+// for that of 1/r;
+// 28 instructions instead of 45.
 // Without contraction and with its FMAs written out, as in rates(): a stage
 // forms the previous trial state's derivatives of x, y and z2 again, and they
 // are the bits that the previous stage checked its successor's trial position
@@ -78,10 +92,16 @@ struct Drift {
 
 __device__ __forceinline__ Drift drift_of(const Physics& ph, double pr, double pi, double g) {
 #pragma clang fp contract(off)
-    const double invg = 1.0 / g;
-    const double s = fma(ph.aw * ph.aw, fma(pr, pr, pi * pi), 1.0);
-    const double p2 = ((1.0 / sqrt(fma(-(ph.inv_gr2 * invg * invg), s, 1.0))) - 1.0) * ph.inv_eta;
-    return {p2, fma(ph.eta, p2, 1.0) * invg};
+    const double invg = __builtin_amdgcn_div_fixup(reciprocal(g), g, 1.0);   // as 1/g at 0, infinity and NaN
+    const double D = fma(-(ph.inv_gr2 * invg * invg), fma(ph.aw2, fma(pr, pr, pi * pi), 1.0), 1.0);
+    const double y = __builtin_amdgcn_rsq(D);
+    const double r0 = D * y, h0 = 0.5 * y;
+    const double e = fma(-h0, r0, 0.5);
+    const double r1 = fma(r0, e, r0), h1 = fma(h0, e, h0);
+    const double r = fma(fma(-r1, r1, D), h1, r1);
+    const double q = h1 + h1;
+    const double um1 = fma(q, fma(-r, q, 1.0), q) - 1.0;
+    return {um1 * ph.inv_eta, fma(um1, invg, invg)};
 }
 
 // Derivatives of x, y and z2 (puffin_equations.f90:115-117, 144-146, 172):
@@ -96,7 +116,7 @@ template <typename R>
 __device__ __forceinline__ Rates<R> rates(const Physics& ph, const Drift& d, R pr, R pi) {
 #pragma clang fp contract(off)
     if (!ph.electrons_evolve) return {(R)0, (R)0, 0.0};
-    const R v = (R)ph.c_dx * (R)d.fac;
+    const R v = ph.template scale<R>().c_dx * (R)d.fac;
     return {v * pr, -v * pi, d.p2};
 }
 
@@ -113,16 +133,16 @@ struct Trial {
 
 template <typename R, int STAGE>
 __device__ __forceinline__ Trial<R> trial_state(const Physics& ph, R x0, R y0, double z20, R pr0, R pi0, double g0,
-                                                R kr, R ki, R kg, R qr, R qi, R qg, double cin, double cprev) {
+                                                R kr, R ki, R kg, R qr, R qi, R qg, double cin, double cprev, R c,
+                                                R cp) {
     Trial<R> t;
     R ppr = pr0, ppi = pi0;
     double pg = g0;
     if (STAGE > 2) {
-        ppr = fma((R)cprev, qr, pr0);
-        ppi = fma((R)cprev, qi, pi0);
+        ppr = fma(cp, qr, pr0);
+        ppi = fma(cp, qi, pi0);
         pg = fma(cprev, (double)qg, g0);
     }
-    const R c = (R)cin;
     t.v = rates<R>(ph, drift_of(ph, (double)ppr, (double)ppi, pg), ppr, ppi);
     t.x = fma(c, t.v.x, x0);
     t.y = fma(c, t.v.y, y0);
@@ -135,22 +155,24 @@ __device__ __forceinline__ Trial<R> trial_state(const Physics& ph, R x0, R y0, d
 
 // Scaled undulator field at one particle from the stage coefficients
 // (bfields.f90): see stage_scalars() on the host for the coefficient map.
-template <typename R>
+// POLE = false: compiled without the hyperbolic functions of the plane-pole
+// and curved-pole types (15 to 20 registers of a stage kernel).
+template <typename R, bool POLE = true>
 __device__ __forceinline__ void bfield(const StageScalars& s, R x, R y, R& bx,
                                        R& by, R& bz) {
-    if (s.und_type == PUFF_UND_PLANEPOLE) {
-        bx = (R)s.c[3] * y;
-        by = (R)s.c[1] + (R)s.c[4] * x;
-        bz = (R)s.c[2] * sinh((R)s.c[7] * y);
-    } else if (s.und_type == PUFF_UND_CURVED) {
-        const R kx = (R)s.c[5], ky = (R)s.c[6];
-        bx = (R)s.c[0] * sinh(kx * x) * sinh(ky * y) + (R)s.c[3] * y;
-        by = (R)s.c[1] * cosh(kx * x) * cosh(ky * y) + (R)s.c[4] * x;
-        bz = (R)s.c[2] * cosh(kx * x) * sinh(ky * y);
+    if (POLE && s.und_type == PUFF_UND_PLANEPOLE) {
+        bx = s.template coef<R>(3) * y;
+        by = s.template coef<R>(1) + s.template coef<R>(4) * x;
+        bz = s.template coef<R>(2) * sinh(s.template coef<R>(7) * y);
+    } else if (POLE && s.und_type == PUFF_UND_CURVED) {
+        const R kx = s.template coef<R>(5), ky = s.template coef<R>(6);
+        bx = s.template coef<R>(0) * sinh(kx * x) * sinh(ky * y) + s.template coef<R>(3) * y;
+        by = s.template coef<R>(1) * cosh(kx * x) * cosh(ky * y) + s.template coef<R>(4) * x;
+        bz = s.template coef<R>(2) * cosh(kx * x) * sinh(ky * y);
     } else {
-        bx = (R)s.c[0] + (R)s.c[3] * y;
-        by = (R)s.c[1] + (R)s.c[4] * x;
-        bz = (R)s.c[5] * x + (R)s.c[6] * y;
+        bx = s.template coef<R>(0) + s.template coef<R>(3) * y;
+        by = s.template coef<R>(1) + s.template coef<R>(4) * x;
+        bz = s.template coef<R>(5) * x + s.template coef<R>(6) * y;
     }
 }
 
@@ -197,54 +219,70 @@ struct TileBox {
     int extra;     // block maximum of workgroup_box's `extra` (NX = 7)
 };
 
-// NX = 7 also reduces `extra` (a non-negative int per lane) to its block
-// maximum, returned in TileBox::extra.
-template <typename R, int NX = 6>
-__device__ __forceinline__ TileBox workgroup_box(const MeshGeom& m, bool ok, const Cell<R>& c,
-                                                 Box* box, int extra = 0) {
-    __shared__ int s_red[NX][MAX_BOX_WAVES];
-    __shared__ int s_bb[NX];
+// Lane's cell bounds over its macroparticles: x, y, z2 as (lo, -hi), so that
+// every entry reduces by minimum; and `extra` (negated, a block maximum).
+struct LaneBox {
+    int v[7];
+};
+
+__device__ __forceinline__ LaneBox lane_box() {
+    return {{0x7fffffff, 1, 0x7fffffff, 1, 0x7fffffff, 1, 0}};
+}
+
+template <typename R>
+__device__ __forceinline__ void lane_box_add(LaneBox& b, bool ok, const Cell<R>& c, int extra = 0) {
+    if (ok) {
+        b.v[0] = min(b.v[0], c.ix());
+        b.v[1] = min(b.v[1], -c.ix());
+        b.v[2] = min(b.v[2], c.iy());
+        b.v[3] = min(b.v[3], -c.iy());
+        b.v[4] = min(b.v[4], c.iz0);
+        b.v[5] = min(b.v[5], -c.iz0);
+    }
+    b.v[6] = min(b.v[6], -extra);
+}
+
+// NX = 7 also reduces `extra` to its block maximum, returned in
+// TileBox::extra.  One barrier: every thread combines the wavefronts' minima
+// itself (scalar values from there on).
+template <int NX = 6>
+__device__ __forceinline__ TileBox workgroup_box(const MeshGeom& m, const LaneBox& lb, Box* box) {
+    __shared__ int s_red[MAX_BOX_WAVES][8];
     const int lane = threadIdx.x & 63;
     const int wv = threadIdx.x >> 6;
-    // max values are reduced as min of their negatives
     int v[NX];
-    v[0] = ok ? c.ix : 0x7fffffff;
-    v[1] = ok ? -c.ix : 1;
-    v[2] = ok ? c.iy : 0x7fffffff;
-    v[3] = ok ? -c.iy : 1;
-    v[4] = ok ? c.iz0 : 0x7fffffff;
-    v[5] = ok ? -c.iz0 : 1;
-    if constexpr (NX > 6) v[6] = -extra;
+#pragma unroll
+    for (int d = 0; d < NX; ++d) v[d] = wave_min(lb.v[d]);
+    if (lane == 0) {
+#pragma unroll
+        for (int d = 0; d < NX; ++d) s_red[wv][d] = v[d];
+    }
+    __syncthreads();
 #pragma unroll
     for (int d = 0; d < NX; ++d) {
-        v[d] = wave_min(v[d]);
-        if (lane == 0) s_red[d][wv] = v[d];
+        int r = s_red[0][d];
+#pragma unroll
+        for (int k = 1; k < MAX_BOX_WAVES; ++k) r = min(r, s_red[k][d]);
+        v[d] = __builtin_amdgcn_readfirstlane(r);
     }
-    __syncthreads();
-    if (threadIdx.x < NX) {
-        const int d = threadIdx.x;
-        int r = s_red[d][0];
-        for (int k = 1; k < (int)(blockDim.x >> 6); ++k) r = min(r, s_red[d][k]);
-        s_bb[d] = (d & 1) ? -r : r;
-        const bool empty = (d & 1) ? (r == 1) : (r == 0x7fffffff);
-        if (d < 6 && !empty) {
-            Box* b = box + (blockIdx.x % BOX_COPIES);
-            if (d & 1) atomicMax(&b->hi[d >> 1], -r);
-            else atomicMin(&b->lo[d >> 1], r);
-        }
-    }
-    __syncthreads();
     TileBox t;
     t.extra = 0;
-    if constexpr (NX > 6) t.extra = -s_bb[NX - 1];
-    t.any = s_bb[1] >= 0;
-    t.bx0 = s_bb[0];
-    t.by0 = s_bb[2];
-    t.bz0 = s_bb[4];
-    t.hz = s_bb[5];
-    t.tx = t.any ? (m.one_d ? 1 : s_bb[1] - t.bx0 + 2) : 0;
-    t.ty = t.any ? (m.one_d ? 1 : s_bb[3] - t.by0 + 2) : 0;
-    t.tz = t.any ? s_bb[5] - t.bz0 + 2 : 0;
+    if constexpr (NX > 6) t.extra = -v[6];
+    t.any = v[1] <= 0;
+    if (t.any && threadIdx.x < 6) {
+        const int d = threadIdx.x >> 1;
+        Box* b = box + (blockIdx.x % BOX_COPIES);
+        const int lo = d == 0 ? v[0] : (d == 1 ? v[2] : v[4]), hi = d == 0 ? v[1] : (d == 1 ? v[3] : v[5]);
+        if (threadIdx.x & 1) atomicMax(&b->hi[d], -hi);
+        else atomicMin(&b->lo[d], lo);
+    }
+    t.bx0 = v[0];
+    t.by0 = v[2];
+    t.bz0 = v[4];
+    t.hz = -v[5];
+    t.tx = t.any ? (m.one_d ? 1 : -v[1] - t.bx0 + 2) : 0;
+    t.ty = t.any ? (m.one_d ? 1 : -v[3] - t.by0 + 2) : 0;
+    t.tz = t.any ? -v[5] - t.bz0 + 2 : 0;
     return t;
 }
 
@@ -305,17 +343,20 @@ template <typename R>
 __device__ __forceinline__ CellRef cell_ref(const MeshGeom& m, bool ok, const Cell<R>& c,
                                             const TileBox& t, int lane) {
     CellRef r;
+    // the upper z2 plane, wrapping on a periodic mesh (on a temporal mesh
+    // locate keeps iz0 below nzp - 1)
+    const int iz1 = (c.iz0 + 1 == m.nzp) ? 0 : c.iz0 + 1;
     if (m.one_d) {
         r.b0 = ok ? c.iz0 : 0;
-        r.b1 = ok ? c.iz1 : 0;
+        r.b1 = ok ? iz1 : 0;
         r.t0 = ok ? c.iz0 - t.bz0 : 0;
         r.key = ok ? c.iz0 : -1 - lane;
         return r;
     }
     const int ntr = m.nx * m.ny;
-    r.b0 = ok ? c.iz0 * ntr + c.iy * m.nx + c.ix : 0;
-    r.b1 = ok ? c.iz1 * ntr + c.iy * m.nx + c.ix : 0;
-    r.t0 = ok ? ((c.iz0 - t.bz0) * t.ty + (c.iy - t.by0)) * t.tx + (c.ix - t.bx0) : 0;
+    r.b0 = ok ? c.iz0 * ntr + c.iy() * m.nx + c.ix() : 0;
+    r.b1 = ok ? iz1 * ntr + c.iy() * m.nx + c.ix() : 0;
+    r.t0 = ok ? ((c.iz0 - t.bz0) * t.ty + (c.iy() - t.by0)) * t.tx + (c.ix() - t.bx0) : 0;
     r.key = ok ? r.b0 : -1 - lane;
     return r;
 }
@@ -386,92 +427,99 @@ __device__ __forceinline__ int corner_tile(const MeshGeom& m, const TileBox& t, 
     return r.t0 + (k & 1) + ((k & 2) ? t.tx : 0) + ((k & 4) ? t.tx * t.ty : 0);
 }
 
-// out[node_k] += w_k (sr, si) for every lane with a cell (sr = si = 0 on
-// lanes without one).
-//   use_tile: accumulation in an LDS tile over the workgroup's node box
-//             (real parts, then imaginary parts; element type D), then one
-//             global atomic per touched node and component.  Each lane visits the corners in a
-//             rotated order so that lanes of one cell do not hit the same LDS
-//             address in the same instruction.
-//   else:     lanes of a wavefront that share a cell are summed first (runs
-//             of equal keys), then one global atomic per run and corner.
-// s_tile: the LDS tile, 2 elements of type D per node of the box.  use_tile
-// must be block-uniform; every thread of the workgroup must call.
+// The deposit out[node_k] += w_k (sr, si) of a workgroup, in one of two ways
+// (use_tile, block-uniform):
+//   an LDS tile over the workgroup's node box (real parts, then imaginary
+//     parts; element type D), cleared (tile_clear), added to by every lane
+//     with a cell (tile_add) and flushed with one global atomic per touched
+//     node and component (tile_flush), a barrier between each.  Each lane
+//     visits the corners in a rotated order so that lanes of one cell do not
+//     hit the same LDS address in the same instruction;
+//   global_add: lanes of a wavefront that share a cell are summed first (runs
+//     of equal keys), then one global atomic per run and corner (sr = si = 0
+//     on lanes without a cell; all lanes call).
+
+template <typename D>
+__device__ __forceinline__ void tile_clear(D* tile, int words) {
+    for (int q = threadIdx.x; q < words; q += blockDim.x) tile[q] = (D)0;
+}
+
 template <typename R, typename D>
-__device__ __forceinline__ void scatter_cells(const MeshGeom& m, const TileBox& t, bool use_tile,
-                                              bool ok, const Cell<R>& c, const CellRef& cr, R sr,
-                                              R si, cplx<R>* out, D* s_tile) {
+__device__ __forceinline__ void tile_add(const MeshGeom& m, const TileBox& t, const Cell<R>& c, const CellRef& cr,
+                                         R sr, R si, D* s_tile) {
     const int lane = threadIdx.x & 63;
-    const int nnb = m.one_d ? 2 : 8;
-    if (use_tile) {
-        const int nt = t.tx * t.ty * t.tz;
-        for (int q = threadIdx.x; q < 2 * nt; q += blockDim.x) s_tile[q] = (D)0;
-        __syncthreads();
-        if (ok) {
-            const D dsr = (D)sr, dsi = (D)si;
-            if (!m.one_d) {
-                const CornerSet<R> cs = corner_set<R>(c, t, lane & 7);
+    const int nt = t.tx * t.ty * t.tz;
+    const D dsr = (D)sr, dsi = (D)si;
+    if (!m.one_d) {
+        const CornerSet<R> cs = corner_set<R>(c, t, lane & 7);
 #pragma unroll
-                for (int q = 0; q < 8; ++q) {
-                    const D wk = (D)(cs.xy[q & 3] * cs.z[q >> 2]);
-                    const int tk = cr.t0 + cs.oxy[q & 3] + cs.oz[q >> 2];
-                    atomicAdd(&s_tile[tk], wk * dsr);
-                    atomicAdd(&s_tile[nt + tk], wk * dsi);
-                }
-            } else {
-                for (int q = 0; q < nnb; ++q) {
-                    const int k = (q + lane) & (nnb - 1);
-                    const D wk = (D)corner_weight<R>(m, c, k);
-                    const int tk = corner_tile(m, t, cr, k);
-                    atomicAdd(&s_tile[tk], wk * dsr);
-                    atomicAdd(&s_tile[nt + tk], wk * dsi);
-                }
-            }
-        }
-        __syncthreads();
-        // flush: lanes 2j and 2j + 1 take the real and imaginary parts of
-        // node j, so that one atomic instruction covers both parts of 32
-        // nodes (each device-scope atomic is a memory-side request per
-        // 32-byte sector and instruction: half the requests of one
-        // instruction per part)
-        const int ntr = m.nx * m.ny;
-        const BoxDiv bd = box_div(t);
-        R* outc = reinterpret_cast<R*>(out);
-        for (int e = threadIdx.x; e < 2 * nt; e += blockDim.x) {
-            const int q = e >> 1, part = e & 1;
-            const D v = s_tile[part * nt + q];
-            if (v != (D)0) {
-                int lx, ly, lz;
-                box_coords(bd, q, lx, ly, lz);
-                const int node = (t.bz0 + lz) * ntr + (t.by0 + ly) * m.nx + (t.bx0 + lx);
-                atomic_add(outc + 2 * node + part, (R)v);
-            }
+        for (int q = 0; q < 8; ++q) {
+            const D wk = (D)(cs.xy[q & 3] * cs.z[q >> 2]);
+            const int tk = cr.t0 + cs.oxy[q & 3] + cs.oz[q >> 2];
+            atomicAdd(&s_tile[tk], wk * dsr);
+            atomicAdd(&s_tile[nt + tk], wk * dsi);
         }
     } else {
-        const int prev = __shfl_up(cr.key, 1, 64);
-        const bool head = (lane == 0) || (prev != cr.key);
-        const unsigned long long heads = __ballot(head);
-        const unsigned long long after = (lane == 63) ? 0ull : (heads >> (lane + 1));
-        const int seg_end = after ? lane + __builtin_ctzll(after) : 63;
-        const int maxlen = wave_max(head ? seg_end - lane + 1 : 1);
+        for (int q = 0; q < 2; ++q) {
+            const int k = (q + lane) & 1;
+            const D wk = (D)corner_weight<R>(m, c, k);
+            const int tk = corner_tile(m, t, cr, k);
+            atomicAdd(&s_tile[tk], wk * dsr);
+            atomicAdd(&s_tile[nt + tk], wk * dsi);
+        }
+    }
+}
+
+// Lanes 2j and 2j + 1 take the real and imaginary parts of node j, so that one
+// atomic instruction covers both parts of 32 nodes (each device-scope atomic
+// is a memory-side request per 32-byte sector and instruction: half the
+// requests of one instruction per part).
+template <typename R, typename D>
+__device__ __forceinline__ void tile_flush(const MeshGeom& m, const TileBox& t, cplx<R>* out, const D* s_tile) {
+    const int nt = t.tx * t.ty * t.tz;
+    const int ntr = m.nx * m.ny;
+    const BoxDiv bd = box_div(t);
+    R* outc = reinterpret_cast<R*>(out);
+    for (int e = threadIdx.x; e < 2 * nt; e += blockDim.x) {
+        const int q = e >> 1, part = e & 1;
+        const D v = s_tile[part * nt + q];
+        if (v != (D)0) {
+            int lx, ly, lz;
+            box_coords(bd, q, lx, ly, lz);
+            const int node = (t.bz0 + lz) * ntr + (t.by0 + ly) * m.nx + (t.bx0 + lx);
+            atomic_add(outc + 2 * node + part, (R)v);
+        }
+    }
+}
+
+template <typename R>
+__device__ __forceinline__ void global_add(const MeshGeom& m, bool ok, const Cell<R>& c, const CellRef& cr, R sr,
+                                           R si, cplx<R>* out) {
+    const int lane = threadIdx.x & 63;
+    const int nnb = m.one_d ? 2 : 8;
+    const int prev = __shfl_up(cr.key, 1, 64);
+    const bool head = (lane == 0) || (prev != cr.key);
+    const unsigned long long heads = __ballot(head);
+    const unsigned long long after = (lane == 63) ? 0ull : (heads >> (lane + 1));
+    const int seg_end = after ? lane + __builtin_ctzll(after) : 63;
+    const int maxlen = wave_max(head ? seg_end - lane + 1 : 1);
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            if (k < nnb) {
-                const R wk = ok ? corner_weight<R>(m, c, k) : (R)0;
-                R vr = wk * sr, vi = wk * si;
-                for (int o = 1; o < maxlen; o <<= 1) {
-                    const R tr = __shfl_down(vr, o, 64);
-                    const R ti = __shfl_down(vi, o, 64);
-                    if (lane + o <= seg_end) {
-                        vr += tr;
-                        vi += ti;
-                    }
+    for (int k = 0; k < 8; ++k) {
+        if (k < nnb) {
+            const R wk = ok ? corner_weight<R>(m, c, k) : (R)0;
+            R vr = wk * sr, vi = wk * si;
+            for (int o = 1; o < maxlen; o <<= 1) {
+                const R tr = __shfl_down(vr, o, 64);
+                const R ti = __shfl_down(vi, o, 64);
+                if (lane + o <= seg_end) {
+                    vr += tr;
+                    vi += ti;
                 }
-                if (ok && head) {
-                    const int node = corner_node(m, cr, k);
-                    atomic_add(&out[node].x, vr);
-                    atomic_add(&out[node].y, vi);
-                }
+            }
+            if (ok && head) {
+                const int node = corner_node(m, cr, k);
+                atomic_add(&out[node].x, vr);
+                atomic_add(&out[node].y, vi);
             }
         }
     }
@@ -482,13 +530,13 @@ __device__ __forceinline__ void scatter_cells(const MeshGeom& m, const TileBox& 
 // One LDS atomic per corner for both components: each contribution becomes
 // the integers qr = rint(w sr S), qi = rint(w si S) with the workgroup's
 // power-of-two scale S, and qr 2^32 + qi is added to one 64-bit word of the
-// tile.  S keeps every node's sums below 2^30 in magnitude (STAGE_THREADS lanes, each
-// adding at most the workgroup's largest |s| to a node), so the low half
-// never carries into the high half beyond what its sign extension undoes:
-// the word is sum qr 2^32 + sum qi exactly, and sum qi is its low 32 bits
-// read as signed.  Integer sums are exact (and independent of the atomics'
-// order); each contribution is rounded once, to 2^-31 of the largest node
-// sum the scale allows.  The flush divides by S and adds in FP32.
+// tile.  S puts the largest |s| at 2^21 .. 2^22 - 4, so a node's sums, of at
+// most PACK_MAX contributions of at most the largest |s|, stay below 2^31 in
+// magnitude: the low half never carries into the high half beyond what its
+// sign extension undoes, the word is sum qr 2^32 + sum qi exactly, and sum qi
+// is its low 32 bits read as signed.  Integer sums are exact (and independent
+// of the atomics' order); each contribution is rounded once, to 2^-22 of the
+// largest |s|.  The flush divides by S and adds in FP32.
 //
 // In 3-D each contribution (wx wy) (wz s S) is rounded to an integer by one
 // FMA with 1.5 2^23 added (|w s S| < 2^22 puts the sum in [2^23, 2^24), where
@@ -498,55 +546,55 @@ __device__ __forceinline__ void scatter_cells(const MeshGeom& m, const TileBox& 
 constexpr float PACK_MAGIC = 12582912.0f;                      // 1.5 2^23
 constexpr unsigned long long PACK_MAGIC2 = 0x4B4000004B400000ull;   // its pattern, twice
 
-// log2 of S for the workgroup's largest |s| (its bit pattern, max_bits).
+constexpr int PACK_MAX = 512;   // macroparticles of a workgroup
+static_assert(PACK_MAX >= STAGE_THREADS * STAGE_WIDE, "node sums below 2^31");
+
+// log2 of S for the workgroup's largest |s| (its bit pattern, max_bits): with
+// e taken 2^-20 above it, |s| S < 2^22 (1 - 2^-21), so |q| <= 2^22 - 1.
 __device__ __forceinline__ int packed_scale_log2(int max_bits) {
     const float mx = __int_as_float(max_bits);
     if (!(mx > 0.0f)) return 0;
     int e = 0;
-    frexpf(mx, &e);      // mx < 2^e
-    return 30 - STAGE_THREADS_LOG2 - e;   // STAGE_THREADS mx S < 2^30
+    frexpf(mx * 1.00000095367431640625f, &e);
+    return 22 - e;
 }
 
-__device__ __forceinline__ void scatter_cells_packed(const MeshGeom& m, const TileBox& t, bool ok,
-                                                     const Cell<float>& c, const CellRef& cr, float sr,
-                                                     float si, int log2S, cplx<float>* out,
-                                                     unsigned long long* s_tile) {
+__device__ __forceinline__ void packed_add(const MeshGeom& m, const TileBox& t, const Cell<float>& c,
+                                           const CellRef& cr, float sr, float si, int log2S,
+                                           unsigned long long* s_tile) {
     const int lane = threadIdx.x & 63;
-    const int nnb = m.one_d ? 2 : 8;
-    const int nt = t.tx * t.ty * t.tz;
-    for (int q = threadIdx.x; q < nt; q += blockDim.x) s_tile[q] = 0ull;
-    __syncthreads();
-    if (ok) {
-        const float ssr = ldexpf(sr, log2S), ssi = ldexpf(si, log2S);
-        if (!m.one_d) {
-            const CornerSet<float> cs = corner_set<float>(c, t, lane & 7);
-            const float zr[2] = {cs.z[0] * ssr, cs.z[1] * ssr};
-            const float zi[2] = {cs.z[0] * ssi, cs.z[1] * ssi};
+    const float ssr = ldexpf(sr, log2S), ssi = ldexpf(si, log2S);
+    if (!m.one_d) {
+        const CornerSet<float> cs = corner_set<float>(c, t, lane & 7);
+        const float zr[2] = {cs.z[0] * ssr, cs.z[1] * ssr};
+        const float zi[2] = {cs.z[0] * ssi, cs.z[1] * ssi};
 #pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                const float vr = fmaf(cs.xy[q & 3], zr[q >> 2], PACK_MAGIC);
-                const float vi = fmaf(cs.xy[q & 3], zi[q >> 2], PACK_MAGIC);
-                const unsigned long long wq =
-                    (((unsigned long long)__float_as_uint(vr) << 32) | __float_as_uint(vi)) - PACK_MAGIC2;
-                atomicAdd(&s_tile[cr.t0 + cs.oxy[q & 3] + cs.oz[q >> 2]], wq);
-            }
-        } else {
-            for (int q = 0; q < nnb; ++q) {
-                const int k = (q + lane) & (nnb - 1);
-                const float wk = corner_weight<float>(m, c, k);
-                const long long qr = (long long)(int)rintf(wk * ssr);
-                const long long qi = (long long)(int)rintf(wk * ssi);
-                atomicAdd(&s_tile[corner_tile(m, t, cr, k)], (unsigned long long)(qr * 4294967296LL + qi));
-            }
+        for (int q = 0; q < 8; ++q) {
+            const float vr = fmaf(cs.xy[q & 3], zr[q >> 2], PACK_MAGIC);
+            const float vi = fmaf(cs.xy[q & 3], zi[q >> 2], PACK_MAGIC);
+            const unsigned long long wq =
+                (((unsigned long long)__float_as_uint(vr) << 32) | __float_as_uint(vi)) - PACK_MAGIC2;
+            atomicAdd(&s_tile[cr.t0 + cs.oxy[q & 3] + cs.oz[q >> 2]], wq);
+        }
+    } else {
+        for (int q = 0; q < 2; ++q) {
+            const int k = (q + lane) & 1;
+            const float wk = corner_weight<float>(m, c, k);
+            const long long qr = (long long)(int)rintf(wk * ssr);
+            const long long qi = (long long)(int)rintf(wk * ssi);
+            atomicAdd(&s_tile[corner_tile(m, t, cr, k)], (unsigned long long)(qr * 4294967296LL + qi));
         }
     }
-    __syncthreads();
+}
+
+__device__ __forceinline__ void packed_flush(const MeshGeom& m, const TileBox& t, int log2S, cplx<float>* out,
+                                             const unsigned long long* s_tile) {
+    const int nt = t.tx * t.ty * t.tz;
     const int ntr = m.nx * m.ny;
     const BoxDiv bd = box_div(t);
     const float inv = ldexpf(1.0f, -log2S);
     float* outc = reinterpret_cast<float*>(out);
-    // lanes 2j and 2j + 1: real and imaginary part of node j (as in
-    // scatter_cells: one atomic instruction per 32 nodes' both parts)
+    // lanes 2j and 2j + 1: real and imaginary part of node j (as tile_flush)
     for (int e = threadIdx.x; e < 2 * nt; e += blockDim.x) {
         const int q = e >> 1, part = e & 1;
         const long long w = (long long)s_tile[q];
@@ -576,85 +624,85 @@ __device__ __forceinline__ void det_split(double v, double scale, unsigned long 
     lo = (unsigned long long)(long long)rint((t - r) * (double)(1ull << DET_LO_BITS));
 }
 
-// out[node_k] += w_k (sr, si) in fixed point for every lane with a cell.
-// The same two paths as scatter_cells (LDS tile over the workgroup's node
-// box, or runs of lanes that share a cell), with integer adds throughout, so
-// neither the order of the LDS atomics nor that of the global ones changes a
-// bit.  s_tile: DET_WORDS x nt words (Re hi | Re lo | Im hi | Im lo); out:
-// DET_WORDS words per mesh node.
-__device__ __forceinline__ void scatter_cells_det(const MeshGeom& m, const TileBox& t, bool use_tile,
-                                                  bool ok, const Cell<double>& c, const CellRef& cr,
-                                                  double sr, double si, double scale,
-                                                  unsigned long long* out, unsigned long long* s_tile) {
+// The deposit in fixed point: the same two ways as above (LDS tile over the
+// workgroup's node box, or runs of lanes that share a cell), with integer adds
+// throughout, so neither the order of the LDS atomics nor that of the global
+// ones changes a bit.  s_tile: DET_WORDS x nt words (Re hi | Re lo | Im hi |
+// Im lo); out: DET_WORDS words per mesh node.
+__device__ __forceinline__ void det_add(const MeshGeom& m, const TileBox& t, const Cell<double>& c,
+                                        const CellRef& cr, double sr, double si, double scale,
+                                        unsigned long long* s_tile) {
+    const int lane = threadIdx.x & 63;
+    const int nt = t.tx * t.ty * t.tz;
+    auto add = [&](double wk, int tk) {
+        unsigned long long h, l;
+        det_split(wk * sr, scale, h, l);
+        atomicAdd(&s_tile[tk], h);
+        atomicAdd(&s_tile[nt + tk], l);
+        det_split(wk * si, scale, h, l);
+        atomicAdd(&s_tile[2 * nt + tk], h);
+        atomicAdd(&s_tile[3 * nt + tk], l);
+    };
+    if (!m.one_d) {
+        const CornerSet<double> cs = corner_set<double>(c, t, lane & 7);
+#pragma unroll
+        for (int q = 0; q < 8; ++q) add(cs.xy[q & 3] * cs.z[q >> 2], cr.t0 + cs.oxy[q & 3] + cs.oz[q >> 2]);
+    } else {
+        for (int q = 0; q < 2; ++q) {
+            const int k = (q + lane) & 1;
+            add(corner_weight<double>(m, c, k), corner_tile(m, t, cr, k));
+        }
+    }
+}
+
+// Lanes DET_WORDS j .. DET_WORDS j + 3 take the words of node j (one 32-byte
+// sector): one atomic instruction covers 16 nodes.
+__device__ __forceinline__ void det_flush(const MeshGeom& m, const TileBox& t, unsigned long long* out,
+                                          const unsigned long long* s_tile) {
+    const int nt = t.tx * t.ty * t.tz;
+    const int64_t ntr = (int64_t)m.nx * m.ny;
+    const BoxDiv bd = box_div(t);
+    for (int e = threadIdx.x; e < DET_WORDS * nt; e += blockDim.x) {
+        const int q = e / DET_WORDS, j = e % DET_WORDS;
+        const unsigned long long w = s_tile[j * nt + q];
+        if (w) {
+            int lx, ly, lz;
+            box_coords(bd, q, lx, ly, lz);
+            const int64_t node = (int64_t)(t.bz0 + lz) * ntr + (int64_t)(t.by0 + ly) * m.nx + (t.bx0 + lx);
+            atomicAdd(out + DET_WORDS * node + j, w);
+        }
+    }
+}
+
+__device__ __forceinline__ void det_global_add(const MeshGeom& m, bool ok, const Cell<double>& c, const CellRef& cr,
+                                               double sr, double si, double scale, unsigned long long* out) {
     const int lane = threadIdx.x & 63;
     const int nnb = m.one_d ? 2 : 8;
-    if (use_tile) {
-        const int nt = t.tx * t.ty * t.tz;
-        for (int q = threadIdx.x; q < DET_WORDS * nt; q += blockDim.x) s_tile[q] = 0ull;
-        __syncthreads();
-        if (ok) {
-            auto add = [&](double wk, int tk) {
-                unsigned long long h, l;
-                det_split(wk * sr, scale, h, l);
-                atomicAdd(&s_tile[tk], h);
-                atomicAdd(&s_tile[nt + tk], l);
-                det_split(wk * si, scale, h, l);
-                atomicAdd(&s_tile[2 * nt + tk], h);
-                atomicAdd(&s_tile[3 * nt + tk], l);
-            };
-            if (!m.one_d) {
-                const CornerSet<double> cs = corner_set<double>(c, t, lane & 7);
+    const int prev = __shfl_up(cr.key, 1, 64);
+    const bool head = (lane == 0) || (prev != cr.key);
+    const unsigned long long heads = __ballot(head);
+    const unsigned long long after = (lane == 63) ? 0ull : (heads >> (lane + 1));
+    const int seg_end = after ? lane + __builtin_ctzll(after) : 63;
+    const int maxlen = wave_max(head ? seg_end - lane + 1 : 1);
 #pragma unroll
-                for (int q = 0; q < 8; ++q) add(cs.xy[q & 3] * cs.z[q >> 2], cr.t0 + cs.oxy[q & 3] + cs.oz[q >> 2]);
-            } else {
-                for (int q = 0; q < nnb; ++q) {
-                    const int k = (q + lane) & (nnb - 1);
-                    add(corner_weight<double>(m, c, k), corner_tile(m, t, cr, k));
+    for (int k = 0; k < 8; ++k) {
+        if (k < nnb) {
+            const double wk = ok ? corner_weight<double>(m, c, k) : 0.0;
+            unsigned long long w[DET_WORDS];
+            det_split(wk * sr, scale, w[0], w[1]);
+            det_split(wk * si, scale, w[2], w[3]);
+            for (int o = 1; o < maxlen; o <<= 1) {
+#pragma unroll
+                for (int j = 0; j < DET_WORDS; ++j) {
+                    const unsigned long long u = __shfl_down(w[j], o, 64);
+                    if (lane + o <= seg_end) w[j] += u;
                 }
             }
-        }
-        __syncthreads();
-        const int64_t ntr = (int64_t)m.nx * m.ny;
-        const BoxDiv bd = box_div(t);
-        // lanes DET_WORDS j .. DET_WORDS j + 3 take the words of node j (one
-        // 32-byte sector): one atomic instruction covers 16 nodes
-        for (int e = threadIdx.x; e < DET_WORDS * nt; e += blockDim.x) {
-            const int q = e / DET_WORDS, j = e % DET_WORDS;
-            const unsigned long long w = s_tile[j * nt + q];
-            if (w) {
-                int lx, ly, lz;
-                box_coords(bd, q, lx, ly, lz);
-                const int64_t node = (int64_t)(t.bz0 + lz) * ntr + (int64_t)(t.by0 + ly) * m.nx + (t.bx0 + lx);
-                atomicAdd(out + DET_WORDS * node + j, w);
-            }
-        }
-    } else {
-        const int prev = __shfl_up(cr.key, 1, 64);
-        const bool head = (lane == 0) || (prev != cr.key);
-        const unsigned long long heads = __ballot(head);
-        const unsigned long long after = (lane == 63) ? 0ull : (heads >> (lane + 1));
-        const int seg_end = after ? lane + __builtin_ctzll(after) : 63;
-        const int maxlen = wave_max(head ? seg_end - lane + 1 : 1);
+            if (ok && head) {
+                unsigned long long* o = out + DET_WORDS * (int64_t)corner_node(m, cr, k);
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            if (k < nnb) {
-                const double wk = ok ? corner_weight<double>(m, c, k) : 0.0;
-                unsigned long long w[DET_WORDS];
-                det_split(wk * sr, scale, w[0], w[1]);
-                det_split(wk * si, scale, w[2], w[3]);
-                for (int o = 1; o < maxlen; o <<= 1) {
-#pragma unroll
-                    for (int j = 0; j < DET_WORDS; ++j) {
-                        const unsigned long long u = __shfl_down(w[j], o, 64);
-                        if (lane + o <= seg_end) w[j] += u;
-                    }
-                }
-                if (ok && head) {
-                    unsigned long long* o = out + DET_WORDS * (int64_t)corner_node(m, cr, k);
-#pragma unroll
-                    for (int j = 0; j < DET_WORDS; ++j)
-                        if (w[j]) atomicAdd(o + j, w[j]);
-                }
+                for (int j = 0; j < DET_WORDS; ++j)
+                    if (w[j]) atomicAdd(o + j, w[j]);
             }
         }
     }
