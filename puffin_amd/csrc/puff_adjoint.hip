@@ -154,7 +154,8 @@ __global__ __launch_bounds__(ADJ_THREADS) void k_adj_stage(AdjArgs<R> a) {
     const int wv = threadIdx.x >> 6;
     LaneBox lb = lane_box();
     lane_box_add<R>(lb, ok, c);
-    const TileBox tb = workgroup_box<6>(m, lb, a.box);
+    __shared__ WaveBoxes s_red;
+    const TileBox tb = workgroup_box<6>(m, lb, a.box, s_red);
     const bool scat = ph.coupling && ph.electrons_evolve;
     const bool use_tile = scat && tile_fits<ADJ_TILE_NODES>(m, tb);
     const int nnb = m.one_d ? 2 : 8;
@@ -240,21 +241,6 @@ __global__ __launch_bounds__(ADJ_THREADS) void k_adj_stage(AdjArgs<R> a) {
     }
     if (!ph.coupling) { fr = 0; fi = 0; }   // rhs.f90:221-224
 
-    // ---- field cotangent of this stage: w_k (dL/dFr, dL/dFi) at the nodes
-    if (scat) {
-        const R sr = ok ? (R)Lfr : (R)0, si = ok ? (R)Lfi : (R)0;
-        if (use_tile) {
-            __shared__ double s_tile[2 * ADJ_TILE_NODES];
-            for (int t = threadIdx.x; t < 2 * tb.tx * tb.ty * tb.tz; t += blockDim.x) s_tile[t] = 0.0;
-            __syncthreads();
-            if (ok) tile_add<R, double>(m, tb, c, cr, sr, si, s_tile);
-            __syncthreads();
-            tile_flush<R, double>(m, tb, a.mAout, s_tile);
-        } else {
-            global_add<R>(m, ok, c, cr, sr, si, a.mAout);
-        }
-    }
-
     // ---- dJ/dn2col of this stage: workgroup sum into a spread accumulator
     {
         double dn = 0.0;
@@ -271,8 +257,6 @@ __global__ __launch_bounds__(ADJ_THREADS) void k_adj_stage(AdjArgs<R> a) {
             if (t != 0.0) atomicAdd(&a.dn2[blockIdx.x % DN2_COPIES], t);
         }
     }
-    if (!in) return;
-
     // ---- particle cotangent mu_s
     double mx = 0, my = 0, mz2 = 0, mpr = 0, mpi = 0, mg = 0;
     if (ok) {
@@ -296,14 +280,14 @@ __global__ __launch_bounds__(ADJ_THREADS) void k_adj_stage(AdjArgs<R> a) {
         my = sy + Lbx * bg[1] + Lby * bg[3] + Lbz * bg[5];
         mz2 = sz;
     }
-    if (STAGE > 1) {
+    if (in && STAGE > 1) {
         a.mout.x[i] = (R)mx;
         a.mout.y[i] = (R)my;
         a.mout.z2[i] = mz2;
         a.mout.pr[i] = (R)mpr;
         a.mout.pi[i] = (R)mpi;
         a.mout.g[i] = mg;
-    } else {
+    } else if (in) {
         // L <- L + mu_1 + mu_2 + mu_3 + mu_4
         a.L.x[i] = (R)((double)a.L.x[i] + mx + (double)a.mnext.x[i] + (double)a.m3.x[i] + (double)a.m4.x[i]);
         a.L.y[i] = (R)((double)a.L.y[i] + my + (double)a.mnext.y[i] + (double)a.m3.y[i] + (double)a.m4.y[i]);
@@ -311,6 +295,27 @@ __global__ __launch_bounds__(ADJ_THREADS) void k_adj_stage(AdjArgs<R> a) {
         a.L.pr[i] = (R)((double)a.L.pr[i] + mpr + (double)a.mnext.pr[i] + (double)a.m3.pr[i] + (double)a.m4.pr[i]);
         a.L.pi[i] = (R)((double)a.L.pi[i] + mpi + (double)a.mnext.pi[i] + (double)a.m3.pi[i] + (double)a.m4.pi[i]);
         a.L.g[i] = a.L.g[i] + mg + a.mnext.g[i] + a.m3.g[i] + a.m4.g[i];
+    }
+
+    // ---- field cotangent of this stage: w_k (dL/dFr, dL/dFi) at the nodes;
+    // last, when nothing else is live
+    if (scat) {
+        const R sr = ok ? (R)Lfr : (R)0, si = ok ? (R)Lfi : (R)0;
+        __shared__ double s_tile[2 * ADJ_TILE_NODES];
+        auto clear = [&](const TileBox& t) { tile_clear(s_tile, 2 * t.tx * t.ty * t.tz); };
+        auto add = [&](const TileBox& t) {
+            hold(c.fx);
+            hold(c.fy);
+            hold(c.fz);
+            if (ok) tile_add<R, double>(m, t, c, cell_ref<R>(m, true, c, t, lane), sr, si, s_tile);
+        };
+        auto flush = [&](const TileBox& t) { tile_flush<R, double>(m, t, a.mAout, s_tile); };
+        if (use_tile) {
+            clear(tb);
+            __syncthreads();
+        }
+        tile_deposit<ADJ_TILE_NODES>(m, tb, use_tile, s_red, clear, add, flush,
+                                     [&]() { global_add<R>(m, ok, c, cr, sr, si, a.mAout); });
     }
 }
 

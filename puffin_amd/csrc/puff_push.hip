@@ -18,12 +18,6 @@
 
 namespace puff {
 
-// A value through an empty asm statement: computed here, not later.
-template <typename T>
-__device__ __forceinline__ void hold(T& v) {
-    asm volatile("" : "+v"(v));
-}
-
 // One RK4 stage.  STAGE = 1..4 (rk4par's four derivs calls), P macroparticles
 // per thread (STAGE_THREADS apart).  DET: the deterministic fixed-point
 // deposit (FP64 form only; see DetState).
@@ -219,7 +213,8 @@ __global__ __launch_bounds__(STAGE_THREADS) void k_stage(StageArgs<R> a) {
     // ---- node box of this workgroup's cells and the step's active box (and,
     // for the packed fixed-point tile, the workgroup's largest |s|)
     const int lane = threadIdx.x & 63;
-    const TileBox tb = workgroup_box<PACKED ? 7 : 6>(m, lb, a.box);
+    __shared__ WaveBoxes s_red;
+    const TileBox tb = workgroup_box<PACKED ? 7 : 6>(m, lb, a.box, s_red);
     const bool use_tile = ph.field_evolve && tile_fits<TILE>(m, tb);
     if (threadIdx.x == 0 && ph.field_evolve && tb.any && !use_tile) atomicAdd(a.flags + FLAG_WORD_FALLBACK, 1);
 
@@ -321,47 +316,52 @@ __global__ __launch_bounds__(STAGE_THREADS) void k_stage(StageArgs<R> a) {
         }
         if (!ph.coupling) { fr[p] = 0; fi[p] = 0; }   // rhs.f90:221-224
 
-        if (!POLE) equations(p);
+        equations(p);
     }
 
     // ---- deposit w_k s into dA_s (getSource)
-    if (ph.field_evolve) {
+    auto add = [&](const TileBox& t) {
 #pragma unroll
         for (int p = 0; p < P; ++p) {
             // the deposit's weights are formed here, not beside the gather's
             hold(c[p].fx);
             hold(c[p].fy);
             hold(c[p].fz);
-            const CellRef cr = cell_ref<R>(m, ok[p], c[p], tb, lane);
-            if constexpr (DET) {
-                // n |s| 2^F <= 2^62 keeps every node's integer sums in range
-                const double lim = ldexp(1.0, 62) / det_scale / (double)a.n;
-                if (ok[p] && (fabs((double)sr[p]) > lim || fabs((double)si[p]) > lim))
-                    atomicOr(a.flags, FLAG_DET_RANGE);
-                if (!use_tile)
-                    det_global_add(m, ok[p], c[p], cr, (double)sr[p], (double)si[p], det_scale, a.det.acc);
-                else if (ok[p])
-                    det_add(m, tb, c[p], cr, (double)sr[p], (double)si[p], det_scale,
-                            reinterpret_cast<unsigned long long*>(s_dep));
-            } else if (!use_tile) {
-                global_add<R>(m, ok[p], c[p], cr, sr[p], si[p], a.dAout);
-            } else if (ok[p]) {
-                if constexpr (PACKED) packed_add(m, tb, c[p], cr, (float)sr[p], (float)si[p], log2S, s_dep);
-                else tile_add<R, D>(m, tb, c[p], cr, sr[p], si[p], s_dep);
-            }
+            if (!ok[p]) continue;
+            const CellRef cr = cell_ref<R>(m, true, c[p], t, lane);
+            if constexpr (DET)
+                det_add(m, t, c[p], cr, (double)sr[p], (double)si[p], det_scale,
+                        reinterpret_cast<unsigned long long*>(s_dep));
+            else if constexpr (PACKED) packed_add(m, t, c[p], cr, (float)sr[p], (float)si[p], log2S, s_dep);
+            else tile_add<R, D>(m, t, c[p], cr, sr[p], si[p], s_dep);
         }
+    };
+    auto flush = [&](const TileBox& t) {
+        if constexpr (DET) det_flush(m, t, a.det.acc, reinterpret_cast<const unsigned long long*>(s_dep));
+        else if constexpr (PACKED) packed_flush(m, t, log2S, reinterpret_cast<cplx<float>*>(a.dAout), s_dep);
+        else tile_flush<R, D>(m, t, a.dAout, s_dep);
+    };
+    if constexpr (DET) {
+        // n |s| 2^F <= 2^62 keeps every node's integer sums in range
+        const double lim = ldexp(1.0, 62) / det_scale / (double)a.n;
+        if (ph.field_evolve && ok[0] && (fabs((double)sr[0]) > lim || fabs((double)si[0]) > lim))
+            atomicOr(a.flags, FLAG_DET_RANGE);
+    }
+    if (ph.field_evolve) {
+        tile_deposit<TILE>(
+            m, tb, use_tile, s_red, [&](const TileBox& t) { tile_clear(s_dep, WORDS * t.tx * t.ty * t.tz); }, add,
+            flush,
+            [&]() {
+#pragma unroll
+                for (int p = 0; p < P; ++p) {
+                    const CellRef cr = cell_ref<R>(m, ok[p], c[p], tb, lane);
+                    if constexpr (DET)
+                        det_global_add(m, ok[p], c[p], cr, (double)sr[p], (double)si[p], det_scale, a.det.acc);
+                    else global_add<R>(m, ok[p], c[p], cr, sr[p], si[p], a.dAout);
+                }
+            });
     }
 
-    if constexpr (POLE) {   // the hyperbolic functions' registers after the deposit's
-#pragma unroll
-        for (int p = 0; p < P; ++p) equations(p);
-    }
-    if (use_tile) {
-        __syncthreads();
-        if constexpr (DET) det_flush(m, tb, a.det.acc, reinterpret_cast<const unsigned long long*>(s_dep));
-        else if constexpr (PACKED) packed_flush(m, tb, log2S, reinterpret_cast<cplx<float>*>(a.dAout), s_dep);
-        else tile_flush<R, D>(m, tb, a.dAout, s_dep);
-    }
 }
 
 // Start of a step: clear flags and the active box.

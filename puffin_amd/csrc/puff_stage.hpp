@@ -15,6 +15,12 @@
 
 namespace puff {
 
+// A value through an empty asm statement: computed here, not later.
+template <typename T>
+__device__ __forceinline__ void hold(T& v) {
+    asm volatile("" : "+v"(v));
+}
+
 // Cell of one particle and its interpolation fractions.  ix and iy share a
 // register (an FFT line fits a workgroup's LDS, so both are below 2^13).
 template <typename R>
@@ -242,40 +248,21 @@ __device__ __forceinline__ void lane_box_add(LaneBox& b, bool ok, const Cell<R>&
     b.v[6] = min(b.v[6], -extra);
 }
 
-// NX = 7 also reduces `extra` to its block maximum, returned in
-// TileBox::extra.  One barrier: every thread combines the wavefronts' minima
-// itself (scalar values from there on).
-template <int NX = 6>
-__device__ __forceinline__ TileBox workgroup_box(const MeshGeom& m, const LaneBox& lb, Box* box) {
-    __shared__ int s_red[MAX_BOX_WAVES][8];
-    const int lane = threadIdx.x & 63;
-    const int wv = threadIdx.x >> 6;
+// Minima of the workgroup's wavefronts (LDS), for workgroup_box.
+struct WaveBoxes {
+    int v[MAX_BOX_WAVES][8];
+};
+
+// Box of a set of minima, all lanes equal (scalar values from here on).
+template <int NX>
+__device__ __forceinline__ TileBox tile_box(const MeshGeom& m, const int (&r)[NX]) {
     int v[NX];
 #pragma unroll
-    for (int d = 0; d < NX; ++d) v[d] = wave_min(lb.v[d]);
-    if (lane == 0) {
-#pragma unroll
-        for (int d = 0; d < NX; ++d) s_red[wv][d] = v[d];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int d = 0; d < NX; ++d) {
-        int r = s_red[0][d];
-#pragma unroll
-        for (int k = 1; k < MAX_BOX_WAVES; ++k) r = min(r, s_red[k][d]);
-        v[d] = __builtin_amdgcn_readfirstlane(r);
-    }
+    for (int d = 0; d < NX; ++d) v[d] = __builtin_amdgcn_readfirstlane(r[d]);
     TileBox t;
     t.extra = 0;
     if constexpr (NX > 6) t.extra = -v[6];
     t.any = v[1] <= 0;
-    if (t.any && threadIdx.x < 6) {
-        const int d = threadIdx.x >> 1;
-        Box* b = box + (blockIdx.x % BOX_COPIES);
-        const int lo = d == 0 ? v[0] : (d == 1 ? v[2] : v[4]), hi = d == 0 ? v[1] : (d == 1 ? v[3] : v[5]);
-        if (threadIdx.x & 1) atomicMax(&b->hi[d], -hi);
-        else atomicMin(&b->lo[d], lo);
-    }
     t.bx0 = v[0];
     t.by0 = v[2];
     t.bz0 = v[4];
@@ -284,6 +271,47 @@ __device__ __forceinline__ TileBox workgroup_box(const MeshGeom& m, const LaneBo
     t.ty = t.any ? (m.one_d ? 1 : -v[3] - t.by0 + 2) : 0;
     t.tz = t.any ? -v[5] - t.bz0 + 2 : 0;
     return t;
+}
+
+// NX = 7 also reduces `extra` to its block maximum, returned in
+// TileBox::extra.  One barrier: every thread combines the wavefronts' minima
+// itself.
+template <int NX = 6>
+__device__ __forceinline__ TileBox workgroup_box(const MeshGeom& m, const LaneBox& lb, Box* box, WaveBoxes& s_red) {
+    const int lane = threadIdx.x & 63;
+    const int wv = threadIdx.x >> 6;
+    int v[NX];
+#pragma unroll
+    for (int d = 0; d < NX; ++d) v[d] = wave_min(lb.v[d]);
+    if (lane == 0) {
+#pragma unroll
+        for (int d = 0; d < NX; ++d) s_red.v[wv][d] = v[d];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int d = 0; d < NX; ++d) {
+        int r = s_red.v[0][d];
+#pragma unroll
+        for (int k = 1; k < MAX_BOX_WAVES; ++k) r = min(r, s_red.v[k][d]);
+        v[d] = r;
+    }
+    const TileBox t = tile_box<NX>(m, v);
+    if (t.any && threadIdx.x < 6) {
+        const int d = threadIdx.x >> 1;
+        Box* b = box + (blockIdx.x % BOX_COPIES);
+        const int lo = d == 0 ? v[0] : (d == 1 ? v[2] : v[4]), hi = d == 0 ? v[1] : (d == 1 ? v[3] : v[5]);
+        if (threadIdx.x & 1) atomicMax(&b->hi[d], -hi);
+        else atomicMin(&b->lo[d], lo);
+    }
+    return t;
+}
+
+// Box of wavefront k of the workgroup.
+__device__ __forceinline__ TileBox wave_box(const MeshGeom& m, const WaveBoxes& s_red, int k) {
+    int v[6];
+#pragma unroll
+    for (int d = 0; d < 6; ++d) v[d] = s_red.v[k][d];
+    return tile_box<6>(m, v);
 }
 
 // Node q of a box -> (lx, ly, lz), x fastest, without integer division: the
@@ -427,17 +455,21 @@ __device__ __forceinline__ int corner_tile(const MeshGeom& m, const TileBox& t, 
     return r.t0 + (k & 1) + ((k & 2) ? t.tx : 0) + ((k & 4) ? t.tx * t.ty : 0);
 }
 
-// The deposit out[node_k] += w_k (sr, si) of a workgroup, in one of two ways
-// (use_tile, block-uniform):
+// The deposit out[node_k] += w_k (sr, si) of a workgroup, in one of three ways:
 //   an LDS tile over the workgroup's node box (real parts, then imaginary
 //     parts; element type D), cleared (tile_clear), added to by every lane
 //     with a cell (tile_add) and flushed with one global atomic per touched
 //     node and component (tile_flush), a barrier between each.  Each lane
 //     visits the corners in a rotated order so that lanes of one cell do not
 //     hit the same LDS address in the same instruction;
-//   global_add: lanes of a wavefront that share a cell are summed first (runs
-//     of equal keys), then one global atomic per run and corner (sr = si = 0
-//     on lanes without a cell; all lanes call).
+//   where the workgroup's box does not fit the tile, the same for one
+//     wavefront after the other (tile_deposit): a run of slots that crosses
+//     from one row of bricks to the next has a box across the whole beam, but
+//     only in the one wavefront that holds the crossing;
+//   global_add, for a wavefront whose own box does not fit: lanes of a
+//     wavefront that share a cell are summed first (runs of equal keys), then
+//     one global atomic per run and corner (sr = si = 0 on lanes without a
+//     cell; all lanes call).
 
 template <typename D>
 __device__ __forceinline__ void tile_clear(D* tile, int words) {
@@ -522,6 +554,41 @@ __device__ __forceinline__ void global_add(const MeshGeom& m, bool ok, const Cel
                 atomic_add(&out[node].y, vi);
             }
         }
+    }
+}
+
+// The tile deposits of a workgroup: add(t) (the lanes of the box t) and
+// flush(t), once for the whole workgroup when its box fits the tile (which is
+// clear then, a barrier passed), else for one wavefront after the other, with
+// clear(t) before and spill() on the lanes of a wavefront whose own box does
+// not fit.  One loop for both, so that the code is there once: the two
+// together, inlined, took 18 to 40 registers more.
+// 2^20 macroparticles on 129 x 129 x 1024 (14 to 23 % of the FP64 workgroups
+// do not fit, 5 % of the mixed ones): a stage 200 us (mixed 89) with global
+// atomics for the whole workgroup, 97 (62) wavefront by wavefront; 2 10^5 of
+// them (all workgroups): 147 and 80 us.  With 2^24 (0.8 and 0.3 %) no change.
+template <int TILE, typename C, typename A, typename F, typename S>
+__device__ __forceinline__ void tile_deposit(const MeshGeom& m, const TileBox& tb, bool whole,
+                                             const WaveBoxes& s_red, C clear, A add, F flush, S spill) {
+    const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int groups = whole ? 1 : MAX_BOX_WAVES;
+#pragma unroll 1
+    for (int k = 0; k < groups; ++k) {
+        TileBox t = tb;
+        if (!whole) {
+            t = wave_box(m, s_red, k);
+            if (!t.any) continue;
+            if (!tile_fits<TILE>(m, t)) {
+                if (wv == k) spill();
+                continue;
+            }
+            __syncthreads();   // the tile may be in use
+            clear(t);
+            __syncthreads();
+        }
+        if (whole || wv == k) add(t);
+        __syncthreads();
+        flush(t);
     }
 }
 
