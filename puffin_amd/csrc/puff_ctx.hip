@@ -69,6 +69,7 @@ struct Ctx {
     double* kx = nullptr;
     double* ky = nullptr;
     double* kz = nullptr;
+    double phase_rate = 0;   // largest (kx^2 + ky^2) / |2 kz|, kz != 0
     double* kzr = nullptr;   // 1/(2 kz), 1/sqrt|2 kz| per kz (the mixed form's spectral factor)
     double* mxy = nullptr;
     double* mz = nullptr;
@@ -681,6 +682,14 @@ static int create(Ctx* c) {
                 kzr[2 * i + 1] = 1.0 / std::sqrt(std::fabs(2.0 * kz[i]));
             }
         }
+        auto largest = [](const std::vector<double>& k) {
+            double m = 0.0;
+            for (double v : k) m = std::max(m, v * v);
+            return m;
+        };
+        for (size_t i = 0; i < kz.size(); ++i)
+            if (kz[i] != 0.0)
+                c->phase_rate = std::max(c->phase_rate, (largest(kx) + largest(ky)) * std::fabs(kzr[2 * i]));
         PUFF_TRY(dalloc(c, (void**)&c->kzr, sizeof(double) * kzr.size()));
         PUFF_HIP(hipMemcpy(c->kzr, kzr.data(), sizeof(double) * kzr.size(), hipMemcpyHostToDevice));
         PUFF_HIP(hipMemcpy(c->mxy, mxy.data(), sizeof(double) * mxy.size(), hipMemcpyHostToDevice));
@@ -979,6 +988,7 @@ static int diffraction(Ctx* c, double h) {
     a.ky = c->ky;
     a.kz = c->kz;
     a.kzr = c->kzr;
+    a.phase_max = std::fabs(h) * c->phase_rate;
     a.mxy = c->mxy;
     a.mz = c->mz;
     a.nx = c->p.nx;
@@ -1592,6 +1602,7 @@ static int diffraction_adjoint(Ctx* c, double h) {
     a.ky = c->ky;
     a.kz = c->kz;
     a.kzr = c->kzr;
+    a.phase_max = std::fabs(h) * c->phase_rate;
     a.mxy = c->mxy;
     a.mz = c->mz;
     a.nx = c->p.nx;

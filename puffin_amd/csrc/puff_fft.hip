@@ -38,24 +38,16 @@ namespace puff {
 #ifndef PUFF_LDS_PAD_X
 #define PUFF_LDS_PAD_X 1
 #endif
-//
-// SW (interleaved buffers of the z2 passes, 0: none) swizzles instead of
-// padding: flat index e becomes e ^ ((e >> (SW & 255)) & (SW >> 8)).  With
-// B lines interleaved, the first radix-16 pass writes lane i's outputs 16 B
-// elements apart (512 bytes for two FP64 or four FP32 lines: one LDS bank);
-// XOR-ing the block number 16 B (shift log2(16 B)) into the low bits, within
-// the block, puts the lanes on different banks.  A padded buffer would need
-// 3 % more LDS, one workgroup per CU fewer at 32 KiB.
-template <bool IL, int SW = 0>
+template <bool IL>
 __host__ __device__ constexpr int lpad(int e) {
-    return (!IL && PUFF_LDS_PAD_X) ? e + (e >> 4) : ((IL && SW) ? e ^ ((e >> (SW & 255)) & (SW >> 8)) : e);
+    return (!IL && PUFF_LDS_PAD_X) ? e + (e >> 4) : e;
 }
 
 // LDS index of element j of line b.  Interleaved layout (b fastest) keeps
 // the strided y / z2 loads conflict free; line-major suits contiguous x lines.
-template <bool IL, int SW = 0>
+template <bool IL>
 __device__ __forceinline__ int lidx(int b, int j, int B, int N) {
-    return lpad<IL, SW>(IL ? j * B + b : b * N + j);
+    return lpad<IL>(IL ? j * B + b : b * N + j);
 }
 
 // Line staging between global memory and LDS with U loads (or stores) per
@@ -71,7 +63,7 @@ constexpr int STAGE_UNROLL = 8;
 #endif
 
 // dst[lpad<IL>(w)] = get(w) for 0 <= w < n.
-template <bool IL, int U, int SW = 0, typename R, typename F>
+template <bool IL, int U, typename R, typename F>
 __device__ __forceinline__ void lds_fill(cplx<R>* dst, int n, F get) {
     for (int w0 = threadIdx.x; w0 < n; w0 += U * (int)blockDim.x) {
         cplx<R> v[U];
@@ -83,7 +75,7 @@ __device__ __forceinline__ void lds_fill(cplx<R>* dst, int n, F get) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int w = w0 + u * (int)blockDim.x;
-            if (w < n) dst[lpad<IL, SW>(w)] = v[u];
+            if (w < n) dst[lpad<IL>(w)] = v[u];
         }
     }
 }
@@ -92,14 +84,14 @@ __device__ __forceinline__ void lds_fill(cplx<R>* dst, int n, F get) {
 // (element 0 stands in past n), so that v stays in registers: with
 // conditional reads the compiler kept v in scratch memory (144 bytes per
 // lane in FP64).
-template <bool IL, int U, int SW = 0, typename R, typename F>
+template <bool IL, int U, typename R, typename F>
 __device__ __forceinline__ void lds_drain(const cplx<R>* src, int n, F put) {
     for (int w0 = threadIdx.x; w0 < n; w0 += U * (int)blockDim.x) {
         cplx<R> v[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int w = w0 + u * (int)blockDim.x;
-            v[u] = src[lpad<IL, SW>(w < n ? w : 0)];
+            v[u] = src[lpad<IL>(w < n ? w : 0)];
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -185,11 +177,6 @@ struct CtPlan {
     };
 PUFF_CT_PLAN(33, 11, 3)
 PUFF_CT_PLAN(129, 43, 3)
-PUFF_CT_PLAN(128, 16, 4, 2)
-PUFF_CT_PLAN(256, 16, 16)
-PUFF_CT_PLAN(1024, 16, 16, 4)
-PUFF_CT_PLAN(4096, 16, 16, 16)
-PUFF_CT_PLAN(64, 16, 4)   // the four-step sub-lines of 4096-point z2 lines
 #undef PUFF_CT_PLAN
 
 // Direct DFT pass for an odd prime r (a radix pass of lds_pass), folded:
@@ -577,62 +564,49 @@ __device__ __forceinline__ void small_radix(cplx<R>* v, int r, int sign) {
 // into registers, the workgroup passes a barrier, and the outputs overwrite
 // the same buffer.  Half the LDS of the ping-pong form, hence more
 // workgroups per CU.
-template <typename R, bool IL, int KB = 1, int SW = 0>
+template <typename R, bool IL>
 __device__ __forceinline__ void inplace_pass(cplx<R>* buf, int B, int N, int r, int p, const cplx<R>* tw,
                                              int sign, int LD) {
-    // KB butterflies per thread: all their inputs are read into registers
-    // before the barrier, all outputs written after it
     const int T = N / r;
     const int twst = N / (p * r);   // j k twst < N, as in lds_pass
-    int b[KB], ob[KB];
-    bool act[KB];
-    cplx<R> v[KB][16];
-    const int tid = opaque_tid();
+    const int w = opaque_tid();
+    const bool act = w < B * T;
+    int b = 0, ob = 0;
+    cplx<R> v[16];
+    if (act) {
+        int i;
+        if (IL) { b = w % B; i = w / B; } else { i = w % T; b = w / T; }
+        const int k = i % p;
+        ob = (i / p) * p * r + k;
+        if (r == 16) {
 #pragma unroll
-    for (int it = 0; it < KB; ++it) {
-        const int w = tid + it * (int)blockDim.x;
-        act[it] = w < B * T;
-        b[it] = 0;
-        ob[it] = 0;
-        if (act[it]) {
-            int i;
-            if (IL) { b[it] = w % B; i = w / B; } else { i = w % T; b[it] = w / T; }
-            const int k = i % p;
-            ob[it] = (i / p) * p * r + k;
-            if (r == 16) {
-#pragma unroll
-                for (int j = 0; j < 16; ++j) {
-                    v[it][j] = buf[lidx<IL, SW>(b[it], i + j * T, B, LD)];
-                    if (j > 0 && k > 0) v[it][j] = cmul(v[it][j], tw_get(tw, j * k * twst, sign));
-                }
-                dft16(v[it], sign);
-            } else {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    if (j < r) {
-                        v[it][j] = buf[lidx<IL, SW>(b[it], i + j * T, B, LD)];
-                        if (j > 0 && k > 0) v[it][j] = cmul(v[it][j], tw_get(tw, j * k * twst, sign));
-                    }
-                }
-                small_radix(v[it], r, sign);
+            for (int j = 0; j < 16; ++j) {
+                v[j] = buf[lidx<IL>(b, i + j * T, B, LD)];
+                if (j > 0 && k > 0) v[j] = cmul(v[j], tw_get(tw, j * k * twst, sign));
             }
+            dft16(v, sign);
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                if (j < r) {
+                    v[j] = buf[lidx<IL>(b, i + j * T, B, LD)];
+                    if (j > 0 && k > 0) v[j] = cmul(v[j], tw_get(tw, j * k * twst, sign));
+                }
+            }
+            small_radix(v, r, sign);
         }
     }
     __syncthreads();
+    if (act) {
+        if (r == 16) {
 #pragma unroll
-    for (int it = 0; it < KB; ++it) {
-        if (act[it]) {
-            if (r == 16) {
+            for (int q0 = 0; q0 < 4; ++q0)
 #pragma unroll
-                for (int q0 = 0; q0 < 4; ++q0)
+                for (int q1 = 0; q1 < 4; ++q1) buf[lidx<IL>(b, ob + (q0 + 4 * q1) * p, B, LD)] = v[4 * q0 + q1];
+        } else {
 #pragma unroll
-                    for (int q1 = 0; q1 < 4; ++q1)
-                        buf[lidx<IL, SW>(b[it], ob[it] + (q0 + 4 * q1) * p, B, LD)] = v[it][4 * q0 + q1];
-            } else {
-#pragma unroll
-                for (int q = 0; q < 4; ++q)
-                    if (q < r) buf[lidx<IL, SW>(b[it], ob[it] + q * p, B, LD)] = v[it][q];
-            }
+            for (int q = 0; q < 4; ++q)
+                if (q < r) buf[lidx<IL>(b, ob + q * p, B, LD)] = v[q];
         }
     }
 }
@@ -649,42 +623,6 @@ __device__ __forceinline__ void lds_passes_inplace(cplx<R>* buf, int B, int N, i
     }
 }
 
-// Butterflies per thread of an in-place pass of radix r over B lines of N.
-constexpr int inplace_kb(int B, int N, int r, int threads) {
-    return (B * (N / r) + threads - 1) / threads;
-}
-
-// The passes of CtPlan<NC> in place over BC lines stored LD apart, with THR
-// threads per workgroup.
-template <typename R, bool IL, int NC, int BC, int LD = NC, int THR = PUFF_Z_THREADS, int SW = 0, int K = 0,
-          int P = 1>
-__device__ __forceinline__ void ct_passes_inplace(cplx<R>* buf, const cplx<R>* tw, int sign) {
-    if constexpr (K < CtPlan<NC>::np) {
-        constexpr int r = CtPlan<NC>::r[K];
-        constexpr int KB = inplace_kb(BC, NC, r, THR);
-        inplace_pass<R, IL, KB, SW>(buf, BC, NC, r, P, tw, sign, LD);
-        __syncthreads();
-        ct_passes_inplace<R, IL, NC, BC, LD, THR, SW, K + 1, P * r>(buf, tw, sign);
-    }
-}
-
-// The z2 buffers' swizzle (lpad's SW) for B interleaved lines of N points
-// of R: B a power of two whose 16 B elements fill whole 256-byte rows of
-// LDS banks, so that the first radix-16 pass's writes would land on one
-// bank; the block number goes into the low bits.  N a multiple of 16, so
-// that the buffer is whole blocks and the swizzle permutes within it.
-#ifndef PUFF_Z_SWIZZLE
-#define PUFF_Z_SWIZZLE 1
-#endif
-template <typename R, int B, int N>
-constexpr int z_swizzle() {
-    if (!PUFF_Z_SWIZZLE || B <= 0 || (B & (B - 1)) != 0 || N % 16 != 0) return 0;
-    if ((16 * B * (int)sizeof(cplx<R>)) % 256 != 0) return 0;
-    int sh = 0;
-    while ((1 << sh) < 16 * B) ++sh;
-    return sh | ((16 * B - 1) << 8);
-}
-
 template <typename R, bool IL, int NC>
 __device__ __forceinline__ cplx<R>* lds_fft(cplx<R>* src, cplx<R>* dst, int B, const FftAxis& ax,
                                             const cplx<R>* tw, int sign) {
@@ -697,15 +635,14 @@ __device__ __forceinline__ cplx<R>* lds_fft(cplx<R>* src, cplx<R>* dst, int B, c
 }
 
 // z2-line transform: in place (one LDS buffer) or ping-pong.
-template <typename R, bool INPLACE, int NC, int BC>
-__device__ __forceinline__ cplx<R>* z_fft(cplx<R>* src, cplx<R>* dst, int B, const FftAxis& ax,
-                                          const cplx<R>* tw, int sign) {
+template <typename R, bool INPLACE>
+__device__ __forceinline__ cplx<R>* z_fft(cplx<R>* src, cplx<R>* dst, int B, const FftAxis& ax, const cplx<R>* tw,
+                                          int sign) {
     if constexpr (INPLACE) {
-        if constexpr (NC > 0) ct_passes_inplace<R, true, NC, BC, NC, PUFF_Z_THREADS, z_swizzle<R, BC, NC>()>(src, tw, sign);
-        else lds_passes_inplace<R, true>(src, B, ax.n, ax.npass, ax.radix, tw, sign);
+        lds_passes_inplace<R, true>(src, B, ax.n, ax.npass, ax.radix, tw, sign);
         return src;
     } else {
-        return lds_fft<R, true, NC>(src, dst, B, ax, tw, sign);
+        return lds_fft<R, true, 0>(src, dst, B, ax, tw, sign);
     }
 }
 
@@ -1131,61 +1068,101 @@ __global__ __launch_bounds__(256) void k_fft_y(DiffArgs<R> a, int Bp, int sign) 
     });
 }
 
+// Sine and cosine of the propagator's phase, an FP64 number below PHASE_LIMIT:
+// reduced by multiples n of pi / 2 (a double and its remainder, each product
+// in one FMA: exact to 1e-17 while n is), then Taylor sums.  FP64: to x^17 and
+// x^18, with the rounding errors of the reduction and of x^2 carried along:
+// within 9.5e-17 of the true values up to 3e13 (half an ulp of 1 is 1.1e-16).  FP32: the
+// rotated field is rounded to 6e-8 anyway; sums to x^9 and x^10 of the reduced
+// phase rounded to FP32 (|r| <= pi / 4).  40 and 20 instructions without
+// branches; the library's functions carry a second path for large arguments
+// at each of their places in a kernel.
+constexpr double PHASE_LIMIT = 1e13;   // n stays below 2^43
+template <typename R>
+struct SinCos {
+    R s, c;
+};
+template <typename R>
+__device__ __forceinline__ SinCos<R> sincos_phase(double th) {
+    constexpr double hi = 1.57079632679489661923, lo = 6.123233995736766036e-17;
+    const double n = rint(th * 0.63661977236758134308);
+    const double r0 = fma(-n, hi, th);
+    const double r = fma(-n, lo, r0);
+    R sn, cs;
+    if constexpr (sizeof(R) == 8) {
+        const double e = fma(-n, lo, r0 - r);
+        const double z = r * r;
+        double p = fma(z, 1.0 / 355687428096000.0, -1.0 / 1307674368000.0);
+        p = fma(z, p, 1.0 / 6227020800.0);
+        p = fma(z, p, -1.0 / 39916800.0);
+        p = fma(z, p, 1.0 / 362880.0);
+        p = fma(z, p, -1.0 / 5040.0);
+        p = fma(z, p, 1.0 / 120.0);
+        p = fma(z, p, -1.0 / 6.0);
+        sn = r + fma(r * z, p, e);
+        double q = fma(z, -1.0 / 6402373705728000.0, 1.0 / 20922789888000.0);
+        q = fma(z, q, -1.0 / 87178291200.0);
+        q = fma(z, q, 1.0 / 479001600.0);
+        q = fma(z, q, -1.0 / 3628800.0);
+        q = fma(z, q, 1.0 / 40320.0);
+        q = fma(z, q, -1.0 / 720.0);
+        q = fma(z, q, 1.0 / 24.0);
+        const double hz = 0.5 * z, w = 1.0 - hz;
+        cs = w + fma(z * z, q, fma(-r, e, fma(-0.5, fma(r, r, -z), (1.0 - w) - hz)));
+    } else {
+        const float x = (float)r, z = x * x;
+        float p = fmaf(z, 1.0f / 362880.0f, -1.0f / 5040.0f);
+        p = fmaf(z, p, 1.0f / 120.0f);
+        p = fmaf(z, p, -1.0f / 6.0f);
+        sn = fmaf(x * z, p, x);
+        float q = fmaf(z, -1.0f / 3628800.0f, 1.0f / 40320.0f);
+        q = fmaf(z, q, -1.0f / 720.0f);
+        q = fmaf(z, q, 1.0f / 24.0f);
+        q = fmaf(z, q, -0.5f);
+        cs = fmaf(z, q, 1.0f);
+    }
+    const int m = (int)(int64_t)n;
+    const R a = (m & 1) ? cs : sn, b = (m & 1) ? sn : cs;
+    return {(m & 2) ? -a : a, ((m + 1) & 2) ? -b : b};
+}
+
 // The spectral factor between the forward and inverse z2 transforms, at
 // wavenumbers (kx, ky, kz): multiplyexp's propagator (with its filter) or
 // AbsorptionStep's damping.  FP64 form: in FP64, rounded once.  Mixed form
-// (an FP32 field): the propagator phase is formed in FP64 and reduced
-// modulo 2 pi there (Cody-Waite, with 2 pi split into a double and its
-// remainder), so that the FP32 sine and cosine see |r| <= pi; the damping
-// exponent is formed in FP64 and exponentiated in FP32.  FP64 sine, cosine
-// and exponential per node cost C4's event 1.2 ms of 22.7.  The mixed form
-// also takes rz, 1/(2 kz) (propagator) or 1/sqrt|2 kz| (damping), from a
+// (an FP32 field): the propagator phase is formed and reduced in FP64; the
+// damping exponent is formed in FP64 and exponentiated in FP32.  The mixed
+// form also takes rz, 1/(2 kz) (propagator) or 1/sqrt|2 kz| (damping), from a
 // per-wavenumber table (kzr) instead of an FP64 divide and square root per
-// node; the FP64 form ignores it.
-template <typename R>
+// node; the FP64 form ignores it.  SMALL: the phases are below PHASE_LIMIT.
+template <typename R, bool SMALL>
 __device__ __forceinline__ cplx<R> spectral_op(const DiffArgs<R>& a, int op, double kx, double ky, double kz,
                                                double rz, cplx<R> v) {
-    if constexpr (sizeof(R) == 4) {
-        if (op == SPEC_PROPAGATE) {
-            if ((kz > a.cutoff) || (kz < -a.cutoff)) {
-                if (kz != 0.0) {
-                    constexpr double two_pi_hi = 6.283185307179586232;      // 2 pi rounded to double
-                    constexpr double two_pi_lo = 2.4492935982947064e-16;    // 2 pi - two_pi_hi
-                    constexpr double inv_two_pi = 0.15915494309189533577;
-                    const double th = a.h * (kx * kx + ky * ky) * rz;
-                    const double n = rint(th * inv_two_pi);
-                    const double r = fma(-n, two_pi_lo, fma(-n, two_pi_hi, th));
-                    float sn, cs;
-                    sincosf((float)r, &sn, &cs);
-                    v = {cs * v.x - sn * v.y, sn * v.x + cs * v.y};
-                }
-            } else if (a.filter) {
-                v = {0.0f, 0.0f};
-            }
-        } else if (kz != 0.0) {
-            const float f = expf((float)(-a.h * a.beta * (fabs(kx) + fabs(ky)) * rz));
-            v = {f * v.x, f * v.y};
-        }
-        return v;
-    }
     if (op == SPEC_PROPAGATE) {
         // multiplyexp (diffraction.f90:150-168)
         if ((kz > a.cutoff) || (kz < -a.cutoff)) {
             if (kz != 0.0) {
-                const double th = a.h * (kx * kx + ky * ky) / (2.0 * kz);
-                double sn, cs;
-                sincos(th, &sn, &cs);
-                const double vr = (double)v.x, vi = (double)v.y;
-                v = {(R)(cs * vr - sn * vi), (R)(sn * vr + cs * vi)};
+                const double th = sizeof(R) == 4 ? a.h * (kx * kx + ky * ky) * rz : a.h * (kx * kx + ky * ky) / (2.0 * kz);
+                SinCos<R> t;
+                if constexpr (SMALL) {
+                    t = sincos_phase<R>(th);
+                } else {
+                    double sn, cs;
+                    sincos(th, &sn, &cs);
+                    t = {(R)sn, (R)cs};
+                }
+                v = {t.c * v.x - t.s * v.y, t.s * v.x + t.c * v.y};
             }
         } else if (a.filter) {
             v = {(R)0, (R)0};
         }
-    } else {
+    } else if (kz != 0.0) {
         // AbsorptionStep damping (diffraction.f90:484-497)
-        if (kz != 0.0) {
+        if constexpr (sizeof(R) == 4) {
+            const float f = expf((float)(-a.h * a.beta * (fabs(kx) + fabs(ky)) * rz));
+            v = {f * v.x, f * v.y};
+        } else {
             const double f = exp(-a.h * a.beta * (fabs(kx) + fabs(ky)) / (sqrt(fabs(2.0 * kz))));
-            v = {(R)(f * (double)v.x), (R)(f * (double)v.y)};
+            v = {f * v.x, f * v.y};
         }
     }
     return v;
@@ -1193,11 +1170,10 @@ __device__ __forceinline__ cplx<R> spectral_op(const DiffArgs<R>& a, int op, dou
 
 // ---- z2 lines (stride nx ny), B consecutive x per block ----------------------
 // op < 0: plain transform with `sign`; else forward, spectral op, inverse.
-template <typename R, bool INPLACE, int NC, int BC>
-__global__ __launch_bounds__(PUFF_Z_THREADS) void k_fft_z(DiffArgs<R> a, int Bp, int op, int sign) {
+template <typename R, bool INPLACE>
+__global__ __launch_bounds__(PUFF_Z_THREADS) void k_fft_z(DiffArgs<R> a, int B, int op, int sign) {
     extern __shared__ unsigned char smem_raw[];
-    const int N = NC ? NC : a.nzp;
-    const int B = BC ? BC : Bp;
+    const int N = a.nzp;
     const FftAxis& az = a.az;
     cplx<R>* s0 = reinterpret_cast<cplx<R>*>(smem_raw);
     cplx<R>* s1 = INPLACE ? s0 : s0 + lpad<true>(B * N);
@@ -1213,161 +1189,327 @@ __global__ __launch_bounds__(PUFF_Z_THREADS) void k_fft_z(DiffArgs<R> a, int Bp,
     // few lines per workgroup here: the twiddles stay in global memory (L2)
     const cplx<R>* tw = reinterpret_cast<const cplx<R>*>(az.tw);
     cplx<R>* base = a.a + (int64_t)iy * a.nx + x0;
-    // the in-place compile-time passes' swizzled buffer (identity otherwise)
-    constexpr int SW = (INPLACE && NC > 0) ? z_swizzle<R, BC, NC>() : 0;
-    // FP64 compile-time plans: kx and the kz of the thread's elements for the
-    // spectral op, loaded with the lines (a load per element in the spectral
-    // loop waits on the memory latency each time); the thread's elements
-    // share one x-column
-    constexpr int KPT = (sizeof(R) == 8 && NC > 0 && BC > 0 && (BC * NC) % PUFF_Z_THREADS == 0 &&
-                         PUFF_Z_THREADS % BC == 0)
-                            ? (BC * NC) / PUFF_Z_THREADS
-                            : 0;
-    double kzp[KPT > 0 ? KPT : 1];
-    double kxp = 0.0;
-    if constexpr (KPT > 0) {
-        if (op >= 0) {
-            const int b = (int)threadIdx.x % BC;
-            kxp = a.kx[x0 + (b < nb ? b : 0)];
-#pragma unroll
-            for (int it = 0; it < KPT; ++it) kzp[it] = a.kz[((int)threadIdx.x + it * PUFF_Z_THREADS) / BC];
-        }
-    }
-    lds_fill<true, PUFF_Z_UNROLL, SW>(s0, B * N, [&](int w) {
+    lds_fill<true, PUFF_Z_UNROLL>(s0, B * N, [&](int w) {
         const int b = w % B, j = w / B;
         return (b < nb) ? base[(int64_t)j * ntr + b] : cplx<R>{0, 0};
     });
     __syncthreads();
     cplx<R>* res;
     if (op < 0) {
-        res = z_fft<R, INPLACE, NC, BC>(s0, s1, B, az, tw, sign);
+        res = z_fft<R, INPLACE>(s0, s1, B, az, tw, sign);
     } else {
-        res = z_fft<R, INPLACE, NC, BC>(s0, s1, B, az, tw, -1);
+        res = z_fft<R, INPLACE>(s0, s1, B, az, tw, -1);
         const double ky = a.ky[iy];
-        if constexpr (KPT > 0) {
-#pragma unroll
-            for (int it = 0; it < KPT; ++it) {
-                const int w = (int)threadIdx.x + it * PUFF_Z_THREADS;
-                if (w % BC < nb) res[lpad<true, SW>(w)] = spectral_op(a, op, kxp, ky, kzp[it], 0.0, res[lpad<true, SW>(w)]);
-            }
-        } else {
-            for (int w = threadIdx.x; w < B * N; w += blockDim.x) {
-                const int b = w % B, q = w / B;
-                if (b >= nb) continue;
-                const double rz = sizeof(R) == 4 ? a.kzr[2 * q + (op == SPEC_ABSORB ? 1 : 0)] : 0.0;
-                res[lpad<true, SW>(w)] = spectral_op(a, op, a.kx[x0 + b], ky, a.kz[q], rz, res[lpad<true, SW>(w)]);
-            }
+        const bool small_phase = a.phase_max < PHASE_LIMIT;
+        for (int w = threadIdx.x; w < B * N; w += blockDim.x) {
+            const int b = w % B, q = w / B;
+            if (b >= nb) continue;
+            const double rz = sizeof(R) == 4 ? a.kzr[2 * q + (op == SPEC_ABSORB ? 1 : 0)] : 0.0;
+            const cplx<R> v = res[lpad<true>(w)];
+            res[lpad<true>(w)] = small_phase ? spectral_op<R, true>(a, op, a.kx[x0 + b], ky, a.kz[q], rz, v)
+                                             : spectral_op<R, false>(a, op, a.kx[x0 + b], ky, a.kz[q], rz, v);
         }
         __syncthreads();
         cplx<R>* other = (res == s0) ? s1 : s0;
-        res = z_fft<R, INPLACE, NC, BC>(res, other, B, az, tw, +1);
+        res = z_fft<R, INPLACE>(res, other, B, az, tw, +1);
     }
-    lds_drain<true, PUFF_Z_UNROLL, SW>(res, B * N, [&](int w, const cplx<R>& v) {
+    lds_drain<true, PUFF_Z_UNROLL>(res, B * N, [&](int w, const cplx<R>& v) {
         const int b = w % B, j = w / B;
         if (b < nb) base[(int64_t)j * ntr + b] = v;
     });
 }
 
-// ---- z2 lines of 4096 points as 64 x 64 (four-step) ---------------------------
-// A 4096-point line fills 32 KiB of LDS (FP32), so a single-pass workgroup
-// holds one or two x-columns and reads 8 or 16 useful bytes of every cache
-// line of the 4096 planes it visits (C4's z2 pass fetched 1.4x and wrote
-// 3.5x its bytes).  Split as n = 64 n1 + n2, k = k1 + 64 k2:
-//   X[k1 + 64 k2] = sum_n2 W64^(n2 k2) W^(n2 k1) sum_n1 x[64 n1 + n2] W64^(n1 k1)
-// (W = exp(-2 pi i / 4096)), the transform runs as passes over 64-point
-// sub-lines, each workgroup holding BX adjacent x-columns (one 128-byte row
-// of every plane it visits) of SETS sub-lines:
-//   Z4_FIRST, set n2: transform over n1 (planes 64 n1 + n2), times
-//     W^(s n2 k1); result k1 back in plane 64 k1 + n2.
-//   Z4_MID, set k1: transform over n2 (planes 64 k1 + n2) -> X[k1 + 64 k2].
-//     With a spectral op: the op at q = k1 + 64 k2, the inverse transform
-//     over k2 and W^(-n2 k1) (the first steps of the inverse four-step),
-//     back in plane 64 k1 + n2.  Without one (plain transform): X written
-//     to plane k1 + 64 k2 of `out`.
-//   Z4_LAST, set n2: transform over k1 (planes 64 k1 + n2) -> x[64 n1 + n2].
-// Each pass moves the field once through HBM in whole rows.
-enum { Z4_FIRST = 0, Z4_MID = 1, Z4_LAST = 2 };
-constexpr int Z4_M = 64;
-template <typename R, int BX, int SETS, int PASS>
-__global__ __launch_bounds__(PUFF_Z_THREADS) void k_fft_z4(DiffArgs<R> a, int op, int sign, cplx<R>* out) {
-    constexpr int M = Z4_M;
-    constexpr int N = M * M;
-    constexpr int L = BX * SETS;   // sub-lines per workgroup: b = xi + BX si
-    constexpr int NSG = M / SETS;
+// ---- z2 lines of a power of two, in registers ---------------------------------
+// A thread holds 16 points of one column (FP64) or of two neighbouring columns
+// (FP32) of the mesh, 16 bytes per point either way; N / 16 threads share a
+// column group and a workgroup takes BG groups, rows of 16 BG bytes (64 to 512)
+// of every plane.  With N = 16 M, M = 16 L (M = L up to 256 points):
+//   X[q + 16 (q2 + 16 p)] = sum_v W_L^(v p) W_M^(v q2) sum_j W16^(j q2) W_N^(u q) sum_i W16^(i q) x[u + M i],
+// u = v + L j: a 16-point DFT per thread, an exchange, a second one, an
+// exchange, and 16 / L DFTs of L points; after them a thread holds its
+// wavenumbers, applies the spectral factor to them, and the inverse retraces
+// the steps.  Nothing is brought into natural order.  An exchange moves the
+// real parts through LDS and then the imaginary parts, in words of 8 bytes, so
+// that a workgroup's LDS is half of what it holds in registers: two workgroups
+// a CU at 1024 points, one at 4096.
+//   layout 1, of (q, u): q-major, a spare row of BG words after every q;
+//   layout 2, of (v, q, q2): v-major, a spare row after every v.
+// Both spread the lanes of a write and of a read over all banks.
+template <int N>
+struct ZReg {
+    static constexpr int M = N / 16;                                  // threads per column group
+    static constexpr int L = M > 16 ? M / 16 : M;                     // points of the last DFT
+    static constexpr bool TWO = M > 16;                               // two exchanges
+    static constexpr int G = 16 / L;
+    static constexpr int BG = N >= 2048 ? 4 : (N >= 512 ? 8 : 4096 / N);
+    static constexpr int THREADS = M * BG;
+    static constexpr int ROW1 = M * BG + BG;
+    static constexpr int ROW2 = 256 * BG + BG;
+    static constexpr int WORDS = TWO ? (16 * ROW1 > L * ROW2 ? 16 * ROW1 : L * ROW2) : 16 * ROW1;
+    static_assert(L >= 2 && L <= 16 && WORDS * 8 <= 160 * 1024, "128 to 4096 points");
+};
+
+// One component (8 bytes) and one point (16 bytes) of a thread's columns.
+template <typename R>
+struct ZWord;
+template <>
+struct ZWord<double> {
+    static constexpr int C = 1;   // columns
+    using type = double;
+    static __device__ __forceinline__ double pack(double a, double) { return a; }
+    static __device__ __forceinline__ double get(double w, int) { return w; }
+};
+template <>
+struct ZWord<float> {
+    static constexpr int C = 2;
+    struct alignas(8) type {   // (not a vector type: see zreg_exchange)
+        float x, y;
+    };
+    static __device__ __forceinline__ type pack(float a, float b) { return type{a, b}; }
+    static __device__ __forceinline__ float get(type w, int c) { return c ? w.y : w.x; }
+};
+
+struct alignas(8) ZPair {
+    float x, y, z, w;
+};
+
+// The columns' element wr(i) of the thread that writes word wa(i) to element i
+// of the thread that reads that word as ra(i).  Starts and ends with the buffer
+// free.  (The words of two columns are structs and the columns arrays of their
+// own: of vectors built from array elements, and of rows of one array, the
+// compiler makes vector loads of the array, which then stays in memory.)
+template <typename R, typename WA, typename WR, typename RA>
+__device__ __forceinline__ void zreg_exchange(cplx<R> (&v)[16], cplx<R> (&w)[16], typename ZWord<R>::type* buf, WA wa,
+                                              WR wr, RA ra) {
+    cplx<R> tv[16], tw[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) buf[wa(i)] = ZWord<R>::pack(v[wr(i)].x, w[wr(i)].x);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const auto e = buf[ra(i)];
+        tv[i].x = ZWord<R>::get(e, 0);
+        tw[i].x = ZWord<R>::get(e, 1);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 16; ++i) buf[wa(i)] = ZWord<R>::pack(v[wr(i)].y, w[wr(i)].y);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const auto e = buf[ra(i)];
+        v[i] = {tv[i].x, ZWord<R>::get(e, 0)};
+        w[i] = {tw[i].x, ZWord<R>::get(e, 1)};
+    }
+    __syncthreads();
+}
+
+// The G DFTs of L points of v (group g: v[g L ..], natural order in and out).
+template <typename R, int L>
+__device__ __forceinline__ void zreg_last(cplx<R> (&v)[16], int sign) {
+    if constexpr (L == 2) {
+#pragma unroll
+        for (int g = 0; g < 8; ++g) {
+            const cplx<R> t = v[2 * g];
+            v[2 * g] = cadd(t, v[2 * g + 1]);
+            v[2 * g + 1] = csub(t, v[2 * g + 1]);
+        }
+    } else if constexpr (L == 4) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) dft4(v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3], sign);
+    } else if constexpr (L == 8) {
+        const R h = (R)0.70710678118654752440;
+        const R sg = (R)(sign < 0 ? -1 : 1);
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+            cplx<R>* x = v + 8 * g;
+            dft4(x[0], x[2], x[4], x[6], sign);
+            dft4(x[1], x[3], x[5], x[7], sign);
+            const cplx<R> o1 = cmul(x[3], cplx<R>{h, sg * h}), o3 = cmul(x[7], cplx<R>{-h, sg * h});
+            const cplx<R> o2 = (sign < 0) ? cplx<R>{x[5].y, -x[5].x} : cplx<R>{-x[5].y, x[5].x};
+            const cplx<R> e[4] = {x[0], x[2], x[4], x[6]}, o[4] = {x[1], o1, o2, o3};
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                x[k] = cadd(e[k], o[k]);
+                x[4 + k] = csub(e[k], o[k]);
+            }
+        }
+    } else {
+        dft16(v, sign);
+        cplx<R> t[16];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) t[k] = v[dft16_at(k)];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) v[k] = t[k];
+    }
+}
+
+// OP < 0: plain transform with `sign`; else forward, spectral factor (phases
+// below PHASE_LIMIT), inverse.
+template <typename R, int N, int OP>
+__global__ __launch_bounds__(ZReg<N>::THREADS, 4) void k_fft_zreg(DiffArgs<R> a, int sign) {
+    using Z = ZReg<N>;
+    constexpr int C = ZWord<R>::C, M = Z::M, L = Z::L, G = Z::G, BG = Z::BG;
     extern __shared__ unsigned char smem_raw[];
-    cplx<R>* buf = reinterpret_cast<cplx<R>*>(smem_raw);
-    cplx<R>* tw = buf + lpad<true>(L * M);   // W64^e = W^(64 e), e < 64
-    const cplx<R>* twn = reinterpret_cast<const cplx<R>*>(a.az.tw);
-    for (int w = threadIdx.x; w < M; w += blockDim.x) tw[w] = twn[w * (N / M)];
-    // x-blocks fastest, then set groups, then rows: neighbouring x-blocks
-    // share the cache lines at their edges and go to one XCD
-    const int nxb = (a.nx + BX - 1) / BX;
-    const int64_t nblk = (int64_t)nxb * NSG * a.ny;
+    auto* buf = reinterpret_cast<typename ZWord<R>::type*>(smem_raw);
+    // columns counted over x, then y; neighbouring blocks share the cache
+    // lines of every plane, so they go to one XCD
+    const int64_t ntr = (int64_t)a.nx * a.ny;
+    const int64_t nblk = (ntr + BG * C - 1) / (BG * C);
     const int64_t blk = xcd_block(nblk);
     if (blk >= nblk) return;
-    const int x0 = (int)(blk % nxb) * BX;
-    const int sg = (int)((blk / nxb) % NSG) * SETS;
-    const int iy = (int)(blk / ((int64_t)nxb * NSG));
-    const int nb = min(BX, a.nx - x0);
-    const int64_t ntr = (int64_t)a.nx * a.ny;
-    const int64_t row = (int64_t)iy * a.nx + x0;
-    cplx<R>* base = a.a + row;
-    // the spectral op's kz and rz of the workgroup's z2 wavenumbers
-    // (sg + si) + 64 k2, entry si + SETS k2, staged with the line loads (a
-    // load per element in the spectral loop waits on the memory latency
-    // each time)
-    double* kzt = reinterpret_cast<double*>(tw + M);
-    const bool fused = PASS == Z4_MID && op >= 0;
-    // a thread's elements w = tid + 256 u share b = tid mod L (L divides
-    // 256), hence its x-column and kx
-    static_assert(PUFF_Z_THREADS % L == 0, "one x-column per thread");
-    const int xt = ((int)threadIdx.x % L) % BX;
-    double kxt = 0.0;
-    if (fused) {
-        kxt = a.kx[x0 + (xt < nb ? xt : 0)];
-        for (int w = threadIdx.x; w < SETS * M; w += blockDim.x) {
-            const int iz = (sg + w % SETS) + M * (w / SETS);
-            kzt[w] = a.kz[iz];
-            kzt[SETS * M + w] = sizeof(R) == 4 ? a.kzr[2 * iz + (op == SPEC_ABSORB ? 1 : 0)] : 0.0;
+    int b = (int)threadIdx.x % BG, t = (int)threadIdx.x / BG;
+    // the thread's columns, moved back to the mesh's last ones past its end; of
+    // those only the columns that no other thread holds are stored
+    const int64_t col0 = (blk * BG + b) * C;
+    const int64_t col = min(col0, ntr - C);
+    const cplx<R>* tw = reinterpret_cast<const cplx<R>*>(a.az.tw);
+    int q1 = t / L, v1 = t % L;   // (q, v) of the middle step
+    uint32_t off = (uint32_t)((t * ntr + col) * (int64_t)sizeof(cplx<R>));
+    // addresses are formed again after it, not held
+    auto refresh = [&]() { asm volatile("" : "+v"(b), "+v"(t), "+v"(q1), "+v"(v1), "+v"(off)); };
+
+    cplx<R> v[16], w[16];   // the two columns (w: FP32 only)
+    // planes t + M i: a scalar row of planes and the thread's 32-bit offset
+    auto place = [&](int i) { return reinterpret_cast<cplx<R>*>(reinterpret_cast<char*>(a.a + (int64_t)(M * i) * ntr) + off); };
+    auto put = [&](cplx<R>* p, int i) {
+        if constexpr (C == 1) *p = v[i];
+        else *reinterpret_cast<ZPair*>(p) = ZPair{v[i].x, v[i].y, w[i].x, w[i].y};
+    };
+    // element at(i) of the thread to p(i)
+    auto store = [&](auto p, auto at) {
+        if (col0 == col) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) put(p(i), at(i));
+        } else if (C > 1 && col0 == ntr - 1) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) p(i)[C - 1] = w[at(i)];
+        }
+    };
+    // four rotations in flight: all fifteen, loaded at once, spill
+    auto twiddle = [&](int k, int i, int e, int sg) {
+        if (k % 4 == 0) __builtin_amdgcn_sched_barrier(0);
+        const cplx<R> r = tw_get(tw, e, sg);
+        v[i] = cmul(v[i], r);
+        if constexpr (C > 1) w[i] = cmul(w[i], r);
+    };
+    auto dft = [&](int sg) {
+        dft16(v, sg);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (C > 1) {
+            dft16(w, sg);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    auto last = [&](int sg) {
+        zreg_last<R, L>(v, sg);
+        if constexpr (C > 1) zreg_last<R, L>(w, sg);
+    };
+    // words of (q, u), of (v, q 16 + q2), and of the last step's (group, point)
+    auto w1 = [&](int q, int u) { return q * Z::ROW1 + u * BG + b; };
+    auto w2 = [&](int vv, int c) { return vv * Z::ROW2 + c * BG + b; };
+    auto w3 = [&](int i) {
+        const int g = i / L, p = i % L;
+        return Z::TWO ? w2(p, t + M * g) : w1(t + M * g, p);
+    };
+    auto same = [](int i) { return i; };
+    // wavenumber of element i after the last step
+    auto wave = [&](int i) {
+        const int c = t + M * (i / L), p = i % L;
+        return Z::TWO ? (c >> 4) + 16 * (c & 15) + 256 * p : c + 16 * p;
+    };
+
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const cplx<R>* p = place(i);
+        if constexpr (C == 1) {
+            v[i] = *p;
+        } else {   // 16 bytes at once, aligned to the 8 of a node
+            const ZPair e = *reinterpret_cast<const ZPair*>(p);
+            v[i] = {e.x, e.y};
+            w[i] = {e.z, e.w};
         }
     }
-    // plane of element j of set s
-    auto plane = [](int s, int j) { return PASS == Z4_MID ? M * s + j : M * j + s; };
-    constexpr int SW = z_swizzle<R, L, M>();
-    lds_fill<true, (L * M) / PUFF_Z_THREADS, SW>(buf, L * M, [&](int w) {
-        const int b = w % L, j = w / L;
-        const int xi = b % BX, si = b / BX;
-        return xi < nb ? base[(int64_t)plane(sg + si, j) * ntr + xi] : cplx<R>{0, 0};
-    });
-    __syncthreads();
-    ct_passes_inplace<R, true, M, L, M, PUFF_Z_THREADS, SW>(buf, tw, fused ? -1 : sign);
-    if (fused) {
-        const double ky = a.ky[iy];
-        for (int w = threadIdx.x; w < L * M; w += blockDim.x) {
-            const int b = w % L, k2 = w / L;
-            const int xi = b % BX, si = b / BX;
-            if (xi >= nb) continue;
-            const int e = si + SETS * k2;
-            buf[lpad<true, SW>(w)] = spectral_op(a, op, kxt, ky, kzt[e], kzt[SETS * M + e], buf[lpad<true, SW>(w)]);
+    // the plain transform of sign +1 is the conjugate of the conjugate's
+    const bool mirror = OP < 0 && sign > 0;
+    auto conjugate = [&]() {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            v[i].y = -v[i].y;
+            if constexpr (C > 1) w[i].y = -w[i].y;
         }
-        __syncthreads();
-        ct_passes_inplace<R, true, M, L, M, PUFF_Z_THREADS, SW>(buf, tw, +1);
+    };
+    if (mirror) conjugate();
+    dft(-1);
+#pragma unroll
+    for (int q = 1; q < 16; ++q) twiddle(q, dft16_at(q), t * q, -1);
+    if constexpr (Z::TWO) {
+        refresh();
+        zreg_exchange<R>(v, w, buf, [&](int q) { return w1(q, t); }, dft16_at, [&](int j) { return w1(q1, v1 + L * j); });
+        dft(-1);
+        refresh();
+#pragma unroll
+        for (int q = 1; q < 16; ++q) twiddle(q, dft16_at(q), 16 * v1 * q, -1);
+        refresh();
+        zreg_exchange<R>(v, w, buf, [&](int q) { return w2(v1, 16 * q1 + q); }, dft16_at, w3);
+    } else {
+        refresh();
+        zreg_exchange<R>(v, w, buf, [&](int q) { return w1(q, t); }, dft16_at, w3);
     }
-    lds_drain<true, (L * M) / PUFF_Z_THREADS, SW>(buf, L * M, [&](int w, const cplx<R>& v) {
-        const int b = w % L, j = w / L;
-        const int xi = b % BX, si = b / BX;
-        if (xi >= nb) return;
-        const int st = sg + si;
-        if (PASS == Z4_FIRST) {
-            base[(int64_t)plane(st, j) * ntr + xi] = cmul(v, tw_get(twn, st * j, sign));   // W^(s n2 k1)
-        } else if (PASS == Z4_MID && !fused) {
-            out[(int64_t)(st + M * j) * ntr + row + xi] = v;   // X[k1 + 64 k2]
-        } else if (PASS == Z4_MID) {
-            base[(int64_t)plane(st, j) * ntr + xi] = cmul(v, tw_get(twn, st * j, +1));     // W^(-n2 k1)
-        } else {
-            base[(int64_t)plane(st, j) * ntr + xi] = v;
+    refresh();
+    last(-1);
+
+    if constexpr (OP < 0) {
+        if (mirror) conjugate();
+        // every thread of the columns has read them: two barriers back at least
+        store([&](int i) { return a.a + wave(i) * ntr + col; }, same);
+        return;
+    }
+
+    double kx[C], ky[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        kx[c] = a.kx[(col + c) % a.nx];
+        ky[c] = a.ky[(col + c) / a.nx];
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        refresh();
+        const int k = wave(i);
+        const double kz = a.kz[k];
+        const double rz = sizeof(R) == 4 ? a.kzr[2 * k + (OP == SPEC_ABSORB ? 1 : 0)] : 0.0;
+        v[i] = spectral_op<R, true>(a, OP, kx[0], ky[0], kz, rz, v[i]);
+        asm volatile("" : "+v"(v[i].x), "+v"(v[i].y));   // one after the other
+        if constexpr (C > 1) {
+            w[i] = spectral_op<R, true>(a, OP, kx[C - 1], ky[C - 1], kz, rz, w[i]);
+            asm volatile("" : "+v"(w[i].x), "+v"(w[i].y));
         }
-    });
+    }
+
+    refresh();
+    last(+1);
+    if constexpr (Z::TWO) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+            if (i % L) twiddle(i, i, 16 * (i % L) * ((t + M * (i / L)) & 15), +1);
+        refresh();
+        zreg_exchange<R>(v, w, buf, w3, same, [&](int q) { return w2(v1, 16 * q1 + q); });
+        dft(+1);
+        refresh();
+#pragma unroll
+        for (int j = 0; j < 16; ++j) twiddle(j, dft16_at(j), (v1 + L * j) * q1, +1);
+        refresh();
+        zreg_exchange<R>(v, w, buf, [&](int j) { return w1(q1, v1 + L * j); }, dft16_at, [&](int q) { return w1(q, t); });
+    } else {
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+            if (i % L) twiddle(i, i, (i % L) * (t + M * (i / L)), +1);
+        refresh();
+        zreg_exchange<R>(v, w, buf, w3, same, [&](int q) { return w1(q, t); });
+    }
+    dft(+1);
+    refresh();
+    store(place, dft16_at);
 }
 
 // ---- host side -----------------------------------------------------------------
@@ -1437,36 +1579,6 @@ template <typename R, int NC>
 static constexpr int ct_lines_y() {
     return lines_per_block(NC, sizeof(cplx<R>), 16, PUFF_Y_LDS_BUDGET, true);
 }
-// Compile-time plans may give a thread several butterflies of an in-place
-// pass (inplace_pass<KB>), up to Z_MAX_HELD complex values per thread
-// (64 VGPRs), so their lines per workgroup follow the LDS budget alone.
-template <typename R>
-constexpr int z_max_held() { return sizeof(R) == 8 ? 16 : 32; }
-template <typename R, int NC>
-static constexpr ZPlan ct_zplan() {
-    bool inplace = true;
-    for (int k = 0; k < CtPlan<NC>::np; ++k) {
-        const int r = CtPlan<NC>::r[k];
-        if (r != 2 && r != 3 && r != 4 && r != 16) inplace = false;
-    }
-    const size_t elem = sizeof(cplx<R>);
-    int B2 = (int)((PUFF_Z_LDS_BUDGET) / (2 * (size_t)NC * elem));
-    B2 = B2 < 1 ? 1 : (B2 > 16 ? 16 : B2);
-    if (!inplace) return ZPlan{B2, false};
-    int Bi = (int)((PUFF_Z_LDS_BUDGET) / ((size_t)NC * elem));
-    Bi = Bi > 16 ? 16 : Bi;
-    for (; Bi > 1; --Bi) {
-        bool fits = true;
-        for (int k = 0; k < CtPlan<NC>::np; ++k) {
-            const int r = CtPlan<NC>::r[k];
-            if (inplace_kb(Bi, NC, r, PUFF_Z_THREADS) * r > z_max_held<R>()) fits = false;
-        }
-        if (fits) break;
-    }
-    if (Bi >= 1 && Bi >= B2) return ZPlan{Bi, true};
-    return ZPlan{B2, false};
-}
-
 template <typename R, int NC, int BC, int OP>
 static void launch_x_op(const DiffArgs<R>& a, int B, int sign, hipStream_t s) {
     const int64_t nlines = (int64_t)a.ny * a.nzp;
@@ -1540,76 +1652,43 @@ static void run_y(const DiffArgs<R>& a, int sign, hipStream_t s) {
     launch_y<R, 0, 0>(a, B, sign, s);
 }
 
-template <typename R, bool IP, int NC, int BC>
+template <typename R, bool IP>
 static void launch_z(const DiffArgs<R>& a, int B, int op, int sign, hipStream_t s) {
     const size_t sh = (IP ? 1 : 2) * (size_t)lpad<true>(B * a.nzp) * sizeof(cplx<R>);
     const int64_t blocks = xcd_grid((int64_t)((a.nx + B - 1) / B) * a.ny);
-    lds_opt_in(reinterpret_cast<const void*>(&k_fft_z<R, IP, NC, BC>), sh);
-    hipLaunchKernelGGL((k_fft_z<R, IP, NC, BC>), dim3((unsigned)blocks), dim3(PUFF_Z_THREADS), sh, s, a, B, op,
+    lds_opt_in(reinterpret_cast<const void*>(&k_fft_z<R, IP>), sh);
+    hipLaunchKernelGGL((k_fft_z<R, IP>), dim3((unsigned)blocks), dim3(PUFF_Z_THREADS), sh, s, a, B, op,
                        sign);
 }
 
-template <typename R, int NC>
-static bool launch_z_ct(const DiffArgs<R>& a, int op, int sign, hipStream_t s) {
-    if (a.nzp != NC) return false;
-    constexpr ZPlan zp = ct_zplan<R, NC>();
-    launch_z<R, zp.inplace, NC, zp.B>(a, zp.B, op, sign, s);
+// Powers of two from 128 to 4096 points run in registers (k_fft_zreg), other
+// lengths through LDS.
+template <typename R, int N>
+static bool launch_zreg(const DiffArgs<R>& a, int op, int sign, hipStream_t s) {
+    const int64_t ntr = (int64_t)a.nx * a.ny;
+    if (a.nzp != N || ntr < ZWord<R>::C || ntr * (N / 16) * (int64_t)sizeof(cplx<R>) >= ((int64_t)1 << 32) || (op == SPEC_PROPAGATE && !(a.phase_max < PHASE_LIMIT))) return false;
+    using Z = ZReg<N>;
+    constexpr int cols = Z::BG * ZWord<R>::C;
+    const int64_t blocks = xcd_grid((ntr + cols - 1) / cols);
+    auto launch = [&](auto kernel) {
+        lds_opt_in(reinterpret_cast<const void*>(kernel), Z::WORDS * 8);
+        hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(Z::THREADS), Z::WORDS * 8, s, a, sign);
+    };
+    if (op < 0) launch(&k_fft_zreg<R, N, -1>);
+    else if (op == SPEC_ABSORB) launch(&k_fft_zreg<R, N, SPEC_ABSORB>);
+    else launch(&k_fft_zreg<R, N, SPEC_PROPAGATE>);
     return true;
-}
-
-// Four-step z2 transform of 4096-point lines (FP64 always: a whole line and
-// its twiddles do not fit one workgroup's LDS; FP32 unless PUFF_Z4 is 0).
-#ifndef PUFF_Z4
-#define PUFF_Z4 1
-#endif
-#ifndef PUFF_Z4_SETS
-#define PUFF_Z4_SETS 2
-#endif
-template <typename R>
-static bool z4_line(int n) {
-    return n == Z4_M * Z4_M && (sizeof(R) == 8 || PUFF_Z4);
-}
-
-template <typename R, int PASS>
-static void launch_z4(const DiffArgs<R>& a, int op, int sign, cplx<R>* out, hipStream_t s) {
-    constexpr int BX = 128 / (int)sizeof(cplx<R>);   // one 128-byte row per plane
-    constexpr int SETS = PUFF_Z4_SETS;
-    constexpr int L = BX * SETS;
-    static_assert((L * Z4_M) % PUFF_Z_THREADS == 0, "whole loads per thread");
-    // line buffer, twiddles, the middle pass's kz and rz
-    const size_t sh = ((size_t)lpad<true>(L * Z4_M) + Z4_M) * sizeof(cplx<R>) + 2 * SETS * Z4_M * sizeof(double);
-    const int nxb = (a.nx + BX - 1) / BX;
-    const int64_t blocks = xcd_grid((int64_t)nxb * (Z4_M / SETS) * a.ny);
-    lds_opt_in(reinterpret_cast<const void*>(&k_fft_z4<R, BX, SETS, PASS>), sh);
-    hipLaunchKernelGGL((k_fft_z4<R, BX, SETS, PASS>), dim3((unsigned)blocks), dim3(PUFF_Z_THREADS), sh, s, a, op,
-                       sign, out);
-}
-
-// op >= 0: forward, spectral op, inverse, in place.  op < 0: plain transform
-// with `sign`, its middle pass writing to tmp (a field-sized buffer), then
-// copied back.
-template <typename R>
-static void run_z4(const DiffArgs<R>& a, int op, int sign, cplx<R>* tmp, hipStream_t s) {
-    if (op >= 0) {
-        launch_z4<R, Z4_FIRST>(a, op, -1, nullptr, s);
-        launch_z4<R, Z4_MID>(a, op, 0, nullptr, s);
-        launch_z4<R, Z4_LAST>(a, op, +1, nullptr, s);
-    } else {
-        launch_z4<R, Z4_FIRST>(a, op, sign, nullptr, s);
-        launch_z4<R, Z4_MID>(a, op, sign, tmp, s);
-        (void)hipMemcpyAsync(a.a, tmp, sizeof(cplx<R>) * (size_t)a.nx * a.ny * a.nzp, hipMemcpyDeviceToDevice, s);
-    }
 }
 
 template <typename R>
 static void run_z(const DiffArgs<R>& a, int op, int sign, hipStream_t s) {
-    if (z4_line<R>(a.nzp)) return run_z4(a, op, sign, a.anb, s);
-    if (launch_z_ct<R, 1024>(a, op, sign, s) || launch_z_ct<R, 4096>(a, op, sign, s) ||
-        launch_z_ct<R, 128>(a, op, sign, s) || launch_z_ct<R, 256>(a, op, sign, s))
+    if (launch_zreg<R, 128>(a, op, sign, s) || launch_zreg<R, 256>(a, op, sign, s) ||
+        launch_zreg<R, 512>(a, op, sign, s) || launch_zreg<R, 1024>(a, op, sign, s) ||
+        launch_zreg<R, 2048>(a, op, sign, s) || launch_zreg<R, 4096>(a, op, sign, s))
         return;
     const ZPlan zp = z_plan(a.nzp, sizeof(cplx<R>), a.az.rader, a.az.npass, a.az.radix);
-    if (zp.inplace) launch_z<R, true, 0, 0>(a, zp.B, op, sign, s);
-    else launch_z<R, false, 0, 0>(a, zp.B, op, sign, s);
+    if (zp.inplace) launch_z<R, true>(a, zp.B, op, sign, s);
+    else launch_z<R, false>(a, zp.B, op, sign, s);
 }
 
 template <typename R>

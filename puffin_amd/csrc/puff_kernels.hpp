@@ -382,6 +382,7 @@ struct DiffArgs {
     const double* ky;
     const double* kz;
     const double* kzr;   // per kz: 1/(2 kz), 1/sqrt|2 kz| (0 at kz = 0)
+    double phase_max;    // bound of the propagator's phase |h| (kx^2 + ky^2) / |2 kz|
     const double* mxy;   // transverse mask
     const double* mz;    // z2 mask
     int nx, ny, nz2, nzp, periodic, filter;
