@@ -201,7 +201,7 @@ __global__ __launch_bounds__(STAGE_THREADS) void k_stage(StageArgs<R> a) {
             if (in[p] && !rejected) {
                 at(a.y0.x, i) = fma(a.h6_r, v.x, x0[p]);
                 at(a.y0.y, i) = fma(a.h6_r, v.y, y0[p]);
-                at(a.y0.z2, i) = fma(a.h6, v.z2, z20[p]);
+                at(a.y0.z2, i) = fma(a.h6, ph.electrons_evolve ? dr.p2 : 0.0, z20[p]);   // k_4: as it is
             }
         }
         if (flag) atomicOr(a.flags, flag);
@@ -259,8 +259,11 @@ __global__ __launch_bounds__(STAGE_THREADS) void k_stage(StageArgs<R> a) {
             bfield<R, POLE>(a.s, x[p], y[p], bx, by, bz);
             const R facr = (R)fac[p];
             const R n2col = a.s.template strength<R>(), kappa = ph.template scale<R>().kappa, inv2rho = ph.template scale<R>().inv2rho;
-            kpr = inv2rho * (n2col * by - ep2k[p] * fr[p]) + kappa * pi[p] * facr * n2col * bz;
-            kpi = inv2rho * (n2col * bx - ep2k[p] * fi[p]) - kappa * pr[p] * facr * n2col * bz;
+            // the roundings written out: a different contraction moves the
+            // mixed form's p_r by 2e-6 and z2 by 2e-9 over a lattice
+            const R pull_r = inv2rho * fma(n2col, by, -(ep2k[p] * fr[p]));
+            kpr = fma(kappa * pi[p] * facr * n2col, bz, pull_r);
+            kpi = fma(inv2rho, fma(n2col, bx, -(ep2k[p] * fi[p])), -(kappa * pr[p] * facr * n2col * bz));
             kg = -ph.rho * fac[p] * 2.0 * ((double)pr[p] * (double)fr[p] + (double)pi[p] * (double)fi[p]);
         }
         if (STAGE < 4) {

@@ -111,7 +111,8 @@ __device__ __forceinline__ Drift drift_of(const Physics& ph, double pr, double p
 }
 
 // Derivatives of x, y and z2 (puffin_equations.f90:115-117, 144-146, 172):
-// zero when the electrons do not evolve (rhs.f90:301-308).
+// zero when the electrons do not evolve (rhs.f90:301-308).  z2's is rounded to
+// the type of the stored derivatives, as k_1 to k_3 of the momenta are.
 template <typename R>
 struct Rates {
     R x, y;
@@ -123,7 +124,7 @@ __device__ __forceinline__ Rates<R> rates(const Physics& ph, const Drift& d, R p
 #pragma clang fp contract(off)
     if (!ph.electrons_evolve) return {(R)0, (R)0, 0.0};
     const R v = ph.template scale<R>().c_dx * (R)d.fac;
-    return {v * pr, -v * pi, d.p2};
+    return {v * pr, -v * pi, (double)(R)d.p2};
 }
 
 // Trial state y0 + c k_{s-1} of one macroparticle (puffin_mpi_RK4.f90:190-195
