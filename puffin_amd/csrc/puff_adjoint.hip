@@ -325,30 +325,17 @@ __global__ __launch_bounds__(ADJ_THREADS) void k_adj_stage(AdjArgs<R> a) {
 template <typename R>
 __global__ __launch_bounds__(256) void k_adj_combine(AdjCombineArgs<R> a) {
     if (blockIdx.x == 0 && threadIdx.x == 0 && a.flags[0]) atomicOr(a.flags + FLAG_WORD_STICKY, a.flags[0]);
-    const Box b = merged_box(a.box);
-    if (b.hi[0] < 0) return;
-    const int x0 = b.lo[0], x1 = min(b.hi[0] + 1, a.nx - 1);
-    const int y0 = a.one_d ? 0 : b.lo[1], y1 = a.one_d ? 0 : min(b.hi[1] + 1, a.ny - 1);
-    int z0, z1;
-    if (a.periodic) {
-        z0 = 0;
-        z1 = a.nzp - 1;
-    } else {
-        z0 = b.lo[2];
-        z1 = min(b.hi[2] + 1, a.nzp - 1);
-    }
-    const int lx = x1 - x0 + 1, ly = y1 - y0 + 1, lz = z1 - z0 + 1;
-    const int64_t vol = (int64_t)lx * ly * lz;
     const int64_t ntr = (int64_t)a.nx * a.ny;
     const cplx<R> zero = {(R)0, (R)0};
-    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < vol;
-         t += (int64_t)gridDim.x * blockDim.x) {
-        const int ix = x0 + (int)(t % lx);
-        const int64_t r = t / lx;
-        const int iy = y0 + (int)(r % ly);
-        const int iz = z0 + (int)(r / ly);
+    each_active_node(merged_box(a.box), a.nx, a.ny, a.nzp, a.periodic, a.one_d, [&](int ix, int iy, int iz) {
         const int64_t j = (int64_t)iz * ntr + (int64_t)iy * a.nx + ix;
+        if (a.clear_dA) {
+            a.dA[0][j] = zero;
+            a.dA[1][j] = zero;
+            a.dA[2][j] = zero;
+        }
         const cplx<R> m0 = a.mA[0][j], m1 = a.mA[1][j], m2 = a.mA[2][j], m3 = a.mA[3][j];
+        if (all_zero(m0, m1) && all_zero(m2, m3)) return;
         cplx<R> v = a.LA[j];
         v.x = (R)((double)v.x + (double)m0.x + (double)m1.x + (double)m2.x + (double)m3.x);
         v.y = (R)((double)v.y + (double)m0.y + (double)m1.y + (double)m2.y + (double)m3.y);
@@ -357,12 +344,7 @@ __global__ __launch_bounds__(256) void k_adj_combine(AdjCombineArgs<R> a) {
         a.mA[1][j] = zero;
         a.mA[2][j] = zero;
         a.mA[3][j] = zero;
-        if (a.clear_dA) {
-            a.dA[0][j] = zero;
-            a.dA[1][j] = zero;
-            a.dA[2][j] = zero;
-        }
-    }
+    });
 }
 
 // Cotangent of J = sum_iz wz[iz] power(iz), power(iz) = transverse trapezoid

@@ -382,45 +382,31 @@ __global__ void k_step_begin(int* flags, Box* box) {
 // (puffin_mpi_RK4.f90:281-282, 314-315), then clear the deposits there (all
 // four, or only the last when the first three are kept for the adjoint).
 // The periodic mesh keeps its aliased last plane equal to plane 0.
+// Bound by memory: 160 bytes per node in FP64, of which a node that took no
+// deposit (the corners of the box around a round beam) needs only the 64 of
+// the reads.
 template <typename R>
 __global__ __launch_bounds__(256) void k_field_combine(CombineArgs<R> a) {
     if (blockIdx.x == 0 && threadIdx.x == 0 && a.flags[0]) atomicOr(a.flags + FLAG_WORD_STICKY, a.flags[0]);
-    const Box b = merged_box(a.box);
-    if (b.hi[0] < 0) return;   // no particle deposited
-    const int x0 = b.lo[0], x1 = min(b.hi[0] + 1, a.nx - 1);
-    const int y0 = a.one_d ? 0 : b.lo[1], y1 = a.one_d ? 0 : min(b.hi[1] + 1, a.ny - 1);
-    int z0, z1;
-    if (a.periodic) {
-        z0 = 0;
-        z1 = a.nzp - 1;
-    } else {
-        z0 = b.lo[2];
-        z1 = min(b.hi[2] + 1, a.nzp - 1);
-    }
-    const int lx = x1 - x0 + 1, ly = y1 - y0 + 1, lz = z1 - z0 + 1;
-    const int64_t vol = (int64_t)lx * ly * lz;
     const bool update = (*a.flags == 0);
     const R h6 = (R)a.h6;
     const int64_t ntr = (int64_t)a.nx * a.ny;
-    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < vol;
-         t += (int64_t)gridDim.x * blockDim.x) {
-        const int ix = x0 + (int)(t % lx);
-        const int64_t r = t / lx;
-        const int iy = y0 + (int)(r % ly);
-        const int iz = z0 + (int)(r / ly);
+    each_active_node(merged_box(a.box), a.nx, a.ny, a.nzp, a.periodic, a.one_d, [&](int ix, int iy, int iz) {
         const int64_t j = (int64_t)iz * ntr + (int64_t)iy * a.nx + ix;
         const cplx<R> d0 = a.d[0][j], d1 = a.d[1][j], d2 = a.d[2][j], d3 = a.d[3][j];
+        const bool alias = a.periodic && iz == 0;
+        if (all_zero(d0, d1) && all_zero(d2, d3) && !alias) return;
         if (update) {
             cplx<R> v = a.A[j];
             const R tx = d1.x + d2.x, ty = d1.y + d2.y;
             v.x = v.x + h6 * (d0.x + d3.x + (R)2 * tx);
             v.y = v.y + h6 * (d0.y + d3.y + (R)2 * ty);
             a.A[j] = v;
-            if (a.periodic && iz == 0) a.A[(int64_t)(a.nz2 - 1) * ntr + (int64_t)iy * a.nx + ix] = v;
+            if (alias) a.A[(int64_t)(a.nz2 - 1) * ntr + (int64_t)iy * a.nx + ix] = v;
         }
         const cplx<R> zero = {(R)0, (R)0};
         for (int k = a.clear_from; k < 4; ++k) a.d[k][j] = zero;
-    }
+    });
 }
 
 // ---- deterministic deposit ---------------------------------------------------
@@ -464,23 +450,10 @@ __global__ void k_det_shift(unsigned long long* bound, int* shift, int64_t n) {
 // active box so far, clearing the integer sums there.
 __global__ __launch_bounds__(256) void k_det_convert(DetState d, cplx<double>* dA, const Box* box, int nx,
                                                      int ny, int nzp, int periodic, int one_d) {
-    const Box b = merged_box(box);
-    if (b.hi[0] < 0) return;
-    const int x0 = b.lo[0], x1 = min(b.hi[0] + 1, nx - 1);
-    const int y0 = one_d ? 0 : b.lo[1], y1 = one_d ? 0 : min(b.hi[1] + 1, ny - 1);
-    const int z0 = periodic ? 0 : b.lo[2];
-    const int z1 = periodic ? nzp - 1 : min(b.hi[2] + 1, nzp - 1);
-    const int lx = x1 - x0 + 1, ly = y1 - y0 + 1, lz = z1 - z0 + 1;
-    const int64_t vol = (int64_t)lx * ly * lz;
     const int F = *d.shift;
     const double inv_hi = ldexp(1.0, -F), inv_lo = ldexp(1.0, -(F + DET_LO_BITS));
     const int64_t ntr = (int64_t)nx * ny;
-    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < vol;
-         t += (int64_t)gridDim.x * blockDim.x) {
-        const int ix = x0 + (int)(t % lx);
-        const int64_t r = t / lx;
-        const int iy = y0 + (int)(r % ly);
-        const int iz = z0 + (int)(r / ly);
+    each_active_node(merged_box(box), nx, ny, nzp, periodic, one_d, [&](int ix, int iy, int iz) {
         const int64_t j = (int64_t)iz * ntr + (int64_t)iy * nx + ix;
         unsigned long long* w = d.acc + DET_WORDS * j;
         const long long rh = (long long)w[0], rl = (long long)w[1], ih = (long long)w[2], il = (long long)w[3];
@@ -491,7 +464,7 @@ __global__ __launch_bounds__(256) void k_det_convert(DetState d, cplx<double>* d
             w[2] = 0ull;
             w[3] = 0ull;
         }
-    }
+    });
 }
 
 // Periodic z2 wrap (para_field.f90:212-215).

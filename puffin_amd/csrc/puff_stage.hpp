@@ -354,6 +354,40 @@ __device__ __forceinline__ Box merged_box(const Box* box) {
     return b;
 }
 
+// f(ix, iy, iz) for every node that the cells of box b touch (all planes of a
+// periodic mesh), x fastest, over the whole grid of workgroups.  The indexes
+// are split with 32-bit divisions where they fit (a 64-bit one is some hundred
+// instructions).  With the skipped nodes of k_field_combine: 104 -> 97 us on
+// 129 x 129 x 1024 with 2^24 macroparticles (FP64), 56 -> 53 us (mixed).
+template <typename F>
+__device__ __forceinline__ void each_active_node(const Box& b, int nx, int ny, int nzp, int periodic, int one_d, F f) {
+    if (b.hi[0] < 0) return;   // no particle deposited
+    const int x0 = b.lo[0], x1 = min(b.hi[0] + 1, nx - 1);
+    const int y0 = one_d ? 0 : b.lo[1], y1 = one_d ? 0 : min(b.hi[1] + 1, ny - 1);
+    const int z0 = periodic ? 0 : b.lo[2];
+    const int z1 = periodic ? nzp - 1 : min(b.hi[2] + 1, nzp - 1);
+    const uint32_t lx = (uint32_t)(x1 - x0 + 1), ly = (uint32_t)(y1 - y0 + 1);
+    const int64_t vol = (int64_t)lx * ly * (z1 - z0 + 1);
+    const int64_t first = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, step = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t t = first; t < vol; t += step) {
+        uint32_t x, r;
+        if (vol <= 0xffffffffll) {
+            r = (uint32_t)t / lx;
+            x = (uint32_t)t - r * lx;
+        } else {
+            r = (uint32_t)(t / lx);   // a row: fewer than 2^32
+            x = (uint32_t)(t - (int64_t)r * lx);
+        }
+        const uint32_t z = r / ly;
+        f(x0 + (int)x, y0 + (int)(r - z * ly), z0 + (int)z);
+    }
+}
+
+template <typename R>
+__device__ __forceinline__ bool all_zero(const cplx<R>& a, const cplx<R>& b) {
+    return a.x == (R)0 && a.y == (R)0 && b.x == (R)0 && b.y == (R)0;
+}
+
 // Whether the workgroup's node box fits the LDS tile and does not wrap
 // around a periodic mesh (block-uniform).
 template <int TILE>
