@@ -203,28 +203,44 @@ static int powmod(int b, int e, int n) {
     return (int)r;
 }
 
-// Radix passes of an n-point line: prime factors of 5 and more (direct DFT
-// passes) first, largest first, so that the costliest pass runs with p = 1
-// and needs no input twiddles; then 16s, 4s, 2s and 3s.
+// Fewest radices of 2 to 16, each at most `top` and in falling order, with
+// product m (the smallest largest one where the count is the same); the number
+// of them, or 99.
+static int radices(int m, int top, int* out) {
+    if (m == 1) return 0;
+    int best = 99;
+    for (int r = 2; r <= top && r <= m; ++r) {
+        if (m % r) continue;
+        int rest[32];
+        const int k = 1 + radices(m / r, r, rest);
+        if (k < best) {
+            best = k;
+            out[0] = r;
+            std::copy(rest, rest + k - 1, out + 1);
+        }
+    }
+    return best;
+}
+
+// Passes of an n-point transform: prime factors above 13 as direct passes, the
+// rest in the fewest passes of up to 16 points (every pass is a round trip
+// through LDS and a barrier): 420 = 10 x 7 x 6, 90 = 10 x 9, 75 = 15 x 5.
 static void factorize(int n, FftAxis& ax) {
     ax.n = n;
     ax.npass = 0;
     int m = n;
-    int n16 = 0, n4 = 0, n2 = 0, n3 = 0;
-    while (m % 16 == 0) { ++n16; m /= 16; }
-    while (m % 4 == 0) { ++n4; m /= 4; }
-    while (m % 2 == 0) { ++n2; m /= 2; }
-    while (m % 3 == 0) { ++n3; m /= 3; }
+    for (int f : {2, 3, 5, 7, 11, 13})
+        while (m % f == 0) m /= f;
+    const int small = n / m;
     int big[32];
     int nbig = 0;
-    for (int f = 5; m > 1 && (int64_t)f * f <= m; f += 2)
+    for (int f = 17; m > 1 && (int64_t)f * f <= m; f += 2)
         while (m % f == 0) { big[nbig++] = f; m /= f; }
     if (m > 1) big[nbig++] = m;
     for (int k = nbig - 1; k >= 0; --k) ax.radix[ax.npass++] = big[k];
-    for (int k = 0; k < n16; ++k) ax.radix[ax.npass++] = 16;
-    for (int k = 0; k < n4; ++k) ax.radix[ax.npass++] = 4;
-    for (int k = 0; k < n2; ++k) ax.radix[ax.npass++] = 2;
-    for (int k = 0; k < n3; ++k) ax.radix[ax.npass++] = 3;
+    int r[32];
+    const int k = radices(small, 16, r);
+    for (int q = 0; q < k; ++q) ax.radix[ax.npass++] = r[q];
 }
 
 template <typename R>

@@ -119,29 +119,213 @@ __device__ __forceinline__ cplx<R> tw_get(const cplx<R>* tw, int e, int sign) {
     return w;
 }
 
-// 4-point DFT in place (x_k = sum_n x_n W4^(nk), W4 = exp(sign 2 pi i / 4)).
+// Index of X_k in dft16's output.
+__host__ __device__ constexpr int dft16_at(int k) { return 4 * (k & 3) + (k >> 2); }
 template <typename R>
-__device__ __forceinline__ void dft4(cplx<R>& x0, cplx<R>& x1, cplx<R>& x2, cplx<R>& x3, int sign) {
-    const cplx<R> a0 = cadd(x0, x2), a1 = csub(x0, x2);
-    const cplx<R> b0 = cadd(x1, x3), b1 = csub(x1, x3);
-    // W4 b1: sign -1 -> -i b1, sign +1 -> +i b1
-    const cplx<R> wb = (sign < 0) ? cplx<R>{b1.y, -b1.x} : cplx<R>{-b1.y, b1.x};
-    x0 = cadd(a0, b0);
-    x1 = cadd(a1, wb);
-    x2 = csub(a0, b0);
-    x3 = csub(a1, wb);
+__device__ __forceinline__ void dft16(cplx<R>* v, R sg);
+
+// ---- DFTs of up to 16 points in registers ---------------------------------------
+// In place, natural order in; on return X_q stands at at(q).  The sign enters as
+// the factor sg = -1 or +1 of the sines, in FMAs that round the same value.
+template <int RR>
+struct OddTable;   // cos and sin of 2 pi m / RR, m = 1 .. (RR - 1) / 2
+template <>
+struct OddTable<3> {
+    static constexpr double c[] = {-0.5};
+    static constexpr double s[] = {0.86602540378443864676};
+};
+template <>
+struct OddTable<5> {
+    static constexpr double c[] = {0.3090169943749474241, -0.8090169943749474241};
+    static constexpr double s[] = {0.95105651629515357212, 0.58778525229247312917};
+};
+template <>
+struct OddTable<7> {
+    static constexpr double c[] = {0.62348980185873353053, -0.22252093395631440429, -0.90096886790241912624};
+    static constexpr double s[] = {0.78183148246802980871, 0.97492791218182360702, 0.43388373911755812048};
+};
+template <>
+struct OddTable<11> {
+    static constexpr double c[] = {0.84125353283118116886, 0.41541501300188642553, -0.14231483827328514044, -0.65486073394528506406, -0.95949297361449738989};
+    static constexpr double s[] = {0.54064081745559758211, 0.90963199535451837141, 0.98982144188093273238, 0.75574957435425828377, 0.28173255684142969771};
+};
+template <>
+struct OddTable<13> {
+    static constexpr double c[] = {0.8854560256532098959, 0.56806474673115580251, 0.12053668025532305335, -0.35460488704253562597, -0.74851074817110109863, -0.97094181742605202716};
+    static constexpr double s[] = {0.46472317204376854566, 0.82298386589365639458, 0.9927088740980539928, 0.93501624268541482344, 0.66312265824079520238, 0.23931566428755776715};
+};
+
+template <typename R>
+__device__ __forceinline__ cplx<R> plus_i(const cplx<R>& a, const cplx<R>& b, R sg) {   // a + i sg b
+    return {fma(-sg, b.y, a.x), fma(sg, b.x, a.y)};
+}
+
+// An odd prime, folded as in direct_pass.
+template <typename R, int RR>
+__device__ __forceinline__ void dft_odd(cplx<R>* v, R sg) {
+    constexpr int h = (RR - 1) / 2;
+    cplx<R> u[h + 1], d[h + 1];
+#pragma unroll
+    for (int j = 1; j <= h; ++j) {
+        u[j] = cadd(v[j], v[RR - j]);
+        d[j] = csub(v[j], v[RR - j]);
+    }
+    const cplx<R> y0 = v[0];
+    cplx<R> sum = y0;
+#pragma unroll
+    for (int j = 1; j <= h; ++j) sum = cadd(sum, u[j]);
+    v[0] = sum;
+#pragma unroll
+    for (int q = 1; q <= h; ++q) {
+        cplx<R> c = y0, t = {0, 0};
+#pragma unroll
+        for (int j = 1; j <= h; ++j) {
+            const int m = (j * q) % RR;
+            const R cc = (R)OddTable<RR>::c[(m <= h ? m : RR - m) - 1];
+            const R ss = (R)(m <= h ? OddTable<RR>::s[m - 1] : -OddTable<RR>::s[RR - m - 1]);
+            c = {fma(u[j].x, cc, c.x), fma(u[j].y, cc, c.y)};
+            t = {fma(d[j].x, ss, t.x), fma(d[j].y, ss, t.y)};
+        }
+        v[q] = plus_i(c, t, sg);
+        v[RR - q] = plus_i(c, t, -sg);
+    }
+}
+
+template <typename R, int RR>
+struct SmallDft {
+    static constexpr int at(int q) { return q; }
+    static __device__ __forceinline__ void run(cplx<R>* v, R sg) { dft_odd<R, RR>(v, sg); }
+};
+template <typename R>
+struct SmallDft<R, 2> {
+    static constexpr int at(int q) { return q; }
+    static __device__ __forceinline__ void run(cplx<R>* v, R) {
+        const cplx<R> t = v[0];
+        v[0] = cadd(t, v[1]);
+        v[1] = csub(t, v[1]);
+    }
+};
+template <typename R>
+struct SmallDft<R, 4> {
+    static constexpr int at(int q) { return q; }
+    static __device__ __forceinline__ void run(cplx<R>* v, R sg) {
+        const cplx<R> a0 = cadd(v[0], v[2]), a1 = csub(v[0], v[2]);
+        const cplx<R> b0 = cadd(v[1], v[3]), b1 = csub(v[1], v[3]);
+        v[0] = cadd(a0, b0);
+        v[1] = plus_i(a1, b1, sg);
+        v[2] = csub(a0, b0);
+        v[3] = plus_i(a1, b1, -sg);
+    }
+};
+// N1 N2 points with a rotation between the steps: n = N2 n1 + n2, X at
+// q = q1 + N1 q2.
+template <typename R>
+struct SmallDft<R, 8> {
+    static constexpr int at(int q) { return q; }
+    static __device__ __forceinline__ void run(cplx<R>* v, R sg) {
+        const R h = (R)0.70710678118654752440;
+        cplx<R> e[4] = {v[0], v[2], v[4], v[6]}, o[4] = {v[1], v[3], v[5], v[7]};
+        SmallDft<R, 4>::run(e, sg);
+        SmallDft<R, 4>::run(o, sg);
+        const cplx<R> z = {0, 0};
+        o[1] = cmul(o[1], cplx<R>{h, sg * h});
+        o[2] = plus_i(z, o[2], sg);
+        o[3] = cmul(o[3], cplx<R>{-h, sg * h});
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            v[k] = cadd(e[k], o[k]);
+            v[4 + k] = csub(e[k], o[k]);
+        }
+    }
+};
+template <typename R>
+struct SmallDft<R, 9> {
+    static constexpr int at(int q) { return q; }
+    static __device__ __forceinline__ void run(cplx<R>* v, R sg) {
+        cplx<R> t[3][3];
+#pragma unroll
+        for (int n2 = 0; n2 < 3; ++n2) {
+#pragma unroll
+            for (int n1 = 0; n1 < 3; ++n1) t[n2][n1] = v[3 * n1 + n2];
+            dft_odd<R, 3>(t[n2], sg);
+        }
+        const cplx<R> w1 = {(R)0.7660444431189780352, sg * (R)0.64278760968653932632}, w2 = {(R)0.17364817766693034885, sg * (R)0.98480775301220805937};
+        const cplx<R> w4 = {(R)-0.93969262078590838405, sg * (R)0.34202014332566873304};
+        t[1][1] = cmul(t[1][1], w1);
+        t[1][2] = cmul(t[1][2], w2);
+        t[2][1] = cmul(t[2][1], w2);
+        t[2][2] = cmul(t[2][2], w4);
+#pragma unroll
+        for (int q1 = 0; q1 < 3; ++q1) {
+            cplx<R> x[3] = {t[0][q1], t[1][q1], t[2][q1]};
+            dft_odd<R, 3>(x, sg);
+#pragma unroll
+            for (int q2 = 0; q2 < 3; ++q2) v[q1 + 3 * q2] = x[q2];
+        }
+    }
+};
+template <typename R>
+struct SmallDft<R, 16> {
+    static constexpr int at(int q) { return dft16_at(q); }
+    static __device__ __forceinline__ void run(cplx<R>* v, R sg) { dft16(v, sg); }
+};
+// N1 N2 points, coprime: n = N2 n1 + N1 n2 and the Chinese remainders q1, q2 of
+// q need no rotations.
+template <typename R, int N1, int N2>
+struct CoprimeDft {
+    static constexpr int at(int q) { return q; }
+    static __device__ __forceinline__ void run(cplx<R>* v, R sg) {
+        constexpr int N = N1 * N2;
+        cplx<R> t[N2][N1];
+#pragma unroll
+        for (int n2 = 0; n2 < N2; ++n2) {
+#pragma unroll
+            for (int n1 = 0; n1 < N1; ++n1) t[n2][n1] = v[(N2 * n1 + N1 * n2) % N];
+            SmallDft<R, N1>::run(t[n2], sg);
+        }
+#pragma unroll
+        for (int q1 = 0; q1 < N1; ++q1) {
+            cplx<R> x[N2];
+#pragma unroll
+            for (int n2 = 0; n2 < N2; ++n2) x[n2] = t[n2][q1];
+            SmallDft<R, N2>::run(x, sg);
+#pragma unroll
+            for (int q = 0; q < N; ++q)
+                if (q % N1 == q1) v[q] = x[q % N2];
+        }
+    }
+};
+template <typename R>
+struct SmallDft<R, 6> : CoprimeDft<R, 2, 3> {};
+template <typename R>
+struct SmallDft<R, 10> : CoprimeDft<R, 2, 5> {};
+template <typename R>
+struct SmallDft<R, 12> : CoprimeDft<R, 4, 3> {};
+template <typename R>
+struct SmallDft<R, 14> : CoprimeDft<R, 2, 7> {};
+template <typename R>
+struct SmallDft<R, 15> : CoprimeDft<R, 3, 5> {};
+
+// 4-point DFT in place (x_k = sum_n x_n W4^(nk), W4 = exp(sg 2 pi i / 4)).
+template <typename R>
+__device__ __forceinline__ void dft4(cplx<R>& x0, cplx<R>& x1, cplx<R>& x2, cplx<R>& x3, R sg) {
+    cplx<R> v[4] = {x0, x1, x2, x3};
+    SmallDft<R, 4>::run(v, sg);
+    x0 = v[0];
+    x1 = v[1];
+    x2 = v[2];
+    x3 = v[3];
 }
 
 // 16-point DFT in registers as 4 x 4 (Cooley-Tukey): with j = 4 j1 + j0 and
 // q = q0 + 4 q1, X_q = sum_j0 W4^(j0 q1) [w^(j0 q0) sum_j1 v_(4 j1 + j0) W4^(j1 q0)],
-// w = exp(sign 2 pi i / 16).  On return v[4 q0 + q1] = X_(q0 + 4 q1).
+// w = exp(sg 2 pi i / 16).  On return v[4 q0 + q1] = X_(q0 + 4 q1).
 template <typename R>
-__device__ __forceinline__ void dft16(cplx<R>* v, int sign) {
+__device__ __forceinline__ void dft16(cplx<R>* v, R sg) {
     const R c1 = (R)0.92387953251128675613, s1 = (R)0.38268343236508977173;   // cos, sin of pi/8
     const R c2 = (R)0.70710678118654752440;                                    // cos pi/4
-    const R sg = (R)(sign < 0 ? -1 : 1);
 #pragma unroll
-    for (int j0 = 0; j0 < 4; ++j0) dft4(v[j0], v[4 + j0], v[8 + j0], v[12 + j0], sign);
+    for (int j0 = 0; j0 < 4; ++j0) dft4(v[j0], v[4 + j0], v[8 + j0], v[12 + j0], sg);
     // v[4 q0 + j0] = Y[j0][q0]; twiddle by w^(j0 q0): m = 1, 2, 3 | 2, 4, 6 | 3, 6, 9
     const cplx<R> w1 = {c1, sg * s1}, w2 = {c2, sg * c2}, w3 = {s1, sg * c1};
     const cplx<R> w6 = {-c2, sg * c2}, w9 = {-c1, -sg * s1};
@@ -149,13 +333,13 @@ __device__ __forceinline__ void dft16(cplx<R>* v, int sign) {
     v[9] = cmul(v[9], w2);
     v[13] = cmul(v[13], w3);
     v[6] = cmul(v[6], w2);
-    v[10] = (sign < 0) ? cplx<R>{v[10].y, -v[10].x} : cplx<R>{-v[10].y, v[10].x};   // w^4 = W4
+    v[10] = {-sg * v[10].y, sg * v[10].x};   // w^4 = W4
     v[14] = cmul(v[14], w6);
     v[7] = cmul(v[7], w3);
     v[11] = cmul(v[11], w6);
     v[15] = cmul(v[15], w9);
 #pragma unroll
-    for (int q0 = 0; q0 < 4; ++q0) dft4(v[4 * q0], v[4 * q0 + 1], v[4 * q0 + 2], v[4 * q0 + 3], sign);
+    for (int q0 = 0; q0 < 4; ++q0) dft4(v[4 * q0], v[4 * q0 + 1], v[4 * q0 + 2], v[4 * q0 + 3], sg);
 }
 
 // ---- compile-time line plans --------------------------------------------------
@@ -178,6 +362,31 @@ struct CtPlan {
 PUFF_CT_PLAN(33, 11, 3)
 PUFF_CT_PLAN(129, 43, 3)
 #undef PUFF_CT_PLAN
+
+// How a runtime plan runs (line_plan): all passes of at most 16 points, in
+// place; a large prime first, on the matrix cores, then the same; or with two
+// line buffers.  A kernel each: the matrix pass's accumulators take a
+// wavefront per SIMD from the others.
+enum { LINE_SMALL = 0, LINE_PRIME = 1, LINE_TWO = 2 };
+
+// Quotients of 0 <= a < 2^16 by 1 <= d < 2^13: the high word of a ceil(2^32 / d).
+struct Div {
+    uint32_t m;   // 0: d = 1
+};
+__device__ __forceinline__ Div div_by(int d) { return {d > 1 ? 0xffffffffu / (uint32_t)d + 1 : 0}; }
+__device__ __forceinline__ int over(int a, Div d) { return d.m ? (int)__umulhi((uint32_t)a, d.m) : a; }
+
+// Line b and butterfly i (of T) of work item w: b fastest in interleaved buffers.
+template <bool IL>
+__device__ __forceinline__ void pass_item(int w, int B, Div by_b, int T, Div by_t, int& b, int& i) {
+    if (IL) {
+        i = over(w, by_b);
+        b = w - i * B;
+    } else {
+        b = over(w, by_t);
+        i = w - b * T;
+    }
+}
 
 // Direct DFT pass for an odd prime r (a radix pass of lds_pass), folded:
 // with the pre-twiddled inputs y_j = x_j W^(j k twst), u_j = y_j + y_(r-j),
@@ -205,12 +414,14 @@ __device__ __forceinline__ void direct_pass(const cplx<R>* src, cplx<R>* dst, in
     const int nr = N / r;
     const int hq = (r + 1) / 2;
     const int nqq = (hq + NQ - 1) / NQ;
+    const Div by_b = div_by(B), by_t = div_by(T), by_tq = div_by(T * nqq), by_p = div_by(p);
     for (int w = threadIdx.x; w < B * T * nqq; w += blockDim.x) {
         int b, t;
-        if (IL) { b = w % B; t = w / B; } else { t = w % (T * nqq); b = w / (T * nqq); }
-        const int q0 = NQ * (t / T);
-        const int i = t % T;
-        const int k = i % p;
+        pass_item<IL>(w, B, by_b, T * nqq, by_tq, b, t);
+        const int qq = over(t, by_t);
+        const int q0 = NQ * qq;
+        const int i = t - qq * T;
+        const int k = i - over(i, by_p) * p;
         const int dk = k * twst;
         int dq[NQ], f[NQ];
 #pragma unroll
@@ -247,7 +458,7 @@ __device__ __forceinline__ void direct_pass(const cplx<R>* src, cplx<R>* dst, in
             e1 += dk;
             e2 -= dk;
         }
-        const int ob = (i / p) * p * r + k;
+        const int ob = (i - k) * r + k;
 #pragma unroll
         for (int m = 0; m < NQ; ++m) {
             const int q = q0 + m;
@@ -372,89 +583,200 @@ __device__ __forceinline__ void direct_pass_ct(const cplx<R>* src, cplx<R>* dst,
     }
 }
 
-// One radix-r pass (after passes whose radices multiply to p) of an in-LDS
-// mixed-radix transform of length N over elements 0..N-1 of B lines laid
-// out with line length LD (N <= LD; elements N..LD-1 are left alone): src
-// to dst.  With constant arguments (ct_passes) every index division folds.
+// One pass of radix RR <= 16 (after passes whose radices multiply to p) of an
+// in-LDS mixed-radix transform of length N over elements 0..N-1 of B lines
+// laid out with line length LD (N <= LD; elements N..LD-1 are left alone).
+// TWO buffers: src to dst, any number of butterflies.  Otherwise in place
+// (src = dst): a thread reads its 16 / RR butterflies or fewer into registers,
+// the workgroup passes a barrier, and the outputs overwrite the buffer; half
+// the LDS, hence more workgroups per CU; B N / RR <= 16 / RR blockDim (checked
+// on the host).
+template <typename R, bool IL, int RR, bool TWO>
+__device__ __forceinline__ void radix_pass(const cplx<R>* src, cplx<R>* dst, int B, int LD, int N, int p,
+                                           const cplx<R>* tw, int sign) {
+    constexpr int KB = TWO ? 1 : 16 / RR;
+    const int T = N / RR;
+    const int twst = T / p;   // twiddle exponents j k twst (j < RR, k < p) stay below N: no reduction
+    const R sg = (R)sign;
+    const Div by_b = div_by(B), by_t = div_by(T), by_p = div_by(p);
+    const int tid = opaque_tid();
+    for (int w0 = tid; !TWO || w0 < B * T; w0 += (int)blockDim.x) {
+        cplx<R> v[KB][RR];
+        int b[KB], ob[KB];
+#pragma unroll
+        for (int it = 0; it < KB; ++it) {
+            const int w = w0 + it * (int)blockDim.x;
+            int i;
+            pass_item<IL>(w < B * T ? w : 0, B, by_b, T, by_t, b[it], i);
+            const int k = i - over(i, by_p) * p;
+            ob[it] = (i - k) * RR + k;
+#pragma unroll
+            for (int j = 0; j < RR; ++j) v[it][j] = src[lidx<IL>(b[it], i + j * T, B, LD)];
+            if (p > 1) {
+#pragma unroll
+                for (int j = 1; j < RR; ++j) v[it][j] = cmul(v[it][j], tw_get(tw, j * k * twst, sign));
+            }
+            SmallDft<R, RR>::run(v[it], sg);
+        }
+        if (!TWO) __syncthreads();
+#pragma unroll
+        for (int it = 0; it < KB; ++it) {
+            if (!TWO && w0 + it * (int)blockDim.x >= B * T) continue;
+#pragma unroll
+            for (int q = 0; q < RR; ++q) dst[lidx<IL>(b[it], ob[it] + q * p, B, LD)] = v[it][SmallDft<R, RR>::at(q)];
+        }
+        if (!TWO) break;
+    }
+}
+
+// A pass of runtime radix.
+template <typename R, bool IL, bool TWO>
+__device__ __forceinline__ void lds_pass(const cplx<R>* src, cplx<R>* dst, int B, int LD, int N, int r, int p,
+                                         const cplx<R>* tw, int sign) {
+    switch (r) {
+#define PUFF_RADIX(RR) \
+    case RR: return radix_pass<R, IL, RR, TWO>(src, dst, B, LD, N, p, tw, sign);
+        PUFF_RADIX(2)
+        PUFF_RADIX(3)
+        PUFF_RADIX(4)
+        PUFF_RADIX(5)
+        PUFF_RADIX(6)
+        PUFF_RADIX(7)
+        PUFF_RADIX(8)
+        PUFF_RADIX(9)
+        PUFF_RADIX(10)
+        PUFF_RADIX(11)
+        PUFF_RADIX(12)
+        PUFF_RADIX(13)
+        PUFF_RADIX(14)
+        PUFF_RADIX(15)
+        PUFF_RADIX(16)
+#undef PUFF_RADIX
+        default: break;
+    }
+    if constexpr (TWO) {
+        if (r >= PUFF_DFT_WIDE_MIN) direct_pass<R, IL, PUFF_DFT_WIDE>(src, dst, B, LD, N, r, p, tw, sign);
+        else direct_pass<R, IL, 2>(src, dst, B, LD, N, r, p, tw, sign);
+    }
+}
+
+// ---- the first pass for a large prime, on the matrix cores ------------------------
+// direct_pass's folded sums for p = 1 (no input rotations) as two products
+//   C = [cos 2 pi j q / r] U,  S = [sin] V,  q = 0 .. h, j = 1 .. h = (r - 1) / 2,
+// with one real column per line, butterfly and component: tiles of 16 q by 16
+// columns (8 butterflies), four j per MFMA.  Each operand is read once per
+// 1024 FMAs instead of once per 4 (direct_pass reads 6 LDS words of 16 bytes
+// for 16 FMAs per lane and is bound by that).  In place: the tiles stay in
+// accumulators until every input is read; the wavefronts deal the tiles out,
+// at most MFMA_TILES each (checked on the host).
+//   Operands: lane l holds A[row l % 16][k = l / 16] and B[k = l / 16][column l % 16];
+//   results: column l % 16, row l / 16 + 4 v (FP64) or 4 (l / 16) + v (FP32), v < 4.
+template <typename R>
+struct Mfma;
+template <>
+struct Mfma<double> {
+    typedef double T __attribute__((ext_vector_type(4)));
+    static __device__ __forceinline__ T fma(double a, double b, T c) {
+        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ int row(int l, int v) { return (l >> 4) + 4 * v; }
+};
+template <>
+struct Mfma<float> {
+    typedef float T __attribute__((ext_vector_type(4)));
+    static __device__ __forceinline__ T fma(float a, float b, T c) {
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ int row(int l, int v) { return 4 * (l >> 4) + v; }
+};
+constexpr int MFMA_TILES = 4;
+constexpr int mfma_tiles(int B, int n, int r) { return (B * (n / r) + 7) / 8 * (((r - 1) / 2 + 16) / 16); }
+
 template <typename R, bool IL>
-__device__ __forceinline__ void lds_pass(const cplx<R>* src, cplx<R>* dst, int B, int LD, int N, int r,
-                                         int p, const cplx<R>* tw, int sign) {
-    const int T = N / r;
-    // twiddle exponents j k twst (j < r, k < p) stay below N: no reduction
-    const int twst = N / (p * r);
-    if (r == 16) {
-        for (int w = threadIdx.x; w < B * T; w += blockDim.x) {
+__device__ __forceinline__ void mfma_pass(cplx<R>* buf, int B, int N, int r, const cplx<R>* tw, int sign) {
+    using M = Mfma<R>;
+    const int T = N / r, cols = B * T, h = (r - 1) / 2, qt = (h + 16) / 16;
+    const int units = (cols + 7) / 8 * qt;
+    const int l = opaque_tid() & 63, k = l >> 4, n = l & 15, part = n & 1;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const Div by_b = div_by(B), by_t = div_by(T), by_q = div_by(qt), by_r = div_by(r);
+    const R* in = reinterpret_cast<const R*>(buf);
+    typename M::T C[MFMA_TILES], S[MFMA_TILES];
+    R y0[MFMA_TILES];
+#pragma unroll
+    for (int m = 0; m < MFMA_TILES; ++m) {
+        C[m] = S[m] = typename M::T{0, 0, 0, 0};
+        y0[m] = 0;
+        const int unit = wave + 4 * m;
+        if (unit < units) {
+            const int ct = over(unit, by_q), q = 16 * (unit - ct * qt) + n;
+            const int item = 8 * ct + (n >> 1);
             int b, i;
-            if (IL) { b = w % B; i = w / B; } else { i = w % T; b = w / T; }
-            const int k = i % p;
-            const int ob = (i / p) * p * 16 + k;
-            cplx<R> v[16];
-#pragma unroll
-            for (int j = 0; j < 16; ++j) {
-                v[j] = src[lidx<IL>(b, i + j * T, B, LD)];
-                if (j > 0 && k > 0) v[j] = cmul(v[j], tw_get(tw, j * k * twst, sign));
-            }
-            dft16(v, sign);
-#pragma unroll
-            for (int q0 = 0; q0 < 4; ++q0)
-#pragma unroll
-                for (int q1 = 0; q1 < 4; ++q1)
-                    dst[lidx<IL>(b, ob + (q0 + 4 * q1) * p, B, LD)] = v[4 * q0 + q1];
-        }
-    } else if (r == 2 || r == 3 || r == 4) {
-        for (int w = threadIdx.x; w < B * T; w += blockDim.x) {
-            int b, i;
-            if (IL) { b = w % B; i = w / B; } else { i = w % T; b = w / T; }
-            const int k = i % p;
-            const int ob = (i / p) * p * r + k;
-            cplx<R> v[4];
-            for (int j = 0; j < r; ++j) {
-                v[j] = src[lidx<IL>(b, i + j * T, B, LD)];
-                if (j > 0 && k > 0) v[j] = cmul(v[j], tw_get(tw, j * k * twst, sign));
-            }
-            if (r == 2) {
-                dst[lidx<IL>(b, ob, B, LD)] = cadd(v[0], v[1]);
-                dst[lidx<IL>(b, ob + p, B, LD)] = csub(v[0], v[1]);
-            } else if (r == 3) {
-                const R s3 = (R)0.86602540378443864676 * (R)(sign < 0 ? -1 : 1);
-                const cplx<R> t1 = cadd(v[1], v[2]);
-                const cplx<R> t2 = {v[0].x - (R)0.5 * t1.x, v[0].y - (R)0.5 * t1.y};
-                const cplx<R> d = csub(v[1], v[2]);
-                const cplx<R> t3 = {-s3 * d.y, s3 * d.x};   // i s s3 (x1 - x2)
-                dst[lidx<IL>(b, ob, B, LD)] = cadd(v[0], t1);
-                dst[lidx<IL>(b, ob + p, B, LD)] = cadd(t2, t3);
-                dst[lidx<IL>(b, ob + 2 * p, B, LD)] = csub(t2, t3);
-            } else {
-                const cplx<R> a0 = cadd(v[0], v[2]), a1 = csub(v[0], v[2]);
-                const cplx<R> b0 = cadd(v[1], v[3]), b1 = csub(v[1], v[3]);
-                // W4 b1: sign -1 -> -i b1, sign +1 -> +i b1
-                const cplx<R> wb = (sign < 0) ? cplx<R>{b1.y, -b1.x} : cplx<R>{-b1.y, b1.x};
-                dst[lidx<IL>(b, ob, B, LD)] = cadd(a0, b0);
-                dst[lidx<IL>(b, ob + p, B, LD)] = cadd(a1, wb);
-                dst[lidx<IL>(b, ob + 2 * p, B, LD)] = csub(a0, b0);
-                dst[lidx<IL>(b, ob + 3 * p, B, LD)] = csub(a1, wb);
+            pass_item<IL>(item < cols ? item : 0, B, by_b, T, by_t, b, i);
+            auto at = [&](int j) { return in[2 * lidx<IL>(b, i + j * T, B, N) + part]; };
+            y0[m] = at(0);
+            const int d0 = (q <= h ? q : 0) * (k + 1), d4 = 4 * (q <= h ? q : 0);
+            int e = d0 - over(d0, by_r) * r;
+            const int d = d4 - over(d4, by_r) * r;
+            for (int j0 = 1; j0 <= h; j0 += 4) {
+                const int j = j0 + k, jj = j <= h ? j : 1;
+                const R xa = at(jj), xb = at(r - jj);
+                const cplx<R> w = tw[e * T];
+                C[m] = M::fma(w.x, j <= h ? xa + xb : (R)0, C[m]);
+                S[m] = M::fma(w.y, j <= h ? xa - xb : (R)0, S[m]);
+                e += d;
+                e = (int)min((uint32_t)e, (uint32_t)(e - r));
             }
         }
-    } else if (r >= PUFF_DFT_WIDE_MIN) {
-        direct_pass<R, IL, PUFF_DFT_WIDE>(src, dst, B, LD, N, r, p, tw, sign);
-    } else {
-        direct_pass<R, IL, 2>(src, dst, B, LD, N, r, p, tw, sign);
+    }
+    __syncthreads();
+    // i S: the other component of the same column, one lane away.  The table
+    // is the forward one (sin negated), the sign turns S.
+    const R sg = (R)((sign < 0) == (part == 0) ? -1 : 1);
+    R* out = reinterpret_cast<R*>(buf);
+#pragma unroll
+    for (int m = 0; m < MFMA_TILES; ++m) {
+        const int unit = wave + 4 * m;
+        if (unit < units) {
+            const int ct = over(unit, by_q);
+            const int item = 8 * ct + (n >> 1);
+            int b, i;
+            pass_item<IL>(item < cols ? item : 0, B, by_b, T, by_t, b, i);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int q = 16 * (unit - ct * qt) + M::row(l, v);
+                const R other = __shfl_xor(S[m][v], 1, 64);
+                const R a = y0[m] + C[m][v], t = sg * other;
+                if (item < cols && q <= h) {
+                    out[2 * lidx<IL>(b, i * r + q, B, N) + part] = a + t;
+                    if (q > 0) out[2 * lidx<IL>(b, i * r + r - q, B, N) + part] = a - t;
+                }
+            }
+        }
     }
 }
 
 // The passes of a runtime plan.  src holds the input; returns the buffer
-// holding the output (src or dst).
-template <typename R, bool IL>
+// holding the output (src or dst; in place: src).
+template <typename R, bool IL, int KIND>
 __device__ __forceinline__ cplx<R>* lds_passes(cplx<R>* src, cplx<R>* dst, int B, int LD, int N, int npass,
                                                const int* radix, const cplx<R>* tw, int sign) {
-    int p = 1;
-    for (int ps = 0; ps < npass; ++ps) {
-        const int r = radix[ps];
-        lds_pass<R, IL>(src, dst, B, LD, N, r, p, tw, sign);
+    constexpr bool TWO = KIND == LINE_TWO;
+    int p = 1, ps = 0;
+    if constexpr (KIND == LINE_PRIME) {
+        mfma_pass<R, IL>(src, B, N, radix[0], tw, sign);
         __syncthreads();
-        cplx<R>* t = src;
-        src = dst;
-        dst = t;
+        p = radix[ps++];
+    }
+    for (; ps < npass; ++ps) {
+        const int r = radix[ps];
+        lds_pass<R, IL, TWO>(src, TWO ? dst : src, B, LD, N, r, p, tw, sign);
+        __syncthreads();
+        if (TWO) {
+            cplx<R>* t = src;
+            src = dst;
+            dst = t;
+        }
         p *= r;
     }
     return src;
@@ -469,11 +791,11 @@ __device__ __forceinline__ cplx<R>* ct_passes(cplx<R>* src, cplx<R>* dst, int B,
         return src;
     } else {
         constexpr int r = CtPlan<NC>::r[K];
-        if constexpr (r != 2 && r != 3 && r != 4 && r != 16) {
+        if constexpr (r > 3) {
             constexpr int nq = r >= PUFF_DFT_WIDE_MIN ? PUFF_DFT_WIDE : 2;
             direct_pass_ct<R, IL, nq, NC, r, P>(src, dst, B, tw, sign);
         } else {
-            lds_pass<R, IL>(src, dst, B, LD, N, r, P, tw, sign);
+            radix_pass<R, IL, r, true>(src, dst, B, LD, N, P, tw, sign);
         }
         __syncthreads();
         return ct_passes<R, IL, NC, K + 1, P * r>(dst, src, B, LD, N, tw, sign);
@@ -498,7 +820,7 @@ __device__ __forceinline__ cplx<R>* lds_rader(cplx<R>* src, cplx<R>* dst, int B,
         P[lidx<IL>(b, j, B, N)] = src[lidx<IL>(b, j < M ? ax.rperm[j] : 0, B, N)];
     }
     __syncthreads();
-    cplx<R>* res = lds_passes<R, IL>(P, Q, B, N, M, ax.npass, ax.radix, tw, -1);
+    cplx<R>* res = lds_passes<R, IL, LINE_TWO>(P, Q, B, N, M, ax.npass, ax.radix, tw, -1);
     for (int w = threadIdx.x; w < B * M; w += blockDim.x) {
         int b, k;
         if (IL) { b = w % B; k = w / B; } else { k = w % M; b = w / M; }
@@ -511,7 +833,7 @@ __device__ __forceinline__ cplx<R>* lds_rader(cplx<R>* src, cplx<R>* dst, int B,
     }
     __syncthreads();
     cplx<R>* other = (res == P) ? Q : P;
-    res = lds_passes<R, IL>(res, other, B, N, M, ax.npass, ax.radix, tw, +1);
+    res = lds_passes<R, IL, LINE_TWO>(res, other, B, N, M, ax.npass, ax.radix, tw, +1);
     cplx<R>* out = (res == P) ? Q : P;
     // every output element except element M (which holds x_0 or X_0 in out)
     const int qm = M / 2;   // g^-(M/2) = -1 = M (mod N)
@@ -535,114 +857,17 @@ __device__ __forceinline__ cplx<R>* lds_rader(cplx<R>* src, cplx<R>* dst, int B,
 }
 
 // In-LDS transform of B lines of length ax.n.  src holds the input; returns
-// the buffer holding the output (src or dst).
-// Radix-2/3/4 butterfly in place on v[0..r-1] (same arithmetic as the
-// ping-pong passes).
-template <typename R>
-__device__ __forceinline__ void small_radix(cplx<R>* v, int r, int sign) {
-    if (r == 2) {
-        const cplx<R> t = v[0];
-        v[0] = cadd(t, v[1]);
-        v[1] = csub(t, v[1]);
-    } else if (r == 3) {
-        const R s3 = (R)0.86602540378443864676 * (R)(sign < 0 ? -1 : 1);
-        const cplx<R> t1 = cadd(v[1], v[2]);
-        const cplx<R> t2 = {v[0].x - (R)0.5 * t1.x, v[0].y - (R)0.5 * t1.y};
-        const cplx<R> d = csub(v[1], v[2]);
-        const cplx<R> t3 = {-s3 * d.y, s3 * d.x};
-        v[0] = cadd(v[0], t1);
-        v[1] = cadd(t2, t3);
-        v[2] = csub(t2, t3);
-    } else {
-        dft4(v[0], v[1], v[2], v[3], sign);
-    }
-}
-
-// In-place form of lds_passes for lines whose passes are all radix 16, 4, 3
-// or 2, with at most one butterfly per thread in every pass (B N / r <=
-// blockDim, checked on the host): each thread reads its butterfly's inputs
-// into registers, the workgroup passes a barrier, and the outputs overwrite
-// the same buffer.  Half the LDS of the ping-pong form, hence more
-// workgroups per CU.
-template <typename R, bool IL>
-__device__ __forceinline__ void inplace_pass(cplx<R>* buf, int B, int N, int r, int p, const cplx<R>* tw,
-                                             int sign, int LD) {
-    const int T = N / r;
-    const int twst = N / (p * r);   // j k twst < N, as in lds_pass
-    const int w = opaque_tid();
-    const bool act = w < B * T;
-    int b = 0, ob = 0;
-    cplx<R> v[16];
-    if (act) {
-        int i;
-        if (IL) { b = w % B; i = w / B; } else { i = w % T; b = w / T; }
-        const int k = i % p;
-        ob = (i / p) * p * r + k;
-        if (r == 16) {
-#pragma unroll
-            for (int j = 0; j < 16; ++j) {
-                v[j] = buf[lidx<IL>(b, i + j * T, B, LD)];
-                if (j > 0 && k > 0) v[j] = cmul(v[j], tw_get(tw, j * k * twst, sign));
-            }
-            dft16(v, sign);
-        } else {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                if (j < r) {
-                    v[j] = buf[lidx<IL>(b, i + j * T, B, LD)];
-                    if (j > 0 && k > 0) v[j] = cmul(v[j], tw_get(tw, j * k * twst, sign));
-                }
-            }
-            small_radix(v, r, sign);
-        }
-    }
-    __syncthreads();
-    if (act) {
-        if (r == 16) {
-#pragma unroll
-            for (int q0 = 0; q0 < 4; ++q0)
-#pragma unroll
-                for (int q1 = 0; q1 < 4; ++q1) buf[lidx<IL>(b, ob + (q0 + 4 * q1) * p, B, LD)] = v[4 * q0 + q1];
-        } else {
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-                if (q < r) buf[lidx<IL>(b, ob + q * p, B, LD)] = v[q];
-        }
-    }
-}
-
-template <typename R, bool IL>
-__device__ __forceinline__ void lds_passes_inplace(cplx<R>* buf, int B, int N, int npass, const int* radix,
-                                                   const cplx<R>* tw, int sign) {
-    int p = 1;
-    for (int ps = 0; ps < npass; ++ps) {
-        const int r = radix[ps];
-        inplace_pass<R, IL>(buf, B, N, r, p, tw, sign, N);
-        __syncthreads();
-        p *= r;
-    }
-}
-
-template <typename R, bool IL, int NC>
+// the buffer holding the output (src or dst; one buffer: src).
+template <typename R, bool IL, int NC, int KIND>
 __device__ __forceinline__ cplx<R>* lds_fft(cplx<R>* src, cplx<R>* dst, int B, const FftAxis& ax,
                                             const cplx<R>* tw, int sign) {
     if constexpr (NC > 0) {
         return ct_passes<R, IL, NC>(src, dst, B, NC, NC, tw, sign);
     } else {
-        if (ax.rader) return lds_rader<R, IL>(src, dst, B, ax, tw, sign);
-        return lds_passes<R, IL>(src, dst, B, ax.n, ax.n, ax.npass, ax.radix, tw, sign);
-    }
-}
-
-// z2-line transform: in place (one LDS buffer) or ping-pong.
-template <typename R, bool INPLACE>
-__device__ __forceinline__ cplx<R>* z_fft(cplx<R>* src, cplx<R>* dst, int B, const FftAxis& ax, const cplx<R>* tw,
-                                          int sign) {
-    if constexpr (INPLACE) {
-        lds_passes_inplace<R, true>(src, B, ax.n, ax.npass, ax.radix, tw, sign);
-        return src;
-    } else {
-        return lds_fft<R, true, 0>(src, dst, B, ax, tw, sign);
+        if constexpr (KIND == LINE_TWO) {
+            if (ax.rader) return lds_rader<R, IL>(src, dst, B, ax, tw, sign);
+        }
+        return lds_passes<R, IL, KIND>(src, dst, B, ax.n, ax.n, ax.npass, ax.radix, tw, sign);
     }
 }
 
@@ -720,9 +945,6 @@ __device__ __forceinline__ int rad_at(int b, int e) {
     return XL ? b * RAD_LD + e + (e >> 4) : (e + (e >> 4)) * BL + b;
 }
 
-// Index of X_k in dft16's output.
-__host__ __device__ constexpr int dft16_at(int k) { return 4 * (k & 3) + (k >> 2); }
-
 // v[j] = a[u + 16 j] -> v[j] = c[u + 16 j]; returns A_0 (in thread u = 0).
 // rb: the table of the transform's sign (global memory, L2).  The buffer may
 // be in use when called; every thread has passed a barrier after its last
@@ -730,7 +952,7 @@ __host__ __device__ constexpr int dft16_at(int k) { return 4 * (k & 3) + (k >> 2
 template <typename R, int BL, bool XL>
 __device__ __forceinline__ cplx<R> rader_core(cplx<R> (&v)[16], int b, int u, cplx<R>* buf, const cplx<R>* tw,
                                               const cplx<R>* rb) {
-    dft16(v, -1);
+    dft16(v, (R)-1);
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < 16; ++q) {
@@ -740,12 +962,12 @@ __device__ __forceinline__ cplx<R> rader_core(cplx<R> (&v)[16], int b, int u, cp
     __syncthreads();
 #pragma unroll
     for (int t = 0; t < 16; ++t) v[t] = buf[rad_at<BL, XL>(b, u * 16 + t)];
-    dft16(v, -1);
+    dft16(v, (R)-1);
     const cplx<R> a0 = v[0];
     cplx<R> c[16];
 #pragma unroll
     for (int p = 0; p < 16; ++p) c[p] = cmul(v[dft16_at(p)], rb[u + 16 * p]);
-    dft16(c, +1);
+    dft16(c, (R)+1);
     // back to the elements this thread read: no barrier before the writes
 #pragma unroll
     for (int t = 0; t < 16; ++t) {
@@ -755,7 +977,7 @@ __device__ __forceinline__ cplx<R> rader_core(cplx<R> (&v)[16], int b, int u, cp
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < 16; ++q) c[q] = buf[rad_at<BL, XL>(b, q * 16 + u)];
-    dft16(c, +1);
+    dft16(c, (R)+1);
 #pragma unroll
     for (int j = 0; j < 16; ++j) v[j] = c[dft16_at(j)];
     return a0;
@@ -919,9 +1141,10 @@ __global__ __launch_bounds__(16 * rad_lines<R>()) void k_rader_x(DiffArgs<R> a, 
 // ---- x lines (contiguous) --------------------------------------------------
 // OP (an XOP_ value) is a template parameter: each fused operation gets its
 // own register allocation.
-template <typename R, int NC, int BC, int OP>
-__global__ __launch_bounds__(256) void k_fft_x(DiffArgs<R> a, int Bp, int sign) {
+template <typename R, int NC, int BC, int KIND, int OP>
+__global__ __launch_bounds__(256, 4) void k_fft_x(DiffArgs<R> a, int Bp, int sign) {
     constexpr int op = OP;
+    constexpr bool TWO = KIND == LINE_TWO;
     extern __shared__ unsigned char smem_raw[];
     const int N = NC ? NC : a.nx;
     const int B = BC ? BC : Bp;
@@ -932,7 +1155,7 @@ __global__ __launch_bounds__(256) void k_fft_x(DiffArgs<R> a, int Bp, int sign) 
     const int64_t L0 = (int64_t)blockIdx.x * B;
     const int nb = (int)min<int64_t>(B, nlines - L0);
     const cplx<R>* twg = reinterpret_cast<const cplx<R>*>(ax.tw);
-    cplx<R>* tw = s1 + lpad<false>(B * N);   // twiddle table staged in LDS
+    cplx<R>* tw = TWO ? s1 + lpad<false>(B * N) : s1;   // twiddle table staged in LDS
     for (int w = threadIdx.x; w < N; w += blockDim.x) tw[w] = twg[w];
     cplx<R>* base = a.a + L0 * N;
     const int64_t ntr = (int64_t)a.nx * a.ny;
@@ -940,15 +1163,16 @@ __global__ __launch_bounds__(256) void k_fft_x(DiffArgs<R> a, int Bp, int sign) 
     // counted on from there (b < B)
     const int iy0 = (int)(L0 % a.ny), iz0 = (int)(L0 / a.ny);
     const double rff = 1.0 / a.ffact;
+    const Div by_n = div_by(N);
     if (op == XOP_ADJ_FOLD_SAVE_FWD) {
         for (int w = threadIdx.x; w < B * N; w += blockDim.x) {
-            const int b = w / N;
+            const int b = over(w, by_n);
             cplx<R> v = (b < nb) ? base[w] : cplx<R>{0, 0};
             if (b < nb) {
                 const int64_t L = L0 + b;
                 if (a.periodic && L < a.ny) {
                     // the output's aliased plane copies plane 1: fold its cotangent
-                    cplx<R>* al = a.a + (int64_t)(a.nz2 - 1) * ntr + L * N + (w % N);
+                    cplx<R>* al = a.a + (int64_t)(a.nz2 - 1) * ntr + L * N + (w - b * N);
                     const cplx<R> t = *al;
                     v.x += t.x;
                     v.y += t.y;
@@ -970,12 +1194,12 @@ __global__ __launch_bounds__(256) void k_fft_x(DiffArgs<R> a, int Bp, int sign) 
         if constexpr (sizeof(R) == 8) return (double)v / a.ffact;
         else return (double)v * rff;
     };
-    cplx<R>* res = lds_fft<R, false, NC>(s0, s1, B, ax, tw, first_sign);
+    cplx<R>* res = lds_fft<R, false, NC, KIND>(s0, s1, B, ax, tw, first_sign);
     if (op == XOP_ADJ_INV_MIX_FWD) {
         // adjoint of the absorption split: (1 - m) cotangent + m W^H G W cotangent / ffact
         const cplx<R>* lam = a.anb + L0 * N;
         for (int w = threadIdx.x; w < nb * N; w += blockDim.x) {
-            const int b = w / N, j = w % N;
+            const int b = over(w, by_n), j = w - b * N;
             const int lb = iy0 + b;   // (iy, iz) of line L0 + b
             const int iy = lb % a.ny, iz = iz0 + lb / a.ny;
             const double mxy = a.mxy[(int64_t)iy * a.nx + j];
@@ -986,8 +1210,8 @@ __global__ __launch_bounds__(256) void k_fft_x(DiffArgs<R> a, int Bp, int sign) 
                             (R)((1.0 - m) * (double)l.y + m * unscale(v.y))};
         }
         __syncthreads();
-        cplx<R>* other = (res == s0) ? s1 : s0;
-        res = lds_fft<R, false, NC>(res, other, B, ax, tw, -1);
+        cplx<R>* other = (TWO && res == s0) ? s1 : s0;
+        res = lds_fft<R, false, NC, KIND>(res, other, B, ax, tw, -1);
     } else if (op == XOP_ADJ_INV_SCALE) {
         for (int w = threadIdx.x; w < nb * N; w += blockDim.x) {
             const cplx<R> v = res[lpad<false>(w)];
@@ -998,7 +1222,7 @@ __global__ __launch_bounds__(256) void k_fft_x(DiffArgs<R> a, int Bp, int sign) 
         // /ffact then AbsorptionStep's split (diffraction.f90:310, 454-470)
         cplx<R>* anb = a.anb + L0 * N;
         for (int w = threadIdx.x; w < nb * N; w += blockDim.x) {
-            const int b = w / N, j = w % N;
+            const int b = over(w, by_n), j = w - b * N;
             const int lb = iy0 + b;   // (iy, iz) of line L0 + b
             const int iy = lb % a.ny, iz = iz0 + lb / a.ny;
             const double mxy = a.mxy[(int64_t)iy * a.nx + j];
@@ -1009,8 +1233,8 @@ __global__ __launch_bounds__(256) void k_fft_x(DiffArgs<R> a, int Bp, int sign) 
             res[lpad<false>(w)] = {(R)(m * vr), (R)(m * vi)};
         }
         __syncthreads();
-        cplx<R>* other = (res == s0) ? s1 : s0;
-        res = lds_fft<R, false, NC>(res, other, B, ax, tw, -1);
+        cplx<R>* other = (TWO && res == s0) ? s1 : s0;
+        res = lds_fft<R, false, NC, KIND>(res, other, B, ax, tw, -1);
     } else if (op == XOP_INV_RECOMBINE) {
         // /ffact + interior (diffraction.f90:513-517)
         const cplx<R>* anb = a.anb + L0 * N;
@@ -1029,15 +1253,17 @@ __global__ __launch_bounds__(256) void k_fft_x(DiffArgs<R> a, int Bp, int sign) 
     if (op == XOP_INV_RECOMBINE && a.periodic) {
         // keep the aliased plane NZ2 equal to plane 1 (para_field.f90:3197-3244)
         for (int w = threadIdx.x; w < nb * N; w += blockDim.x) {
-            const int64_t L = L0 + w / N;
-            if (L < a.ny) a.a[(int64_t)(a.nz2 - 1) * ntr + L * N + (w % N)] = res[lpad<false>(w)];
+            const int b = over(w, by_n);
+            const int64_t L = L0 + b;
+            if (L < a.ny) a.a[(int64_t)(a.nz2 - 1) * ntr + L * N + (w - b * N)] = res[lpad<false>(w)];
         }
     }
 }
 
 // ---- y lines (stride nx), B consecutive x per block -------------------------
-template <typename R, int NC, int BC>
-__global__ __launch_bounds__(256) void k_fft_y(DiffArgs<R> a, int Bp, int sign) {
+template <typename R, int NC, int BC, int KIND>
+__global__ __launch_bounds__(256, 4) void k_fft_y(DiffArgs<R> a, int Bp, int sign) {
+    constexpr bool TWO = KIND == LINE_TWO;
     extern __shared__ unsigned char smem_raw[];
     const int N = NC ? NC : a.ny;
     const int B = BC ? BC : Bp;
@@ -1053,17 +1279,18 @@ __global__ __launch_bounds__(256) void k_fft_y(DiffArgs<R> a, int Bp, int sign) 
     const int iz = (int)(blk / nxb);
     const int nb = min(B, a.nx - x0);
     const cplx<R>* twg = reinterpret_cast<const cplx<R>*>(ay.tw);
-    cplx<R>* tw = s1 + lpad<true>(B * N);   // twiddle table staged in LDS
+    cplx<R>* tw = TWO ? s1 + lpad<true>(B * N) : s1;   // twiddle table staged in LDS
     for (int w = threadIdx.x; w < N; w += blockDim.x) tw[w] = twg[w];
+    const Div by_b = div_by(B);
     cplx<R>* base = a.a + (int64_t)iz * a.nx * a.ny + x0;
     lds_fill<true, STAGE_UNROLL>(s0, B * N, [&](int w) {
-        const int b = w % B, j = w / B;
+        const int j = over(w, by_b), b = w - j * B;
         return (b < nb) ? base[(int64_t)j * a.nx + b] : cplx<R>{0, 0};
     });
     __syncthreads();
-    cplx<R>* res = lds_fft<R, true, NC>(s0, s1, B, ay, tw, sign);
+    cplx<R>* res = lds_fft<R, true, NC, KIND>(s0, s1, B, ay, tw, sign);
     lds_drain<true, STAGE_UNROLL>(res, B * N, [&](int w, const cplx<R>& v) {
-        const int b = w % B, j = w / B;
+        const int j = over(w, by_b), b = w - j * B;
         if (b < nb) base[(int64_t)j * a.nx + b] = v;
     });
 }
@@ -1170,13 +1397,14 @@ __device__ __forceinline__ cplx<R> spectral_op(const DiffArgs<R>& a, int op, dou
 
 // ---- z2 lines (stride nx ny), B consecutive x per block ----------------------
 // op < 0: plain transform with `sign`; else forward, spectral op, inverse.
-template <typename R, bool INPLACE>
-__global__ __launch_bounds__(PUFF_Z_THREADS) void k_fft_z(DiffArgs<R> a, int B, int op, int sign) {
+template <typename R, int KIND>
+__global__ __launch_bounds__(PUFF_Z_THREADS, 4) void k_fft_z(DiffArgs<R> a, int B, int op, int sign) {
+    constexpr bool TWO = KIND == LINE_TWO;
     extern __shared__ unsigned char smem_raw[];
     const int N = a.nzp;
     const FftAxis& az = a.az;
     cplx<R>* s0 = reinterpret_cast<cplx<R>*>(smem_raw);
-    cplx<R>* s1 = INPLACE ? s0 : s0 + lpad<true>(B * N);
+    cplx<R>* s1 = TWO ? s0 + lpad<true>(B * N) : s0;
     // blocks of B x-columns, x fastest; neighbouring blocks share the cache
     // lines of every z2 plane, so they go to one XCD
     const int nxb = (a.nx + B - 1) / B;
@@ -1186,23 +1414,30 @@ __global__ __launch_bounds__(PUFF_Z_THREADS) void k_fft_z(DiffArgs<R> a, int B, 
     const int iy = (int)(blk / nxb);
     const int nb = min(B, a.nx - x0);
     const int64_t ntr = (int64_t)a.nx * a.ny;
-    // few lines per workgroup here: the twiddles stay in global memory (L2)
+    // few lines per workgroup here: the twiddles stay in global memory (L2),
+    // except for the matrix cores' pass, whose lanes read them at random
     const cplx<R>* tw = reinterpret_cast<const cplx<R>*>(az.tw);
+    if constexpr (KIND == LINE_PRIME) {
+        cplx<R>* t = s0 + lpad<true>(B * N);
+        for (int w = threadIdx.x; w < N; w += blockDim.x) t[w] = tw[w];
+        tw = t;
+    }
     cplx<R>* base = a.a + (int64_t)iy * a.nx + x0;
+    const Div by_b = div_by(B);
     lds_fill<true, PUFF_Z_UNROLL>(s0, B * N, [&](int w) {
-        const int b = w % B, j = w / B;
+        const int j = over(w, by_b), b = w - j * B;
         return (b < nb) ? base[(int64_t)j * ntr + b] : cplx<R>{0, 0};
     });
     __syncthreads();
     cplx<R>* res;
     if (op < 0) {
-        res = z_fft<R, INPLACE>(s0, s1, B, az, tw, sign);
+        res = lds_fft<R, true, 0, KIND>(s0, s1, B, az, tw, sign);
     } else {
-        res = z_fft<R, INPLACE>(s0, s1, B, az, tw, -1);
+        res = lds_fft<R, true, 0, KIND>(s0, s1, B, az, tw, -1);
         const double ky = a.ky[iy];
         const bool small_phase = a.phase_max < PHASE_LIMIT;
         for (int w = threadIdx.x; w < B * N; w += blockDim.x) {
-            const int b = w % B, q = w / B;
+            const int q = over(w, by_b), b = w - q * B;
             if (b >= nb) continue;
             const double rz = sizeof(R) == 4 ? a.kzr[2 * q + (op == SPEC_ABSORB ? 1 : 0)] : 0.0;
             const cplx<R> v = res[lpad<true>(w)];
@@ -1210,11 +1445,11 @@ __global__ __launch_bounds__(PUFF_Z_THREADS) void k_fft_z(DiffArgs<R> a, int B, 
                                              : spectral_op<R, false>(a, op, a.kx[x0 + b], ky, a.kz[q], rz, v);
         }
         __syncthreads();
-        cplx<R>* other = (res == s0) ? s1 : s0;
-        res = z_fft<R, INPLACE>(res, other, B, az, tw, +1);
+        cplx<R>* other = (TWO && res == s0) ? s1 : s0;
+        res = lds_fft<R, true, 0, KIND>(res, other, B, az, tw, +1);
     }
     lds_drain<true, PUFF_Z_UNROLL>(res, B * N, [&](int w, const cplx<R>& v) {
-        const int b = w % B, j = w / B;
+        const int j = over(w, by_b), b = w - j * B;
         if (b < nb) base[(int64_t)j * ntr + b] = v;
     });
 }
@@ -1240,7 +1475,6 @@ struct ZReg {
     static constexpr int M = N / 16;                                  // threads per column group
     static constexpr int L = M > 16 ? M / 16 : M;                     // points of the last DFT
     static constexpr bool TWO = M > 16;                               // two exchanges
-    static constexpr int G = 16 / L;
     static constexpr int BG = N >= 2048 ? 4 : (N >= 512 ? 8 : 4096 / N);
     static constexpr int THREADS = M * BG;
     static constexpr int ROW1 = M * BG + BG;
@@ -1304,43 +1538,17 @@ __device__ __forceinline__ void zreg_exchange(cplx<R> (&v)[16], cplx<R> (&w)[16]
     __syncthreads();
 }
 
-// The G DFTs of L points of v (group g: v[g L ..], natural order in and out).
+// The 16 / L DFTs of L points of v (group g: v[g L ..], natural order in and out).
 template <typename R, int L>
-__device__ __forceinline__ void zreg_last(cplx<R> (&v)[16], int sign) {
-    if constexpr (L == 2) {
+__device__ __forceinline__ void zreg_last(cplx<R> (&v)[16], R sg) {
 #pragma unroll
-        for (int g = 0; g < 8; ++g) {
-            const cplx<R> t = v[2 * g];
-            v[2 * g] = cadd(t, v[2 * g + 1]);
-            v[2 * g + 1] = csub(t, v[2 * g + 1]);
-        }
-    } else if constexpr (L == 4) {
+    for (int g = 0; g < 16 / L; ++g) {
+        cplx<R> x[L];
 #pragma unroll
-        for (int g = 0; g < 4; ++g) dft4(v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3], sign);
-    } else if constexpr (L == 8) {
-        const R h = (R)0.70710678118654752440;
-        const R sg = (R)(sign < 0 ? -1 : 1);
+        for (int k = 0; k < L; ++k) x[k] = v[g * L + k];
+        SmallDft<R, L>::run(x, sg);
 #pragma unroll
-        for (int g = 0; g < 2; ++g) {
-            cplx<R>* x = v + 8 * g;
-            dft4(x[0], x[2], x[4], x[6], sign);
-            dft4(x[1], x[3], x[5], x[7], sign);
-            const cplx<R> o1 = cmul(x[3], cplx<R>{h, sg * h}), o3 = cmul(x[7], cplx<R>{-h, sg * h});
-            const cplx<R> o2 = (sign < 0) ? cplx<R>{x[5].y, -x[5].x} : cplx<R>{-x[5].y, x[5].x};
-            const cplx<R> e[4] = {x[0], x[2], x[4], x[6]}, o[4] = {x[1], o1, o2, o3};
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                x[k] = cadd(e[k], o[k]);
-                x[4 + k] = csub(e[k], o[k]);
-            }
-        }
-    } else {
-        dft16(v, sign);
-        cplx<R> t[16];
-#pragma unroll
-        for (int k = 0; k < 16; ++k) t[k] = v[dft16_at(k)];
-#pragma unroll
-        for (int k = 0; k < 16; ++k) v[k] = t[k];
+        for (int k = 0; k < L; ++k) v[g * L + k] = x[SmallDft<R, L>::at(k)];
     }
 }
 
@@ -1349,7 +1557,7 @@ __device__ __forceinline__ void zreg_last(cplx<R> (&v)[16], int sign) {
 template <typename R, int N, int OP>
 __global__ __launch_bounds__(ZReg<N>::THREADS, 4) void k_fft_zreg(DiffArgs<R> a, int sign) {
     using Z = ZReg<N>;
-    constexpr int C = ZWord<R>::C, M = Z::M, L = Z::L, G = Z::G, BG = Z::BG;
+    constexpr int C = ZWord<R>::C, M = Z::M, L = Z::L, BG = Z::BG;
     extern __shared__ unsigned char smem_raw[];
     auto* buf = reinterpret_cast<typename ZWord<R>::type*>(smem_raw);
     // columns counted over x, then y; neighbouring blocks share the cache
@@ -1394,16 +1602,16 @@ __global__ __launch_bounds__(ZReg<N>::THREADS, 4) void k_fft_zreg(DiffArgs<R> a,
         if constexpr (C > 1) w[i] = cmul(w[i], r);
     };
     auto dft = [&](int sg) {
-        dft16(v, sg);
+        dft16(v, (R)sg);
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (C > 1) {
-            dft16(w, sg);
+            dft16(w, (R)sg);
             __builtin_amdgcn_sched_barrier(0);
         }
     };
     auto last = [&](int sg) {
-        zreg_last<R, L>(v, sg);
-        if constexpr (C > 1) zreg_last<R, L>(w, sg);
+        zreg_last<R, L>(v, (R)sg);
+        if constexpr (C > 1) zreg_last<R, L>(w, (R)sg);
     };
     // words of (q, u), of (v, q 16 + q2), and of the last step's (group, point)
     auto w1 = [&](int q, int u) { return q * Z::ROW1 + u * BG + b; };
@@ -1521,51 +1729,52 @@ static void lds_opt_in(const void* kernel, size_t bytes) {
         (void)hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
 }
 
-// Lines per workgroup: two LDS line buffers and the twiddle table within
-// `budget` bytes.
+// Lines per workgroup (B) and its LDS buffers: one line buffer, or two (TWO)
+// where the plan has a pass of more than 16 points, is Rader's, or holds more
+// butterflies in a pass than the threads do in registers with one line already.
+// tw: the twiddle table in LDS too (x and y lines).  In place every pass's
+// butterflies must fit (radix_pass), and a line of 420 points in FP64 takes
+// 27 KiB for four lines instead of two in two buffers: 154 -> 51 us per z2 pass
+// over 90 x 75 x 420 with the passes of 5, 7, ... points in registers.
 #ifndef PUFF_Z_LDS_BUDGET
 #define PUFF_Z_LDS_BUDGET (32 * 1024)
 #endif
 #ifndef PUFF_XY_LDS_BUDGET
 #define PUFF_XY_LDS_BUDGET (32 * 1024)
 #endif
-static constexpr int lines_per_block(int n, size_t elem, int cap, size_t budget, bool il) {
-    const size_t tw = (size_t)n * elem;
+static constexpr int lines_per_block(int n, size_t elem, int cap, size_t budget, bool il, bool two, bool tw) {
     int b = cap;
-    while (b > 1 && (2 * (size_t)(il ? lpad<true>(b * n) : lpad<false>(b * n)) * elem + tw) > budget) --b;
+    while (b > 1 &&
+           ((two ? 2 : 1) * (size_t)(il ? lpad<true>(b * n) : lpad<false>(b * n)) + (tw ? n : 0)) * elem > budget)
+        --b;
     return b;
 }
-
-// z2 lines per workgroup and whether the pass runs in place (one LDS
-// buffer): in place when every pass is radix 16, 4, 3 or 2 with at most one
-// butterfly per thread, and that leaves at least as many lines per workgroup
-// as two buffers do: C1's 1024-point lines in FP64 (616 -> 454 us per pass)
-// and C4's 4096-point lines (7.50 -> 6.92 ms).  Otherwise two line buffers,
-// no twiddle table (wider workgroups with longer runs along x measured
-// slower: occupancy matters more than coalescing here).
-struct ZPlan {
-    int B;
-    bool inplace;
+struct LinePlan {
+    int B, kind;
 };
-static constexpr ZPlan z_plan(int n, size_t elem, bool rader, int npass, const int* radix) {
-    bool inplace = !rader;
-    int minr = 16;
-    for (int k = 0; k < npass; ++k) {
-        const int r = radix[k];
-        if (r != 2 && r != 3 && r != 4 && r != 16) inplace = false;
-        if (r < minr) minr = r;
+static LinePlan line_plan(const FftAxis& ax, size_t elem, int cap, size_t budget, bool il, bool tw) {
+    int kind = ax.rader ? LINE_TWO : LINE_SMALL;
+    int fit = cap;   // lines whose butterflies fit the registers
+    for (int k = 0; k < ax.npass; ++k) {
+        const int r = ax.radix[k];
+        if (r > 16 && k > 0) {
+            kind = LINE_TWO;
+        } else if (r > 16) {
+            if (kind == LINE_SMALL) kind = LINE_PRIME;
+            while (fit > 0 && mfma_tiles(fit, ax.n, r) > 4 * MFMA_TILES) --fit;
+        } else {
+            fit = std::min(fit, (16 / r) * 256 / (ax.n / r));
+        }
     }
-    int B = (int)((PUFF_Z_LDS_BUDGET) / (2 * (size_t)n * elem));
-    B = B < 1 ? 1 : (B > 16 ? 16 : B);   // lines per workgroup with two buffers
-    if (inplace) {
-        int Bi = (int)((PUFF_Z_LDS_BUDGET) / ((size_t)n * elem));
-        Bi = Bi > 16 ? 16 : Bi;
-        const int bt = PUFF_Z_THREADS / (n / minr);   // one butterfly per thread
-        Bi = Bi > bt ? bt : Bi;
-        inplace = Bi >= 1 && Bi >= B;
-        if (inplace) B = Bi;
+    if (fit < 1) kind = LINE_TWO;
+    if (kind == LINE_PRIME) {
+        tw = true;
+        // whole tiles of 8 butterflies, where 64 KiB have room for them
+        const int whole = (8 + ax.n / ax.radix[0] - 1) / (ax.n / ax.radix[0]);
+        if (lines_per_block(ax.n, elem, whole, 2 * budget, il, false, true) == whole) budget *= 2;
     }
-    return ZPlan{B, inplace};
+    const bool two = kind == LINE_TWO;
+    return {lines_per_block(ax.n, elem, two ? cap : fit, budget, il, two, tw), kind};
 }
 
 #ifndef PUFF_Y_LDS_BUDGET
@@ -1573,18 +1782,18 @@ static constexpr ZPlan z_plan(int n, size_t elem, bool rader, int npass, const i
 #endif
 template <typename R, int NC>
 static constexpr int ct_lines_x() {
-    return lines_per_block(NC, sizeof(cplx<R>), 64, PUFF_XY_LDS_BUDGET, false);
+    return lines_per_block(NC, sizeof(cplx<R>), 64, PUFF_XY_LDS_BUDGET, false, true, true);
 }
 template <typename R, int NC>
 static constexpr int ct_lines_y() {
-    return lines_per_block(NC, sizeof(cplx<R>), 16, PUFF_Y_LDS_BUDGET, true);
+    return lines_per_block(NC, sizeof(cplx<R>), 16, PUFF_Y_LDS_BUDGET, true, true, true);
 }
-template <typename R, int NC, int BC, int OP>
+template <typename R, int NC, int BC, int KIND, int OP>
 static void launch_x_op(const DiffArgs<R>& a, int B, int sign, hipStream_t s) {
     const int64_t nlines = (int64_t)a.ny * a.nzp;
-    const size_t sh = (2 * (size_t)lpad<false>(B * a.nx) + a.nx) * sizeof(cplx<R>);
-    lds_opt_in(reinterpret_cast<const void*>(&k_fft_x<R, NC, BC, OP>), sh);
-    hipLaunchKernelGGL((k_fft_x<R, NC, BC, OP>), dim3((unsigned)((nlines + B - 1) / B)), dim3(256), sh, s, a, B,
+    const size_t sh = ((KIND == LINE_TWO ? 2 : 1) * (size_t)lpad<false>(B * a.nx) + a.nx) * sizeof(cplx<R>);
+    lds_opt_in(reinterpret_cast<const void*>(&k_fft_x<R, NC, BC, KIND, OP>), sh);
+    hipLaunchKernelGGL((k_fft_x<R, NC, BC, KIND, OP>), dim3((unsigned)((nlines + B - 1) / B)), dim3(256), sh, s, a, B,
                        sign);
 }
 
@@ -1607,34 +1816,38 @@ static void run_rader_x(const DiffArgs<R>& a, int op, int sign, hipStream_t s) {
     }
 }
 
-template <typename R, int NC, int BC>
+template <typename R, int NC, int BC, int KIND>
 static void launch_x(const DiffArgs<R>& a, int B, int op, int sign, hipStream_t s) {
     if (BC) B = BC;   // compile-time plans fix their lines per workgroup
     switch (op) {
-        case XOP_FORWARD: return launch_x_op<R, NC, BC, XOP_FORWARD>(a, B, sign, s);
-        case XOP_INV_SPLIT_FWD: return launch_x_op<R, NC, BC, XOP_INV_SPLIT_FWD>(a, B, sign, s);
-        case XOP_INV_RECOMBINE: return launch_x_op<R, NC, BC, XOP_INV_RECOMBINE>(a, B, sign, s);
-        case XOP_ADJ_FOLD_SAVE_FWD: return launch_x_op<R, NC, BC, XOP_ADJ_FOLD_SAVE_FWD>(a, B, sign, s);
-        case XOP_ADJ_INV_MIX_FWD: return launch_x_op<R, NC, BC, XOP_ADJ_INV_MIX_FWD>(a, B, sign, s);
-        default: return launch_x_op<R, NC, BC, XOP_ADJ_INV_SCALE>(a, B, sign, s);
+        case XOP_FORWARD: return launch_x_op<R, NC, BC, KIND, XOP_FORWARD>(a, B, sign, s);
+        case XOP_INV_SPLIT_FWD: return launch_x_op<R, NC, BC, KIND, XOP_INV_SPLIT_FWD>(a, B, sign, s);
+        case XOP_INV_RECOMBINE: return launch_x_op<R, NC, BC, KIND, XOP_INV_RECOMBINE>(a, B, sign, s);
+        case XOP_ADJ_FOLD_SAVE_FWD: return launch_x_op<R, NC, BC, KIND, XOP_ADJ_FOLD_SAVE_FWD>(a, B, sign, s);
+        case XOP_ADJ_INV_MIX_FWD: return launch_x_op<R, NC, BC, KIND, XOP_ADJ_INV_MIX_FWD>(a, B, sign, s);
+        default: return launch_x_op<R, NC, BC, KIND, XOP_ADJ_INV_SCALE>(a, B, sign, s);
     }
 }
 
 template <typename R>
 static void run_x(const DiffArgs<R>& a, int op, int sign, hipStream_t s) {
     if (a.nx == RAD_N) return run_rader_x(a, op, sign, s);
-    const int B = lines_per_block(a.nx, sizeof(cplx<R>), 64, PUFF_XY_LDS_BUDGET, false);
-    if (a.nx == 129) return launch_x<R, 129, ct_lines_x<R, 129>()>(a, B, op, sign, s);
-    if (a.nx == 33) return launch_x<R, 33, ct_lines_x<R, 33>()>(a, B, op, sign, s);
-    launch_x<R, 0, 0>(a, B, op, sign, s);
+    if (a.nx == 129) return launch_x<R, 129, ct_lines_x<R, 129>(), LINE_TWO>(a, 0, op, sign, s);
+    if (a.nx == 33) return launch_x<R, 33, ct_lines_x<R, 33>(), LINE_TWO>(a, 0, op, sign, s);
+    const LinePlan lp = line_plan(a.ax, sizeof(cplx<R>), 64, PUFF_XY_LDS_BUDGET, false, true);
+    switch (lp.kind) {
+        case LINE_SMALL: return launch_x<R, 0, 0, LINE_SMALL>(a, lp.B, op, sign, s);
+        case LINE_PRIME: return launch_x<R, 0, 0, LINE_PRIME>(a, lp.B, op, sign, s);
+        default: return launch_x<R, 0, 0, LINE_TWO>(a, lp.B, op, sign, s);
+    }
 }
 
-template <typename R, int NC, int BC>
+template <typename R, int NC, int BC, int KIND>
 static void launch_y(const DiffArgs<R>& a, int B, int sign, hipStream_t s) {
     if (BC) B = BC;   // compile-time plans fix their lines per workgroup
-    const size_t sh = (2 * (size_t)lpad<true>(B * a.ny) + a.ny) * sizeof(cplx<R>);
-    lds_opt_in(reinterpret_cast<const void*>(&k_fft_y<R, NC, BC>), sh);
-    hipLaunchKernelGGL((k_fft_y<R, NC, BC>), dim3((unsigned)xcd_grid((int64_t)((a.nx + B - 1) / B) * a.nzp)),
+    const size_t sh = ((KIND == LINE_TWO ? 2 : 1) * (size_t)lpad<true>(B * a.ny) + a.ny) * sizeof(cplx<R>);
+    lds_opt_in(reinterpret_cast<const void*>(&k_fft_y<R, NC, BC, KIND>), sh);
+    hipLaunchKernelGGL((k_fft_y<R, NC, BC, KIND>), dim3((unsigned)xcd_grid((int64_t)((a.nx + B - 1) / B) * a.nzp)),
                        dim3(256), sh, s, a, B, sign);
 }
 
@@ -1646,18 +1859,22 @@ static void run_y(const DiffArgs<R>& a, int sign, hipStream_t s) {
         hipLaunchKernelGGL((k_rader_y<R>), dim3((unsigned)blocks), dim3(16 * BL), 0, s, a, sign);
         return;
     }
-    const int B = lines_per_block(a.ny, sizeof(cplx<R>), 16, PUFF_Y_LDS_BUDGET, true);
-    if (a.ny == 129) return launch_y<R, 129, ct_lines_y<R, 129>()>(a, B, sign, s);
-    if (a.ny == 33) return launch_y<R, 33, ct_lines_y<R, 33>()>(a, B, sign, s);
-    launch_y<R, 0, 0>(a, B, sign, s);
+    if (a.ny == 129) return launch_y<R, 129, ct_lines_y<R, 129>(), LINE_TWO>(a, 0, sign, s);
+    if (a.ny == 33) return launch_y<R, 33, ct_lines_y<R, 33>(), LINE_TWO>(a, 0, sign, s);
+    const LinePlan lp = line_plan(a.ay, sizeof(cplx<R>), 16, PUFF_Y_LDS_BUDGET, true, true);
+    switch (lp.kind) {
+        case LINE_SMALL: return launch_y<R, 0, 0, LINE_SMALL>(a, lp.B, sign, s);
+        case LINE_PRIME: return launch_y<R, 0, 0, LINE_PRIME>(a, lp.B, sign, s);
+        default: return launch_y<R, 0, 0, LINE_TWO>(a, lp.B, sign, s);
+    }
 }
 
-template <typename R, bool IP>
+template <typename R, int KIND>
 static void launch_z(const DiffArgs<R>& a, int B, int op, int sign, hipStream_t s) {
-    const size_t sh = (IP ? 1 : 2) * (size_t)lpad<true>(B * a.nzp) * sizeof(cplx<R>);
+    const size_t sh = ((KIND == LINE_TWO ? 2 : 1) * (size_t)lpad<true>(B * a.nzp) + (KIND == LINE_PRIME ? a.nzp : 0)) * sizeof(cplx<R>);
     const int64_t blocks = xcd_grid((int64_t)((a.nx + B - 1) / B) * a.ny);
-    lds_opt_in(reinterpret_cast<const void*>(&k_fft_z<R, IP>), sh);
-    hipLaunchKernelGGL((k_fft_z<R, IP>), dim3((unsigned)blocks), dim3(PUFF_Z_THREADS), sh, s, a, B, op,
+    lds_opt_in(reinterpret_cast<const void*>(&k_fft_z<R, KIND>), sh);
+    hipLaunchKernelGGL((k_fft_z<R, KIND>), dim3((unsigned)blocks), dim3(PUFF_Z_THREADS), sh, s, a, B, op,
                        sign);
 }
 
@@ -1686,9 +1903,12 @@ static void run_z(const DiffArgs<R>& a, int op, int sign, hipStream_t s) {
         launch_zreg<R, 512>(a, op, sign, s) || launch_zreg<R, 1024>(a, op, sign, s) ||
         launch_zreg<R, 2048>(a, op, sign, s) || launch_zreg<R, 4096>(a, op, sign, s))
         return;
-    const ZPlan zp = z_plan(a.nzp, sizeof(cplx<R>), a.az.rader, a.az.npass, a.az.radix);
-    if (zp.inplace) launch_z<R, true>(a, zp.B, op, sign, s);
-    else launch_z<R, false>(a, zp.B, op, sign, s);
+    const LinePlan lp = line_plan(a.az, sizeof(cplx<R>), 16, PUFF_Z_LDS_BUDGET, true, false);
+    switch (lp.kind) {
+        case LINE_SMALL: return launch_z<R, LINE_SMALL>(a, lp.B, op, sign, s);
+        case LINE_PRIME: return launch_z<R, LINE_PRIME>(a, lp.B, op, sign, s);
+        default: return launch_z<R, LINE_TWO>(a, lp.B, op, sign, s);
+    }
 }
 
 template <typename R>
