@@ -37,13 +37,14 @@ def log(msg: str) -> None:
 # and chi and writes k_s; stage 4 also reads k1, k2 and writes y) and per
 # active node per stage; the field combination and the diffraction per node.
 def stage_bytes(precision: int):
-    if precision == 0:   # FP64: six-vector 48 B, chi 8 B, complex 16 B
-        part = [48 + 8 + 48, 48 + 48 + 8 + 48, 48 + 48 + 8 + 48, 4 * 48 + 8 + 48]
+    # derivatives are kept of p_r, p_i and Gamma; those of x, y and z2 are
+    # formed again from the momenta (stage 3 reads k1 and k2, stage 4 all three)
+    if precision == 0:   # FP64: state 48 B, derivative 24 B, chi 8 B, complex 16 B
+        part = [48 + 8 + 24, 48 + 24 + 8 + 24, 48 + 2 * 24 + 8 + 24, 48 + 3 * 24 + 8 + 48]
         node = [2 * 16, 3 * 16, 3 * 16, 3 * 16]
         comb, diff = 6 * 16, 14 * 16
-    else:                # mixed: state 32 B (z2, Gamma FP64), derivative k 24 B (all FP32),
-        # chi 4 B, complex 8 B
-        part = [32 + 4 + 24, 32 + 24 + 4 + 24, 32 + 24 + 4 + 24, 32 + 3 * 24 + 4 + 32]
+    else:                # mixed: state 32 B (z2, Gamma FP64), derivative 12 B, chi 4 B, complex 8 B
+        part = [32 + 4 + 12, 32 + 12 + 4 + 12, 32 + 2 * 12 + 4 + 12, 32 + 3 * 12 + 4 + 32]
         node = [2 * 8, 3 * 8, 3 * 8, 3 * 8]
         comb, diff = 6 * 8, 14 * 8
     return part, node, comb, diff

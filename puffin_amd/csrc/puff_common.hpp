@@ -60,7 +60,7 @@ constexpr int BOX_COPIES = 64;
 
 // Workgroup of the RK4 stage kernels (one macroparticle per thread) and the
 // node capacity of its LDS deposit tile.  Four-wave workgroups (one wave per
-// SIMD each); the stage kernels hold 42-76 VGPRs, so the LDS tiles set how
+// SIMD each); the stage kernels hold 60-80 VGPRs, so the LDS tiles set how
 // many workgroups share a CU: 1280 nodes (2 FP64 each, 20 KiB) in the FP64
 // form, 3072 (one packed 8-byte word each, 24 KiB) in the mixed form.
 // Measured on the C1 beam: FP64 tiles of 768 and 2048 nodes gave 3.17 and
@@ -71,20 +71,9 @@ constexpr int BOX_COPIES = 64;
 #define PUFF_STAGE_THREADS 256
 #endif
 constexpr int STAGE_THREADS = PUFF_STAGE_THREADS;
-// Macroparticles per thread of a stage workgroup, and its workgroups.
-#ifndef PUFF_STAGE_WIDE
-#define PUFF_STAGE_WIDE 1
-#endif
-constexpr int STAGE_WIDE = PUFF_STAGE_WIDE;
-constexpr int64_t STAGE_WIDE_MIN = (int64_t)4 * 256 * STAGE_THREADS * STAGE_WIDE;
-inline int stage_per_thread(int stage, int64_t n, int precision, bool general) {
-    return (precision == PUFF_MIXED && stage < 4 && n >= STAGE_WIDE_MIN && !general) ? STAGE_WIDE : 1;
-}
+// Undulator types with hyperbolic fields: the stage kernels' POLE instances.
 inline bool stage_pole(int und_type) { return und_type == PUFF_UND_PLANEPOLE || und_type == PUFF_UND_CURVED; }
-inline int64_t stage_workgroups(int64_t n, int per_thread) {
-    const int64_t w = (int64_t)STAGE_THREADS * per_thread;
-    return (n + w - 1) / w;
-}
+inline int64_t stage_workgroups(int64_t n) { return (n + STAGE_THREADS - 1) / STAGE_THREADS; }
 #ifndef PUFF_TILE_NODES_FP64
 #define PUFF_TILE_NODES_FP64 1280
 #endif
@@ -104,8 +93,7 @@ constexpr int stage_tile_nodes() {
 }
 // Node capacity of the stage kernels' LDS copy of the field over the
 // workgroup's node box (one complex per node; larger boxes gather from
-// global memory); the box of two macroparticles per thread fits 512 nodes as
-// often as that of one fits 256.
+// global memory): what fits behind the first 512 nodes of either deposit tile.
 #ifndef PUFF_FIELD_TILE_NODES
 #define PUFF_FIELD_TILE_NODES 512
 #endif
@@ -116,8 +104,8 @@ constexpr int FIELD_TILE_NODES = PUFF_FIELD_TILE_NODES;
 constexpr int ADJ_THREADS = 256;
 // Deposit tile (two doubles per node): 2000 nodes keep a workgroup's LDS
 // (with the field tile) under 40 KiB, four workgroups per CU, as many as the
-// kernel's 116 VGPRs allow.  1024 nodes sent more of C4's sparse-beam
-// workgroups to global atomics: its adjoint stages took 969 ms per 30 steps
+// kernel's 118 VGPRs allow.  With 1024 nodes more of C4's sparse-beam
+// workgroups overflowed it (and took global atomics then): its adjoint stages took 969 ms per 30 steps
 // against 888 ms.
 constexpr int ADJ_TILE_NODES = 2000;
 constexpr int ADJ_FIELD_TILE_NODES = 256;   // LDS copy of the trial field and source cotangent

@@ -246,8 +246,8 @@ static void factorize(int n, FftAxis& ax) {
 template <typename R>
 static int make_axis(Ctx* c, int n, FftAxis& ax, bool z2_axis = false) {
     // one line, its ping-pong buffer and the twiddle table share a
-    // workgroup's LDS (160 KiB on gfx950); 4096-point z2 lines run as
-    // 64 x 64 (four-step) in either form
+    // workgroup's LDS (160 KiB on gfx950); 4096-point z2 lines stay in
+    // registers (k_fft_zreg), or take one buffer and no table (k_fft_z)
     if (3 * (size_t)n * sizeof(cplx<R>) > 160 * 1024 && !(z2_axis && n == 4096)) {
         set_error("FFT line of " + std::to_string(n) + " points does not fit one workgroup's LDS");
         return PUFF_ERR_ARG;
@@ -968,10 +968,7 @@ static int rk4par(Ctx* c, double sz, double h, char* cap = nullptr, void* cap_hd
         // could not use the LDS tile exceeds twice its value after the sort
         // (measured on the bunched C1 beam: sorting at that point beats
         // letting the share grow until the fallback has cost one sort)
-        const bool general = c->det || stage_pole(c->p.und_type);
-        double groups = 0.0;
-        for (int st = 1; st <= 4; ++st)
-            groups += (double)stage_workgroups(c->n, stage_per_thread(st, c->n, c->precision, general));
+        const double groups = 4.0 * (double)stage_workgroups(c->n);
         const double share = groups > 0 ? (double)c->h_flags[FLAG_WORD_FALLBACK] / groups : 0.0;
         c->fallback_last = share;
         if (c->steps_since_sort == 1) c->fallback_base = share;
@@ -1188,7 +1185,7 @@ static int download_field(Ctx* c, int kind, double* ar, double* ai) {
 template <typename R>
 static int transform(Ctx* c, int sign) {
     if (c->p.one_d) return PUFF_ERR_STATE;
-    launch_fft3d<R>(reinterpret_cast<cplx<R>*>(c->A), reinterpret_cast<cplx<R>*>(c->anb), c->p.nx, c->p.ny,
+    launch_fft3d<R>(reinterpret_cast<cplx<R>*>(c->A), c->p.nx, c->p.ny,
                     c->nzp(), c->ax, c->ay, c->az, sign, c->stream);
     PUFF_HIP(hipGetLastError());
     PUFF_HIP(hipStreamSynchronize(c->stream));
@@ -1799,7 +1796,6 @@ constexpr uint64_t CAPTURE_MAGIC = 0x3150414346465550ull;   // "PUFFCAP1"
 // stage sources in the capture; a host copy of the header to cap_hdr.
 template <typename R>
 static void capture_start(Ctx* c, char* cap, void* cap_hdr, CaptureView<R>& v, const double* taper0) {
-    Particles<R>& P = parts<R>(c);
     capture_view<R>(c, cap, &v);
     Words64 words{};
     BlobHeader* hd = reinterpret_cast<BlobHeader*>(words.w);

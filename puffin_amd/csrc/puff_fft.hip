@@ -5,19 +5,18 @@
 // sign -1 forward, +1 backward, unnormalised; the backward result is divided
 // by ffact = NX NY NZ2' afterwards (diffraction.f90:310, 513).
 //
-// Each workgroup holds B whole lines in LDS and runs a Stockham autosort
-// transform (natural order in and out), one radix pass per LDS round trip.
-// Radices 2, 3, 4 and 16 have explicit butterflies (16 as 4 x 4 in
-// registers, halving the passes and barriers of power-of-two lines); any
-// other factor (11, 43, 127, ...) is a direct DFT pass; a prime line length
-// with a power-of-two n - 1 (17, 257) uses Rader's algorithm (transverse lines
-// of 257 points with their own kernels, k_rader_x and k_rader_y).
+// Routes by line length: z2 lines of a power of two from 128 to 4096 in
+// registers (k_fft_zreg); transverse lines of 257 points by Rader's algorithm in
+// registers (k_rader_x, k_rader_y); all others as whole lines in LDS, a
+// workgroup B of them, in Stockham passes (natural order in and out), one LDS
+// round trip each: compiled plans for 33 and 129 points, and runtime plans of
+// passes of 2 to 16 points, a large prime on the matrix cores, or direct sums
+// for what is larger still (line_plan).
 //
 // DiffractionStep (diffraction.f90:209-348) becomes nine line passes:
 //   x fwd | y fwd | z fwd . multiplyexp . z inv | y inv |
 //   x inv . /ffact . mask split . x fwd | y fwd | z fwd . damping . z inv |
 //   y inv | x inv . /ffact . + interior
-// (4096-point z2 lines: each z2 pass as three four-step passes, k_fft_z4).
 #include "puff_common.hpp"
 #include "puff_kernels.hpp"
 
@@ -668,7 +667,9 @@ __device__ __forceinline__ void lds_pass(const cplx<R>* src, cplx<R>* dst, int B
 // 1024 FMAs instead of once per 4 (direct_pass reads 6 LDS words of 16 bytes
 // for 16 FMAs per lane and is bound by that).  In place: the tiles stay in
 // accumulators until every input is read; the wavefronts deal the tiles out,
-// at most MFMA_TILES each (checked on the host).
+// at most MFMA_TILES each (checked on the host).  A spectral pass over 61 x 47
+// lines of 389 points, FP64: 200 -> 124 us (bound by LDS latency at two
+// workgroups a CU).
 //   Operands: lane l holds A[row l % 16][k = l / 16] and B[k = l / 16][column l % 16];
 //   results: column l % 16, row l / 16 + 4 v (FP64) or 4 (l / 16) + v (FP32), v < 4.
 template <typename R>
@@ -1470,6 +1471,10 @@ __global__ __launch_bounds__(PUFF_Z_THREADS, 4) void k_fft_z(DiffArgs<R> a, int 
 //   layout 1, of (q, u): q-major, a spare row of BG words after every q;
 //   layout 2, of (v, q, q2): v-major, a spare row after every v.
 // Both spread the lanes of a write and of a read over all banks.
+// A spectral pass over 129 x 129 lines of 1024 points (FP64; 112 us at the rate
+// of a large copy) took 269 us with two lines a workgroup in LDS; a diffraction
+// step, two such passes of nine, went from 1895 to 1797 us.  257 x 257 lines of
+// 4096 (FP32): three passes of memory became one, 19.4 -> 16.7 ms.
 template <int N>
 struct ZReg {
     static constexpr int M = N / 16;                                  // threads per column group
@@ -1729,13 +1734,14 @@ static void lds_opt_in(const void* kernel, size_t bytes) {
         (void)hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
 }
 
-// Lines per workgroup (B) and its LDS buffers: one line buffer, or two (TWO)
-// where the plan has a pass of more than 16 points, is Rader's, or holds more
-// butterflies in a pass than the threads do in registers with one line already.
-// tw: the twiddle table in LDS too (x and y lines).  In place every pass's
-// butterflies must fit (radix_pass), and a line of 420 points in FP64 takes
-// 27 KiB for four lines instead of two in two buffers: 154 -> 51 us per z2 pass
-// over 90 x 75 x 420 with the passes of 5, 7, ... points in registers.
+// Lines per workgroup (B) and the plan's kind.  In place every pass's
+// butterflies must fit the threads' registers (radix_pass) and the matrix
+// pass's tiles their accumulators; where one line already does not, or a plan
+// has Rader's or a second large prime, two buffers.  tw: the twiddle table in
+// LDS too (x and y lines).  Both sides of the line, one diffraction step:
+// 90 x 75 x 420 (FP64) 816 us in two buffers with direct sums of 5 and 7,
+// 364 us in place; 61 x 47 x 389 640 us with direct sums, 375 us on the matrix
+// cores; 76 x 42 x 457 (mixed) 615 and 335 us.
 #ifndef PUFF_Z_LDS_BUDGET
 #define PUFF_Z_LDS_BUDGET (32 * 1024)
 #endif
@@ -1949,11 +1955,10 @@ void launch_diffraction_adjoint(const DiffArgs<R>& a, hipStream_t s) {
 }
 
 template <typename R>
-void launch_fft3d(cplx<R>* data, cplx<R>* tmp, int nx, int ny, int nz, const FftAxis& ax, const FftAxis& ay,
-                  const FftAxis& az, int sign, hipStream_t s) {
+void launch_fft3d(cplx<R>* data, int nx, int ny, int nz, const FftAxis& ax, const FftAxis& ay, const FftAxis& az,
+                  int sign, hipStream_t s) {
     DiffArgs<R> a{};
     a.a = data;
-    a.anb = tmp;
     a.nx = nx;
     a.ny = ny;
     a.nz2 = nz;
@@ -1970,9 +1975,9 @@ template void launch_diffraction<double>(const DiffArgs<double>&, hipStream_t);
 template void launch_diffraction<float>(const DiffArgs<float>&, hipStream_t);
 template void launch_diffraction_adjoint<double>(const DiffArgs<double>&, hipStream_t);
 template void launch_diffraction_adjoint<float>(const DiffArgs<float>&, hipStream_t);
-template void launch_fft3d<double>(cplx<double>*, cplx<double>*, int, int, int, const FftAxis&,
-                                   const FftAxis&, const FftAxis&, int, hipStream_t);
-template void launch_fft3d<float>(cplx<float>*, cplx<float>*, int, int, int, const FftAxis&, const FftAxis&,
-                                  const FftAxis&, int, hipStream_t);
+template void launch_fft3d<double>(cplx<double>*, int, int, int, const FftAxis&, const FftAxis&, const FftAxis&, int,
+                                   hipStream_t);
+template void launch_fft3d<float>(cplx<float>*, int, int, int, const FftAxis&, const FftAxis&, const FftAxis&, int,
+                                  hipStream_t);
 
 }  // namespace puff

@@ -18,15 +18,17 @@
 
 namespace puff {
 
-// One RK4 stage.  STAGE = 1..4 (rk4par's four derivs calls), P macroparticles
-// per thread (STAGE_THREADS apart).  DET: the deterministic fixed-point
-// deposit (FP64 form only; see DetState).
+// One RK4 stage.  STAGE = 1..4 (rk4par's four derivs calls).  DET: the
+// deterministic fixed-point deposit (FP64 form only; see DetState).
 //
-// Two macroparticles per thread halve what a workgroup pays per macroparticle
-// for its node box, field tile, flush and barriers, and give the memory twice
-// the loads per wavefront.
-template <typename R, int STAGE, bool DET, int P, bool POLE>
+// One macroparticle per thread (P): with two, a workgroup's box, field tile and
+// flush serve twice as many, which took 20 % off the mixed stage 1 of 2^24 on
+// 129 x 129 x 1024, and added 40 to 120 % to the stages of thin beams, whose
+// boxes then grow past the tile.  (Written without the loops over P the
+// compiler specialises the gather's branches: 1 to 3 % slower stages.)
+template <typename R, int STAGE, bool DET, bool POLE>
 __global__ __launch_bounds__(STAGE_THREADS) void k_stage(StageArgs<R> a) {
+    constexpr int P = 1;
     // Deposit tiles: two doubles per node in the FP64 form; DET_WORDS 8-byte
     // integers in its deterministic mode; one 8-byte packed fixed-point word
     // in the mixed form (packed_add: one ds_add_u64 per corner for
@@ -258,7 +260,8 @@ __global__ __launch_bounds__(STAGE_THREADS) void k_stage(StageArgs<R> a) {
             R bx, by, bz;
             bfield<R, POLE>(a.s, x[p], y[p], bx, by, bz);
             const R facr = (R)fac[p];
-            const R n2col = a.s.template strength<R>(), kappa = ph.template scale<R>().kappa, inv2rho = ph.template scale<R>().inv2rho;
+            const R n2col = a.s.template strength<R>();
+            const R kappa = ph.template scale<R>().kappa, inv2rho = ph.template scale<R>().inv2rho;
             // the roundings written out: a different contraction moves the
             // mixed form's p_r by 2e-6 and z2 by 2e-9 over a lattice
             const R pull_r = inv2rho * fma(n2col, by, -(ep2k[p] * fr[p]));
@@ -364,7 +367,6 @@ __global__ __launch_bounds__(STAGE_THREADS) void k_stage(StageArgs<R> a) {
                 }
             });
     }
-
 }
 
 // Start of a step: clear flags and the active box.
@@ -477,24 +479,16 @@ __global__ void k_wrap_z2(double* z2, int64_t n, double lenz2) {
 
 template <typename R, int STAGE>
 static void launch_stage_n(const StageArgs<R>& a, hipStream_t s) {
-    const bool pole = stage_pole(a.s.und_type);
-    const int per = stage_per_thread(STAGE, a.n, sizeof(R) == 8 ? PUFF_FP64 : PUFF_MIXED, pole || a.det.acc);
-    const int64_t blocks = stage_workgroups(a.n, per);
+    const int64_t blocks = stage_workgroups(a.n);
     const dim3 grid((unsigned)(blocks > 0 ? blocks : 1)), thr(STAGE_THREADS);
     if constexpr (sizeof(R) == 8) {
         if (a.det.acc) {
-            hipLaunchKernelGGL((k_stage<R, STAGE, true, 1, true>), grid, thr, 0, s, a);
+            hipLaunchKernelGGL((k_stage<R, STAGE, true, true>), grid, thr, 0, s, a);
             return;
         }
     }
-    if constexpr (sizeof(R) == 4 && STAGE < 4) {
-        if (per > 1) {
-            hipLaunchKernelGGL((k_stage<R, STAGE, false, STAGE_WIDE, false>), grid, thr, 0, s, a);
-            return;
-        }
-    }
-    if (pole) hipLaunchKernelGGL((k_stage<R, STAGE, false, 1, true>), grid, thr, 0, s, a);
-    else hipLaunchKernelGGL((k_stage<R, STAGE, false, 1, false>), grid, thr, 0, s, a);
+    if (stage_pole(a.s.und_type)) hipLaunchKernelGGL((k_stage<R, STAGE, false, true>), grid, thr, 0, s, a);
+    else hipLaunchKernelGGL((k_stage<R, STAGE, false, false>), grid, thr, 0, s, a);
 }
 
 template <typename R>

@@ -649,7 +649,7 @@ constexpr float PACK_MAGIC = 12582912.0f;                      // 1.5 2^23
 constexpr unsigned long long PACK_MAGIC2 = 0x4B4000004B400000ull;   // its pattern, twice
 
 constexpr int PACK_MAX = 512;   // macroparticles of a workgroup
-static_assert(PACK_MAX >= STAGE_THREADS * STAGE_WIDE, "node sums below 2^31");
+static_assert(PACK_MAX >= STAGE_THREADS, "node sums below 2^31");
 
 // log2 of S for the workgroup's largest |s| (its bit pattern, max_bits): with
 // e taken 2^-20 above it, |s| S < 2^22 (1 - 2^-21), so |q| <= 2^22 - 1.
