@@ -114,7 +114,7 @@ static_assert(STAGE_THREADS == ADJ_THREADS, "one count of wavefronts per workgro
 
 // Flag words of the step kernels: [0] flag bits of the current step;
 // [FLAG_WORD_FALLBACK] the stage workgroups of the step whose node box did not
-// fit the LDS tile (global-atomic deposit): the host re-sorts the particles
+// fit the LDS tile (deposit wavefront by wavefront): the host re-sorts them
 // when that share grows; [FLAG_WORD_STICKY] the OR of the step flags since
 // the host last read them (deferred status).
 constexpr int FLAG_WORDS = 3;

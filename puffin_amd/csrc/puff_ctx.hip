@@ -107,8 +107,8 @@ struct Ctx {
     bool sorted = false;
     int sort_every = 30;
     int64_t steps_since_sort = 0;
-    // adaptive re-sort: share of stage workgroups that fell back to global
-    // atomics on the first step after the last sort, and the due flag
+    // adaptive re-sort: share of stage workgroups that overflowed their LDS
+    // tile on the first step after the last sort, and the due flag
     double fallback_base = 0.0;
     double fallback_last = 0.0;   // share of the last synchronised step
     bool sort_due = false;
