@@ -47,6 +47,15 @@ __global__ __launch_bounds__(STAGE_THREADS) void k_stage(StageArgs<R> a) {
         PACKED, unsigned long long,
         typename std::conditional<sizeof(R) == 4 && PUFF_MIXED_TILE == 2, float, double>::type>::type;
     constexpr int WORDS = DET ? DET_WORDS : (PACKED ? 1 : 2);
+    // Wavefronts that deposit in turn (tile_deposit) add in FP64, two words per
+    // node, in the mixed form too: the packed words round to 2^-22 of the
+    // workgroup's largest source, which a workgroup spread over the beam may
+    // hold far from its smallest.  A step on 129 x 129 x 1024 of 2^17 (all
+    // workgroups overflow), 2^20 (5 %) and 2^24 macroparticles (0.3 %): 326, 363
+    // and 1570 us; packed words for the single wavefronts too, 238, 326 and 1535;
+    // global atomics for whole workgroups, 482, 510 and 1680.
+    constexpr int WAVE_WORDS = PACKED ? 2 : WORDS;
+    constexpr int WAVE_TILE = TILE * WORDS / WAVE_WORDS;
     static_assert(WORDS * FIELD_TILE_NODES * sizeof(D) + FIELD_TILE_NODES * sizeof(cplx<R>) <=
                       WORDS * TILE * sizeof(D), "field tile inside the deposit tile");
     __shared__ D s_dep[WORDS * TILE];
@@ -338,14 +347,18 @@ __global__ __launch_bounds__(STAGE_THREADS) void k_stage(StageArgs<R> a) {
             if constexpr (DET)
                 det_add(m, t, c[p], cr, (double)sr[p], (double)si[p], det_scale,
                         reinterpret_cast<unsigned long long*>(s_dep));
-            else if constexpr (PACKED) packed_add(m, t, c[p], cr, (float)sr[p], (float)si[p], log2S, s_dep);
-            else tile_add<R, D>(m, t, c[p], cr, sr[p], si[p], s_dep);
+            else if constexpr (PACKED) {
+                if (use_tile) packed_add(m, t, c[p], cr, (float)sr[p], (float)si[p], log2S, s_dep);
+                else tile_add<R, double>(m, t, c[p], cr, sr[p], si[p], reinterpret_cast<double*>(s_dep));
+            } else tile_add<R, D>(m, t, c[p], cr, sr[p], si[p], s_dep);
         }
     };
     auto flush = [&](const TileBox& t) {
         if constexpr (DET) det_flush(m, t, a.det.acc, reinterpret_cast<const unsigned long long*>(s_dep));
-        else if constexpr (PACKED) packed_flush(m, t, log2S, reinterpret_cast<cplx<float>*>(a.dAout), s_dep);
-        else tile_flush<R, D>(m, t, a.dAout, s_dep);
+        else if constexpr (PACKED) {
+            if (use_tile) packed_flush(m, t, log2S, reinterpret_cast<cplx<float>*>(a.dAout), s_dep);
+            else tile_flush<R, double>(m, t, a.dAout, reinterpret_cast<const double*>(s_dep));
+        } else tile_flush<R, D>(m, t, a.dAout, s_dep);
     };
     if constexpr (DET) {
         // n |s| 2^F <= 2^62 keeps every node's integer sums in range
@@ -354,9 +367,9 @@ __global__ __launch_bounds__(STAGE_THREADS) void k_stage(StageArgs<R> a) {
             atomicOr(a.flags, FLAG_DET_RANGE);
     }
     if (ph.field_evolve) {
-        tile_deposit<TILE>(
-            m, tb, use_tile, s_red, [&](const TileBox& t) { tile_clear(s_dep, WORDS * t.tx * t.ty * t.tz); }, add,
-            flush,
+        tile_deposit<WAVE_TILE>(
+            m, tb, use_tile, s_red, [&](const TileBox& t) { tile_clear(s_dep, WAVE_WORDS * t.tx * t.ty * t.tz); },
+            add, flush,
             [&]() {
 #pragma unroll
                 for (int p = 0; p < P; ++p) {

@@ -599,9 +599,9 @@ __device__ __forceinline__ void global_add(const MeshGeom& m, bool ok, const Cel
 // not fit.  One loop for both, so that the code is there once: the two
 // together, inlined, took 18 to 40 registers more.
 // 2^20 macroparticles on 129 x 129 x 1024 (14 to 23 % of the FP64 workgroups
-// do not fit, 5 % of the mixed ones): a stage 200 us (mixed 89) with global
-// atomics for the whole workgroup, 97 (62) wavefront by wavefront; 2 10^5 of
-// them (all workgroups): 147 and 80 us.  With 2^24 (0.8 and 0.3 %) no change.
+// do not fit): a stage 200 us with global atomics for the whole workgroup, 97
+// wavefront by wavefront; 2 10^5 of them (all workgroups): 147 and 80 us.  With
+// 2^24 (0.8 %) no change.  (Mixed form: k_stage.)
 template <int TILE, typename C, typename A, typename F, typename S>
 __device__ __forceinline__ void tile_deposit(const MeshGeom& m, const TileBox& tb, bool whole,
                                              const WaveBoxes& s_red, C clear, A add, F flush, S spill) {
@@ -627,7 +627,7 @@ __device__ __forceinline__ void tile_deposit(const MeshGeom& m, const TileBox& t
     }
 }
 
-// ---- packed fixed-point tile (mixed form) -------------------------------------
+// ---- packed fixed-point tile of a whole workgroup (mixed form) -----------------
 
 // One LDS atomic per corner for both components: each contribution becomes
 // the integers qr = rint(w sr S), qi = rint(w si S) with the workgroup's
