@@ -29,6 +29,7 @@ namespace puff {
 template <typename R, int STAGE, bool DET, bool POLE>
 __global__ __launch_bounds__(STAGE_THREADS) void k_stage(StageArgs<R> a) {
     constexpr int P = 1;
+    static_assert(P == 1 || !DET, "the deterministic range checks take one macroparticle per thread");
     // Deposit tiles: two doubles per node in the FP64 form; DET_WORDS 8-byte
     // integers in its deterministic mode; one 8-byte packed fixed-point word
     // in the mixed form (packed_add: one ds_add_u64 per corner for
@@ -65,8 +66,10 @@ __global__ __launch_bounds__(STAGE_THREADS) void k_stage(StageArgs<R> a) {
     // they write only the step's scratch (k_s, dA_s), and a particle whose
     // trial position is off the mesh takes no part in the gather and deposit
     // (locate raises the flag again).  Stage 4 writes the state, and only
-    // when no flag is set: read here, with the particle loads (no kernel of
-    // stage 4 raises a flag: stage 3 checked its trial positions).
+    // when no flag is set: read here, with the particle loads.  No workgroup of
+    // stage 4 raises a flag, or others would have written by then: stage 3
+    // checks stage 4's trial positions and, for the deterministic deposit, its
+    // sources.
     const int rejected = (STAGE == 4) ? *a.flags : 0;
     // Slots of the workgroup: s0 + t, with s0 scalar and t 32 bits, so that an
     // access is a scalar base and one register of offset (64-bit lane addresses
@@ -183,6 +186,7 @@ __global__ __launch_bounds__(STAGE_THREADS) void k_stage(StageArgs<R> a) {
     R ep2k[P], sr[P], si[P];
     Cell<R> c[P];
     bool ok[P];
+    bool next_ok = false;   // (DET) the next stage's trial position is on the mesh
     LaneBox lb = lane_box();
 #pragma unroll
     for (int p = 0; p < P; ++p) {
@@ -205,7 +209,11 @@ __global__ __launch_bounds__(STAGE_THREADS) void k_stage(StageArgs<R> a) {
             // it does)
             const R cn = a.cnext_r;
             Cell<R> cc;
-            if (in[p]) flag |= locate<R>(m, fma(cn, v.x, x0[p]), fma(cn, v.y, y0[p]), fma(a.cnext, v.z2, z20[p]), cc);
+            if (in[p]) {
+                const int off = locate<R>(m, fma(cn, v.x, x0[p]), fma(cn, v.y, y0[p]), fma(a.cnext, v.z2, z20[p]), cc);
+                next_ok = off == 0;
+                flag |= off;
+            }
         } else {
             // x, y and z2 of the step's end do not wait for the field
             const unsigned i = threadIdx.x + p * STAGE_THREADS;
@@ -260,6 +268,12 @@ __global__ __launch_bounds__(STAGE_THREADS) void k_stage(StageArgs<R> a) {
     const int nnb = m.one_d ? 2 : 8;
     const int log2S = PACKED ? packed_scale_log2(tb.extra) : 0;
     R fr[P], fi[P];
+    double det_scale = 0.0, det_lim = 0.0;
+    if constexpr (DET) {
+        // n |s| 2^F <= 2^62 keeps every node's integer sums in range
+        det_scale = ldexp(1.0, *a.det.shift);
+        det_lim = ldexp(1.0, 62) / det_scale / (double)a.n;
+    }
     // ---- momentum equations (puffin_equations.f90:17-104)
     auto equations = [&](int p) {
         const unsigned i = threadIdx.x + p * STAGE_THREADS;
@@ -284,6 +298,13 @@ __global__ __launch_bounds__(STAGE_THREADS) void k_stage(StageArgs<R> a) {
                 at(a.kout.pi, i) = kpi;
                 at(a.kout.g, i) = (R)kg;   // FP32 in the mixed form (see KPtrs)
             }
+            if constexpr (DET && STAGE == 3) {
+                // stage 4's sources, as it will form them
+                const double r4 = fma(a.cnext, kpr, pr0[p]), i4 = fma(a.cnext, kpi, pi0[p]);
+                const double q4 = chi[p] * ph.inv_dV3 * drift_of(ph, r4, i4, fma(a.cnext, kg, g0[p])).fac;
+                if (ph.field_evolve && next_ok && (fabs(q4 * r4) > det_lim || fabs(q4 * i4) > det_lim))
+                    atomicOr(a.flags, FLAG_DET_RANGE);
+            }
         } else if (in[p] && !rejected) {
             // y = (y0 + h/6 (k1 + 2 (k2 + k3))) + h/6 k4 (puffin_mpi_RK4.f90:274-279, 307-312)
             at(a.y0.pr, i) = fma(a.h6_r, kpr, pr0[p]);
@@ -291,8 +312,6 @@ __global__ __launch_bounds__(STAGE_THREADS) void k_stage(StageArgs<R> a) {
             at(a.y0.g, i) = fma(a.h6, kg, g0[p]);
         }
     };
-    double det_scale = 0.0;
-    if constexpr (DET) det_scale = ldexp(1.0, *a.det.shift);
 #pragma unroll
     for (int p = 0; p < P; ++p) {
         const CellRef cr = cell_ref<R>(m, ok[p], c[p], tb, lane);
@@ -360,10 +379,8 @@ __global__ __launch_bounds__(STAGE_THREADS) void k_stage(StageArgs<R> a) {
             else tile_flush<R, double>(m, t, a.dAout, reinterpret_cast<const double*>(s_dep));
         } else tile_flush<R, D>(m, t, a.dAout, s_dep);
     };
-    if constexpr (DET) {
-        // n |s| 2^F <= 2^62 keeps every node's integer sums in range
-        const double lim = ldexp(1.0, 62) / det_scale / (double)a.n;
-        if (ph.field_evolve && ok[0] && (fabs((double)sr[0]) > lim || fabs((double)si[0]) > lim))
+    if constexpr (DET && STAGE < 4) {
+        if (ph.field_evolve && ok[0] && (fabs((double)sr[0]) > det_lim || fabs((double)si[0]) > det_lim))
             atomicOr(a.flags, FLAG_DET_RANGE);
     }
     if (ph.field_evolve) {
