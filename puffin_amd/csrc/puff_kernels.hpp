@@ -2,6 +2,7 @@
 #pragma once
 
 #include "puff_common.hpp"
+#include "puff_plan.hpp"
 
 namespace puff {
 

@@ -554,7 +554,7 @@ __device__ __forceinline__ void tile_flush(const MeshGeom& m, const TileBox& t, 
             int lx, ly, lz;
             box_coords(bd, q, lx, ly, lz);
             const int node = (t.bz0 + lz) * ntr + (t.by0 + ly) * m.nx + (t.bx0 + lx);
-            atomic_add(outc + 2 * node + part, (R)v);
+            atomic_add(outc + node_component(node, part), (R)v);
         }
     }
 }
@@ -706,7 +706,7 @@ __device__ __forceinline__ void packed_flush(const MeshGeom& m, const TileBox& t
             int lx, ly, lz;
             box_coords(bd, q, lx, ly, lz);
             const int node = (t.bz0 + lz) * ntr + (t.by0 + ly) * m.nx + (t.bx0 + lx);
-            atomic_add(outc + 2 * node + part, (float)v * inv);
+            atomic_add(outc + node_component(node, part), (float)v * inv);
         }
     }
 }
