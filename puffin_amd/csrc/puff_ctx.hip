@@ -698,14 +698,7 @@ static int create(Ctx* c) {
                 kzr[2 * i + 1] = 1.0 / std::sqrt(std::fabs(2.0 * kz[i]));
             }
         }
-        auto largest = [](const std::vector<double>& k) {
-            double m = 0.0;
-            for (double v : k) m = std::max(m, v * v);
-            return m;
-        };
-        for (size_t i = 0; i < kz.size(); ++i)
-            if (kz[i] != 0.0)
-                c->phase_rate = std::max(c->phase_rate, (largest(kx) + largest(ky)) * std::fabs(kzr[2 * i]));
+        c->phase_rate = largest_phase_rate(kx, ky, kz);
         PUFF_TRY(dalloc(c, (void**)&c->kzr, sizeof(double) * kzr.size()));
         PUFF_HIP(hipMemcpy(c->kzr, kzr.data(), sizeof(double) * kzr.size(), hipMemcpyHostToDevice));
         PUFF_HIP(hipMemcpy(c->mxy, mxy.data(), sizeof(double) * mxy.size(), hipMemcpyHostToDevice));
