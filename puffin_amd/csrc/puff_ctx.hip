@@ -187,13 +187,6 @@ static int dalloc(Ctx* c, void** p, size_t bytes) {
 
 // ---- FFT plans ----------------------------------------------------------------
 
-static bool is_prime(int n) {
-    if (n < 2) return false;
-    for (int f = 2; (int64_t)f * f <= n; ++f)
-        if (n % f == 0) return false;
-    return true;
-}
-
 static int powmod(int b, int e, int n) {
     int64_t r = 1, x = b % n;
     for (; e > 0; e >>= 1) {
@@ -203,52 +196,12 @@ static int powmod(int b, int e, int n) {
     return (int)r;
 }
 
-// Fewest radices of 2 to 16, each at most `top` and in falling order, with
-// product m (the smallest largest one where the count is the same); the number
-// of them, or 99.
-static int radices(int m, int top, int* out) {
-    if (m == 1) return 0;
-    int best = 99;
-    for (int r = 2; r <= top && r <= m; ++r) {
-        if (m % r) continue;
-        int rest[32];
-        const int k = 1 + radices(m / r, r, rest);
-        if (k < best) {
-            best = k;
-            out[0] = r;
-            std::copy(rest, rest + k - 1, out + 1);
-        }
-    }
-    return best;
-}
-
-// Passes of an n-point transform: prime factors above 13 as direct passes, the
-// rest in the fewest passes of up to 16 points (every pass is a round trip
-// through LDS and a barrier): 420 = 10 x 7 x 6, 90 = 10 x 9, 75 = 15 x 5.
-static void factorize(int n, FftAxis& ax) {
-    ax.n = n;
-    ax.npass = 0;
-    int m = n;
-    for (int f : {2, 3, 5, 7, 11, 13})
-        while (m % f == 0) m /= f;
-    const int small = n / m;
-    int big[32];
-    int nbig = 0;
-    for (int f = 17; m > 1 && (int64_t)f * f <= m; f += 2)
-        while (m % f == 0) { big[nbig++] = f; m /= f; }
-    if (m > 1) big[nbig++] = m;
-    for (int k = nbig - 1; k >= 0; --k) ax.radix[ax.npass++] = big[k];
-    int r[32];
-    const int k = radices(small, 16, r);
-    for (int q = 0; q < k; ++q) ax.radix[ax.npass++] = r[q];
-}
-
 template <typename R>
 static int make_axis(Ctx* c, int n, FftAxis& ax, bool z2_axis = false) {
     // one line, its ping-pong buffer and the twiddle table share a
     // workgroup's LDS (160 KiB on gfx950); 4096-point z2 lines stay in
     // registers (k_fft_zreg), or take one buffer and no table (k_fft_z)
-    if (3 * (size_t)n * sizeof(cplx<R>) > 160 * 1024 && !(z2_axis && n == 4096)) {
+    if (3 * (size_t)n * sizeof(cplx<R>) > LDS_BYTES && !(z2_axis && n == 4096)) {
         set_error("FFT line of " + std::to_string(n) + " points does not fit one workgroup's LDS");
         return PUFF_ERR_ARG;
     }
@@ -311,6 +264,19 @@ static int make_axis(Ctx* c, int n, FftAxis& ax, bool z2_axis = false) {
         ax.riperm = static_cast<const int*>(dq);
         ax.rb = db;
     }
+    return PUFF_OK;
+}
+
+// Before the first pass of a transform: a later one that cannot be launched
+// would leave the field half transformed.
+template <typename R>
+static int check_lines(const Ctx* c) {
+    const FftAxis* ax[3] = {&c->ax, &c->ay, &c->az};
+    for (int k = 0; k < 3; ++k)
+        if (!line_fits(*ax[k], sizeof(cplx<R>), k)) {
+            set_error("FFT line of " + std::to_string(ax[k]->n) + " points does not fit one workgroup's LDS");
+            return PUFF_ERR_ARG;
+        }
     return PUFF_OK;
 }
 
@@ -987,6 +953,7 @@ static int diffraction(Ctx* c, double h) {
         set_error("no diffraction on a 1-D mesh (read_base_input.f90:389)");
         return PUFF_ERR_STATE;
     }
+    PUFF_TRY(check_lines<R>(c));
     DiffArgs<R> a{};
     a.a = reinterpret_cast<cplx<R>*>(c->A);
     a.anb = reinterpret_cast<cplx<R>*>(c->anb);
@@ -1178,6 +1145,7 @@ static int download_field(Ctx* c, int kind, double* ar, double* ai) {
 template <typename R>
 static int transform(Ctx* c, int sign) {
     if (c->p.one_d) return PUFF_ERR_STATE;
+    PUFF_TRY(check_lines<R>(c));
     launch_fft3d<R>(reinterpret_cast<cplx<R>*>(c->A), c->p.nx, c->p.ny,
                     c->nzp(), c->ax, c->ay, c->az, sign, c->stream);
     PUFF_HIP(hipGetLastError());
@@ -1601,6 +1569,7 @@ static int diffraction_adjoint(Ctx* c, double h) {
         set_error("no diffraction on a 1-D mesh (read_base_input.f90:389)");
         return PUFF_ERR_STATE;
     }
+    PUFF_TRY(check_lines<R>(c));
     DiffArgs<R> a{};
     a.a = reinterpret_cast<cplx<R>*>(c->LA);
     a.anb = reinterpret_cast<cplx<R>*>(c->anb);

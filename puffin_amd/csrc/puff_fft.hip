@@ -28,20 +28,6 @@ namespace puff {
 #ifndef PUFF_Z_THREADS
 #define PUFF_Z_THREADS 256
 #endif
-// LDS word of flat element e of a line-major buffer (IL false): one spare
-// slot after every 16 elements.  A radix-16 pass with p = 1 has each lane
-// write 16 consecutive outputs, so lanes write 16 elements apart, all on the
-// same LDS banks; with the spare slots they land 17 apart and 16 lanes cover
-// all the banks.  Interleaved buffers (IL: y and z2 lines, b fastest) put
-// consecutive lanes on consecutive elements and are not padded.
-#ifndef PUFF_LDS_PAD_X
-#define PUFF_LDS_PAD_X 1
-#endif
-template <bool IL>
-__host__ __device__ constexpr int lpad(int e) {
-    return (!IL && PUFF_LDS_PAD_X) ? e + (e >> 4) : e;
-}
-
 // LDS index of element j of line b.  Interleaved layout (b fastest) keeps
 // the strided y / z2 loads conflict free; line-major suits contiguous x lines.
 template <bool IL>
@@ -361,12 +347,6 @@ struct CtPlan {
 PUFF_CT_PLAN(33, 11, 3)
 PUFF_CT_PLAN(129, 43, 3)
 #undef PUFF_CT_PLAN
-
-// How a runtime plan runs (line_plan): all passes of at most 16 points, in
-// place; a large prime first, on the matrix cores, then the same; or with two
-// line buffers.  A kernel each: the matrix pass's accumulators take a
-// wavefront per SIMD from the others.
-enum { LINE_SMALL = 0, LINE_PRIME = 1, LINE_TWO = 2 };
 
 // Quotients of 0 <= a < 2^16 by 1 <= d < 2^13: the high word of a ceil(2^32 / d).
 struct Div {
@@ -690,8 +670,6 @@ struct Mfma<float> {
     }
     static __device__ __forceinline__ int row(int l, int v) { return 4 * (l >> 4) + v; }
 };
-constexpr int MFMA_TILES = 4;
-constexpr int mfma_tiles(int B, int n, int r) { return (B * (n / r) + 7) / 8 * (((r - 1) / 2 + 16) / 16); }
 
 template <typename R, bool IL>
 __device__ __forceinline__ void mfma_pass(cplx<R>* buf, int B, int N, int r, const cplx<R>* tw, int sign) {
@@ -1485,7 +1463,7 @@ struct ZReg {
     static constexpr int ROW1 = M * BG + BG;
     static constexpr int ROW2 = 256 * BG + BG;
     static constexpr int WORDS = TWO ? (16 * ROW1 > L * ROW2 ? 16 * ROW1 : L * ROW2) : 16 * ROW1;
-    static_assert(L >= 2 && L <= 16 && WORDS * 8 <= 160 * 1024, "128 to 4096 points");
+    static_assert(L >= 2 && L <= 16 && WORDS * 8 <= LDS_BYTES, "128 to 4096 points");
 };
 
 // One component (8 bytes) and one point (16 bytes) of a thread's columns.
@@ -1727,65 +1705,12 @@ __global__ __launch_bounds__(ZReg<N>::THREADS, 4) void k_fft_zreg(DiffArgs<R> a,
 
 // ---- host side -----------------------------------------------------------------
 
-
 // Dynamic LDS above 64 KiB needs the kernel's opt-in (up to 160 KiB).
 static void lds_opt_in(const void* kernel, size_t bytes) {
     if (bytes > 64 * 1024)
-        (void)hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        (void)hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
 }
 
-// Lines per workgroup (B) and the plan's kind.  In place every pass's
-// butterflies must fit the threads' registers (radix_pass) and the matrix
-// pass's tiles their accumulators; where one line already does not, or a plan
-// has Rader's or a second large prime, two buffers.  tw: the twiddle table in
-// LDS too (x and y lines).  Both sides of the line, one diffraction step:
-// 90 x 75 x 420 (FP64) 816 us in two buffers with direct sums of 5 and 7,
-// 364 us in place; 61 x 47 x 389 640 us with direct sums, 375 us on the matrix
-// cores; 76 x 42 x 457 (mixed) 615 and 335 us.
-#ifndef PUFF_Z_LDS_BUDGET
-#define PUFF_Z_LDS_BUDGET (32 * 1024)
-#endif
-#ifndef PUFF_XY_LDS_BUDGET
-#define PUFF_XY_LDS_BUDGET (32 * 1024)
-#endif
-static constexpr int lines_per_block(int n, size_t elem, int cap, size_t budget, bool il, bool two, bool tw) {
-    int b = cap;
-    while (b > 1 &&
-           ((two ? 2 : 1) * (size_t)(il ? lpad<true>(b * n) : lpad<false>(b * n)) + (tw ? n : 0)) * elem > budget)
-        --b;
-    return b;
-}
-struct LinePlan {
-    int B, kind;
-};
-static LinePlan line_plan(const FftAxis& ax, size_t elem, int cap, size_t budget, bool il, bool tw) {
-    int kind = ax.rader ? LINE_TWO : LINE_SMALL;
-    int fit = cap;   // lines whose butterflies fit the registers
-    for (int k = 0; k < ax.npass; ++k) {
-        const int r = ax.radix[k];
-        if (r > 16 && k > 0) {
-            kind = LINE_TWO;
-        } else if (r > 16) {
-            if (kind == LINE_SMALL) kind = LINE_PRIME;
-            while (fit > 0 && mfma_tiles(fit, ax.n, r) > 4 * MFMA_TILES) --fit;
-        } else {
-            fit = std::min(fit, (16 / r) * 256 / (ax.n / r));
-        }
-    }
-    if (fit < 1) kind = LINE_TWO;
-    if (kind == LINE_PRIME) {
-        tw = true;
-        // whole tiles of 8 butterflies, where 64 KiB have room for them
-        const int whole = (8 + ax.n / ax.radix[0] - 1) / (ax.n / ax.radix[0]);
-        if (lines_per_block(ax.n, elem, whole, 2 * budget, il, false, true) == whole) budget *= 2;
-    }
-    const bool two = kind == LINE_TWO;
-    return {lines_per_block(ax.n, elem, two ? cap : fit, budget, il, two, tw), kind};
-}
-
-#ifndef PUFF_Y_LDS_BUDGET
-#define PUFF_Y_LDS_BUDGET PUFF_XY_LDS_BUDGET
-#endif
 template <typename R, int NC>
 static constexpr int ct_lines_x() {
     return lines_per_block(NC, sizeof(cplx<R>), 64, PUFF_XY_LDS_BUDGET, false, true, true);
@@ -1797,7 +1722,7 @@ static constexpr int ct_lines_y() {
 template <typename R, int NC, int BC, int KIND, int OP>
 static void launch_x_op(const DiffArgs<R>& a, int B, int sign, hipStream_t s) {
     const int64_t nlines = (int64_t)a.ny * a.nzp;
-    const size_t sh = ((KIND == LINE_TWO ? 2 : 1) * (size_t)lpad<false>(B * a.nx) + a.nx) * sizeof(cplx<R>);
+    const size_t sh = line_lds(B, a.nx, KIND, sizeof(cplx<R>), 0);
     lds_opt_in(reinterpret_cast<const void*>(&k_fft_x<R, NC, BC, KIND, OP>), sh);
     hipLaunchKernelGGL((k_fft_x<R, NC, BC, KIND, OP>), dim3((unsigned)((nlines + B - 1) / B)), dim3(256), sh, s, a, B,
                        sign);
@@ -1840,7 +1765,7 @@ static void run_x(const DiffArgs<R>& a, int op, int sign, hipStream_t s) {
     if (a.nx == RAD_N) return run_rader_x(a, op, sign, s);
     if (a.nx == 129) return launch_x<R, 129, ct_lines_x<R, 129>(), LINE_TWO>(a, 0, op, sign, s);
     if (a.nx == 33) return launch_x<R, 33, ct_lines_x<R, 33>(), LINE_TWO>(a, 0, op, sign, s);
-    const LinePlan lp = line_plan(a.ax, sizeof(cplx<R>), 64, PUFF_XY_LDS_BUDGET, false, true);
+    const LinePlan lp = axis_plan(a.ax, sizeof(cplx<R>), 0);
     switch (lp.kind) {
         case LINE_SMALL: return launch_x<R, 0, 0, LINE_SMALL>(a, lp.B, op, sign, s);
         case LINE_PRIME: return launch_x<R, 0, 0, LINE_PRIME>(a, lp.B, op, sign, s);
@@ -1851,7 +1776,7 @@ static void run_x(const DiffArgs<R>& a, int op, int sign, hipStream_t s) {
 template <typename R, int NC, int BC, int KIND>
 static void launch_y(const DiffArgs<R>& a, int B, int sign, hipStream_t s) {
     if (BC) B = BC;   // compile-time plans fix their lines per workgroup
-    const size_t sh = ((KIND == LINE_TWO ? 2 : 1) * (size_t)lpad<true>(B * a.ny) + a.ny) * sizeof(cplx<R>);
+    const size_t sh = line_lds(B, a.ny, KIND, sizeof(cplx<R>), 1);
     lds_opt_in(reinterpret_cast<const void*>(&k_fft_y<R, NC, BC, KIND>), sh);
     hipLaunchKernelGGL((k_fft_y<R, NC, BC, KIND>), dim3((unsigned)xcd_grid((int64_t)((a.nx + B - 1) / B) * a.nzp)),
                        dim3(256), sh, s, a, B, sign);
@@ -1867,7 +1792,7 @@ static void run_y(const DiffArgs<R>& a, int sign, hipStream_t s) {
     }
     if (a.ny == 129) return launch_y<R, 129, ct_lines_y<R, 129>(), LINE_TWO>(a, 0, sign, s);
     if (a.ny == 33) return launch_y<R, 33, ct_lines_y<R, 33>(), LINE_TWO>(a, 0, sign, s);
-    const LinePlan lp = line_plan(a.ay, sizeof(cplx<R>), 16, PUFF_Y_LDS_BUDGET, true, true);
+    const LinePlan lp = axis_plan(a.ay, sizeof(cplx<R>), 1);
     switch (lp.kind) {
         case LINE_SMALL: return launch_y<R, 0, 0, LINE_SMALL>(a, lp.B, sign, s);
         case LINE_PRIME: return launch_y<R, 0, 0, LINE_PRIME>(a, lp.B, sign, s);
@@ -1877,7 +1802,7 @@ static void run_y(const DiffArgs<R>& a, int sign, hipStream_t s) {
 
 template <typename R, int KIND>
 static void launch_z(const DiffArgs<R>& a, int B, int op, int sign, hipStream_t s) {
-    const size_t sh = ((KIND == LINE_TWO ? 2 : 1) * (size_t)lpad<true>(B * a.nzp) + (KIND == LINE_PRIME ? a.nzp : 0)) * sizeof(cplx<R>);
+    const size_t sh = line_lds(B, a.nzp, KIND, sizeof(cplx<R>), 2);
     const int64_t blocks = xcd_grid((int64_t)((a.nx + B - 1) / B) * a.ny);
     lds_opt_in(reinterpret_cast<const void*>(&k_fft_z<R, KIND>), sh);
     hipLaunchKernelGGL((k_fft_z<R, KIND>), dim3((unsigned)blocks), dim3(PUFF_Z_THREADS), sh, s, a, B, op,
@@ -1909,7 +1834,7 @@ static void run_z(const DiffArgs<R>& a, int op, int sign, hipStream_t s) {
         launch_zreg<R, 512>(a, op, sign, s) || launch_zreg<R, 1024>(a, op, sign, s) ||
         launch_zreg<R, 2048>(a, op, sign, s) || launch_zreg<R, 4096>(a, op, sign, s))
         return;
-    const LinePlan lp = line_plan(a.az, sizeof(cplx<R>), 16, PUFF_Z_LDS_BUDGET, true, false);
+    const LinePlan lp = axis_plan(a.az, sizeof(cplx<R>), 2);
     switch (lp.kind) {
         case LINE_SMALL: return launch_z<R, LINE_SMALL>(a, lp.B, op, sign, s);
         case LINE_PRIME: return launch_z<R, LINE_PRIME>(a, lp.B, op, sign, s);

@@ -1,9 +1,11 @@
 // Plain C++ of the library, shared by kernels and host code and compiled alone
-// by the tests: index arithmetic of the mesh, bounds.
+// by the tests: index arithmetic of the mesh, bounds,
+// plans of the FFT lines.
 #pragma once
 
 #include <algorithm>
 #include <cmath>
+#include <cstddef>
 #include <cstdint>
 
 #if defined(__HIPCC__)
@@ -31,6 +33,158 @@ double largest_phase_rate(const V& kx, const V& ky, const V& kz) {
     for (double v : kz)
         if (v != 0.0) rate = std::max(rate, k2 * std::fabs(1.0 / (2.0 * v)));
     return rate;
+}
+
+// ---- FFT lines ----------------------------------------------------------------
+
+inline bool is_prime(int n) {
+    if (n < 2) return false;
+    for (int f = 2; (int64_t)f * f <= n; ++f)
+        if (n % f == 0) return false;
+    return true;
+}
+
+// Fewest radices of 2 to 16, each at most `top` and in falling order, with
+// product m (the smallest largest one where the count is the same); the number
+// of them, or 99.
+inline int radices(int m, int top, int* out) {
+    if (m == 1) return 0;
+    int best = 99;
+    for (int r = 2; r <= top && r <= m; ++r) {
+        if (m % r) continue;
+        int rest[32];
+        const int k = 1 + radices(m / r, r, rest);
+        if (k < best) {
+            best = k;
+            out[0] = r;
+            std::copy(rest, rest + k - 1, out + 1);
+        }
+    }
+    return best;
+}
+
+// Passes of an n-point transform: prime factors above 13 as direct passes, the
+// rest in the fewest passes of up to 16 points (every pass is a round trip
+// through LDS and a barrier): 420 = 10 x 7 x 6, 90 = 10 x 9, 75 = 15 x 5.
+template <typename Axis>
+void factorize(int n, Axis& ax) {
+    ax.n = n;
+    ax.npass = 0;
+    int m = n;
+    for (int f : {2, 3, 5, 7, 11, 13})
+        while (m % f == 0) m /= f;
+    const int small = n / m;
+    int big[32];
+    int nbig = 0;
+    for (int f = 17; m > 1 && (int64_t)f * f <= m; f += 2)
+        while (m % f == 0) { big[nbig++] = f; m /= f; }
+    if (m > 1) big[nbig++] = m;
+    for (int k = nbig - 1; k >= 0; --k) ax.radix[ax.npass++] = big[k];
+    int r[32];
+    const int k = radices(small, 16, r);
+    for (int q = 0; q < k; ++q) ax.radix[ax.npass++] = r[q];
+}
+
+// LDS word of flat element e of a line-major buffer (IL false): one spare
+// slot after every 16 elements.  A radix-16 pass with p = 1 has each lane
+// write 16 consecutive outputs, so lanes write 16 elements apart, all on the
+// same LDS banks; with the spare slots they land 17 apart and 16 lanes cover
+// all the banks.  Interleaved buffers (IL: y and z2 lines, b fastest) put
+// consecutive lanes on consecutive elements and are not padded.
+#ifndef PUFF_LDS_PAD_X
+#define PUFF_LDS_PAD_X 1
+#endif
+template <bool IL>
+PUFF_BOTH constexpr int lpad(int e) {
+    return (!IL && PUFF_LDS_PAD_X) ? e + (e >> 4) : e;
+}
+
+// How a runtime plan runs (line_plan): all passes of at most 16 points, in
+// place; a large prime first, on the matrix cores, then the same; or with two
+// line buffers.  A kernel each: the matrix pass's accumulators take a
+// wavefront per SIMD from the others.
+enum { LINE_SMALL = 0, LINE_PRIME = 1, LINE_TWO = 2 };
+
+constexpr int MFMA_TILES = 4;
+constexpr int mfma_tiles(int B, int n, int r) { return (B * (n / r) + 7) / 8 * (((r - 1) / 2 + 16) / 16); }
+
+// Lines per workgroup (B) and the plan's kind.  In place every pass's
+// butterflies must fit the threads' registers (radix_pass) and the matrix
+// pass's tiles their accumulators; where one line already does not, or a plan
+// has Rader's or a second large prime, two buffers.  tw: the twiddle table in
+// LDS too (x and y lines).  Both sides of the line, one diffraction step:
+// 90 x 75 x 420 (FP64) 816 us in two buffers with direct sums of 5 and 7,
+// 364 us in place; 61 x 47 x 389 640 us with direct sums, 375 us on the matrix
+// cores; 76 x 42 x 457 (mixed) 615 and 335 us.
+#ifndef PUFF_Z_LDS_BUDGET
+#define PUFF_Z_LDS_BUDGET (32 * 1024)
+#endif
+#ifndef PUFF_XY_LDS_BUDGET
+#define PUFF_XY_LDS_BUDGET (32 * 1024)
+#endif
+#ifndef PUFF_Y_LDS_BUDGET
+#define PUFF_Y_LDS_BUDGET PUFF_XY_LDS_BUDGET
+#endif
+constexpr int lines_per_block(int n, size_t elem, int cap, size_t budget, bool il, bool two, bool tw) {
+    int b = cap;
+    while (b > 1 &&
+           ((two ? 2 : 1) * (size_t)(il ? lpad<true>(b * n) : lpad<false>(b * n)) + (tw ? n : 0)) * elem > budget)
+        --b;
+    return b;
+}
+struct LinePlan {
+    int B, kind;
+};
+template <typename Axis>
+LinePlan line_plan(const Axis& ax, size_t elem, int cap, size_t budget, bool il, bool tw) {
+    int kind = ax.rader ? LINE_TWO : LINE_SMALL;
+    int fit = cap;   // lines whose butterflies fit the registers
+    for (int k = 0; k < ax.npass; ++k) {
+        const int r = ax.radix[k];
+        if (r > 16 && k > 0) {
+            kind = LINE_TWO;
+        } else if (r > 16) {
+            if (kind == LINE_SMALL) kind = LINE_PRIME;
+            while (fit > 0 && mfma_tiles(fit, ax.n, r) > 4 * MFMA_TILES) --fit;
+        } else {
+            fit = std::min(fit, (16 / r) * 256 / (ax.n / r));
+        }
+    }
+    if (fit < 1) kind = LINE_TWO;
+    if (kind == LINE_PRIME) {
+        tw = true;
+        // whole tiles of 8 butterflies, where 64 KiB have room for them
+        const int whole = (8 + ax.n / ax.radix[0] - 1) / (ax.n / ax.radix[0]);
+        if (lines_per_block(ax.n, elem, whole, 2 * budget, il, false, true) == whole) budget *= 2;
+    }
+    const bool two = kind == LINE_TWO;
+    return {lines_per_block(ax.n, elem, two ? cap : fit, budget, il, two, tw), kind};
+}
+
+constexpr size_t LDS_BYTES = 160 * 1024;   // of a CU, all of it one workgroup's at most
+
+// LDS bytes of a workgroup of B lines of an axis (0: x, 1: y, 2: z2).
+inline size_t line_lds(int B, int n, int kind, size_t elem, int axis) {
+    const size_t line = axis ? lpad<true>(B * n) : lpad<false>(B * n);
+    const bool table = axis < 2 || kind == LINE_PRIME;
+    return ((kind == LINE_TWO ? 2 : 1) * line + (table ? n : 0)) * elem;
+}
+
+// The runtime plan of an axis.
+template <typename Axis>
+LinePlan axis_plan(const Axis& ax, size_t elem, int axis) {
+    if (axis == 0) return line_plan(ax, elem, 64, PUFF_XY_LDS_BUDGET, false, true);
+    if (axis == 1) return line_plan(ax, elem, 16, PUFF_Y_LDS_BUDGET, true, true);
+    return line_plan(ax, elem, 16, PUFF_Z_LDS_BUDGET, true, false);
+}
+
+// Whether a workgroup holds one line of the axis's plan.  A context admits
+// lines of three times n elements (two buffers and the table); the spare slots
+// of x lines in two buffers take another n / 8.
+template <typename Axis>
+bool line_fits(const Axis& ax, size_t elem, int axis) {
+    const LinePlan lp = axis_plan(ax, elem, axis);
+    return line_lds(lp.B, ax.n, lp.kind, elem, axis) <= LDS_BYTES;
 }
 
 }  // namespace puff

@@ -14,6 +14,22 @@ SOURCE = r"""
 #include <vector>
 #include "puff_plan.hpp"
 using namespace puff;
+struct Axis { int n, npass, radix[16], rader; };
+static Axis axis_of(int n) {
+    Axis a{};
+    const bool rader = n == 17 || n == 257;
+    factorize(rader ? n - 1 : n, a);
+    a.n = n;
+    a.rader = rader;
+    return a;
+}
+extern "C" void line(int n, int elem, int axis, long long* out) {   // B, kind, LDS bytes, fits, radices
+    const Axis a = axis_of(n);
+    const LinePlan lp = axis_plan(a, elem, axis);
+    const long long v[] = {lp.B, lp.kind, (long long)line_lds(lp.B, n, lp.kind, elem, axis), line_fits(a, elem, axis)};
+    for (int k = 0; k < 4; ++k) out[k] = v[k];
+    for (int k = 0; k < 16; ++k) out[4 + k] = k < a.npass ? a.radix[k] : 0;
+}
 extern "C" uint32_t component(int node, int part) { return node_component(node, part); }
 extern "C" double phase_rate(const double* x, const double* y, const double* z, int nx, int ny, int nz) {
     return largest_phase_rate(std::vector<double>(x, x + nx), std::vector<double>(y, y + ny), std::vector<double>(z, z + nz));
@@ -63,3 +79,26 @@ def test_phase_rate_takes_one_pass_over_each_axis(plan):
     t = time.perf_counter()
     _phase_rate(plan, k, k, k)
     assert time.perf_counter() - t < 5.0
+
+
+@pytest.mark.parametrize("axis", [0, 1, 2])
+@pytest.mark.parametrize("elem", [16, 8])
+def test_plans_of_every_admitted_line(plan, elem, axis):
+    """Lengths of 3 n elements within a CU's 160 KiB of LDS: the plan fits too or
+    is refused, which only x lines within 4 % of the limit are; the butterflies
+    of passes in place fit the registers and the prime pass's tiles the
+    accumulators."""
+    out = (ctypes.c_longlong * 20)()
+    for n in range(2, 160 * 1024 // (3 * elem) + 1):
+        plan.line(n, elem, axis, out)
+        B, kind, lds, fits = out[:4]
+        radix = [r for r in out[4:] if r]
+        assert B >= 1 and (lds <= 160 * 1024) == bool(fits), n
+        assert fits or (axis == 0 and 3 * n * elem > 0.96 * 160 * 1024), n
+        if n not in (17, 257):
+            assert np.prod(radix) == n, n
+        for k, r in enumerate(radix):
+            if kind == 0 or (kind == 1 and k > 0):
+                assert r <= 16 and B * (n // r) <= (16 // r) * 256, n
+            elif kind == 1:
+                assert -(-B * (n // r) // 8) * (((r - 1) // 2 + 16) // 16) <= 16, n
