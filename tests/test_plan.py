@@ -17,7 +17,7 @@ using namespace puff;
 struct Axis { int n, npass, radix[16], rader; };
 static Axis axis_of(int n) {
     Axis a{};
-    const bool rader = n == 17 || n == 257;
+    const bool rader = rader_line(n);
     factorize(rader ? n - 1 : n, a);
     a.n = n;
     a.rader = rader;
@@ -95,7 +95,7 @@ def test_plans_of_every_admitted_line(plan, elem, axis):
         radix = [r for r in out[4:] if r]
         assert B >= 1 and (lds <= 160 * 1024) == bool(fits), n
         assert fits or (axis == 0 and 3 * n * elem > 0.96 * 160 * 1024), n
-        if n not in (17, 257):
+        if n != 257:
             assert np.prod(radix) == n, n
         for k, r in enumerate(radix):
             if kind == 0 or (kind == 1 and k > 0):
