@@ -1752,7 +1752,8 @@ static int state_load(Ctx* c, const void* src, const void* host_header) {
     return PUFF_OK;
 }
 
-constexpr uint64_t CAPTURE_MAGIC = 0x3150414346465550ull;   // "PUFFCAP1"
+// Captures of another layout are refused: 1 held all six stage derivatives.
+constexpr uint64_t CAPTURE_MAGIC = 0x3250414346465550ull;   // "PUFFCAP2"
 
 // Start of a captured step (after its sort): header, start state and cleared
 // stage sources in the capture; a host copy of the header to cap_hdr.
