@@ -55,23 +55,41 @@ __global__ __launch_bounds__(256) void k_power(const cplx<R>* a, int nx, int ny,
 // in many bins (macroparticles not sorted: a change of bin, 12 cross-lane
 // moves per sum, would serve fewer than RUN_MIN lanes), add with an LDS
 // atomic per lane and sum.
+// A wavefront keeps runs at all only if its stretch is longer than `turns` turns
+// of 64 and its first slots are in order (RUN_ORDERED neighbours in one bin);
+// else every lane adds by itself throughout.  Calls with runs and without, in
+// us: slice sums of 20011 sorted slots (one turn) 40 and 35, of 2^19 (two) 46
+// and 67; of 2^22 slots in no order 100 and 89; the current of 2^20 sorted slots
+// (four turns, one sum: little to gain) 41 and 37, of 2^22 (sixteen) 63 and 78.
 constexpr int BIN_THREADS = 256;
 constexpr int RUN_MIN = 16;
+constexpr int RUN_ORDERED = 48;
 
+// Slots of a wavefront's stretch.
+__device__ __forceinline__ int64_t wave_stretch(int64_t n) {
+    const int64_t nw = (int64_t)gridDim.x * (BIN_THREADS / 64);
+    return (n + nw * 64 - 1) / (nw * 64) * 64;
+}
+
+// All wavefront-uniform but the values.
 template <int NV>
 struct RunSums {
-    double v[NV];
-    int bin = -1;   // wavefront-uniform; -1: none yet
+    double v[NV] = {};
+    int bin = -1;   // -1: none yet
+    bool on;        // keeps runs
+    bool first;     // of the stretch
+    __device__ __forceinline__ RunSums(int64_t n, int turns) : on(wave_stretch(n) > 64 * turns), first(true) {}
 };
 
 // acc[k * stride + bin] += the wavefront's sums, and start anew.
 template <int NV>
 __device__ __forceinline__ void run_flush(RunSums<NV>& r, double* sh, int stride) {
+    if (r.bin < 0) return;
     const int lane = threadIdx.x & 63;
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
         const double t = wave_sum(r.v[k]);
-        if (lane == 0 && r.bin >= 0 && t != 0.0) atomicAdd(&sh[k * stride + r.bin], t);
+        if (lane == 0 && t != 0.0) atomicAdd(&sh[k * stride + r.bin], t);
         r.v[k] = 0.0;
     }
 }
@@ -79,24 +97,31 @@ __device__ __forceinline__ void run_flush(RunSums<NV>& r, double* sh, int stride
 // Adds the lanes' values x (bin < 0: none) to their bins.  All lanes call.
 template <int NV>
 __device__ __forceinline__ void run_add(RunSums<NV>& r, int bin, const double (&x)[NV], double* sh, int stride) {
-    unsigned long long left = __ballot(bin >= 0);
-    for (int peel = 0; left && peel < 2; ++peel) {
-        // the lanes of the current bin first, then those of the first other one
-        unsigned long long same = __ballot(bin == r.bin) & left;
-        if (!same) {
-            const int next = __builtin_amdgcn_readlane(bin, __builtin_ctzll(left));
-            same = __ballot(bin == next) & left;
-            if (__builtin_popcountll(same) < RUN_MIN) break;
-            run_flush<NV>(r, sh, stride);
-            r.bin = next;
-        }
-        if ((same >> (threadIdx.x & 63)) & 1ull) {
+    const int lane = threadIdx.x & 63;
+    bool alone = bin >= 0;
+    if (r.on && r.first) r.on = __builtin_popcountll(__ballot(bin == __shfl_up(bin, 1, 64))) >= RUN_ORDERED;
+    r.first = false;
+    if (r.on) {
+        unsigned long long left = __ballot(bin >= 0);
+        for (int peel = 0; left && peel < 2; ++peel) {
+            // the lanes of the current bin first, then those of the first other one
+            unsigned long long same = __ballot(bin == r.bin) & left;
+            if (!same) {
+                const int next = __builtin_amdgcn_readlane(bin, __builtin_ctzll(left));
+                same = __ballot(bin == next) & left;
+                if (__builtin_popcountll(same) < RUN_MIN) break;
+                run_flush<NV>(r, sh, stride);
+                r.bin = next;
+            }
+            if ((same >> lane) & 1ull) {
 #pragma unroll
-            for (int k = 0; k < NV; ++k) r.v[k] += x[k];
+                for (int k = 0; k < NV; ++k) r.v[k] += x[k];
+            }
+            left &= ~same;
         }
-        left &= ~same;
+        alone = (left >> lane) & 1ull;
     }
-    if ((left >> (threadIdx.x & 63)) & 1ull) {
+    if (alone) {
 #pragma unroll
         for (int k = 0; k < NV; ++k) atomicAdd(&sh[k * stride + bin], x[k]);
     }
@@ -106,8 +131,7 @@ __device__ __forceinline__ void run_add(RunSums<NV>& r, int bin, const double (&
 // past the end: all lanes take every turn.
 template <typename F>
 __device__ __forceinline__ void for_wave_slots(int64_t n, F f) {
-    const int64_t nw = (int64_t)gridDim.x * (BIN_THREADS / 64);
-    const int64_t per = (n + nw * 64 - 1) / (nw * 64) * 64;
+    const int64_t per = wave_stretch(n);
     const int64_t w = (int64_t)blockIdx.x * (BIN_THREADS / 64) + (threadIdx.x >> 6);
     const int64_t end = min(n, (w + 1) * per);
     for (int64_t b = w * per; b < end; b += 64) {
@@ -137,8 +161,8 @@ __global__ __launch_bounds__(BIN_THREADS) void k_bunching(const double* z2, cons
     extern __shared__ double sh[];
     for (int t = threadIdx.x; t < 3 * nslices; t += blockDim.x) sh[t] = 0.0;
     __syncthreads();
-    RunSums<3> r{};    // slice is
-    RunSums<2> up{};   // slice is + 1
+    RunSums<3> r(n, 1);    // slice is
+    RunSums<2> up(n, 1);   // slice is + 1
     for_wave_slots(n, [&](int64_t i) {
         double x[3] = {0, 0, 0}, x2[2] = {0, 0};
         int bin = -1, bin2 = -1;
@@ -185,7 +209,7 @@ __global__ __launch_bounds__(BIN_THREADS) void k_slice_moments(PartPtrs<R> y, co
     extern __shared__ double sh[];
     for (int t = threadIdx.x; t < NSLICE_SUMS * nch; t += blockDim.x) sh[t] = 0.0;
     __syncthreads();
-    RunSums<NSLICE_SUMS> r{};
+    RunSums<NSLICE_SUMS> r(n, 1);
     for_wave_slots(n, [&](int64_t i) {
         double v[NSLICE_SUMS];
 #pragma unroll
@@ -231,7 +255,7 @@ __global__ __launch_bounds__(BIN_THREADS) void k_current(const double* z2, const
     for (int t = threadIdx.x; t < nch; t += blockDim.x) sh[t] = 0.0;
     __syncthreads();
     double bad = 0.0;
-    RunSums<1> rl{}, ru{};   // lower and upper node
+    RunSums<1> rl(n, 8), ru(n, 8);   // lower and upper node
     for_wave_slots(n, [&](int64_t i) {
         int lo = 0, hi = 0;
         double x1[1] = {0.0}, x2[1] = {0.0};
