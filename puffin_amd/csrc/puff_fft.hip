@@ -674,7 +674,7 @@ struct Mfma<float> {
 };
 
 template <typename R, bool IL>
-__device__ __forceinline__ void mfma_pass(cplx<R>* buf, int B, int N, int r, const cplx<R>* tw, int sign) {
+__device__ __forceinline__ void mfma_pass(cplx<R>* buf, int B, int N, int r, const cplx<R>* tp, int sign) {
     using M = Mfma<R>;
     const int T = N / r, cols = B * T, h = (r - 1) / 2, qt = (h + 16) / 16;
     const int units = (cols + 7) / 8 * qt;
@@ -702,7 +702,7 @@ __device__ __forceinline__ void mfma_pass(cplx<R>* buf, int B, int N, int r, con
             for (int j0 = 1; j0 <= h; j0 += 4) {
                 const int j = j0 + k, jj = j <= h ? j : 1;
                 const R xa = at(jj), xb = at(r - jj);
-                const cplx<R> w = tw[e * T];
+                const cplx<R> w = tp[e];
                 C[m] = M::fma(w.x, j <= h ? xa + xb : (R)0, C[m]);
                 S[m] = M::fma(w.y, j <= h ? xa - xb : (R)0, S[m]);
                 e += d;
@@ -737,15 +737,25 @@ __device__ __forceinline__ void mfma_pass(cplx<R>* buf, int B, int N, int r, con
     }
 }
 
+// The rotations of the matrix pass, every N / r-th of the table, side by side in
+// LDS: the lanes read them at random, and N / r apart a power of two of them
+// would share banks.
+template <typename R>
+__device__ __forceinline__ const cplx<R>* prime_table(cplx<R>* tp, const cplx<R>* tw, const FftAxis& ax) {
+    const int r = ax.radix[0], T = ax.n / r;
+    for (int e = threadIdx.x; e < r; e += blockDim.x) tp[e] = tw[e * T];
+    return tp;
+}
+
 // The passes of a runtime plan.  src holds the input; returns the buffer
 // holding the output (src or dst; in place: src).
 template <typename R, bool IL, int KIND>
 __device__ __forceinline__ cplx<R>* lds_passes(cplx<R>* src, cplx<R>* dst, int B, int LD, int N, int npass,
-                                               const int* radix, const cplx<R>* tw, int sign) {
+                                               const int* radix, const cplx<R>* tw, const cplx<R>* tp, int sign) {
     constexpr bool TWO = KIND == LINE_TWO;
     int p = 1, ps = 0;
     if constexpr (KIND == LINE_PRIME) {
-        mfma_pass<R, IL>(src, B, N, radix[0], tw, sign);
+        mfma_pass<R, IL>(src, B, N, radix[0], tp, sign);
         __syncthreads();
         p = radix[ps++];
     }
@@ -801,7 +811,7 @@ __device__ __forceinline__ cplx<R>* lds_rader(cplx<R>* src, cplx<R>* dst, int B,
         P[lidx<IL>(b, j, B, N)] = src[lidx<IL>(b, j < M ? ax.rperm[j] : 0, B, N)];
     }
     __syncthreads();
-    cplx<R>* res = lds_passes<R, IL, LINE_TWO>(P, Q, B, N, M, ax.npass, ax.radix, tw, -1);
+    cplx<R>* res = lds_passes<R, IL, LINE_TWO>(P, Q, B, N, M, ax.npass, ax.radix, tw, tw, -1);
     for (int w = threadIdx.x; w < B * M; w += blockDim.x) {
         int b, k;
         if (IL) { b = w % B; k = w / B; } else { k = w % M; b = w / M; }
@@ -814,7 +824,7 @@ __device__ __forceinline__ cplx<R>* lds_rader(cplx<R>* src, cplx<R>* dst, int B,
     }
     __syncthreads();
     cplx<R>* other = (res == P) ? Q : P;
-    res = lds_passes<R, IL, LINE_TWO>(res, other, B, N, M, ax.npass, ax.radix, tw, +1);
+    res = lds_passes<R, IL, LINE_TWO>(res, other, B, N, M, ax.npass, ax.radix, tw, tw, +1);
     cplx<R>* out = (res == P) ? Q : P;
     // every output element except element M (which holds x_0 or X_0 in out)
     const int qm = M / 2;   // g^-(M/2) = -1 = M (mod N)
@@ -841,14 +851,14 @@ __device__ __forceinline__ cplx<R>* lds_rader(cplx<R>* src, cplx<R>* dst, int B,
 // the buffer holding the output (src or dst; one buffer: src).
 template <typename R, bool IL, int NC, int KIND>
 __device__ __forceinline__ cplx<R>* lds_fft(cplx<R>* src, cplx<R>* dst, int B, const FftAxis& ax,
-                                            const cplx<R>* tw, int sign) {
+                                            const cplx<R>* tw, const cplx<R>* tp, int sign) {
     if constexpr (NC > 0) {
         return ct_passes<R, IL, NC>(src, dst, B, NC, NC, tw, sign);
     } else {
         if constexpr (KIND == LINE_TWO) {
             if (ax.rader) return lds_rader<R, IL>(src, dst, B, ax, tw, sign);
         }
-        return lds_passes<R, IL, KIND>(src, dst, B, ax.n, ax.n, ax.npass, ax.radix, tw, sign);
+        return lds_passes<R, IL, KIND>(src, dst, B, ax.n, ax.n, ax.npass, ax.radix, tw, tp, sign);
     }
 }
 
@@ -1140,6 +1150,7 @@ __global__ __launch_bounds__(256, KIND == LINE_TWO ? 1 : 4) void k_fft_x(DiffArg
     const cplx<R>* twg = reinterpret_cast<const cplx<R>*>(ax.tw);
     cplx<R>* tw = TWO ? s1 + lpad<false>(B * N) : s1;   // twiddle table staged in LDS
     for (int w = threadIdx.x; w < N; w += blockDim.x) tw[w] = twg[w];
+    const cplx<R>* tp = KIND == LINE_PRIME ? prime_table(tw + N, twg, ax) : tw;
     cplx<R>* base = a.a + L0 * N;
     const int64_t ntr = (int64_t)a.nx * a.ny;
     // plane and row of the block's first line; line L0 + b is row iy0 + b
@@ -1177,7 +1188,7 @@ __global__ __launch_bounds__(256, KIND == LINE_TWO ? 1 : 4) void k_fft_x(DiffArg
         if constexpr (sizeof(R) == 8) return (double)v / a.ffact;
         else return (double)v * rff;
     };
-    cplx<R>* res = lds_fft<R, false, NC, KIND>(s0, s1, B, ax, tw, first_sign);
+    cplx<R>* res = lds_fft<R, false, NC, KIND>(s0, s1, B, ax, tw, tp, first_sign);
     if (op == XOP_ADJ_INV_MIX_FWD) {
         // adjoint of the absorption split: (1 - m) cotangent + m W^H G W cotangent / ffact
         const cplx<R>* lam = a.anb + L0 * N;
@@ -1194,7 +1205,7 @@ __global__ __launch_bounds__(256, KIND == LINE_TWO ? 1 : 4) void k_fft_x(DiffArg
         }
         __syncthreads();
         cplx<R>* other = (TWO && res == s0) ? s1 : s0;
-        res = lds_fft<R, false, NC, KIND>(res, other, B, ax, tw, -1);
+        res = lds_fft<R, false, NC, KIND>(res, other, B, ax, tw, tp, -1);
     } else if (op == XOP_ADJ_INV_SCALE) {
         for (int w = threadIdx.x; w < nb * N; w += blockDim.x) {
             const cplx<R> v = res[lpad<false>(w)];
@@ -1217,7 +1228,7 @@ __global__ __launch_bounds__(256, KIND == LINE_TWO ? 1 : 4) void k_fft_x(DiffArg
         }
         __syncthreads();
         cplx<R>* other = (TWO && res == s0) ? s1 : s0;
-        res = lds_fft<R, false, NC, KIND>(res, other, B, ax, tw, -1);
+        res = lds_fft<R, false, NC, KIND>(res, other, B, ax, tw, tp, -1);
     } else if (op == XOP_INV_RECOMBINE) {
         // /ffact + interior (diffraction.f90:513-517)
         const cplx<R>* anb = a.anb + L0 * N;
@@ -1264,6 +1275,7 @@ __global__ __launch_bounds__(256, KIND == LINE_TWO ? 1 : 4) void k_fft_y(DiffArg
     const cplx<R>* twg = reinterpret_cast<const cplx<R>*>(ay.tw);
     cplx<R>* tw = TWO ? s1 + lpad<true>(B * N) : s1;   // twiddle table staged in LDS
     for (int w = threadIdx.x; w < N; w += blockDim.x) tw[w] = twg[w];
+    const cplx<R>* tp = KIND == LINE_PRIME ? prime_table(tw + N, twg, ay) : tw;
     const Div by_b = div_by(B);
     cplx<R>* base = a.a + (int64_t)iz * a.nx * a.ny + x0;
     lds_fill<true, STAGE_UNROLL>(s0, B * N, [&](int w) {
@@ -1271,7 +1283,7 @@ __global__ __launch_bounds__(256, KIND == LINE_TWO ? 1 : 4) void k_fft_y(DiffArg
         return (b < nb) ? base[(int64_t)j * a.nx + b] : cplx<R>{0, 0};
     });
     __syncthreads();
-    cplx<R>* res = lds_fft<R, true, NC, KIND>(s0, s1, B, ay, tw, sign);
+    cplx<R>* res = lds_fft<R, true, NC, KIND>(s0, s1, B, ay, tw, tp, sign);
     lds_drain<true, STAGE_UNROLL>(res, B * N, [&](int w, const cplx<R>& v) {
         const int j = over(w, by_b), b = w - j * B;
         if (b < nb) base[(int64_t)j * a.nx + b] = v;
@@ -1397,14 +1409,9 @@ __global__ __launch_bounds__(PUFF_Z_THREADS, KIND == LINE_TWO ? 1 : 4) void k_ff
     const int iy = (int)(blk / nxb);
     const int nb = min(B, a.nx - x0);
     const int64_t ntr = (int64_t)a.nx * a.ny;
-    // few lines per workgroup here: the twiddles stay in global memory (L2),
-    // except for the matrix cores' pass, whose lanes read them at random
+    // few lines per workgroup here: the twiddles stay in global memory (L2)
     const cplx<R>* tw = reinterpret_cast<const cplx<R>*>(az.tw);
-    if constexpr (KIND == LINE_PRIME) {
-        cplx<R>* t = s0 + lpad<true>(B * N);
-        for (int w = threadIdx.x; w < N; w += blockDim.x) t[w] = tw[w];
-        tw = t;
-    }
+    const cplx<R>* tp = KIND == LINE_PRIME ? prime_table(s0 + lpad<true>(B * N), tw, az) : tw;
     cplx<R>* base = a.a + (int64_t)iy * a.nx + x0;
     const Div by_b = div_by(B);
     lds_fill<true, PUFF_Z_UNROLL>(s0, B * N, [&](int w) {
@@ -1414,9 +1421,9 @@ __global__ __launch_bounds__(PUFF_Z_THREADS, KIND == LINE_TWO ? 1 : 4) void k_ff
     __syncthreads();
     cplx<R>* res;
     if (op < 0) {
-        res = lds_fft<R, true, 0, KIND>(s0, s1, B, az, tw, sign);
+        res = lds_fft<R, true, 0, KIND>(s0, s1, B, az, tw, tp, sign);
     } else {
-        res = lds_fft<R, true, 0, KIND>(s0, s1, B, az, tw, -1);
+        res = lds_fft<R, true, 0, KIND>(s0, s1, B, az, tw, tp, -1);
         const double ky = a.ky[iy];
         const bool small_phase = a.phase_max < PHASE_LIMIT;
         for (int w = threadIdx.x; w < B * N; w += blockDim.x) {
@@ -1429,7 +1436,7 @@ __global__ __launch_bounds__(PUFF_Z_THREADS, KIND == LINE_TWO ? 1 : 4) void k_ff
         }
         __syncthreads();
         cplx<R>* other = (TWO && res == s0) ? s1 : s0;
-        res = lds_fft<R, true, 0, KIND>(res, other, B, az, tw, +1);
+        res = lds_fft<R, true, 0, KIND>(res, other, B, az, tw, tp, +1);
     }
     lds_drain<true, PUFF_Z_UNROLL>(res, B * N, [&](int w, const cplx<R>& v) {
         const int j = over(w, by_b), b = w - j * B;
@@ -1717,16 +1724,16 @@ static void lds_opt_in(const void* kernel, size_t bytes) {
 
 template <typename R, int NC>
 static constexpr int ct_lines_x() {
-    return lines_per_block(NC, sizeof(cplx<R>), 64, PUFF_XY_LDS_BUDGET, false, true, true);
+    return lines_per_block(NC, sizeof(cplx<R>), 64, PUFF_XY_LDS_BUDGET, false, true, NC);
 }
 template <typename R, int NC>
 static constexpr int ct_lines_y() {
-    return lines_per_block(NC, sizeof(cplx<R>), 16, PUFF_Y_LDS_BUDGET, true, true, true);
+    return lines_per_block(NC, sizeof(cplx<R>), 16, PUFF_Y_LDS_BUDGET, true, true, NC);
 }
 template <typename R, int NC, int BC, int KIND, int OP>
 static void launch_x_op(const DiffArgs<R>& a, int B, int sign, hipStream_t s) {
     const int64_t nlines = (int64_t)a.ny * a.nzp;
-    const size_t sh = line_lds(B, a.nx, KIND, sizeof(cplx<R>), 0);
+    const size_t sh = line_lds(a.ax, B, KIND, sizeof(cplx<R>), 0);
     lds_opt_in(reinterpret_cast<const void*>(&k_fft_x<R, NC, BC, KIND, OP>), sh);
     hipLaunchKernelGGL((k_fft_x<R, NC, BC, KIND, OP>), dim3((unsigned)((nlines + B - 1) / B)), dim3(256), sh, s, a, B,
                        sign);
@@ -1780,7 +1787,7 @@ static void run_x(const DiffArgs<R>& a, int op, int sign, hipStream_t s) {
 template <typename R, int NC, int BC, int KIND>
 static void launch_y(const DiffArgs<R>& a, int B, int sign, hipStream_t s) {
     if (BC) B = BC;   // compile-time plans fix their lines per workgroup
-    const size_t sh = line_lds(B, a.ny, KIND, sizeof(cplx<R>), 1);
+    const size_t sh = line_lds(a.ay, B, KIND, sizeof(cplx<R>), 1);
     lds_opt_in(reinterpret_cast<const void*>(&k_fft_y<R, NC, BC, KIND>), sh);
     hipLaunchKernelGGL((k_fft_y<R, NC, BC, KIND>), dim3((unsigned)xcd_grid((int64_t)((a.nx + B - 1) / B) * a.nzp)),
                        dim3(256), sh, s, a, B, sign);
@@ -1806,7 +1813,7 @@ static void run_y(const DiffArgs<R>& a, int sign, hipStream_t s) {
 
 template <typename R, int KIND>
 static void launch_z(const DiffArgs<R>& a, int B, int op, int sign, hipStream_t s) {
-    const size_t sh = line_lds(B, a.nzp, KIND, sizeof(cplx<R>), 2);
+    const size_t sh = line_lds(a.az, B, KIND, sizeof(cplx<R>), 2);
     const int64_t blocks = xcd_grid((int64_t)((a.nx + B - 1) / B) * a.ny);
     lds_opt_in(reinterpret_cast<const void*>(&k_fft_z<R, KIND>), sh);
     hipLaunchKernelGGL((k_fft_z<R, KIND>), dim3((unsigned)blocks), dim3(PUFF_Z_THREADS), sh, s, a, B, op,

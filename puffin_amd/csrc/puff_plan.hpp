@@ -122,7 +122,9 @@ constexpr int mfma_tiles(int B, int n, int r) { return (B * (n / r) + 7) / 8 * (
 // LDS too (x and y lines).  Both sides of the line, one diffraction step:
 // 90 x 75 x 420 (FP64) 816 us in two buffers with direct sums of 5 and 7,
 // 364 us in place; 61 x 47 x 389 640 us with direct sums, 375 us on the matrix
-// cores; 76 x 42 x 457 (mixed) 615 and 335 us.
+// cores; 76 x 42 x 457 (mixed) 615 and 335 us.  The matrix pass forms tiles of 8
+// butterflies however few a workgroup has: with 3 of them (61 x 57 x 1047, FP64)
+// 820 us against 1430 in two buffers, with 2 (100 x 90 x 958) 3880 against 3350.
 #ifndef PUFF_Z_LDS_BUDGET
 #define PUFF_Z_LDS_BUDGET (32 * 1024)
 #endif
@@ -132,13 +134,13 @@ constexpr int mfma_tiles(int B, int n, int r) { return (B * (n / r) + 7) / 8 * (
 #ifndef PUFF_Y_LDS_BUDGET
 #define PUFF_Y_LDS_BUDGET PUFF_XY_LDS_BUDGET
 #endif
-constexpr int lines_per_block(int n, size_t elem, int cap, size_t budget, bool il, bool two, bool tw) {
+constexpr int lines_per_block(int n, size_t elem, int cap, size_t budget, bool il, bool two, int table) {
     int b = cap;
-    while (b > 1 &&
-           ((two ? 2 : 1) * (size_t)(il ? lpad<true>(b * n) : lpad<false>(b * n)) + (tw ? n : 0)) * elem > budget)
+    while (b > 1 && ((two ? 2 : 1) * (size_t)(il ? lpad<true>(b * n) : lpad<false>(b * n)) + table) * elem > budget)
         --b;
     return b;
 }
+constexpr int PRIME_LEAST = 3;
 struct LinePlan {
     int B, kind;
 };
@@ -158,23 +160,27 @@ LinePlan line_plan(const Axis& ax, size_t elem, int cap, size_t budget, bool il,
         }
     }
     if (fit < 1) kind = LINE_TWO;
+    const int table = tw ? ax.n : 0;
     if (kind == LINE_PRIME) {
-        tw = true;
         // whole tiles of 8 butterflies, where 64 KiB have room for them
-        const int whole = (8 + ax.n / ax.radix[0] - 1) / (ax.n / ax.radix[0]);
-        if (lines_per_block(ax.n, elem, whole, 2 * budget, il, false, true) == whole) budget *= 2;
+        const int r = ax.radix[0], T = ax.n / r, whole = (8 + T - 1) / T;
+        auto lines = [&](int most, size_t room) { return lines_per_block(ax.n, elem, most, room, il, false, table + r); };
+        const int B = lines(fit, lines(whole, 2 * budget) == whole ? 2 * budget : budget);
+        if (B * T >= PRIME_LEAST) return {B, kind};
+        kind = LINE_TWO;
     }
-    const bool two = kind == LINE_TWO;
-    return {lines_per_block(ax.n, elem, two ? cap : fit, budget, il, two, tw), kind};
+    if (kind == LINE_TWO) return {lines_per_block(ax.n, elem, cap, budget, il, true, table), kind};
+    return {lines_per_block(ax.n, elem, fit, budget, il, false, table), kind};
 }
 
 constexpr size_t LDS_BYTES = 160 * 1024;   // of a CU, all of it one workgroup's at most
 
 // LDS bytes of a workgroup of B lines of an axis (0: x, 1: y, 2: z2).
-inline size_t line_lds(int B, int n, int kind, size_t elem, int axis) {
-    const size_t line = axis ? lpad<true>(B * n) : lpad<false>(B * n);
-    const bool table = axis < 2 || kind == LINE_PRIME;
-    return ((kind == LINE_TWO ? 2 : 1) * line + (table ? n : 0)) * elem;
+template <typename Axis>
+size_t line_lds(const Axis& ax, int B, int kind, size_t elem, int axis) {
+    const size_t line = axis ? lpad<true>(B * ax.n) : lpad<false>(B * ax.n);
+    const int table = (axis < 2 ? ax.n : 0) + (kind == LINE_PRIME ? ax.radix[0] : 0);
+    return ((kind == LINE_TWO ? 2 : 1) * line + table) * elem;
 }
 
 // The runtime plan of an axis.
@@ -191,7 +197,7 @@ LinePlan axis_plan(const Axis& ax, size_t elem, int axis) {
 template <typename Axis>
 bool line_fits(const Axis& ax, size_t elem, int axis) {
     const LinePlan lp = axis_plan(ax, elem, axis);
-    return line_lds(lp.B, ax.n, lp.kind, elem, axis) <= LDS_BYTES;
+    return line_lds(ax, lp.B, lp.kind, elem, axis) <= LDS_BYTES;
 }
 
 }  // namespace puff

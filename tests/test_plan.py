@@ -26,7 +26,7 @@ static Axis axis_of(int n) {
 extern "C" void line(int n, int elem, int axis, long long* out) {   // B, kind, LDS bytes, fits, radices
     const Axis a = axis_of(n);
     const LinePlan lp = axis_plan(a, elem, axis);
-    const long long v[] = {lp.B, lp.kind, (long long)line_lds(lp.B, n, lp.kind, elem, axis), line_fits(a, elem, axis)};
+    const long long v[] = {lp.B, lp.kind, (long long)line_lds(a, lp.B, lp.kind, elem, axis), line_fits(a, elem, axis)};
     for (int k = 0; k < 4; ++k) out[k] = v[k];
     for (int k = 0; k < 16; ++k) out[4 + k] = k < a.npass ? a.radix[k] : 0;
 }
