@@ -1776,7 +1776,7 @@ static void run_x(const DiffArgs<R>& a, int op, int sign, hipStream_t s) {
     if (a.nx == RAD_N) return run_rader_x(a, op, sign, s);
     if (a.nx == 129) return launch_x<R, 129, ct_lines_x<R, 129>(), LINE_TWO>(a, 0, op, sign, s);
     if (a.nx == 33) return launch_x<R, 33, ct_lines_x<R, 33>(), LINE_TWO>(a, 0, op, sign, s);
-    const LinePlan lp = axis_plan(a.ax, sizeof(cplx<R>), 0);
+    const LinePlan lp = axis_plan(a.ax, sizeof(cplx<R>), 0, (int64_t)a.ny * a.nzp, 1);
     switch (lp.kind) {
         case LINE_SMALL: return launch_x<R, 0, 0, LINE_SMALL>(a, lp.B, op, sign, s);
         case LINE_PRIME: return launch_x<R, 0, 0, LINE_PRIME>(a, lp.B, op, sign, s);
@@ -1803,7 +1803,7 @@ static void run_y(const DiffArgs<R>& a, int sign, hipStream_t s) {
     }
     if (a.ny == 129) return launch_y<R, 129, ct_lines_y<R, 129>(), LINE_TWO>(a, 0, sign, s);
     if (a.ny == 33) return launch_y<R, 33, ct_lines_y<R, 33>(), LINE_TWO>(a, 0, sign, s);
-    const LinePlan lp = axis_plan(a.ay, sizeof(cplx<R>), 1);
+    const LinePlan lp = axis_plan(a.ay, sizeof(cplx<R>), 1, a.nx, a.nzp);
     switch (lp.kind) {
         case LINE_SMALL: return launch_y<R, 0, 0, LINE_SMALL>(a, lp.B, sign, s);
         case LINE_PRIME: return launch_y<R, 0, 0, LINE_PRIME>(a, lp.B, sign, s);
@@ -1845,7 +1845,7 @@ static void run_z(const DiffArgs<R>& a, int op, int sign, hipStream_t s) {
         launch_zreg<R, 512>(a, op, sign, s) || launch_zreg<R, 1024>(a, op, sign, s) ||
         launch_zreg<R, 2048>(a, op, sign, s) || launch_zreg<R, 4096>(a, op, sign, s))
         return;
-    const LinePlan lp = axis_plan(a.az, sizeof(cplx<R>), 2);
+    const LinePlan lp = axis_plan(a.az, sizeof(cplx<R>), 2, a.nx, a.ny);
     switch (lp.kind) {
         case LINE_SMALL: return launch_z<R, LINE_SMALL>(a, lp.B, op, sign, s);
         case LINE_PRIME: return launch_z<R, LINE_PRIME>(a, lp.B, op, sign, s);

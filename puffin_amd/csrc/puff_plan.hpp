@@ -144,8 +144,20 @@ constexpr int PRIME_LEAST = 3;
 struct LinePlan {
     int B, kind;
 };
+
+// Half the lines a workgroup, and half again, down to `least`, while the mesh's
+// rows of `cols` lines give work to fewer than three quarters of the CUs.  A
+// diffraction step of 26 x 26 x 236 (FP64; 52 workgroups of 15 z2 lines else)
+// 146 -> 107 us; with two workgroups a CU as the aim, small lines lose
+// (26 x 26 x 260: 116 -> 121 us).
+constexpr int CUS = 256;
+inline int filled(int B, int least, int64_t cols, int64_t rows) {
+    while (B / 2 >= least && (cols + B - 1) / B * rows < 3 * CUS / 4) B /= 2;
+    return B;
+}
+
 template <typename Axis>
-LinePlan line_plan(const Axis& ax, size_t elem, int cap, size_t budget, bool il, bool tw) {
+LinePlan line_plan(const Axis& ax, size_t elem, int cap, size_t budget, bool il, bool tw, int64_t cols, int64_t rows) {
     int kind = ax.rader ? LINE_TWO : LINE_SMALL;
     int fit = cap;   // lines whose butterflies fit the registers
     for (int k = 0; k < ax.npass; ++k) {
@@ -165,12 +177,13 @@ LinePlan line_plan(const Axis& ax, size_t elem, int cap, size_t budget, bool il,
         // whole tiles of 8 butterflies, where 64 KiB have room for them
         const int r = ax.radix[0], T = ax.n / r, whole = (8 + T - 1) / T;
         auto lines = [&](int most, size_t room) { return lines_per_block(ax.n, elem, most, room, il, false, table + r); };
-        const int B = lines(fit, lines(whole, 2 * budget) == whole ? 2 * budget : budget);
-        if (B * T >= PRIME_LEAST) return {B, kind};
+        int B = lines(fit, lines(whole, 2 * budget) == whole ? 2 * budget : budget);
+        if (8 % T == 0 && B > whole) B -= B % whole;   // no part-filled tile
+        if (B * T >= PRIME_LEAST) return {filled(B, std::min(B, whole), cols, rows), kind};
         kind = LINE_TWO;
     }
     if (kind == LINE_TWO) return {lines_per_block(ax.n, elem, cap, budget, il, true, table), kind};
-    return {lines_per_block(ax.n, elem, fit, budget, il, false, table), kind};
+    return {filled(lines_per_block(ax.n, elem, fit, budget, il, false, table), 1, cols, rows), kind};
 }
 
 constexpr size_t LDS_BYTES = 160 * 1024;   // of a CU, all of it one workgroup's at most
@@ -185,10 +198,10 @@ size_t line_lds(const Axis& ax, int B, int kind, size_t elem, int axis) {
 
 // The runtime plan of an axis.
 template <typename Axis>
-LinePlan axis_plan(const Axis& ax, size_t elem, int axis) {
-    if (axis == 0) return line_plan(ax, elem, 64, PUFF_XY_LDS_BUDGET, false, true);
-    if (axis == 1) return line_plan(ax, elem, 16, PUFF_Y_LDS_BUDGET, true, true);
-    return line_plan(ax, elem, 16, PUFF_Z_LDS_BUDGET, true, false);
+LinePlan axis_plan(const Axis& ax, size_t elem, int axis, int64_t cols, int64_t rows) {
+    if (axis == 0) return line_plan(ax, elem, 64, PUFF_XY_LDS_BUDGET, false, true, cols, rows);
+    if (axis == 1) return line_plan(ax, elem, 16, PUFF_Y_LDS_BUDGET, true, true, cols, rows);
+    return line_plan(ax, elem, 16, PUFF_Z_LDS_BUDGET, true, false, cols, rows);
 }
 
 // Whether a workgroup holds one line of the axis's plan.  A context admits
@@ -196,7 +209,7 @@ LinePlan axis_plan(const Axis& ax, size_t elem, int axis) {
 // of x lines in two buffers take another n / 8.
 template <typename Axis>
 bool line_fits(const Axis& ax, size_t elem, int axis) {
-    const LinePlan lp = axis_plan(ax, elem, axis);
+    const LinePlan lp = axis_plan(ax, elem, axis, 1, 1);
     return line_lds(ax, lp.B, lp.kind, elem, axis) <= LDS_BYTES;
 }
 

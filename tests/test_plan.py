@@ -23,9 +23,9 @@ static Axis axis_of(int n) {
     a.rader = rader;
     return a;
 }
-extern "C" void line(int n, int elem, int axis, long long* out) {   // B, kind, LDS bytes, fits, radices
+extern "C" void line(int n, int elem, int axis, int cols, int rows, long long* out) {   // B, kind, LDS, fits, radices
     const Axis a = axis_of(n);
-    const LinePlan lp = axis_plan(a, elem, axis);
+    const LinePlan lp = axis_plan(a, elem, axis, cols, rows);
     const long long v[] = {lp.B, lp.kind, (long long)line_lds(a, lp.B, lp.kind, elem, axis), line_fits(a, elem, axis)};
     for (int k = 0; k < 4; ++k) out[k] = v[k];
     for (int k = 0; k < 16; ++k) out[4 + k] = k < a.npass ? a.radix[k] : 0;
@@ -81,20 +81,26 @@ def test_phase_rate_takes_one_pass_over_each_axis(plan):
     assert time.perf_counter() - t < 5.0
 
 
+@pytest.mark.parametrize("cols,rows", [(10 ** 6, 1000), (26, 26), (1, 1)])
 @pytest.mark.parametrize("axis", [0, 1, 2])
 @pytest.mark.parametrize("elem", [16, 8])
-def test_plans_of_every_admitted_line(plan, elem, axis):
+def test_plans_of_every_admitted_line(plan, elem, axis, cols, rows):
     """Lengths of 3 n elements within a CU's 160 KiB of LDS: the plan fits too or
     is refused, which only x lines within 4 % of the limit are; the butterflies
     of passes in place fit the registers and the prime pass's tiles the
-    accumulators."""
-    out = (ctypes.c_longlong * 20)()
+    accumulators; few lines spread over the chip, but never over part-filled
+    tiles where there could be whole ones."""
+    out, most = (ctypes.c_longlong * 20)(), (ctypes.c_longlong * 20)()
     for n in range(2, 160 * 1024 // (3 * elem) + 1):
-        plan.line(n, elem, axis, out)
+        plan.line(n, elem, axis, cols, rows, out)
+        plan.line(n, elem, axis, 10 ** 6, 1000, most)
         B, kind, lds, fits = out[:4]
         radix = [r for r in out[4:] if r]
-        assert B >= 1 and (lds <= 160 * 1024) == bool(fits), n
+        assert 1 <= B <= most[0] and kind == most[1], n
+        assert (lds <= 160 * 1024) == bool(fits), n
         assert fits or (axis == 0 and 3 * n * elem > 0.96 * 160 * 1024), n
+        if kind != 2 and -(-cols // B) * rows < 192:
+            assert B // 2 < (min(most[0], -(-8 * radix[0] // n)) if kind == 1 else 1), n
         if n != 257:
             assert np.prod(radix) == n, n
         for k, r in enumerate(radix):
