@@ -54,3 +54,34 @@ def test_light_macroparticles_beside_heavy_ones(n):
     got, want = ((r + 1j * i).reshape(shape)[light] for r, i in ((gr, gi), (o.ar, o.ai)))
     assert np.abs(want).max() > 0
     assert np.abs(got - want).max() / np.abs(want).max() < 1e-5
+
+
+@pytest.mark.parametrize("n", [63, 2048, 4099])
+def test_deterministic_deposit_of_thin_sorted_beams(n):
+    """Wavefront by wavefront in fixed point: the bits of the unsorted slots (whose
+    wavefronts deposit straight to memory), and the oracle's values to 1e-10."""
+    mp, p, h = _beam(n)
+    zero = np.zeros(mp.nmesh)
+    o = orc.Oracle(mp, p, (zero.copy(), zero.copy()))
+    out = []
+    for in_order in (False, True):
+        print(f"[gpu-overflow] deterministic n={n} sorted={in_order}", flush=True)
+        with gpu.Integrator(mp, n, FP64) as g:
+            g.set_deterministic(True)
+            g.set_sort_interval(0)
+            g.upload_particles(p)
+            g.upload_field(zero, zero)
+            if in_order:
+                g.sort_now()
+            for k in range(3):
+                assert g.rk4par(k * h, h) == 0
+            out.append((g.download_particles(), g.download_field()))
+    for k in range(3):
+        assert o.rk4par(k * h, h) == 0
+    for k in ("x", "y", "z2", "px", "py", "gam"):
+        assert np.array_equal(out[0][0][k], out[1][0][k]), k
+        assert np.abs(out[1][0][k] - o.parts[k]).max() <= 1e-10 * np.abs(o.parts[k]).max(), k
+    for a, b in zip(out[0][1], out[1][1]):
+        assert np.array_equal(a, b)
+    want = o.ar + 1j * o.ai
+    assert np.abs(out[1][1][0] + 1j * out[1][1][1] - want).max() <= 1e-10 * np.abs(want).max()
