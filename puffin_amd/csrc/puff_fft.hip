@@ -1290,64 +1290,6 @@ __global__ __launch_bounds__(256, KIND == LINE_TWO ? 1 : 4) void k_fft_y(DiffArg
     });
 }
 
-// Sine and cosine of the propagator's phase, an FP64 number below PHASE_LIMIT:
-// reduced by multiples n of pi / 2 (a double and its remainder, each product
-// in one FMA: exact to 1e-17 while n is), then Taylor sums.  FP64: to x^17 and
-// x^18, with the rounding errors of the reduction and of x^2 carried along:
-// within 9.5e-17 of the true values up to 3e13 (half an ulp of 1 is 1.1e-16).  FP32: the
-// rotated field is rounded to 6e-8 anyway; sums to x^9 and x^10 of the reduced
-// phase rounded to FP32 (|r| <= pi / 4).  40 and 20 instructions without
-// branches; the library's functions carry a second path for large arguments
-// at each of their places in a kernel.
-constexpr double PHASE_LIMIT = 1e13;   // n stays below 2^43
-template <typename R>
-struct SinCos {
-    R s, c;
-};
-template <typename R>
-__device__ __forceinline__ SinCos<R> sincos_phase(double th) {
-    constexpr double hi = 1.57079632679489661923, lo = 6.123233995736766036e-17;
-    const double n = rint(th * 0.63661977236758134308);
-    const double r0 = fma(-n, hi, th);
-    const double r = fma(-n, lo, r0);
-    R sn, cs;
-    if constexpr (sizeof(R) == 8) {
-        const double e = fma(-n, lo, r0 - r);
-        const double z = r * r;
-        double p = fma(z, 1.0 / 355687428096000.0, -1.0 / 1307674368000.0);
-        p = fma(z, p, 1.0 / 6227020800.0);
-        p = fma(z, p, -1.0 / 39916800.0);
-        p = fma(z, p, 1.0 / 362880.0);
-        p = fma(z, p, -1.0 / 5040.0);
-        p = fma(z, p, 1.0 / 120.0);
-        p = fma(z, p, -1.0 / 6.0);
-        sn = r + fma(r * z, p, e);
-        double q = fma(z, -1.0 / 6402373705728000.0, 1.0 / 20922789888000.0);
-        q = fma(z, q, -1.0 / 87178291200.0);
-        q = fma(z, q, 1.0 / 479001600.0);
-        q = fma(z, q, -1.0 / 3628800.0);
-        q = fma(z, q, 1.0 / 40320.0);
-        q = fma(z, q, -1.0 / 720.0);
-        q = fma(z, q, 1.0 / 24.0);
-        const double hz = 0.5 * z, w = 1.0 - hz;
-        cs = w + fma(z * z, q, fma(-r, e, fma(-0.5, fma(r, r, -z), (1.0 - w) - hz)));
-    } else {
-        const float x = (float)r, z = x * x;
-        float p = fmaf(z, 1.0f / 362880.0f, -1.0f / 5040.0f);
-        p = fmaf(z, p, 1.0f / 120.0f);
-        p = fmaf(z, p, -1.0f / 6.0f);
-        sn = fmaf(x * z, p, x);
-        float q = fmaf(z, -1.0f / 3628800.0f, 1.0f / 40320.0f);
-        q = fmaf(z, q, -1.0f / 720.0f);
-        q = fmaf(z, q, 1.0f / 24.0f);
-        q = fmaf(z, q, -0.5f);
-        cs = fmaf(z, q, 1.0f);
-    }
-    const int m = (int)(int64_t)n;
-    const R a = (m & 1) ? cs : sn, b = (m & 1) ? sn : cs;
-    return {(m & 2) ? -a : a, ((m + 1) & 2) ? -b : b};
-}
-
 // The spectral factor between the forward and inverse z2 transforms, at
 // wavenumbers (kx, ky, kz): multiplyexp's propagator (with its filter) or
 // AbsorptionStep's damping.  FP64 form: in FP64, rounded once.  Mixed form

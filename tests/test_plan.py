@@ -11,9 +11,25 @@ import pytest
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "puffin_amd", "csrc")
 
 SOURCE = r"""
+#include <random>
 #include <vector>
 #include "puff_plan.hpp"
 using namespace puff;
+template <typename R>
+static double sincos_error(double lo, double hi, int n) {
+    std::mt19937_64 g(1);
+    std::uniform_real_distribution<double> u(std::log(lo), std::log(hi));
+    long double worst = 0;
+    for (int i = 0; i < n; ++i) {
+        const double th = (i & 1 ? -1 : 1) * std::exp(u(g));
+        const SinCos<R> t = sincos_phase<R>(th);
+        worst = std::max({worst, std::fabs((long double)t.s - sinl(th)), std::fabs((long double)t.c - cosl(th))});
+    }
+    return (double)worst;
+}
+extern "C" double sincos_error(int form, double lo, double hi, int n) {
+    return form ? sincos_error<float>(lo, hi, n) : sincos_error<double>(lo, hi, n);
+}
 struct Axis { int n, npass, radix[16], rader; };
 static Axis axis_of(int n) {
     Axis a{};
@@ -42,11 +58,12 @@ def plan(tmp_path_factory):
     d = tmp_path_factory.mktemp("plan")
     src, so = d / "plan.cpp", d / "plan.so"
     src.write_text(SOURCE)
-    subprocess.run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-Wall", "-Werror", f"-I{CSRC}", str(src), "-o", str(so)],
+    subprocess.run(["g++", "-O2", "-std=c++17", "-ffp-contract=off", "-shared", "-fPIC", "-Wall", "-Werror", f"-I{CSRC}", str(src), "-o", str(so)],
                    check=True)
     lib = ctypes.CDLL(str(so))
     lib.component.restype = ctypes.c_uint32
-    lib.phase_rate.restype = ctypes.c_double
+    lib.phase_rate.restype = lib.sincos_error.restype = ctypes.c_double
+    lib.sincos_error.argtypes = [ctypes.c_int, ctypes.c_double, ctypes.c_double, ctypes.c_int]
     return lib
 
 
@@ -108,3 +125,11 @@ def test_plans_of_every_admitted_line(plan, elem, axis, cols, rows):
                 assert r <= 16 and B * (n // r) <= (16 // r) * 256, n
             elif kind == 1:
                 assert -(-B * (n // r) // 8) * (((r - 1) // 2 + 16) // 16) <= 16, n
+
+
+@pytest.mark.parametrize("form,bound", [(0, 9.5e-17), (1, 7.5e-8)])
+@pytest.mark.parametrize("decade", [-6, -1, 0, 1, 3, 5, 8, 10, 12])
+def test_sine_and_cosine_of_phases(plan, decade, form, bound):
+    """The stated bounds against the long double functions (64-bit significand),
+    at phases of either sign up to the limit of 1e13."""
+    assert plan.sincos_error(form, 10.0 ** decade, 10.0 ** (decade + 1), 200000) < bound
