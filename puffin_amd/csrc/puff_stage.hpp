@@ -165,6 +165,9 @@ __device__ __forceinline__ Trial<R> trial_state(const Physics& ph, R x0, R y0, d
 // (bfields.f90): see stage_scalars() on the host for the coefficient map.
 // POLE = false: compiled without the hyperbolic functions of the plane-pole
 // and curved-pole types (15 to 20 registers of a stage kernel).
+// Which product of a sum of two is rounded is written out: left to the compiler
+// it changes with the code around, and the mixed form's z2 by up to 1.4e-9 over 25
+// steps of a focusing curved-pole undulator.
 template <typename R, bool POLE = true>
 __device__ __forceinline__ void bfield(const StageScalars& s, R x, R y, R& bx,
                                        R& by, R& bz) {
@@ -174,13 +177,13 @@ __device__ __forceinline__ void bfield(const StageScalars& s, R x, R y, R& bx,
         bz = s.template coef<R>(2) * sinh(s.template coef<R>(7) * y);
     } else if (POLE && s.und_type == PUFF_UND_CURVED) {
         const R kx = s.template coef<R>(5), ky = s.template coef<R>(6);
-        bx = s.template coef<R>(0) * sinh(kx * x) * sinh(ky * y) + s.template coef<R>(3) * y;
-        by = s.template coef<R>(1) * cosh(kx * x) * cosh(ky * y) + s.template coef<R>(4) * x;
+        bx = fma(s.template coef<R>(3), y, s.template coef<R>(0) * sinh(kx * x) * sinh(ky * y));
+        by = fma(s.template coef<R>(4), x, s.template coef<R>(1) * cosh(kx * x) * cosh(ky * y));
         bz = s.template coef<R>(2) * cosh(kx * x) * sinh(ky * y);
     } else {
         bx = s.template coef<R>(0) + s.template coef<R>(3) * y;
         by = s.template coef<R>(1) + s.template coef<R>(4) * x;
-        bz = s.template coef<R>(5) * x + s.template coef<R>(6) * y;
+        bz = fma(s.template coef<R>(6), y, s.template coef<R>(5) * x);
     }
 }
 
