@@ -364,7 +364,7 @@ class Integrator:
 
     def tile_fallback(self):
         """(last step, first step after the last re-sort): share of stage
-        workgroups that deposited with global atomics."""
+        workgroups whose node box overflowed the LDS tile."""
         a, b = ctypes.c_double(), ctypes.c_double()
         _check(lib().puff_tile_fallback(self._h, ctypes.byref(a), ctypes.byref(b)), "puff_tile_fallback")
         return a.value, b.value
