@@ -182,6 +182,10 @@ int puff_rk4par(puff_ctx* ctx, double sz, double h);
  * Free-space diffraction of the field over distance h.
  * Replaces DiffractionStep(h, sAr, sAi, qOK) (diffraction.f90:209-348):
  * forward 3-D DFT, multiplyexp, backward DFT, /ffact, AbsorptionStep.
+ * PUFF_ERR_ARG with the field as it was where an x line's plan exceeds a
+ * workgroup's LDS (most lengths of 3278 to 3413 points in FP64 and all of 6555
+ * to 6826 in the mixed form; a context admits them for the steps alone).  The
+ * same for puff_transform and the adjoint.
  */
 int puff_diffraction_step(puff_ctx* ctx, double h);
 
