@@ -60,7 +60,7 @@ constexpr int BOX_COPIES = 64;
 
 // Workgroup of the RK4 stage kernels (one macroparticle per thread) and the
 // node capacity of its LDS deposit tile.  Four-wave workgroups (one wave per
-// SIMD each); the stage kernels hold 66-85 VGPRs, so the LDS tiles set how
+// SIMD each); the stage kernels hold 71-81 VGPRs, so the LDS tiles set how
 // many workgroups share a CU: 1280 nodes (2 FP64 each, 20 KiB) in the FP64
 // form, 3072 (one packed 8-byte word each, 24 KiB) in the mixed form.
 // Measured on the C1 beam: FP64 tiles of 768 and 2048 nodes gave 3.17 and

@@ -48,15 +48,6 @@ __global__ __launch_bounds__(STAGE_THREADS) void k_stage(StageArgs<R> a) {
         PACKED, unsigned long long,
         typename std::conditional<sizeof(R) == 4 && PUFF_MIXED_TILE == 2, float, double>::type>::type;
     constexpr int WORDS = DET ? DET_WORDS : (PACKED ? 1 : 2);
-    // Wavefronts that deposit in turn (tile_deposit) add in FP64, two words per
-    // node, in the mixed form too: the packed words round to 2^-22 of the
-    // workgroup's largest source, which a workgroup spread over the beam may
-    // hold far from its smallest.  A step on 129 x 129 x 1024 of 2^17 (all
-    // workgroups overflow), 2^20 (5 %) and 2^24 macroparticles (0.3 %): 326, 363
-    // and 1570 us; packed words for the single wavefronts too, 238, 326 and 1535;
-    // global atomics for whole workgroups, 482, 510 and 1680.
-    constexpr int WAVE_WORDS = PACKED ? 2 : WORDS;
-    constexpr int WAVE_TILE = TILE * WORDS / WAVE_WORDS;
     static_assert(WORDS * FIELD_TILE_NODES * sizeof(D) + FIELD_TILE_NODES * sizeof(cplx<R>) <=
                       WORDS * TILE * sizeof(D), "field tile inside the deposit tile");
     __shared__ D s_dep[WORDS * TILE];
@@ -366,36 +357,49 @@ __global__ __launch_bounds__(STAGE_THREADS) void k_stage(StageArgs<R> a) {
             if constexpr (DET)
                 det_add(m, t, c[p], cr, (double)sr[p], (double)si[p], det_scale,
                         reinterpret_cast<unsigned long long*>(s_dep));
-            else if constexpr (PACKED) {
-                if (use_tile) packed_add(m, t, c[p], cr, (float)sr[p], (float)si[p], log2S, s_dep);
-                else tile_add<R, double>(m, t, c[p], cr, sr[p], si[p], reinterpret_cast<double*>(s_dep));
-            } else tile_add<R, D>(m, t, c[p], cr, sr[p], si[p], s_dep);
+            else if constexpr (PACKED) packed_add(m, t, c[p], cr, (float)sr[p], (float)si[p], log2S, s_dep);
+            else tile_add<R, D>(m, t, c[p], cr, sr[p], si[p], s_dep);
         }
     };
     auto flush = [&](const TileBox& t) {
         if constexpr (DET) det_flush(m, t, a.det.acc, reinterpret_cast<const unsigned long long*>(s_dep));
-        else if constexpr (PACKED) {
-            if (use_tile) packed_flush(m, t, log2S, reinterpret_cast<cplx<float>*>(a.dAout), s_dep);
-            else tile_flush<R, double>(m, t, a.dAout, reinterpret_cast<const double*>(s_dep));
-        } else tile_flush<R, D>(m, t, a.dAout, s_dep);
+        else if constexpr (PACKED) packed_flush(m, t, log2S, reinterpret_cast<cplx<float>*>(a.dAout), s_dep);
+        else tile_flush<R, D>(m, t, a.dAout, s_dep);
     };
     if constexpr (DET && STAGE < 4) {
         if (ph.field_evolve && ok[0] && (fabs((double)sr[0]) > det_lim || fabs((double)si[0]) > det_lim))
             atomicOr(a.flags, FLAG_DET_RANGE);
     }
-    if (ph.field_evolve) {
-        tile_deposit<WAVE_TILE>(
-            m, tb, use_tile, s_red, [&](const TileBox& t) { tile_clear(s_dep, WAVE_WORDS * t.tx * t.ty * t.tz); },
-            add, flush,
-            [&]() {
+    if (!ph.field_evolve) return;
+    auto spill = [&]() {
 #pragma unroll
-                for (int p = 0; p < P; ++p) {
-                    const CellRef cr = cell_ref<R>(m, ok[p], c[p], tb, lane);
-                    if constexpr (DET)
-                        det_global_add(m, ok[p], c[p], cr, (double)sr[p], (double)si[p], det_scale, a.det.acc);
-                    else global_add<R>(m, ok[p], c[p], cr, sr[p], si[p], a.dAout);
-                }
-            });
+        for (int p = 0; p < P; ++p) {
+            const CellRef cr = cell_ref<R>(m, ok[p], c[p], tb, lane);
+            if constexpr (DET)
+                det_global_add(m, ok[p], c[p], cr, (double)sr[p], (double)si[p], det_scale, a.det.acc);
+            else global_add<R>(m, ok[p], c[p], cr, sr[p], si[p], a.dAout);
+        }
+    };
+    if constexpr (PACKED) {
+        // wavefronts that deposit in turn add in FP64: the packed words round to
+        // 2^-22 of the workgroup's largest source, which a workgroup spread over
+        // the beam may hold far from its smallest.  A step on 129 x 129 x 1024 of
+        // 2^17 (all workgroups overflow), 2^20 (5 %) and 2^24 macroparticles
+        // (0.3 %): 258, 347 and 1470 us; packed words for the single wavefronts
+        // too, 238, 324 and 1500; global atomics for whole workgroups, 482, 510
+        // and 1680.
+        static_assert(P == 1, "one macroparticle per thread");
+        if (use_tile) {
+            add(tb);
+            __syncthreads();
+            flush(tb);
+        } else {
+            wave_deposit<TILE, R>(m, s_red, ok[0], c[0], sr[0], si[0], reinterpret_cast<double*>(s_dep), a.dAout, spill);
+        }
+    } else {
+        tile_deposit<TILE>(
+            m, tb, use_tile, s_red, [&](const TileBox& t) { tile_clear(s_dep, WORDS * t.tx * t.ty * t.tz); }, add,
+            flush, spill);
     }
 }
 

@@ -29,7 +29,7 @@ def _beam(n, seed=5):
     return mp, p, h
 
 
-@pytest.mark.parametrize("n", [2048, 4096, 6144])
+@pytest.mark.parametrize("n", [1536, 2048, 3072, 4096, 6144])
 def test_light_macroparticles_beside_heavy_ones(n):
     """The mixed form's field of macroparticles 1e-7 as heavy as others of their
     workgroup, on nodes that only they touch (x > 0; the heavy ones stay 0.2, one
